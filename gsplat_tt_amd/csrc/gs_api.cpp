@@ -1579,10 +1579,24 @@ struct gs_ctx {
                 "train: lambda_dssim must be in [0, 1]");
     }
 
+    // The groups of partial sums of a forward and its loss (t_loss), added up.
+    static constexpr size_t kSumBytes = gs::kTrainSumSlots * sizeof(gs::TrainSums);
+    static gs::TrainSums add_sums(const void* p) {
+        gs::TrainSums t{}, v;
+        for (int k = 0; k < gs::kTrainSumSlots; ++k) {
+            std::memcpy(&v, static_cast<const char*>(p) + k * sizeof(v), sizeof(v));
+            t.l1 += v.l1;
+            t.ssim += v.ssim;
+            t.considered += v.considered;
+            t.blended += v.blended;
+        }
+        return t;
+    }
+
     // SSIM part of the full loss on device images: adds its gradient to dimage
-    // (which holds the L1 part) and its S sum to *ssim_sum.
+    // (which holds the L1 part) and its S sum to the groups of sums.
     void enqueue_ssim(const float* image, const float* target, int H, int W, float lambda,
-                      float loss_scale, float* dimage, double* ssim_sum) {
+                      float loss_scale, float* dimage, gs::TrainSums* sums) {
         const size_t px = (size_t)H * W;
         t_ssim.ensure(px * 36);
         gs::SsimParams sp{};
@@ -1596,7 +1610,7 @@ struct gs_ctx {
         sp.target = target;
         sp.maps = t_ssim.as<float>();
         sp.dimage = dimage;
-        sp.ssim_sum = ssim_sum;
+        sp.sums = sums;
         HIPCHK(gs::launch_ssim(sp, st));
     }
 
@@ -1617,7 +1631,7 @@ struct gs_ctx {
         t_T.ensure(px * 4);
         t_stop.ensure(px * 4);
         t_dimg.ensure(px * 12);
-        t_loss.ensure(32);  // L1 sum, SSIM sum (f64), considered and blended pairs (u64)
+        t_loss.ensure(kSumBytes);
         if (timing)
             for (auto& e : tev)
                 if (!e) HIPCHK(hipEventCreate(&e));
@@ -1625,7 +1639,7 @@ struct gs_ctx {
         HIPCHK(gs::launch_fill_u32(L.fr, 0u, L.fwords, st));
         if (spin_limit) HIPCHK(gs::launch_fill_u32(L.cnt + C_CTL + 1, spin_limit, 1, st));
         tr.cam.ctl = L.cnt + C_CTL;
-        HIPCHK(gs::launch_fill_u32(t_loss.as<uint32_t>(), 0u, 8, st));
+        HIPCHK(gs::launch_fill_u32(t_loss.as<uint32_t>(), 0u, kSumBytes / 4, st));
         gs::Compact cpt{b_rc.as<float4>(), b_dkey.as<uint32_t>(),
                         nullptr, b_src.as<uint32_t>()};
         HIPCHK(gs::launch_train_project(tplanes(t_p), tr.cam, cpt, b_brec.as<float4>(),
@@ -1653,13 +1667,12 @@ struct gs_ctx {
         fp.dimage = t_dimg.as<float>();
         fp.grad_scale = (float)((double)c->loss_scale * (1.0 - (double)c->lambda_dssim) /
                                 (3.0 * (double)px));
-        fp.loss = reinterpret_cast<double*>(t_loss.p);
-        fp.pairs = reinterpret_cast<unsigned long long*>(t_loss.p) + 2;
+        fp.sums = t_loss.as<gs::TrainSums>();
         fp.ctl = L.cnt + C_CTL;
         HIPCHK(gs::launch_train_fwd(b_brec.as<float4>(), tr.ids, b_ranges.as<uint32_t>(), fp, st));
         if (tgt_dev != nullptr && c->lambda_dssim > 0.0f)
             enqueue_ssim(t_img.as<float>(), tgt_dev, H, W, c->lambda_dssim, c->loss_scale,
-                         t_dimg.as<float>(), reinterpret_cast<double*>(t_loss.p) + 1);
+                         t_dimg.as<float>(), t_loss.as<gs::TrainSums>());
         if (timing) HIPCHK(hipEventRecord(tev[1], st));
     }
 
@@ -1685,7 +1698,7 @@ struct gs_ctx {
         for (int attempt = 0;; ++attempt) {
             train_forward_enqueue(v, c, tgt, dbg);
             HIPCHK(hipMemcpyAsync(h_pin, b_frame.p, 64 * 4, hipMemcpyDeviceToHost, st));
-            HIPCHK(hipMemcpyAsync(h_pin + 64, t_loss.p, 32, hipMemcpyDeviceToHost, st));
+            HIPCHK(hipMemcpyAsync(h_pin + 64, t_loss.p, kSumBytes, hipMemcpyDeviceToHost, st));
             sync();
             // The capacity test comes first: an attempt past the capacity has
             // kErrCapacity raised by the count scan, and is re-run (its fill
@@ -1702,16 +1715,13 @@ struct gs_ctx {
         }
         tr.M = h_pin[C_M];
         tr.p_pre = h_pin[C_PPRE];
-        uint64_t pp[2];
-        std::memcpy(pp, h_pin + 68, 16);
-        tr.pixel_pairs = (int64_t)pp[0];
-        tr.pixel_blended = (int64_t)pp[1];
         tr.P = h_pin[C_P];
-        double sums[2];
-        std::memcpy(sums, h_pin + 64, 16);
+        const gs::TrainSums sum = add_sums(h_pin + 64);
+        tr.pixel_pairs = (int64_t)sum.considered;
+        tr.pixel_blended = (int64_t)sum.blended;
         const double lam = c->lambda_dssim;
-        tr.l1 = tgt ? sums[0] / (3.0 * (double)px) : 0.0;
-        tr.ssim = (tgt && lam > 0.0) ? sums[1] / (3.0 * (double)px) : 0.0;
+        tr.l1 = tgt ? sum.l1 / (3.0 * (double)px) : 0.0;
+        tr.ssim = (tgt && lam > 0.0) ? sum.ssim / (3.0 * (double)px) : 0.0;
         tr.loss = tgt ? (double)c->loss_scale * ((1.0 - lam) * tr.l1 + lam * (1.0 - tr.ssim))
                       : 0.0;
         tr.fwd_valid = true;
@@ -2639,27 +2649,28 @@ int gs_train_loss(gs_ctx* ctx, const float* image, const float* target, int heig
         ctx->t_img.ensure(px * 12);
         ctx->t_tgt.ensure(px * 12);
         ctx->t_dimg.ensure(px * 12);
-        ctx->t_loss.ensure(16);
+        ctx->t_loss.ensure(gs_ctx::kSumBytes);
         hipStream_t st = ctx->st;
         HIPCHK(hipMemcpyAsync(ctx->t_img.p, image, px * 12, hipMemcpyHostToDevice, st));
         HIPCHK(hipMemcpyAsync(ctx->t_tgt.p, target, px * 12, hipMemcpyHostToDevice, st));
-        HIPCHK(gs::launch_fill_u32(ctx->t_loss.as<uint32_t>(), 0u, 4, st));
-        double* sums = reinterpret_cast<double*>(ctx->t_loss.p);
+        HIPCHK(gs::launch_fill_u32(ctx->t_loss.as<uint32_t>(), 0u, gs_ctx::kSumBytes / 4, st));
+        gs::TrainSums* sums = ctx->t_loss.as<gs::TrainSums>();
         const float scale = (float)((double)loss_scale * (1.0 - (double)lambda_dssim) /
                                     (3.0 * (double)px));
         HIPCHK(gs::launch_l1(ctx->t_img.as<float>(), ctx->t_tgt.as<float>(), (int64_t)px * 3,
                              scale, ctx->t_dimg.as<float>(), sums, st));
         if (lambda_dssim > 0.0f)
             ctx->enqueue_ssim(ctx->t_img.as<float>(), ctx->t_tgt.as<float>(), height, width,
-                              lambda_dssim, loss_scale, ctx->t_dimg.as<float>(), sums + 1);
-        double h[2];
+                              lambda_dssim, loss_scale, ctx->t_dimg.as<float>(), sums);
+        gs::TrainSums h[gs::kTrainSumSlots];
         HIPCHK(hipMemcpyAsync(dimage, ctx->t_dimg.p, px * 12, hipMemcpyDeviceToHost, st));
-        HIPCHK(hipMemcpyAsync(h, sums, 16, hipMemcpyDeviceToHost, st));
+        HIPCHK(hipMemcpyAsync(h, sums, sizeof(h), hipMemcpyDeviceToHost, st));
         ctx->sync();
         ctx->tr.fwd_valid = false;  // t_dimg / t_img no longer hold a training forward
         if (loss3) {
             const double n = 3.0 * (double)px, lam = lambda_dssim;
-            const double l1 = h[0] / n, ssim = lam > 0.0 ? h[1] / n : 0.0;
+            const gs::TrainSums sum = gs_ctx::add_sums(h);
+            const double l1 = sum.l1 / n, ssim = lam > 0.0 ? sum.ssim / n : 0.0;
             loss3[0] = (double)loss_scale * ((1.0 - lam) * l1 + lam * (1.0 - ssim));
             loss3[1] = l1;
             loss3[2] = ssim;

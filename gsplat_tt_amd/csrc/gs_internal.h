@@ -365,6 +365,17 @@ struct TrainDebug {
     uint8_t* valid;
 };
 
+// Partial sums of a forward and its loss, spread over kTrainSumSlots groups that
+// the host adds up.
+constexpr int kTrainSumSlots = 64;
+struct TrainSums {
+    double l1;    // |image - target|
+    double ssim;  // S of the full loss
+    // (pixel, entry) pairs: considered (each pixel's entries up to its stop) and
+    // blended (the backward evaluates the same pairs)
+    unsigned long long considered, blended;
+};
+
 struct TrainFwdParams {
     int tiles_x, tiles_y, width, height;
     float alpha_max, alpha_min, t_min;
@@ -375,10 +386,7 @@ struct TrainFwdParams {
     const float* target;   // (H,W,3) or null (no loss)
     float* dimage;         // dL/dimage (H,W,3), written with a target
     float grad_scale;      // loss_scale / (3HW)
-    double* loss;          // accumulates sum |image - target|
-    // (pixel, entry) pairs: [0] considered (each pixel's entries up to its
-    // stop), [1] blended; accumulated (the backward evaluates the same pairs)
-    unsigned long long* pairs;
+    TrainSums* sums;       // kTrainSumSlots groups of partial sums, cleared before
     const uint32_t* ctl;   // control words of the forward (nothing is read after an error)
 };
 
@@ -391,12 +399,13 @@ struct SsimParams {
     const float* target;   // (H,W,3)
     float* maps;           // 3 x (H,W,3): w dS/dmu_x, w dS/dE_xx, w dS/dE_xy
     float* dimage;         // (H,W,3): the SSIM gradient is added
-    double* ssim_sum;      // accumulates sum of S over the 3HW values
+    TrainSums* sums;       // kTrainSumSlots groups: the sum of S over the 3HW values
 };
 hipError_t launch_ssim(const SsimParams& sp, hipStream_t st);
-// dimage = scale * sign(image - target); *l1_sum += sum |image - target|.
+// dimage = scale * sign(image - target); sums (kTrainSumSlots groups) gain
+// sum |image - target|.
 hipError_t launch_l1(const float* image, const float* target, int64_t count, float scale,
-                     float* dimage, double* l1_sum, hipStream_t st);
+                     float* dimage, TrainSums* sums, hipStream_t st);
 
 struct TrainBwdParams {
     int tiles_x, tiles_y, width, height;
@@ -415,7 +424,7 @@ struct AdamParams {
 
 // Compact outputs: rect (u, v, rx, ry), cov (a, b, c, 2 ln(op/alpha_min)), depth
 // keys, src (compact -> Gaussian) and the forward record trec (3 float4 per
-// compact Gaussian: (u, v, op), (A, B, C), (r, g, b)); cidx maps Gaussian ->
+// compact Gaussian: (u, v, op, 2 ln(op/alpha_min)), (A, B, C), (r, g, b)); cidx maps Gaussian ->
 // compact index or 0xFFFFFFFF; visible marks the sparse-Adam rows.
 hipError_t launch_train_project(const TrainParamsDev& P, const TrainCam& cam, Compact out,
                                 float4* trec, uint32_t* cidx, uint8_t* visible,

@@ -241,7 +241,7 @@ __global__ __launch_bounds__(kTThreads) void k_train_project(
                                   raw[2] < 0.0f ? 0.0f : raw[2]};
             rect[it] = make_float4(g.u, g.v, rx, ry);
             cov[it] = make_float4(g.a, g.b, g.c, m2thr);
-            r0[it] = make_float4(g.u, g.v, op, 0.0f);
+            r0[it] = make_float4(g.u, g.v, op, m2thr);
             r1[it] = make_float4(g.A, g.B, g.C, 0.0f);
             r2[it] = make_float4(col[0], col[1], col[2], 0.0f);
             depth[it] = g.z;
@@ -307,64 +307,141 @@ __global__ __launch_bounds__(kTThreads) void k_train_project(
     }
 }
 
-// Forward of one 16x16 tile, one pixel per thread, entries staged in LDS in
-// batches of 256 (3DGS rules, train_oracle.py:196-229). Writes the image, the
-// final transmittance, the entry index where the pixel stopped, and - with a
-// target - the L1 gradient and the loss.
-__global__ __launch_bounds__(256) void k_train_fwd(const float4* __restrict__ trec,
-                                                   const uint32_t* __restrict__ sid,
-                                                   const uint32_t* __restrict__ ranges,
-                                                   TrainFwdParams fp) {
-    __shared__ float4 s0[256], s1[256], s2[256];
-    __shared__ double s_loss[4];
-    __shared__ unsigned long long s_pairs[2][4];
+// ---------------------------------------------------------------------------
+// Blend forward and backward. One wave64 (its own workgroup, no barriers
+// between waves) owns a 16x4 pixel band of a 16x16 tile, lane = row * 16 +
+// column, and walks the tile's depth-ordered entries 64 at a time: lane q tests
+// entry q against the whole band (band_keeps) and the kept ones are packed into
+// LDS, so that the per-pixel work is spent on entries that reach the band. The
+// next batch's records are loaded while this one is walked. Both are bound by
+// VALU issue, the longest tile lists by the latency of one wave's chain, which is
+// why a band is a workgroup of its own: four waves per tile finish independently.
+// Measured against 256-thread tile workgroups that evaluated every entry at
+// every pixel behind a barrier per batch (per step, 1M Gaussians at 1280x720):
+// forward 286 -> 124 us, backward 609 -> 318 us; 20K Gaussians at 200x152:
+// 58 -> 17 and 74 -> 26 us.
+// ---------------------------------------------------------------------------
+constexpr int kBandRows = 4;
+constexpr int kBandsPerTile = 16 / kBandRows;
+
+// False only when alpha = op exp(-q/2) stays below alpha_min at every pixel
+// centre of the band whose first centre is (x0, y0): the least q over the
+// rectangle of centres, on the edges facing the Gaussian's centre, is past
+// m2thr = 2 ln(op / alpha_min). The margin covers the rounding of this test and
+// of the per-pixel evaluation (a few ulp of the largest term), so no entry that
+// any pixel would blend is dropped; NaN keeps.
+__device__ __forceinline__ bool band_keeps(float4 r0, float4 r1, float x0, float y0) {
+    const float A = r1.x, B = r1.y, C = r1.z;
+    const float ul = x0 - r0.x, uh = ul + 15.0f;
+    const float vl = y0 - r0.y, vh = vl + (float)(kBandRows - 1);
+    const bool xin = ul <= 0.0f && uh >= 0.0f, yin = vl <= 0.0f && vh >= 0.0f;
+    const float uf = ul > 0.0f ? ul : uh, vf = vl > 0.0f ? vl : vh;
+    const float vs = fminf(fmaxf(-B * uf * __builtin_amdgcn_rcpf(C), vl), vh);
+    const float us = fminf(fmaxf(-B * vf * __builtin_amdgcn_rcpf(A), ul), uh);
+    const float a1 = A * uf * uf, b1 = 2.0f * B * uf * vs, c1 = C * vs * vs;
+    const float a2 = A * us * us, b2 = 2.0f * B * us * vf, c2 = C * vf * vf;
+    const float tol = 4e-6f;
+    const float q1 = (a1 + b1 + c1) - tol * (a1 + fabsf(b1) + c1);
+    const float q2 = (a2 + b2 + c2) - tol * (a2 + fabsf(b2) + c2);
+    const float lim = r0.w + 1e-4f;
+    const bool far1 = !xin && q1 > lim, far2 = !yin && q2 > lim;
+    // the nearest point lies on one of the facing edges: dropped when each of them is far
+    return !((far1 || xin) && (far2 || yin) && !(xin && yin));
+}
+
+// One entry at one pixel: power = -0.5 (A dx^2 + 2 B dx dy + C dy^2) in the order
+// of train_oracle.py:199-203, each operation rounded, the same in the forward
+// and the backward, so both see the same alpha.
+struct Splat {
+    float dx, dy, adx, cdy, power, w, raw;
+};
+__device__ __forceinline__ Splat splat_at(float px, float py, float u, float v, float A, float B,
+                                          float C, float op) {
+    Splat s;
+    s.dx = px - u;
+    s.dy = py - v;
+    s.adx = A * s.dx;
+    s.cdy = C * s.dy;
+    s.power = -0.5f * (s.adx * s.dx + 2.0f * B * s.dx * s.dy + s.cdy * s.dy);
+    s.w = __expf(fminf(s.power, 0.0f));
+    s.raw = op * s.w;
+    return s;
+}
+
+// Forward of one band (3DGS rules, train_oracle.py:196-229). Writes the image,
+// the final transmittance, the entry index where the pixel stopped, and - with
+// a target - the L1 gradient and the loss.
+__global__ __launch_bounds__(GS_WAVE) void k_train_fwd(const float4* __restrict__ trec,
+                                                       const uint32_t* __restrict__ sid,
+                                                       const uint32_t* __restrict__ ranges,
+                                                       TrainFwdParams fp) {
+    __shared__ float4 s0[GS_WAVE], s1[GS_WAVE];
+    __shared__ float2 s2[GS_WAVE];
     // after an earlier give-up the sorted ids may be wrong: read nothing (the
     // flag was raised by an earlier launch, so every thread sees the same value)
     if (upstream_failed(fp.ctl)) return;
-    const int tid = threadIdx.x;
-    const int tile = blockIdx.x;
+    const int lane = threadIdx.x;
+    const int tile = blockIdx.x / kBandsPerTile, band = blockIdx.x % kBandsPerTile;
     const int tx = tile % fp.tiles_x, ty = tile / fp.tiles_x;
-    const int px = tx * 16 + (tid & 15), py = ty * 16 + (tid >> 4);
+    const int px = tx * 16 + (lane & 15), py = ty * 16 + band * kBandRows + (lane >> 4);
     const bool inside = px < fp.width && py < fp.height;
     const float pxc = (float)px + 0.5f, pyc = (float)py + 0.5f;
+    const float bx0 = (float)(tx * 16) + 0.5f, by0 = (float)(ty * 16 + band * kBandRows) + 0.5f;
     const uint32_t start = ranges[2 * tile], end = ranges[2 * tile + 1];
     float T = 1.0f, cr = 0.0f, cg = 0.0f, cb = 0.0f;
     bool done = !inside;
     uint32_t stop = end - start;
-    uint32_t blended = 0;
-    for (uint32_t base = start; base < end; base += 256) {
-        const uint32_t nb = min(256u, end - base);
-        if ((uint32_t)tid < nb) {
-            const uint32_t gi = sid[base + tid];
-            s0[tid] = trec[3 * (size_t)gi + 0];
-            s1[tid] = trec[3 * (size_t)gi + 1];
-            s2[tid] = trec[3 * (size_t)gi + 2];
-        }
-        __syncthreads();
-        if (!done) {
-            for (uint32_t j = 0; j < nb; ++j) {
-                const float4 r0 = s0[j], r1 = s1[j];
-                const float dx = pxc - r0.x, dy = pyc - r0.y;
-                const float power = -0.5f * (r1.x * dx * dx + 2.0f * r1.y * dx * dy + r1.z * dy * dy);
-                const float raw = r0.z * __expf(power < 0.0f ? power : 0.0f);
-                const float alpha = raw > fp.alpha_max ? fp.alpha_max : raw;
-                if (alpha < fp.alpha_min) continue;
-                const float tn = T * (1.0f - alpha);
-                if (tn < fp.t_min) {
-                    done = true;
-                    stop = base - start + j;
-                    break;
-                }
-                const float4 c = s2[j];
-                const float at = alpha * T;
-                cr += at * c.x;
-                cg += at * c.y;
-                cb += at * c.z;
-                T = tn;
-                ++blended;
+    uint32_t blended = 0;  // of the wave
+    if (start < end && __ballot(inside) != 0ull) {
+        uint32_t gi = sid[min(start + lane, end - 1)];
+        float4 r0 = trec[3 * (size_t)gi + 0], r1 = trec[3 * (size_t)gi + 1],
+               r2 = trec[3 * (size_t)gi + 2];
+        gi = sid[min(start + GS_WAVE + lane, end - 1)];
+        for (uint32_t base = start; base < end; base += GS_WAVE) {
+            const bool keep = base + lane < end && band_keeps(r0, r1, bx0, by0);
+            const uint64_t mask = __ballot(keep);
+            const int cnt = __popcll(mask);
+            __syncthreads();  // one wave: orders the LDS reads of the batch before
+            if (keep) {
+                const int k = __popcll(mask & lanemask_lt());
+                s0[k] = make_float4(r0.x, r0.y, r0.z, r1.x);
+                s1[k] = make_float4(r1.y, r1.z, r2.x, r2.y);
+                s2[k] = make_float2(r2.z, __uint_as_float(base - start + lane));
             }
+            if (lane >= cnt && lane < ((cnt + 3) & ~3)) {  // opacity 0: blends nowhere
+                s0[lane] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                s1[lane] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                s2[lane] = make_float2(0.0f, 0.0f);
+            }
+            r0 = trec[3 * (size_t)gi + 0];
+            r1 = trec[3 * (size_t)gi + 1];
+            r2 = trec[3 * (size_t)gi + 2];
+            gi = sid[min(base + 2 * GS_WAVE + lane, end - 1)];
+            __syncthreads();
+            for (int k = 0; k < cnt; k += 4) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const float4 e0 = s0[k + j], e1 = s1[k + j];
+                    const float2 e2 = s2[k + j];
+                    const Splat s = splat_at(pxc, pyc, e0.x, e0.y, e0.w, e1.x, e1.y, e0.z);
+                    const float alpha = fminf(s.raw, fp.alpha_max);
+                    const bool live = alpha >= fp.alpha_min && !done;
+                    const float tn = T * (1.0f - alpha);
+                    const bool hit = live && tn < fp.t_min;
+                    const bool bl = live && !hit;
+                    done = done || hit;
+                    stop = hit ? __float_as_uint(e2.y) : stop;
+                    const float at = bl ? alpha * T : 0.0f;
+                    cr += at * e1.z;
+                    cg += at * e1.w;
+                    cb += at * e2.x;
+                    T = bl ? tn : T;
+                    blended += (uint32_t)__popcll(__ballot(bl));
+                }
+                if (__ballot(!done) == 0ull) break;
+            }
+            if (__ballot(!done) == 0ull) break;
         }
-        if (__syncthreads_count(!done) == 0) break;
     }
     double lsum = 0.0;
     if (inside) {
@@ -385,31 +462,21 @@ __global__ __launch_bounds__(256) void k_train_fwd(const float4* __restrict__ tr
             }
         }
     }
+    // sums into one of kTrainSumSlots groups (one address for all of a
+    // launch's thousands of waves would serialise them); the host adds the groups
+    TrainSums* const slot = fp.sums + blockIdx.x % kTrainSumSlots;
     if (fp.target != nullptr) {
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) lsum += __shfl_xor(lsum, o, GS_WAVE);
-        if (lane_id() == 0) s_loss[tid / GS_WAVE] = lsum;
+        if (lane == 0) atomicAdd(&slot->l1, lsum);
     }
-    if (fp.pairs != nullptr) {
-        unsigned long long pc = inside ? stop : 0u, pb = inside ? blended : 0u;
+    uint32_t pc = inside ? stop : 0u;  // a band's 64 stops, each below 2^26
+    unsigned long long pcw = pc;
 #pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-            pc += __shfl_xor(pc, o, GS_WAVE);
-            pb += __shfl_xor(pb, o, GS_WAVE);
-        }
-        if (lane_id() == 0) {
-            s_pairs[0][tid / GS_WAVE] = pc;
-            s_pairs[1][tid / GS_WAVE] = pb;
-        }
-    }
-    __syncthreads();
-    if (tid == 0) {
-        if (fp.target != nullptr)
-            atomicAdd(fp.loss, s_loss[0] + s_loss[1] + s_loss[2] + s_loss[3]);
-        if (fp.pairs != nullptr) {
-            atomicAdd(&fp.pairs[0], s_pairs[0][0] + s_pairs[0][1] + s_pairs[0][2] + s_pairs[0][3]);
-            atomicAdd(&fp.pairs[1], s_pairs[1][0] + s_pairs[1][1] + s_pairs[1][2] + s_pairs[1][3]);
-        }
+    for (int o = 32; o > 0; o >>= 1) pcw += __shfl_xor(pcw, o, GS_WAVE);
+    if (lane == 0) {
+        atomicAdd(&slot->considered, pcw);
+        atomicAdd(&slot->blended, (unsigned long long)blended);
     }
 }
 
@@ -503,7 +570,9 @@ __global__ __launch_bounds__(256) void k_ssim_fwd(SsimParams sp) {
     for (int o = 32; o > 0; o >>= 1) ssum += __shfl_xor(ssum, o, GS_WAVE);
     if (lane_id() == 0) s_sum[tid / GS_WAVE] = ssum;
     __syncthreads();
-    if (tid == 0) atomicAdd(sp.ssim_sum, (s_sum[0] + s_sum[1]) + (s_sum[2] + s_sum[3]));
+    if (tid == 0)
+        atomicAdd(&sp.sums[blockIdx.x % kTrainSumSlots].ssim,
+                  (s_sum[0] + s_sum[1]) + (s_sum[2] + s_sum[3]));
 }
 
 // Backward: dimage += G*(w dS/dmu_x) + 2 x G*(w dS/dE_xx) + y G*(w dS/dE_xy)
@@ -570,7 +639,7 @@ __global__ __launch_bounds__(256) void k_ssim_bwd(SsimParams sp) {
 __global__ __launch_bounds__(256) void k_l1(const float* __restrict__ image,
                                             const float* __restrict__ target, int64_t count,
                                             float scale, float* __restrict__ dimage,
-                                            double* l1_sum) {
+                                            TrainSums* sums) {
     __shared__ double s_sum[4];
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     double a = 0.0;
@@ -583,74 +652,86 @@ __global__ __launch_bounds__(256) void k_l1(const float* __restrict__ image,
     for (int o = 32; o > 0; o >>= 1) a += __shfl_xor(a, o, GS_WAVE);
     if (lane_id() == 0) s_sum[threadIdx.x / GS_WAVE] = a;
     __syncthreads();
-    if (threadIdx.x == 0) atomicAdd(l1_sum, (s_sum[0] + s_sum[1]) + (s_sum[2] + s_sum[3]));
+    if (threadIdx.x == 0)
+        atomicAdd(&sums[blockIdx.x % kTrainSumSlots].l1,
+                  (s_sum[0] + s_sum[1]) + (s_sum[2] + s_sum[3]));
 }
 
 // v plus the value a DPP move brings into the lane (all lanes active).
-template <int CTRL, int ROWS>
-__device__ __forceinline__ float dpp_add(float v) {
-    const int x = __builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, ROWS, 0xF, false);
-    return v + __int_as_float(x);
+template <int CTRL>
+__device__ __forceinline__ float dpp_add(float keep, float give) {
+    const int x = __builtin_amdgcn_update_dpp(0, __float_as_int(give), CTRL, 0xF, 0xF, false);
+    return keep + __int_as_float(x);
+}
+constexpr int kDppXor1 = 0xB1;         // quad_perm 1,0,3,2
+constexpr int kDppXor2 = 0x4E;         // quad_perm 2,3,0,1
+constexpr int kDppHalfMirror = 0x141;  // lane 7 - l of each 8
+constexpr int kDppRor8 = 0x128;        // lane l ^ 8 of each 16
+
+// Lanes 0-31: the sum of a over lane pairs (l, l + 32); lanes 32-63: that of b.
+__device__ __forceinline__ float pack32(float a, float b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false,
+                                                    false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+// Even rows of 16 lanes: the sum of a over the row and the next one; odd rows: that of b.
+__device__ __forceinline__ float pack16(float a, float b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false,
+                                                    false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
-// Lanes whose per-pair terms are summed together before one of them adds the
-// sums into LDS: fewer LDS atomics against more DPP steps. Measured on the 1M
-// training step (backward ms): 8 lanes 0.99, 16 lanes 0.63, 32 lanes 0.57,
-// 64 lanes 0.58 (LDS float atomics cost more per lane than the DPP adds).
-constexpr int kBwdGroup = 32;
-constexpr int kBwdCopies = GS_WAVE / kBwdGroup;  // LDS accumulator copies, one per group
-constexpr int kBwdBatch = 128;
-
-// Sum over each group of kBwdGroup lanes, complete in the group's last lane
-// (quad swaps, half-row and row mirrors, then row broadcasts across rows).
-__device__ __forceinline__ float group_fsum(float v) {
-    v = dpp_add<0xB1, 0xF>(v);   // quad_perm 1,0,3,2
-    v = dpp_add<0x4E, 0xF>(v);   // quad_perm 2,3,0,1
-    v = dpp_add<0x141, 0xF>(v);  // row_half_mirror
-    if constexpr (kBwdGroup >= 16) v = dpp_add<0x140, 0xF>(v);  // row_mirror
-    // Across rows: v += lane 15 of the row before (rows 1, 3), then v += lane 31
-    // (rows 2, 3). One DPP add each, the rows outside the row mask keeping v; the
-    // s_nop gives the two wait states a DPP read needs after a VALU write.
-    if constexpr (kBwdGroup >= 32)
-        asm volatile("s_nop 1\n\tv_add_f32_dpp %0, %0, %0 row_bcast:15 row_mask:0xa bank_mask:0xf"
-                     : "+v"(v));
-    if constexpr (kBwdGroup >= 64)
-        asm volatile("s_nop 1\n\tv_add_f32_dpp %0, %0, %0 row_bcast:31 row_mask:0xc bank_mask:0xf"
-                     : "+v"(v));
-    return v;
+// Sums the nine terms of two entries over the 64 lanes, all 18 of them in one
+// register: at each halving of the lanes, two registers become one, half of the
+// lanes carrying on with the one's term and half with the other's, so that the
+// 18 sums take 43 vector instructions (one by one, six each: 108). Lane l
+// returns the sum of term_of_lane(l) of entry l / 32.
+__device__ __forceinline__ float sum_terms(const float (&a)[9], const float (&b)[9], bool bit3,
+                                           bool bit2, bool bit1) {
+    float r[9];
+#pragma unroll
+    for (int i = 0; i < 9; ++i) r[i] = pack32(a[i], b[i]);
+    float q[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) q[i] = pack16(r[i], r[i + 4]);
+    float s8 = pack16(r[8], r[8]);
+    float x0 = dpp_add<kDppRor8>(bit3 ? q[1] : q[0], bit3 ? q[0] : q[1]);
+    float x1 = dpp_add<kDppRor8>(bit3 ? q[3] : q[2], bit3 ? q[2] : q[3]);
+    s8 = dpp_add<kDppRor8>(s8, s8);
+    float x = dpp_add<kDppHalfMirror>(bit2 ? x1 : x0, bit2 ? x0 : x1);
+    s8 = dpp_add<kDppHalfMirror>(s8, s8);
+    x = dpp_add<kDppXor2>(bit1 ? s8 : x, bit1 ? x : s8);
+    return dpp_add<kDppXor1>(x, x);
+}
+__device__ __forceinline__ int term_of_lane(int l) {
+    return (l & 2) ? 8 : ((l >> 4) & 1) * 4 + ((l >> 2) & 1) * 2 + ((l >> 3) & 1);
 }
 
-// Backward of one 16x16 tile: entries from the last one any pixel considered
-// down to the first; per pixel the reverse recursion T_i = T_{i+1}/(1 - alpha_i),
-// behind_i = alpha_{i+1} c_{i+1} + (1 - alpha_{i+1}) behind_{i+1},
-// dL/dalpha_i = T_i (c_i - behind_i) . g - T_final bg . g / (1 - alpha_i).
-// Per (wave, entry): the entry's alpha for every lane, a ballot of the lanes
-// that blend it, and only when one does, the nine per-pair terms (dmx dmy dA
-// dB dC dop dr dg db) for every lane with the lanes that do not blend it
-// contributing exact zeros (selects, no divergent branches). The terms are
-// summed over each group of kBwdGroup lanes with DPP moves and the group's last
-// lane adds them into its own LDS accumulator copy (copies interleaved, so the
-// lanes hit distinct banks); the copies' sum goes to the Gaussian's accumulator
-// with one global atomic per term. 1/(1 - alpha) is one reciprocal estimate,
-// exp the hardware exponential (the forward uses the same one, so both see the
-// same alpha).
-__global__ __launch_bounds__(256) void k_train_bwd(const float4* __restrict__ trec,
-                                                   const uint32_t* __restrict__ sid,
-                                                   const uint32_t* __restrict__ ranges,
-                                                   TrainBwdParams bp) {
-    __shared__ float4 s0[kBwdBatch], s1[kBwdBatch], s2[kBwdBatch];
-    __shared__ __align__(16) float s_acc[kBwdBatch][9][kBwdCopies];
-    __shared__ uint32_t s_has[4][kBwdBatch];
-    __shared__ uint32_t s_nmax;
-    const int tid = threadIdx.x, w = tid / GS_WAVE, lane = lane_id();
-    const int tile = blockIdx.x;
+// Backward of one band: entries from the last one any of its pixels considered
+// down to the first; per pixel the reverse recursion T_i = T_{i+1}/(1 - alpha_i)
+// and, with s_i = c_i . g, behind_i = behind_{i+1} + alpha_{i+1} (s_{i+1} -
+// behind_{i+1}) starting from the background's bg . g (the colours behind an
+// entry are only ever needed through their product with the pixel's gradient),
+// dL/dalpha_i = T_i (s_i - behind_i). A lane that does not blend the entry has
+// alpha 0, which leaves T and behind as they are, and contributes exact zeros.
+// The nine per-pair terms (dmx dmy dA dB dC dop dr dg db) of two entries at a
+// time are summed over the wave (sum_terms) and 18 lanes add them to the
+// Gaussians' accumulators, one atomic each. 1/(1 - alpha) is one reciprocal
+// estimate.
+__global__ __launch_bounds__(GS_WAVE) void k_train_bwd(const float4* __restrict__ trec,
+                                                       const uint32_t* __restrict__ sid,
+                                                       const uint32_t* __restrict__ ranges,
+                                                       TrainBwdParams bp) {
+    __shared__ float4 s0[GS_WAVE], s1[GS_WAVE], s2[GS_WAVE];
+    const int lane = threadIdx.x;
+    const int tile = blockIdx.x / kBandsPerTile, band = blockIdx.x % kBandsPerTile;
     const int tx = tile % bp.tiles_x, ty = tile / bp.tiles_x;
-    const int px = tx * 16 + (tid & 15), py = ty * 16 + (tid >> 4);
+    const int px = tx * 16 + (lane & 15), py = ty * 16 + band * kBandRows + (lane >> 4);
     const bool inside = px < bp.width && py < bp.height;
     const float pxc = (float)px + 0.5f, pyc = (float)py + 0.5f;
+    const float bx0 = (float)(tx * 16) + 0.5f, by0 = (float)(ty * 16 + band * kBandRows) + 0.5f;
     const uint32_t start = ranges[2 * tile], end = ranges[2 * tile + 1];
-    if (tid == 0) s_nmax = 0;
-    float T = 1.0f, g0 = 0.0f, g1 = 0.0f, g2 = 0.0f, tbg = 0.0f;
+    float T = 1.0f, g0 = 0.0f, g1 = 0.0f, g2 = 0.0f;
     uint32_t stop = 0;
     if (inside) {
         const size_t p = (size_t)py * bp.width + px;
@@ -659,106 +740,84 @@ __global__ __launch_bounds__(256) void k_train_bwd(const float4* __restrict__ tr
         g0 = bp.dimage[3 * p + 0];
         g1 = bp.dimage[3 * p + 1];
         g2 = bp.dimage[3 * p + 2];
-        tbg = T * (bp.bg[0] * g0 + bp.bg[1] * g1 + bp.bg[2] * g2);
     }
-    __syncthreads();
-    if (stop > 0) atomicMax(&s_nmax, stop);
-    __syncthreads();
-    const uint32_t nmax = min(s_nmax, end - start);
-    // the wave's own last considered entry: entries past it are skipped
-    uint32_t wstop = stop;
+    float behind = bp.bg[0] * g0 + bp.bg[1] * g1 + bp.bg[2] * g2;
+    // the band's last considered entry: entries past it are skipped
+    uint32_t nmax = stop;
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) wstop = max(wstop, (uint32_t)__shfl_xor((int)wstop, o, GS_WAVE));
-    float* const acc_lane = &s_acc[0][0][lane / kBwdGroup];  // this lane's copy (group leaders)
-    const bool leader = (lane % kBwdGroup) == kBwdGroup - 1;
-    float b0 = 0.0f, b1 = 0.0f, b2 = 0.0f;  // colour behind (normalised)
-    for (int32_t hi = (int32_t)nmax; hi > 0; hi -= kBwdBatch) {
-        const int32_t lo = max(0, hi - kBwdBatch);
-        const int32_t nb = hi - lo;
-        if (tid < nb) {
-            const uint32_t gi = sid[start + lo + tid];
-            s0[tid] = trec[3 * (size_t)gi + 0];
-            s1[tid] = trec[3 * (size_t)gi + 1];
-            s2[tid] = trec[3 * (size_t)gi + 2];
+    for (int o = 32; o > 0; o >>= 1) nmax = max(nmax, (uint32_t)__shfl_xor((int)nmax, o, GS_WAVE));
+    nmax = min((uint32_t)__builtin_amdgcn_readfirstlane((int)nmax), end - start);
+    if (nmax == 0) return;
+    // this lane's share of a pair's sums: its term, and the term's scale
+    const int term = term_of_lane(lane);
+    const bool writes = (lane & 3) == 0 || (lane & 31) == 2;
+    const float scale = term == 3 ? -1.0f : ((term == 2 || term == 4) ? -0.5f : 1.0f);
+    const bool bit3 = lane & 8, bit2 = lane & 4, bit1 = lane & 2;
+    // lane q holds the batch's entry hi - 1 - q (the walk's order)
+    int32_t hi = (int32_t)nmax;
+    uint32_t gi = sid[start + max(hi - 1 - lane, 0)];
+    float4 r0 = trec[3 * (size_t)gi + 0], r1 = trec[3 * (size_t)gi + 1],
+           r2 = trec[3 * (size_t)gi + 2];
+    uint32_t gn = sid[start + max(hi - 1 - GS_WAVE - lane, 0)];
+    for (; hi > 0; hi -= GS_WAVE) {
+        const bool keep = hi - 1 - lane >= 0 && band_keeps(r0, r1, bx0, by0);
+        const uint64_t mask = __ballot(keep);
+        const int cnt = __popcll(mask);
+        __syncthreads();  // one wave: orders the LDS reads of the batch before
+        if (keep) {
+            const int k = __popcll(mask & lanemask_lt());
+            s0[k] = make_float4(r0.x, r0.y, r0.z, r1.x);
+            s1[k] = make_float4(r1.y, r1.z, r2.x, r2.y);
+            s2[k] = make_float4(r2.z, __uint_as_float((uint32_t)(hi - 1 - lane)),
+                                __uint_as_float(gi), 0.0f);
         }
-        for (int i = tid; i < kBwdBatch * 9 * kBwdCopies / 4; i += 256)
-            reinterpret_cast<float4*>(&s_acc[0][0][0])[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        for (int i = lane; i < nb; i += GS_WAVE) s_has[w][i] = 0u;
+        if (lane == cnt && (cnt & 1)) {  // opacity 0, past every stop: blends nowhere
+            s0[lane] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            s1[lane] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            s2[lane] = make_float4(0.0f, __uint_as_float(0xFFFFFFFFu), 0.0f, 0.0f);
+        }
+        gi = gn;
+        r0 = trec[3 * (size_t)gi + 0];
+        r1 = trec[3 * (size_t)gi + 1];
+        r2 = trec[3 * (size_t)gi + 2];
+        gn = sid[start + max(hi - 1 - 2 * GS_WAVE - lane, 0)];
         __syncthreads();
-        const int32_t jtop = min(nb, (int32_t)wstop - lo) - 1;
-        for (int32_t j = jtop; j >= 0; --j) {
-            const uint32_t e = (uint32_t)(lo + j);
-            const float4 r0 = s0[j], r1 = s1[j];
-            const float dx = pxc - r0.x, dy = pyc - r0.y;
-            const float power = -0.5f * (r1.x * dx * dx + 2.0f * r1.y * dx * dy + r1.z * dy * dy);
-            const float wgt = __expf(power < 0.0f ? power : 0.0f);
-            const float raw = r0.z * wgt;
-            const bool clamp = raw > bp.alpha_max;
-            const float alpha = fminf(raw, bp.alpha_max);  // raw is finite: = clamp ? max : raw
-            const bool live = e < stop && alpha >= bp.alpha_min;
-            const uint64_t any = __ballot(live);
-            if (any) {
-                const float4 c = s2[j];
-                const float om = 1.0f - alpha;
-                const float rom = __builtin_amdgcn_rcpf(om);
-                const float Tn = T * rom;
-                const float dalpha =
-                    Tn * ((c.x - b0) * g0 + (c.y - b1) * g1 + (c.z - b2) * g2) - tbg * rom;
-                // a lane that does not blend the entry contributes exact zeros
-                const float at = live ? alpha * Tn : 0.0f;
-                const float d5 = (live && !clamp) ? dalpha : 0.0f;  // no gradient through the clamp
-                const float dp = (power <= 0.0f ? d5 : 0.0f) * raw;
-                float v[9];
-                v[0] = dp * (r1.x * dx + r1.y * dy);
-                v[1] = dp * (r1.y * dx + r1.z * dy);
-                v[2] = -0.5f * dp * dx * dx;
-                v[3] = -dp * dx * dy;
-                v[4] = -0.5f * dp * dy * dy;
-                v[5] = d5 * wgt;
-                v[6] = at * g0;
-                v[7] = at * g1;
-                v[8] = at * g2;
-                const float nb0 = alpha * c.x + om * b0;
-                const float nb1 = alpha * c.y + om * b1;
-                const float nb2 = alpha * c.z + om * b2;
-                T = live ? Tn : T;
-                b0 = live ? nb0 : b0;
-                b1 = live ? nb1 : b1;
-                b2 = live ? nb2 : b2;
+        for (int k = 0; k < cnt; k += 2) {
+            float v[2][9];
+            bool any = false;
 #pragma unroll
-                for (int k = 0; k < 9; ++k) {
-                    v[k] = group_fsum(v[k]);
-                    // keep the last step in every lane (one DPP add) rather than
-                    // a DPP move for every lane plus an add in the leaders' branch
-                    asm volatile("" : : "v"(v[k]));
-                }
-                if (leader) {
-#pragma unroll
-                    for (int k = 0; k < 9; ++k) atomicAdd(acc_lane + (j * 9 + k) * kBwdCopies, v[k]);
-                }
+            for (int j = 0; j < 2; ++j) {
+                const float4 e0 = s0[k + j], e1 = s1[k + j], e2 = s2[k + j];
+                const Splat s = splat_at(pxc, pyc, e0.x, e0.y, e0.w, e1.x, e1.y, e0.z);
+                const float alpha = fminf(s.raw, bp.alpha_max);
+                const bool live = __float_as_uint(e2.y) < stop && alpha >= bp.alpha_min;
+                any = any || live;
+                const float a = live ? alpha : 0.0f;
+                const float Tn = T * __builtin_amdgcn_rcpf(1.0f - a);
+                const float d = __builtin_fmaf(e1.z, g0, __builtin_fmaf(e1.w, g1, e2.x * g2)) -
+                                behind;
+                behind = __builtin_fmaf(a, d, behind);
+                T = Tn;
+                const float at = a * Tn;
+                // no gradient through the clamps
+                const float dop = (live && !(s.raw > bp.alpha_max)) ? Tn * d : 0.0f;
+                const float dp = s.power <= 0.0f ? dop * s.raw : 0.0f;
+                const float dpx = dp * s.dx, dpy = dp * s.dy;
+                v[j][0] = dp * __builtin_fmaf(e1.x, s.dy, s.adx);
+                v[j][1] = dp * __builtin_fmaf(e1.x, s.dx, s.cdy);
+                v[j][2] = dpx * s.dx;
+                v[j][3] = dpx * s.dy;
+                v[j][4] = dpy * s.dy;
+                v[j][5] = dop * s.w;
+                v[j][6] = at * g0;
+                v[j][7] = at * g1;
+                v[j][8] = at * g2;
             }
-            if (lane == 0) s_has[w][j] = any ? 1u : 0u;
+            if (__ballot(any) == 0ull) continue;
+            const float sum = sum_terms(v[0], v[1], bit3, bit2, bit1);
+            const uint32_t g = __float_as_uint(s2[k + (lane >> 5)].z);
+            if (writes && sum != 0.0f) atomicAdd(bp.grad2d + 9 * (size_t)g + term, sum * scale);
         }
-        __syncthreads();
-        if (tid < nb) {
-            const bool has = (s_has[0][tid] | s_has[1][tid] | s_has[2][tid] | s_has[3][tid]) != 0u;
-            if (has) {
-                float acc[9];
-#pragma unroll
-                for (int k = 0; k < 9; ++k) {
-                    float a = 0.0f;
-#pragma unroll
-                    for (int c = 0; c < kBwdCopies; ++c) a += s_acc[tid][k][c];
-                    acc[k] = a;
-                }
-                const uint32_t gi = sid[start + lo + tid];
-                float* dst = bp.grad2d + 9 * (size_t)gi;
-#pragma unroll
-                for (int k = 0; k < 9; ++k)
-                    if (acc[k] != 0.0f) atomicAdd(dst + k, acc[k]);
-            }
-        }
-        __syncthreads();
     }
 }
 
@@ -981,7 +1040,7 @@ hipError_t launch_train_fwd(const float4* trec, const uint32_t* sid, const uint3
                             const TrainFwdParams& fp, hipStream_t st) {
     const int tiles = fp.tiles_x * fp.tiles_y;
     if (tiles <= 0) return hipSuccess;
-    k_train_fwd<<<tiles, 256, 0, st>>>(trec, sid, ranges, fp);
+    k_train_fwd<<<tiles * kBandsPerTile, GS_WAVE, 0, st>>>(trec, sid, ranges, fp);
     return hipGetLastError();
 }
 
@@ -997,10 +1056,10 @@ hipError_t launch_ssim(const SsimParams& sp, hipStream_t st) {
 }
 
 hipError_t launch_l1(const float* image, const float* target, int64_t count, float scale,
-                     float* dimage, double* l1_sum, hipStream_t st) {
+                     float* dimage, TrainSums* sums, hipStream_t st) {
     if (count <= 0) return hipSuccess;
     k_l1<<<(unsigned)((count + 255) / 256), 256, 0, st>>>(image, target, count, scale, dimage,
-                                                          l1_sum);
+                                                          sums);
     return hipGetLastError();
 }
 
@@ -1008,7 +1067,7 @@ hipError_t launch_train_bwd(const float4* trec, const uint32_t* sid, const uint3
                             const TrainBwdParams& bp, hipStream_t st) {
     const int tiles = bp.tiles_x * bp.tiles_y;
     if (tiles <= 0) return hipSuccess;
-    k_train_bwd<<<tiles, 256, 0, st>>>(trec, sid, ranges, bp);
+    k_train_bwd<<<tiles * kBandsPerTile, GS_WAVE, 0, st>>>(trec, sid, ranges, bp);
     return hipGetLastError();
 }
 

@@ -268,7 +268,7 @@ struct gs_ctx {
             if (e) (void)hipEventDestroy(e);
         for (auto& e : tev)
             if (e) (void)hipEventDestroy(e);
-        for (DevBuf* b : {&t_p, &t_m, &t_v, &t_g, &t_cidx, &t_vis, &t_grad2d, &t_img, &t_T, &t_stop,
+        for (DevBuf* b : {&t_p, &t_m, &t_v, &t_g, &t_gnz, &t_cidx, &t_vis, &t_grad2d, &t_img, &t_T, &t_stop,
                           &t_dimg, &t_tgt, &t_loss, &t_dbg, &t_ssim})
             b->release();
         if (st) (void)hipStreamDestroy(st);
@@ -1407,7 +1407,7 @@ struct gs_ctx {
     struct TrainState {
         int64_t n = 0;
         int deg = -1;
-        int planes = 0;
+        int row = 0;  // floats per parameter row
         int64_t step = 0;
         bool ready = false;
         bool fwd_valid = false;   // the frame buffers hold the last training forward
@@ -1423,26 +1423,17 @@ struct gs_ctx {
     // Adam moments stored as bf16 bits (gs_train_set_moments), kept across
     // gs_train_init; fp32 by default
     bool t_bf16_mom = false;
-    DevBuf t_p, t_m, t_v, t_g, t_cidx, t_vis, t_grad2d, t_img, t_T, t_stop, t_dimg, t_tgt,
+    // t_gnz: per row of t_g, whether it is not all zero (launch_train_grads)
+    DevBuf t_p, t_m, t_v, t_g, t_gnz, t_cidx, t_vis, t_grad2d, t_img, t_T, t_stop, t_dimg, t_tgt,
         t_loss, t_dbg, t_ssim;
     std::vector<float> t_host;
     hipEvent_t tev[6] = {};
 
-    gs::TrainParamsDev tplanes(DevBuf& b) {
-        gs::TrainParamsDev d{};
-        float* base = b.as<float>();
-        const size_t n = (size_t)tr.n;
-        for (int c = 0; c < 3; ++c) d.mean[c] = base + c * n;
-        for (int c = 0; c < 3; ++c) d.ls[c] = base + (3 + c) * n;
-        for (int c = 0; c < 4; ++c) d.quat[c] = base + (6 + c) * n;
-        d.ol = base + 10 * n;
-        d.sh = base + 11 * n;
-        d.n = tr.n;
-        d.sh_degree = tr.deg;
-        return d;
+    gs::TrainParamsDev train_rows() {
+        return gs::TrainParamsDev{t_p.as<float4>(), tr.n, tr.deg};
     }
 
-    // AoS host arrays <-> SoA planes (mean 3, log-scale 3, quat 4, logit 1, SH 3K).
+    // The caller's arrays <-> rows of tr.row values (gs_internal.h).
     // bf16 bits of x, round to nearest even (a NaN stays a quiet NaN), as
     // torch's float -> bfloat16 conversion rounds
     static uint16_t bf16_rne(float x) {
@@ -1452,31 +1443,29 @@ struct gs_ctx {
         u += 0x7FFFu + ((u >> 16) & 1u);
         return (uint16_t)(u >> 16);
     }
-    // Moments are bf16 planes when t_bf16_mom (gs_train_set_moments).
-    bool bf16_planes(const DevBuf& b) const { return t_bf16_mom && (&b == &t_m || &b == &t_v); }
+    // Moments are bf16 rows when t_bf16_mom (gs_train_set_moments).
+    bool bf16_rows(const DevBuf& b) const { return t_bf16_mom && (&b == &t_m || &b == &t_v); }
 
     void train_upload(DevBuf& b, const gs_train_arrays* a) {
         REQUIRE(a && a->means && a->log_scales && a->quats && a->opacity_logits && a->sh,
                 "train: null parameter array");
         const int64_t n = tr.n;
         const int K = (tr.deg + 1) * (tr.deg + 1);
-        t_host.resize((size_t)tr.planes * (size_t)std::max<int64_t>(n, 1));
+        t_host.resize((size_t)tr.row * (size_t)std::max<int64_t>(n, 1));
         float* h = t_host.data();
         parallel_for(n, [&](int64_t lo, int64_t hi) {
             for (int64_t i = lo; i < hi; ++i) {
-                for (int c = 0; c < 3; ++c) {
-                    h[c * n + i] = a->means[3 * i + c];
-                    h[(3 + c) * n + i] = a->log_scales[3 * i + c];
-                }
-                for (int c = 0; c < 4; ++c) h[(6 + c) * n + i] = a->quats[4 * i + c];
-                h[10 * n + i] = a->opacity_logits[i];
-                for (int k = 0; k < K; ++k)
-                    for (int c = 0; c < 3; ++c)
-                        h[(11 + 3 * k + c) * n + i] = a->sh[(i * K + k) * 3 + c];
+                float* r = h + i * tr.row;
+                std::memcpy(r, a->means + 3 * i, 12);
+                std::memcpy(r + 3, a->log_scales + 3 * i, 12);
+                std::memcpy(r + 6, a->quats + 4 * i, 16);
+                r[10] = a->opacity_logits[i];
+                std::memcpy(r + 11, a->sh + 3 * K * i, (size_t)K * 12);
+                for (int j = 11 + 3 * K; j < tr.row; ++j) r[j] = 0.0f;
             }
         });
-        if (bf16_planes(b)) {
-            std::vector<uint16_t> hb((size_t)tr.planes * (size_t)n);
+        if (bf16_rows(b)) {
+            std::vector<uint16_t> hb((size_t)tr.row * (size_t)n);
             parallel_for((int64_t)hb.size(), [&](int64_t lo, int64_t hi) {
                 for (int64_t i = lo; i < hi; ++i) hb[(size_t)i] = bf16_rne(h[i]);
             });
@@ -1484,7 +1473,7 @@ struct gs_ctx {
             sync();
             return;
         }
-        HIPCHK(hipMemcpyAsync(b.p, h, (size_t)tr.planes * n * 4, hipMemcpyHostToDevice, st));
+        HIPCHK(hipMemcpyAsync(b.p, h, (size_t)tr.row * n * 4, hipMemcpyHostToDevice, st));
         sync();
     }
     void train_download(DevBuf& b, gs_train_arrays* a) {
@@ -1492,10 +1481,10 @@ struct gs_ctx {
                 "train: null output array");
         const int64_t n = tr.n;
         const int K = (tr.deg + 1) * (tr.deg + 1);
-        t_host.resize((size_t)tr.planes * (size_t)std::max<int64_t>(n, 1));
+        t_host.resize((size_t)tr.row * (size_t)std::max<int64_t>(n, 1));
         float* h = t_host.data();
-        if (bf16_planes(b)) {
-            std::vector<uint16_t> hb((size_t)tr.planes * (size_t)n);
+        if (bf16_rows(b)) {
+            std::vector<uint16_t> hb((size_t)tr.row * (size_t)n);
             HIPCHK(hipMemcpyAsync(hb.data(), b.p, hb.size() * 2, hipMemcpyDeviceToHost, st));
             sync();
             parallel_for((int64_t)hb.size(), [&](int64_t lo, int64_t hi) {
@@ -1505,20 +1494,17 @@ struct gs_ctx {
                 }
             });
         } else {
-            HIPCHK(hipMemcpyAsync(h, b.p, (size_t)tr.planes * n * 4, hipMemcpyDeviceToHost, st));
+            HIPCHK(hipMemcpyAsync(h, b.p, (size_t)tr.row * n * 4, hipMemcpyDeviceToHost, st));
             sync();
         }
         parallel_for(n, [&](int64_t lo, int64_t hi) {
             for (int64_t i = lo; i < hi; ++i) {
-                for (int c = 0; c < 3; ++c) {
-                    a->means[3 * i + c] = h[c * n + i];
-                    a->log_scales[3 * i + c] = h[(3 + c) * n + i];
-                }
-                for (int c = 0; c < 4; ++c) a->quats[4 * i + c] = h[(6 + c) * n + i];
-                a->opacity_logits[i] = h[10 * n + i];
-                for (int k = 0; k < K; ++k)
-                    for (int c = 0; c < 3; ++c)
-                        a->sh[(i * K + k) * 3 + c] = h[(11 + 3 * k + c) * n + i];
+                const float* r = h + i * tr.row;
+                std::memcpy(a->means + 3 * i, r, 12);
+                std::memcpy(a->log_scales + 3 * i, r + 3, 12);
+                std::memcpy(a->quats + 4 * i, r + 6, 16);
+                a->opacity_logits[i] = r[10];
+                std::memcpy(a->sh + 3 * K * i, r + 11, (size_t)K * 12);
             }
         });
     }
@@ -1530,8 +1516,8 @@ struct gs_ctx {
         tr = TrainState{};
         tr.n = n;
         tr.deg = deg;
-        tr.planes = 11 + 3 * (deg + 1) * (deg + 1);
-        const size_t bytes = (size_t)tr.planes * (size_t)std::max<int64_t>(n, 1) * 4;
+        tr.row = gs::train_row_floats(deg);
+        const size_t bytes = (size_t)tr.row * (size_t)std::max<int64_t>(n, 1) * 4;
         for (DevBuf* b : {&t_p, &t_m, &t_v, &t_g}) b->ensure(bytes);
         HIPCHK(gs::launch_fill_u32(t_m.as<uint32_t>(), 0u, bytes / 4, st));
         HIPCHK(gs::launch_fill_u32(t_v.as<uint32_t>(), 0u, bytes / 4, st));
@@ -1539,6 +1525,8 @@ struct gs_ctx {
         t_cidx.ensure((size_t)std::max<int64_t>(n, 1) * 4);
         t_vis.ensure((size_t)std::max<int64_t>(n, 1));
         HIPCHK(hipMemsetAsync(t_vis.p, 0, (size_t)std::max<int64_t>(n, 1), st));
+        t_gnz.ensure((size_t)std::max<int64_t>(n, 1));
+        HIPCHK(hipMemsetAsync(t_gnz.p, 0, (size_t)std::max<int64_t>(n, 1), st));
         train_upload(t_p, a);
         tr.ready = true;
     }
@@ -1642,7 +1630,7 @@ struct gs_ctx {
         HIPCHK(gs::launch_fill_u32(t_loss.as<uint32_t>(), 0u, kSumBytes / 4, st));
         gs::Compact cpt{b_rc.as<float4>(), b_dkey.as<uint32_t>(),
                         nullptr, b_src.as<uint32_t>()};
-        HIPCHK(gs::launch_train_project(tplanes(t_p), tr.cam, cpt, b_brec.as<float4>(),
+        HIPCHK(gs::launch_train_project(train_rows(), tr.cam, cpt, b_brec.as<float4>(),
                                         t_cidx.as<uint32_t>(), t_vis.as<uint8_t>(), L.lb_proj,
                                         L.cnt + C_PROJ_TICKET, L.cnt + C_M,
                                         b_phist_proj.as<uint32_t>(), dbg, st));
@@ -1728,9 +1716,9 @@ struct gs_ctx {
         tr.has_dimage = tgt != nullptr;
     }
 
-    // Enqueues the blend backward and the projection backward (gradients in t_g).
-    void train_backward_enqueue(const gs_train_cfg* c) {
-        const int64_t N = tr.n;
+    // Enqueues the blend backward and the gradients of the parameters (in t_g);
+    // with adam, the sparse Adam of the step in the same pass.
+    void train_backward_enqueue(const gs_train_cfg* c, bool adam) {
         t_grad2d.ensure((size_t)std::max<uint32_t>(tr.M, 1) * 36);
         if (timing) HIPCHK(hipEventRecord(tev[2], st));
         HIPCHK(gs::launch_fill_u32(t_grad2d.as<uint32_t>(), 0u, (size_t)tr.M * 9, st));
@@ -1748,13 +1736,19 @@ struct gs_ctx {
         bp.grad2d = t_grad2d.as<float>();
         if (tr.M > 0 && tr.P > 0)
             HIPCHK(gs::launch_train_bwd(b_brec.as<float4>(), tr.ids, b_ranges.as<uint32_t>(), bp, st));
-        HIPCHK(gs::launch_train_param_grads(tplanes(t_p), tr.cam, t_cidx.as<uint32_t>(),
-                                            t_grad2d.as<float>(), tplanes(t_g), st));
-        if (timing) HIPCHK(hipEventRecord(tev[3], st));
-        (void)N;
+        // the device time of a step's Adam is part of its gradient pass
+        if (timing && adam) HIPCHK(hipEventRecord(tev[3], st));
+        if (timing && adam) HIPCHK(hipEventRecord(tev[4], st));
+        const gs::AdamParams ap = adam ? adam_params(c) : gs::AdamParams{};
+        HIPCHK(gs::launch_train_grads(train_rows(), tr.cam, t_cidx.as<uint32_t>(),
+                                      t_grad2d.as<float>(), t_g.as<float4>(), t_gnz.as<uint8_t>(),
+                                      t_m.p, t_v.p, t_vis.as<uint8_t>(), adam ? &ap : nullptr,
+                                      t_bf16_mom, st));
+        if (timing) HIPCHK(hipEventRecord(tev[adam ? 5 : 3], st));
+        if (adam) ++tr.step;
     }
 
-    void train_adam_enqueue(const gs_train_cfg* c) {
+    gs::AdamParams adam_params(const gs_train_cfg* c) const {
         const double b1 = c->beta1, b2 = c->beta2;
         const int64_t t = tr.step + 1;
         const double bc1 = 1.0 - std::pow(b1, (double)t), bc2 = 1.0 - std::pow(b2, (double)t);
@@ -1766,17 +1760,21 @@ struct gs_ctx {
         ap.sqrt_bc2 = (float)std::sqrt(bc2);
         ap.eps = (float)c->eps;
         const double lr_geo[4] = {c->lr_means, c->lr_log_scales, c->lr_quats, c->lr_opacity};
-        const int geo_planes[4] = {3, 3, 4, 1};
+        const int geo_values[4] = {3, 3, 4, 1};
         int j = 0;
         for (int gidx = 0; gidx < 4; ++gidx)
-            for (int k = 0; k < geo_planes[gidx]; ++k) ap.step[j++] = (float)(lr_geo[gidx] / bc1);
+            for (int k = 0; k < geo_values[gidx]; ++k) ap.step[j++] = (float)(lr_geo[gidx] / bc1);
         const int K = (tr.deg + 1) * (tr.deg + 1);
         for (int k = 0; k < K; ++k)
             for (int ch = 0; ch < 3; ++ch)
                 ap.step[j++] = (float)(k == 0 ? c->lr_sh_dc : c->lr_sh_rest) / (float)bc1;
+        return ap;
+    }
+
+    void train_adam_enqueue(const gs_train_cfg* c) {
         if (timing) HIPCHK(hipEventRecord(tev[4], st));
-        HIPCHK(gs::launch_sparse_adam(t_p.as<float>(), t_m.p, t_v.p, t_g.as<float>(),
-                                      t_vis.as<uint8_t>(), tr.n, tr.planes, ap, t_bf16_mom, st));
+        HIPCHK(gs::launch_sparse_adam(train_rows(), t_m.p, t_v.p, t_g.as<float4>(),
+                                      t_vis.as<uint8_t>(), adam_params(c), t_bf16_mom, st));
         if (timing) HIPCHK(hipEventRecord(tev[5], st));
         ++tr.step;
     }
@@ -2464,7 +2462,11 @@ int gs_train_write(gs_ctx* ctx, int which, const gs_train_arrays* in) {
         ctx->sync();
         ctx->train_upload(*b[which], in);
         if (which == 0) ctx->tr.fwd_valid = false;
-        if (which == 3) ctx->tr.grads_valid = true;
+        if (which == 3) {
+            if (ctx->tr.n > 0)
+                HIPCHK(hipMemsetAsync(ctx->t_gnz.p, 1, (size_t)ctx->tr.n, ctx->st));
+            ctx->tr.grads_valid = true;
+        }
     });
 }
 
@@ -2577,7 +2579,7 @@ int gs_train_backward(gs_ctx* ctx, const gs_train_cfg* cfg, const float* dimage,
         const size_t px = (size_t)ctx->tr.H * ctx->tr.W;
         if (dimage)
             HIPCHK(hipMemcpyAsync(ctx->t_dimg.p, dimage, px * 12, hipMemcpyHostToDevice, ctx->st));
-        ctx->train_backward_enqueue(cfg);
+        ctx->train_backward_enqueue(cfg, false);
         if (g2d != nullptr) {
             const int64_t n = ctx->tr.n;
             const uint32_t M = ctx->tr.M;
@@ -2626,8 +2628,7 @@ int gs_train_step(gs_ctx* ctx, const gs_view* view, const gs_train_cfg* cfg, con
         ctx->drain_spec();
         ctx->train_check(view, cfg);
         ctx->train_forward(view, cfg, target, target_on_device != 0, gs::TrainDebug{});
-        ctx->train_backward_enqueue(cfg);
-        ctx->train_adam_enqueue(cfg);
+        ctx->train_backward_enqueue(cfg, true);
         ctx->sync();
         ctx->tr.fwd_valid = false;
         ctx->tr.grads_valid = false;

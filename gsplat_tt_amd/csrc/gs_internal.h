@@ -330,18 +330,17 @@ hipError_t launch_mb_stats(const float4* brec, const uint32_t* sid, const uint32
                            int cull_disabled, unsigned long long* out, const uint32_t* ctl,
                            hipStream_t st);
 
-// ---- train.hip: training step (3DGS forward rules, L1, backward, sparse Adam)
-constexpr int kMaxTrainPlanes = 64;  // 11 geometry/opacity planes + 3 (d+1)^2 SH planes
-
-// Optimizer-space parameters (or gradients / moments of the same shape) as SoA
-// planes of n floats: mean x y z, log-scale 0..2, quaternion w x y z, opacity
-// logit, then SH plane 3k+c for coefficient k, channel c.
+// ---- train.hip: training step (3DGS rules, L1, backward, sparse Adam)
+// Optimizer-space parameters (or gradients / moments of the same shape): one row
+// per Gaussian of train_row_floats(sh_degree) values - mean 3, log-scale 3,
+// quaternion 4, opacity logit, then SH coefficient k channel c at 11 + 3k + c,
+// padded with zeros to whole float4. Rows, because the sparse Adam and the
+// gradients touch some Gaussians and leave the others.
+constexpr int kMaxTrainRow = 60;
+inline int train_row_values(int sh_degree) { return 11 + 3 * (sh_degree + 1) * (sh_degree + 1); }
+inline int train_row_floats(int sh_degree) { return (train_row_values(sh_degree) + 3) & ~3; }
 struct TrainParamsDev {
-    float* mean[3];
-    float* ls[3];
-    float* quat[4];
-    float* ol;
-    float* sh;
+    float4* rows;
     int64_t n;
     int sh_degree;
 };
@@ -419,7 +418,7 @@ struct TrainBwdParams {
 
 struct AdamParams {
     float beta1, beta2, one_minus_beta1, one_minus_beta2, sqrt_bc2, eps;
-    float step[kMaxTrainPlanes];  // learning rate / (1 - beta1^t), per plane
+    float step[kMaxTrainRow];  // learning rate / (1 - beta1^t), per value of a row (0: padding)
 };
 
 // Compact outputs: rect (u, v, rx, ry), cov (a, b, c, 2 ln(op/alpha_min)), depth
@@ -434,12 +433,17 @@ hipError_t launch_train_fwd(const float4* trec, const uint32_t* sid, const uint3
                             const TrainFwdParams& fp, hipStream_t st);
 hipError_t launch_train_bwd(const float4* trec, const uint32_t* sid, const uint32_t* ranges,
                             const TrainBwdParams& bp, hipStream_t st);
-hipError_t launch_train_param_grads(const TrainParamsDev& P, const TrainCam& cam,
-                                    const uint32_t* cidx, const float* grad2d,
-                                    const TrainParamsDev& G, hipStream_t st);
-// m, v: float planes, or bf16 bits (uint16_t planes) with bf16_moments.
-hipError_t launch_sparse_adam(float* p, void* m, void* v, const float* g,
-                              const uint8_t* visible, int64_t n, int planes, const AdamParams& ap,
-                              bool bf16_moments, hipStream_t st);
+// Gradients (G rows) of every Gaussian from its accumulated 2D gradients; gnz[i]
+// marks the rows of G that are not zero (kept from call to call, so that rows
+// that stay zero are not written again). With adam (optional), the sparse Adam
+// of the visible rows in the same pass, as launch_sparse_adam.
+// m, v: float rows, or rows of bf16 bits (uint16_t) with bf16_moments.
+hipError_t launch_train_grads(const TrainParamsDev& P, const TrainCam& cam, const uint32_t* cidx,
+                              const float* grad2d, float4* G, uint8_t* gnz, void* m, void* v,
+                              const uint8_t* visible, const AdamParams* adam, bool bf16_moments,
+                              hipStream_t st);
+hipError_t launch_sparse_adam(const TrainParamsDev& P, void* m, void* v, const float4* G,
+                              const uint8_t* visible, const AdamParams& ap, bool bf16_moments,
+                              hipStream_t st);
 
 }  // namespace gs

@@ -109,9 +109,37 @@ __device__ __forceinline__ float s3(const float* S, int i, int k) {
     return lo == 0 ? S[hi] : (lo == 1 ? S[2 + hi] : S[5]);
 }
 
-__device__ __forceinline__ void geometry(const TrainParamsDev& P, int64_t i, const TrainCam& cam,
-                                         Geo& g) {
-    const float mx = P.mean[0][i], my = P.mean[1][i], mz = P.mean[2][i];
+// Layout of a parameter row (gs_internal.h).
+template <int DEG>
+struct Row {
+    static constexpr int K = (DEG + 1) * (DEG + 1);
+    static constexpr int V = (11 + 3 * K + 3) / 4;  // float4 per row
+    static constexpr int S = 4 * V;
+};
+
+// The first three float4 of a row: mean, log-scale, quaternion, opacity logit
+// and the first SH value.
+struct Head {
+    float4 a, b, c;
+};
+__device__ __forceinline__ Head load_head(const float4* row) { return Head{row[0], row[1], row[2]}; }
+
+// SH values 0 .. 3K-1 of a row (the padding after them is zero).
+template <int DEG>
+__device__ __forceinline__ void load_sh(const float4* row, const Head& h, float* sh) {
+    sh[0] = h.c.w;
+#pragma unroll
+    for (int q = 3; q < Row<DEG>::V; ++q) {
+        const float4 f = row[q];
+        const float t[4] = {f.x, f.y, f.z, f.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (4 * (q - 3) + 1 + e < 3 * Row<DEG>::K) sh[4 * (q - 3) + 1 + e] = t[e];
+    }
+}
+
+__device__ __forceinline__ void geometry(const Head& h, const TrainCam& cam, Geo& g) {
+    const float mx = h.a.x, my = h.a.y, mz = h.a.z;
     const float* R = cam.r;
     g.x = R[0] * mx + R[1] * my + R[2] * mz + cam.t[0];
     g.y = R[3] * mx + R[4] * my + R[5] * mz + cam.t[1];
@@ -121,7 +149,7 @@ __device__ __forceinline__ void geometry(const TrainParamsDev& P, int64_t i, con
     g.iz = 1.0f / zs;
     g.u = cam.fx * g.x * g.iz + cam.cx;
     g.v = cam.fy * g.y * g.iz + cam.cy;
-    const float q0 = P.quat[0][i], q1 = P.quat[1][i], q2 = P.quat[2][i], q3 = P.quat[3][i];
+    const float q0 = h.b.z, q1 = h.b.w, q2 = h.c.x, q3 = h.c.y;
     g.qinv = 1.0f / sqrtf(q0 * q0 + q1 * q1 + q2 * q2 + q3 * q3);
     const float w = q0 * g.qinv, x = q1 * g.qinv, y = q2 * g.qinv, z = q3 * g.qinv;
     g.qn[0] = w; g.qn[1] = x; g.qn[2] = y; g.qn[3] = z;
@@ -129,9 +157,9 @@ __device__ __forceinline__ void geometry(const TrainParamsDev& P, int64_t i, con
     Q[0] = 1.0f - 2.0f * (y * y + z * z); Q[1] = 2.0f * (x * y - w * z); Q[2] = 2.0f * (x * z + w * y);
     Q[3] = 2.0f * (x * y + w * z); Q[4] = 1.0f - 2.0f * (x * x + z * z); Q[5] = 2.0f * (y * z - w * x);
     Q[6] = 2.0f * (x * z - w * y); Q[7] = 2.0f * (y * z + w * x); Q[8] = 1.0f - 2.0f * (x * x + y * y);
-    g.s[0] = expf(P.ls[0][i]);
-    g.s[1] = expf(P.ls[1][i]);
-    g.s[2] = expf(P.ls[2][i]);
+    g.s[0] = expf(h.a.w);
+    g.s[1] = expf(h.b.x);
+    g.s[2] = expf(h.b.y);
     float M[9];
 #pragma unroll
     for (int r = 0; r < 3; ++r)
@@ -166,11 +194,10 @@ __device__ __forceinline__ void geometry(const TrainParamsDev& P, int64_t i, con
 }
 
 template <int DEG>
-__device__ __forceinline__ void colour(const TrainParamsDev& P, int64_t i, const TrainCam& cam,
+__device__ __forceinline__ void colour(const Head& h, const float* sh, const TrainCam& cam,
                                        float* raw, float* dir, float& dnorm) {
-    constexpr int K = (DEG + 1) * (DEG + 1);
-    const float dx = P.mean[0][i] - cam.ccx, dy = P.mean[1][i] - cam.ccy,
-                dz = P.mean[2][i] - cam.ccz;
+    constexpr int K = Row<DEG>::K;
+    const float dx = h.a.x - cam.ccx, dy = h.a.y - cam.ccy, dz = h.a.z - cam.ccz;
     dnorm = sqrtf(dx * dx + dy * dy + dz * dz);
     dir[0] = dx / dnorm; dir[1] = dy / dnorm; dir[2] = dz / dnorm;
     float b[16];
@@ -179,7 +206,7 @@ __device__ __forceinline__ void colour(const TrainParamsDev& P, int64_t i, const
     for (int ch = 0; ch < 3; ++ch) {
         float acc = 0.0f;
 #pragma unroll
-        for (int k = 0; k < K; ++k) acc += b[k] * P.sh[(size_t)(3 * k + ch) * P.n + i];
+        for (int k = 0; k < K; ++k) acc += b[k] * sh[3 * k + ch];
         raw[ch] = acc + 0.5f;
     }
 }
@@ -208,6 +235,11 @@ __global__ __launch_bounds__(kTThreads) void k_train_project(
     float4 rect[kTItems], cov[kTItems], r0[kTItems], r1[kTItems], r2[kTItems];
     float depth[kTItems];
     uint64_t bal[kTItems];
+    // the heads of a thread's rows together (past the end: the last row's)
+    Head head[kTItems];
+#pragma unroll
+    for (int it = 0; it < kTItems; ++it)
+        head[it] = load_head(P.rows + min(base + it * kTThreads + tid, n - 1) * Row<DEG>::V);
 #pragma unroll
     for (int it = 0; it < kTItems; ++it) {
         const int64_t i = base + it * kTThreads + tid;
@@ -215,10 +247,8 @@ __global__ __launch_bounds__(kTThreads) void k_train_project(
         depth[it] = 0.0f;
         if (i < n) {
             Geo g;
-            geometry(P, i, cam, g);
-            const float op = sigmoidf(P.ol[i]);
-            float raw[3], dir[3], dn;
-            colour<DEG>(P, i, cam, raw, dir, dn);
+            geometry(head[it], cam, g);
+            const float op = sigmoidf(head[it].c.z);
             // sparse-Adam rows: 3-sigma box overlaps the image (train_oracle.py:175-181)
             const float rx3 = ceilf(3.0f * sqrtf(fmaxf(g.a, 0.0f)));
             const float ry3 = ceilf(3.0f * sqrtf(fmaxf(g.c, 0.0f)));
@@ -237,6 +267,13 @@ __global__ __launch_bounds__(kTThreads) void k_train_project(
                     (g.v + ry > 0.0f) && (g.v - ry < (float)cam.H);
             }
             keep[it] = k;
+            // the colour of the rest is needed by the parity outputs only
+            float raw[3] = {0.0f, 0.0f, 0.0f};
+            if (k || dbg.means2d != nullptr) {
+                float sh[3 * Row<DEG>::K], dir[3], dn;
+                load_sh<DEG>(P.rows + i * Row<DEG>::V, head[it], sh);
+                colour<DEG>(head[it], sh, cam, raw, dir, dn);
+            }
             const float col[3] = {raw[0] < 0.0f ? 0.0f : raw[0], raw[1] < 0.0f ? 0.0f : raw[1],
                                   raw[2] < 0.0f ? 0.0f : raw[2]};
             rect[it] = make_float4(g.u, g.v, rx, ry);
@@ -821,38 +858,15 @@ __global__ __launch_bounds__(GS_WAVE) void k_train_bwd(const float4* __restrict_
     }
 }
 
-// Optimizer-space gradients of every Gaussian from its accumulated 2D
-// gradients (zero for Gaussians that blended nowhere).
+// Optimizer-space gradient row (Row<DEG>::S values into out) of a Gaussian from
+// its accumulated 2D gradients gg: dmx dmy dA dB dC dop dr dg db.
 template <int DEG>
-__global__ __launch_bounds__(256) void k_train_param_grads(TrainParamsDev P, TrainCam cam,
-                                                           const uint32_t* __restrict__ cidx,
-                                                           const float* __restrict__ grad2d,
-                                                           TrainParamsDev G) {
-    constexpr int K = (DEG + 1) * (DEG + 1);
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= P.n) return;
-    const uint32_t ci = cidx[i];
-    float gg[9];
-    if (ci != 0xFFFFFFFFu) {
-#pragma unroll
-        for (int k = 0; k < 9; ++k) gg[k] = grad2d[9 * (size_t)ci + k];
-    } else {
-#pragma unroll
-        for (int k = 0; k < 9; ++k) gg[k] = 0.0f;
-    }
-    bool any = false;
-#pragma unroll
-    for (int k = 0; k < 9; ++k) any |= gg[k] != 0.0f;
-    if (!any) {
-        for (int c = 0; c < 3; ++c) G.mean[c][i] = 0.0f;
-        for (int c = 0; c < 3; ++c) G.ls[c][i] = 0.0f;
-        for (int c = 0; c < 4; ++c) G.quat[c][i] = 0.0f;
-        G.ol[i] = 0.0f;
-        for (int c = 0; c < 3 * K; ++c) G.sh[(size_t)c * P.n + i] = 0.0f;
-        return;
-    }
+__device__ __forceinline__ void row_gradient(const float4* row, const TrainCam& cam,
+                                             const float (&gg)[9], float4* out) {
+    constexpr int K = Row<DEG>::K;
+    const Head head = load_head(row);
     Geo g;
-    geometry(P, i, cam, g);
+    geometry(head, cam, g);
     const float gu = gg[0], gv = gg[1], gA = gg[2], gB = gg[3], gC = gg[4], gop = gg[5];
     // conic = inv(S2): dL/dS2 = -Q Gq Q, Gq = [[gA, gB/2], [gB/2, gC]]
     const float hB = 0.5f * gB;
@@ -935,83 +949,172 @@ __global__ __launch_bounds__(256) void k_train_param_grads(TrainParamsDev P, Tra
     }
 #pragma unroll
     for (int k = 0; k < 3; ++k) gls[k] *= g.s[k];
-    const float op = sigmoidf(P.ol[i]);
+    const float op = sigmoidf(head.c.z);
     const float gol = gop * op * (1.0f - op);
     // colour = max(SH(d) + 0.5, 0)
+    float sh[3 * K];
+    load_sh<DEG>(row, head, sh);
     float raw[3], dir[3], dn;
-    colour<DEG>(P, i, cam, raw, dir, dn);
+    colour<DEG>(head, sh, cam, raw, dir, dn);
     float gcol[3];
 #pragma unroll
     for (int ch = 0; ch < 3; ++ch) gcol[ch] = raw[ch] >= 0.0f ? gg[6 + ch] : 0.0f;
     float b[16], db[16][3];
     sh_basis<DEG, true>(dir[0], dir[1], dir[2], b, db);
-    float gd[3] = {0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-#pragma unroll
-        for (int ch = 0; ch < 3; ++ch) {
-            G.sh[(size_t)(3 * k + ch) * P.n + i] = b[k] * gcol[ch];
-            if (K > 1) {
-                const float c = P.sh[(size_t)(3 * k + ch) * P.n + i] * gcol[ch];
-                gd[0] += c * db[k][0];
-                gd[1] += c * db[k][1];
-                gd[2] += c * db[k][2];
-            }
-        }
-    }
     if (K > 1) {
+        float gd[3] = {0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int k = 1; k < K; ++k) {
+            const float c = sh[3 * k] * gcol[0] + sh[3 * k + 1] * gcol[1] + sh[3 * k + 2] * gcol[2];
+            gd[0] += c * db[k][0];
+            gd[1] += c * db[k][1];
+            gd[2] += c * db[k][2];
+        }
         const float dd = dir[0] * gd[0] + dir[1] * gd[1] + dir[2] * gd[2];
 #pragma unroll
         for (int k = 0; k < 3; ++k) gm[k] += (gd[k] - dir[k] * dd) / dn;
     }
+    out[0] = make_float4(gm[0], gm[1], gm[2], gls[0]);
+    out[1] = make_float4(gls[1], gls[2], gq[0], gq[1]);
+    out[2] = make_float4(gq[2], gq[3], gol, b[0] * gcol[0]);
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        G.mean[k][i] = gm[k];
-        G.ls[k][i] = gls[k];
+    for (int q = 3; q < Row<DEG>::V; ++q) {
+        float t[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int j = 4 * (q - 3) + 1 + e;  // SH value 3k + channel
+            t[e] = j < 3 * K ? b[j < 3 * K ? j / 3 : 0] * gcol[j % 3] : 0.0f;
+        }
+        out[q] = make_float4(t[0], t[1], t[2], t[3]);
     }
-#pragma unroll
-    for (int k = 0; k < 4; ++k) G.quat[k][i] = gq[k];
-    G.ol[i] = gol;
 }
 
-// Sparse Adam (train_oracle.py:434-470): rows with visible[i] set; every plane
-// of the parameter block, fp32 arithmetic, bias correction folded into the
-// per-plane step sizes and sqrt(1 - beta2^t) computed by the host. Moments
-// stored as MOM: float, or bf16 bits (uint16_t) read exactly into fp32, updated
-// in fp32, the update taken from the fp32 values, stored rounded to nearest
-// even (train_oracle.py:445-470 with moment_dtype bfloat16,
+// Moments of four values of a row: float, or bf16 bits (uint16_t) read exactly
+// into fp32, updated in fp32, the update taken from the fp32 values, stored
+// rounded to nearest even (train_oracle.py:445-470 with moment_dtype bfloat16,
 // t2_param_backward.py:195-224): half the moments' bytes.
-template <typename MOM>
-__device__ __forceinline__ float mom_load(const MOM* a, size_t k);
-template <>
-__device__ __forceinline__ float mom_load<float>(const float* a, size_t k) { return a[k]; }
-template <>
-__device__ __forceinline__ float mom_load<uint16_t>(const uint16_t* a, size_t k) {
-    return bf16_to_f32(a[k]);
+__device__ __forceinline__ float4 mom_load(const float* a, size_t f) {
+    return reinterpret_cast<const float4*>(a)[f];
 }
-__device__ __forceinline__ void mom_store(float* a, size_t k, float x) { a[k] = x; }
-__device__ __forceinline__ void mom_store(uint16_t* a, size_t k, float x) {
-    a[k] = f32_to_bf16_rne(x);
+__device__ __forceinline__ float4 mom_load(const uint16_t* a, size_t f) {
+    const ushort4 u = reinterpret_cast<const ushort4*>(a)[f];
+    return make_float4(bf16_to_f32(u.x), bf16_to_f32(u.y), bf16_to_f32(u.z), bf16_to_f32(u.w));
+}
+__device__ __forceinline__ void mom_store(float* a, size_t f, float4 x) {
+    reinterpret_cast<float4*>(a)[f] = x;
+}
+__device__ __forceinline__ void mom_store(uint16_t* a, size_t f, float4 x) {
+    reinterpret_cast<ushort4*>(a)[f] = make_ushort4(f32_to_bf16_rne(x.x), f32_to_bf16_rne(x.y),
+                                                    f32_to_bf16_rne(x.z), f32_to_bf16_rne(x.w));
 }
 
+// Sparse Adam of one value (train_oracle.py:434-470), fp32 arithmetic, bias
+// correction folded into the step size and sqrt(1 - beta2^t) by the host.
+__device__ __forceinline__ void adam_value(float& p, float& m, float& v, float g, float step,
+                                           const AdamParams& ap) {
+    m = ap.beta1 * m + ap.one_minus_beta1 * g;
+    v = ap.beta2 * v + ap.one_minus_beta2 * g * g;
+    const float den = sqrtf(v) / ap.sqrt_bc2 + ap.eps;
+    p = p - step * (m / den);
+}
 template <typename MOM>
-__global__ __launch_bounds__(256) void k_sparse_adam(float* __restrict__ p, MOM* __restrict__ m,
-                                                     MOM* __restrict__ v,
-                                                     const float* __restrict__ g,
-                                                     const uint8_t* __restrict__ visible,
-                                                     int64_t n, int planes, AdamParams ap) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n || !visible[i]) return;
-    for (int j = 0; j < planes; ++j) {
-        const size_t k = (size_t)j * n + i;
-        const float gj = g[k];
-        const float m1 = ap.beta1 * mom_load(m, k) + ap.one_minus_beta1 * gj;
-        const float v1 = ap.beta2 * mom_load(v, k) + ap.one_minus_beta2 * gj * gj;
-        const float den = sqrtf(v1) / ap.sqrt_bc2 + ap.eps;
-        p[k] = p[k] - ap.step[j] * (m1 / den);
-        mom_store(m, k, m1);
-        mom_store(v, k, v1);
+__device__ __forceinline__ void adam_float4(float4* P, MOM* m, MOM* v, size_t f, float4 g,
+                                            float4 step, const AdamParams& ap) {
+    float4 p = P[f], mm = mom_load(m, f), vv = mom_load(v, f);
+    adam_value(p.x, mm.x, vv.x, g.x, step.x, ap);
+    adam_value(p.y, mm.y, vv.y, g.y, step.y, ap);
+    adam_value(p.z, mm.z, vv.z, g.z, step.z, ap);
+    adam_value(p.w, mm.w, vv.w, g.w, step.w, ap);
+    P[f] = p;
+    mom_store(m, f, mm);
+    mom_store(v, f, vv);
+}
+
+// Gradients of every Gaussian, and with ADAM the sparse Adam of the visible rows
+// in the same pass (the gradient row then never comes back from HBM). A
+// workgroup owns R rows. First a thread per row forms the gradient of a row
+// that blended somewhere into LDS and the rows with work are listed; then the
+// workgroup streams those rows, one float4 per lane, so that every access to
+// G, the parameters and the moments is contiguous within a row and the rows
+// without work (invisible, gradient zero as before) are not touched at all.
+constexpr uint32_t kRowGrad = 1u << 16, kRowZero = 1u << 17, kRowAdam = 1u << 18;
+constexpr int kGradThreads = 256;
+template <int DEG, bool ADAM, typename MOM>
+__global__ __launch_bounds__(kGradThreads) void k_train_grads(
+    TrainParamsDev P, TrainCam cam, const uint32_t* __restrict__ cidx,
+    const float* __restrict__ grad2d, float4* __restrict__ G, uint8_t* __restrict__ gnz,
+    MOM* __restrict__ m, MOM* __restrict__ v, const uint8_t* __restrict__ visible, AdamParams ap) {
+    constexpr int V = Row<DEG>::V;
+    constexpr int R = DEG < 2 ? kGradThreads : kGradThreads / 2;  // rows: 16 to 30 KB of LDS
+    __shared__ float4 s_g[R][V];
+    __shared__ float4 s_step[V];
+    __shared__ uint32_t s_list[R];
+    __shared__ uint32_t s_count;
+    if (upstream_failed(cam.ctl)) return;
+    const int tid = threadIdx.x;
+    const int64_t row0 = (int64_t)blockIdx.x * R;
+    if (tid == 0) s_count = 0;
+    if (ADAM && tid < V)
+        s_step[tid] = make_float4(ap.step[4 * tid], ap.step[4 * tid + 1], ap.step[4 * tid + 2],
+                                  ap.step[4 * tid + 3]);
+    __syncthreads();
+    const int64_t i = row0 + tid;
+    if (tid < R) {
+        uint32_t act = 0;
+        if (i < P.n) {
+            const uint32_t ci = cidx[i];
+            float gg[9];
+            bool any = false;
+#pragma unroll
+            for (int k = 0; k < 9; ++k) {
+                gg[k] = ci != 0xFFFFFFFFu ? grad2d[9 * (size_t)ci + k] : 0.0f;
+                any |= gg[k] != 0.0f;
+            }
+            const bool was = gnz[i] != 0;
+            if (any) {
+                row_gradient<DEG>(P.rows + i * V, cam, gg, s_g[tid]);
+                act = kRowGrad;
+            } else if (was) {
+                act = kRowZero;
+            }
+            if (any != was) gnz[i] = any ? 1 : 0;
+            if (ADAM && visible[i]) act |= kRowAdam;
+        }
+        const uint64_t mask = __ballot(act != 0u);
+        uint32_t at = 0;
+        if (lane_id() == 0 && mask != 0ull) at = atomicAdd(&s_count, (uint32_t)__popcll(mask));
+        at = (uint32_t)__builtin_amdgcn_readfirstlane((int)at);
+        if (act != 0u) s_list[at + (uint32_t)__popcll(mask & lanemask_lt())] = act | (uint32_t)tid;
     }
+    __syncthreads();
+    const uint32_t total = s_count * V;
+    for (uint32_t k = tid; k < total; k += kGradThreads) {
+        const uint32_t e = s_list[k / V], q = k % V, r = e & 0xFFFFu;
+        const size_t f = (size_t)(row0 + r) * V + q;
+        float4 g = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (e & kRowGrad) g = s_g[r][q];
+        if (e & (kRowGrad | kRowZero)) G[f] = g;
+        if (ADAM && (e & kRowAdam)) adam_float4(P.rows, m, v, f, g, s_step[q], ap);
+    }
+}
+
+// The sparse Adam alone, from gradient rows: a lane per float4 of the visible
+// rows.
+template <int DEG, typename MOM>
+__global__ __launch_bounds__(256) void k_sparse_adam(TrainParamsDev P, MOM* __restrict__ m,
+                                                     MOM* __restrict__ v,
+                                                     const float4* __restrict__ G,
+                                                     const uint8_t* __restrict__ visible,
+                                                     AdamParams ap) {
+    constexpr int V = Row<DEG>::V;
+    __shared__ float4 s_step[V];
+    if (threadIdx.x < V)
+        s_step[threadIdx.x] = make_float4(ap.step[4 * threadIdx.x], ap.step[4 * threadIdx.x + 1],
+                                          ap.step[4 * threadIdx.x + 2], ap.step[4 * threadIdx.x + 3]);
+    __syncthreads();
+    const size_t f = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (f >= (size_t)P.n * V || !visible[f / V]) return;
+    adam_float4(P.rows, m, v, f, G[f], s_step[f % V], ap);
 }
 
 }  // namespace
@@ -1071,36 +1174,71 @@ hipError_t launch_train_bwd(const float4* trec, const uint32_t* sid, const uint3
     return hipGetLastError();
 }
 
-hipError_t launch_train_param_grads(const TrainParamsDev& P, const TrainCam& cam,
-                                    const uint32_t* cidx, const float* grad2d,
-                                    const TrainParamsDev& G, hipStream_t st) {
-    if (P.n <= 0) return hipSuccess;
-    const unsigned grid = (unsigned)((P.n + 255) / 256);
-    switch (P.sh_degree) {
-        case 0: k_train_param_grads<0><<<grid, 256, 0, st>>>(P, cam, cidx, grad2d, G); break;
-        case 1: k_train_param_grads<1><<<grid, 256, 0, st>>>(P, cam, cidx, grad2d, G); break;
-        case 2: k_train_param_grads<2><<<grid, 256, 0, st>>>(P, cam, cidx, grad2d, G); break;
-        case 3: k_train_param_grads<3><<<grid, 256, 0, st>>>(P, cam, cidx, grad2d, G); break;
-        default: return hipErrorInvalidValue;
-    }
+namespace {
+template <int DEG>
+hipError_t train_grads_deg(const TrainParamsDev& P, const TrainCam& cam, const uint32_t* cidx,
+                           const float* grad2d, float4* G, uint8_t* gnz, void* m, void* v,
+                           const uint8_t* visible, const AdamParams* adam, bool bf16_moments,
+                           hipStream_t st) {
+    constexpr int R = DEG < 2 ? kGradThreads : kGradThreads / 2;
+    const unsigned grid = (unsigned)((P.n + R - 1) / R);
+    if (adam == nullptr)
+        k_train_grads<DEG, false, float><<<grid, kGradThreads, 0, st>>>(
+            P, cam, cidx, grad2d, G, gnz, nullptr, nullptr, nullptr, AdamParams{});
+    else if (bf16_moments)
+        k_train_grads<DEG, true, uint16_t><<<grid, kGradThreads, 0, st>>>(
+            P, cam, cidx, grad2d, G, gnz, static_cast<uint16_t*>(m), static_cast<uint16_t*>(v),
+            visible, *adam);
+    else
+        k_train_grads<DEG, true, float><<<grid, kGradThreads, 0, st>>>(
+            P, cam, cidx, grad2d, G, gnz, static_cast<float*>(m), static_cast<float*>(v), visible,
+            *adam);
     return hipGetLastError();
 }
 
-hipError_t launch_sparse_adam(float* p, void* m, void* v, const float* g,
-                              const uint8_t* visible, int64_t n, int planes, const AdamParams& ap,
-                              bool bf16_moments, hipStream_t st) {
-    if (n <= 0) return hipSuccess;
-    if (planes > kMaxTrainPlanes) return hipErrorInvalidValue;
-    const unsigned grid = (unsigned)((n + 255) / 256);
+template <int DEG>
+hipError_t sparse_adam_deg(const TrainParamsDev& P, void* m, void* v, const float4* G,
+                           const uint8_t* visible, const AdamParams& ap, bool bf16_moments,
+                           hipStream_t st) {
+    const unsigned grid = (unsigned)(((size_t)P.n * Row<DEG>::V + 255) / 256);
     if (bf16_moments)
-        k_sparse_adam<uint16_t><<<grid, 256, 0, st>>>(p, static_cast<uint16_t*>(m),
-                                                      static_cast<uint16_t*>(v), g, visible, n,
-                                                      planes, ap);
+        k_sparse_adam<DEG, uint16_t><<<grid, 256, 0, st>>>(
+            P, static_cast<uint16_t*>(m), static_cast<uint16_t*>(v), G, visible, ap);
     else
-        k_sparse_adam<float><<<grid, 256, 0, st>>>(p, static_cast<float*>(m),
-                                                   static_cast<float*>(v), g, visible, n, planes,
-                                                   ap);
+        k_sparse_adam<DEG, float><<<grid, 256, 0, st>>>(P, static_cast<float*>(m),
+                                                        static_cast<float*>(v), G, visible, ap);
     return hipGetLastError();
+}
+}  // namespace
+
+hipError_t launch_train_grads(const TrainParamsDev& P, const TrainCam& cam, const uint32_t* cidx,
+                              const float* grad2d, float4* G, uint8_t* gnz, void* m, void* v,
+                              const uint8_t* visible, const AdamParams* adam, bool bf16_moments,
+                              hipStream_t st) {
+    if (P.n <= 0) return hipSuccess;
+#define GS_TG(D) \
+    train_grads_deg<D>(P, cam, cidx, grad2d, G, gnz, m, v, visible, adam, bf16_moments, st)
+    switch (P.sh_degree) {
+        case 0: return GS_TG(0);
+        case 1: return GS_TG(1);
+        case 2: return GS_TG(2);
+        case 3: return GS_TG(3);
+        default: return hipErrorInvalidValue;
+    }
+#undef GS_TG
+}
+
+hipError_t launch_sparse_adam(const TrainParamsDev& P, void* m, void* v, const float4* G,
+                              const uint8_t* visible, const AdamParams& ap, bool bf16_moments,
+                              hipStream_t st) {
+    if (P.n <= 0) return hipSuccess;
+    switch (P.sh_degree) {
+        case 0: return sparse_adam_deg<0>(P, m, v, G, visible, ap, bf16_moments, st);
+        case 1: return sparse_adam_deg<1>(P, m, v, G, visible, ap, bf16_moments, st);
+        case 2: return sparse_adam_deg<2>(P, m, v, G, visible, ap, bf16_moments, st);
+        case 3: return sparse_adam_deg<3>(P, m, v, G, visible, ap, bf16_moments, st);
+        default: return hipErrorInvalidValue;
+    }
 }
 
 }  // namespace gs

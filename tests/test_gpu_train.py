@@ -324,3 +324,67 @@ def test_train_bands_match_oracle(gpu_ctx, n, H, W, op):
     ref = TO.projection_backward(pr, g2, cfg_o)
     for k in TO.PARAM_NAMES:
         assert rel_err(grads[k], ref[k]) < 1e-2, k
+
+
+@pytest.mark.parametrize("n,deg,bf16", [(1, 0, False), (127, 3, False), (129, 2, True),
+                                        (255, 1, True), (257, 0, False), (600, 3, True)])
+def test_train_step_rows(gpu_ctx, n, deg, bf16):
+    """The fused gradient and Adam pass over whole and partial workgroups of rows (128 or
+    256), every SH degree (row lengths 14 to 59 values): moments and parameters follow
+    bit for bit from the step's own gradients, invisible rows keep theirs, and a row
+    whose gradient returns to zero (another view, or gradients written from outside)
+    reads zero again."""
+    print("train step rows", n, deg, bf16, flush=True)
+    rng = np.random.default_rng(n + deg)
+    H, W = 40, 56
+    K = scenes.intrinsics(60.0, 60.0, W / 2, H / 2)
+    side = np.where(rng.random(n) < 0.3, -1.0, 1.0)  # a third behind the camera
+    if n == 1:
+        side[:] = 1.0
+    p = {"means": np.stack([rng.uniform(-0.6, 0.6, n), rng.uniform(-0.4, 0.4, n),
+                            side * rng.uniform(2, 4, n)], 1),
+         "log_scales": rng.normal(-2.5, 0.5, (n, 3)), "quats": rng.standard_normal((n, 4)),
+         "opacity_logits": rng.normal(0, 1.0, n),
+         "sh": rng.uniform(-0.5, 0.5, (n, (deg + 1) ** 2, 3))}
+    p = {k: v.astype(np.float32) for k, v in p.items()}
+    cfg = L.make_train_cfg()
+    view = L.make_view(np.eye(4, dtype=np.float32), K, H, W, tile_size=16)
+    away = L.make_view(np.diag([1, 1, 1, 1]).astype(np.float32) +
+                       np.array([[0, 0, 0, 0], [0, 0, 0, 0], [0, 0, 0, -50], [0, 0, 0, 0]],
+                                np.float32), K, H, W, tile_size=16)
+    target = rng.random((H, W, 3)).astype(np.float32)
+    tr = L.Trainer(gpu_ctx, p, deg)
+    try:
+        tr.set_moments(bf16)
+        _, _, proj, _ = tr.forward(view, cfg, want_proj=True)
+        vis = proj["visible"]
+        tr.step(view, cfg, target)
+        g, m, v, q = tr.read(3), tr.read(1), tr.read(2), tr.read(0)
+        f = np.float32
+        rnd = TO.bf16_round if bf16 else (lambda x: x)
+        bc1, bc2 = 1.0 - 0.9, 1.0 - 0.999
+        lr = {"means": cfg.lr_means, "log_scales": cfg.lr_log_scales, "quats": cfg.lr_quats,
+              "opacity_logits": cfg.lr_opacity}
+        for k in TO.PARAM_NAMES:
+            assert np.abs(g[k]).max() > 0, k
+            m1, v1 = f(1.0 - 0.9) * g[k], f(1.0 - 0.999) * g[k] * g[k]
+            den = np.sqrt(v1) / f(np.sqrt(bc2)) + f(cfg.eps)
+            if k == "sh":
+                step = np.full((1, (deg + 1) ** 2, 1), f(cfg.lr_sh_rest) / f(bc1), f)
+                step[:, 0] = f(cfg.lr_sh_dc) / f(bc1)
+            else:
+                step = f(lr[k] / bc1)
+            row = vis.reshape(-1, *([1] * (g[k].ndim - 1)))
+            assert np.array_equal(m[k], np.where(row, rnd(m1), f(0))), k
+            assert np.array_equal(v[k], np.where(row, rnd(v1), f(0))), k
+            assert np.array_equal(q[k], np.where(row, p[k] - step * (m1 / den), p[k])), k
+        tr.step(away, cfg, target)  # nothing in view: every gradient is zero again
+        assert all(np.all(a == 0) for a in tr.read(3).values())
+        after = tr.read(0)
+        assert all(np.array_equal(after[k], q[k]) for k in TO.PARAM_NAMES)
+        tr.write(3, {k: np.ones_like(a) for k, a in g.items()})
+        tr.forward(away, cfg, target)
+        tr.backward(cfg)
+        assert all(np.all(a == 0) for a in tr.read(3).values())
+    finally:
+        tr.set_moments(False)

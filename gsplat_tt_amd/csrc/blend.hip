@@ -572,6 +572,16 @@ __global__ __launch_bounds__(kStatThreads) void k_mb_stats(
 }
 
 template <int TS>
+const void* blend_ts(int out_format) {
+    switch (out_format) {
+        case 0: return reinterpret_cast<const void*>(&k_blend<TS, 0>);
+        case 1: return reinterpret_cast<const void*>(&k_blend<TS, 1>);
+        case 2: return reinterpret_cast<const void*>(&k_blend<TS, 2>);
+        default: return nullptr;
+    }
+}
+
+template <int TS>
 hipError_t launch_ts(const float4* brec, const uint32_t* sid, const uint32_t* ranges,
                      BlendParams bp, void* out, hipStream_t st) {
     const unsigned grid = (unsigned)(bp.tiles_x * bp.tiles_y * (TS / 16) * (TS / 4));
@@ -603,6 +613,29 @@ hipError_t launch_blend(const float4* brec, const uint32_t* sid, const uint32_t*
     if (bp.tile_size == 16) return launch_ts<16>(brec, sid, ranges, bp, out, st);
     if (bp.tile_size == 32) return launch_ts<32>(brec, sid, ranges, bp, out, st);
     return hipErrorInvalidValue;
+}
+
+const void* blend_kernel(int tile_size, int out_format) {
+    if (tile_size == 16) return blend_ts<16>(out_format);
+    if (tile_size == 32) return blend_ts<32>(out_format);
+    return nullptr;
+}
+
+hipError_t graph_set_blend_out(hipGraphExec_t exec, hipGraphNode_t node, void* out) {
+    hipKernelNodeParams kp;
+    hipError_t e = hipGraphKernelNodeGetParams(node, &kp);
+    if (e != hipSuccess) return e;
+    if (kp.kernelParams == nullptr) return hipErrorInvalidValue;
+    // the node's arguments as launch_blend passed them, the image replaced
+    const float4* a0 = *static_cast<const float4* const*>(kp.kernelParams[0]);
+    const uint32_t* a1 = *static_cast<const uint32_t* const*>(kp.kernelParams[1]);
+    const uint32_t* a2 = *static_cast<const uint32_t* const*>(kp.kernelParams[2]);
+    BlendParams a3 = *static_cast<const BlendParams*>(kp.kernelParams[3]);
+    void* a4 = out;
+    void* args[5] = {&a0, &a1, &a2, &a3, &a4};
+    kp.kernelParams = args;
+    kp.extra = nullptr;
+    return hipGraphExecKernelNodeSetParams(exec, node, &kp);
 }
 
 }  // namespace gs

@@ -1180,11 +1180,13 @@ struct gs_ctx {
     // ------------------------------------------------------------ frame graphs
     // A gs_render_batch frame's kernels (everything frame() enqueues) captured
     // once per frame slot and shape and replayed for the slot's later frames of
-    // that shape, with the view set on the graph's k_project node: one launch
-    // instead of ~20 per frame (100K-Gaussian orbit 12.9K -> 13.4K frames/s; a
+    // that shape, with the view set on the graph's k_project node and the image on
+    // its k_blend node: one launch instead of ~20 per frame (100K-Gaussian orbit
+    // 12.9K -> 13.4K frames/s; 16 views of it into 16 images, whose frames each
+    // captured anew while a graph held its image: 2.63 -> 2.12 ms; a
     // single frame, whose host waits for it, gains nothing and stays direct). A
     // shape is everything the captured launches depend on besides the view's
-    // camera: the view's other fields, the output, the scene size and SH
+    // camera and image: the view's other fields, the scene size and SH
     // degree, the pair capacity, the spin limit, the slot's device buffers
     // (their addresses) and the sort's look-back state — the state-
     // clearing launches of the passes are baked into the graph, so a graph is
@@ -1205,9 +1207,10 @@ struct gs_ctx {
         hipGraph_t graph = nullptr;
         hipGraphExec_t exec = nullptr;
         hipGraphNode_t proj = nullptr;  // null: not replayable (the sort state moved)
+        hipGraphNode_t blend = nullptr;
         gs_view shape{};
         gs::SceneDev sd{};  // the scene's device pointers, held by the projection node
-        void* dout = nullptr;
+        void* dout = nullptr;  // the image the blend node writes now
         int64_t n = -1, T = -1;
         int deg = -2;
         uint64_t pcap = 0, gen = 0;
@@ -1263,8 +1266,7 @@ struct gs_ctx {
         const FrameLayout L = frame_prepare(N, pend.T);  // every allocation before a capture
         const gs_view shape = graph_shape(&pend.v);
         const uint64_t gen = buffers_key();
-        const bool same_shape = fg.dout == pend.dout && fg.n == N && fg.T == pend.T &&
-                                fg.deg == sd.sh_degree && fg.pcap == pair_cap && fg.gen == gen &&
+        const bool same_shape = fg.n == N && fg.T == pend.T && fg.deg == sd.sh_degree && fg.pcap == pair_cap && fg.gen == gen &&
                                 fg.spin == spin_limit && same_scene(fg.sd, sd) &&
                                 std::memcmp(&fg.shape, &shape, sizeof(shape)) == 0;
         // a shape whose frames never leave the sort state as they found it (an
@@ -1274,6 +1276,10 @@ struct gs_ctx {
         if (fg.exec != nullptr && fg.proj != nullptr && same_shape && fg.marks == sort_marks()) {
             const gs::ProjParams p = frame_proj_params(&pend.v, L, N, pend.tiles_x, pend.tiles_y);
             HIPCHK(gs::graph_set_project_params(fg.exec, fg.proj, p));
+            if (fg.dout != pend.dout) {
+                HIPCHK(gs::graph_set_blend_out(fg.exec, fg.blend, pend.dout));
+                fg.dout = pend.dout;
+            }
             HIPCHK(hipGraphLaunch(fg.exec, st));
             ++graph_replays;
             pend.replayed = true;
@@ -1336,22 +1342,24 @@ struct gs_ctx {
             HIPCHK(hipGraphGetNodes(fg.graph, nullptr, &nn));
             std::vector<hipGraphNode_t> nodes(nn);
             if (nn) HIPCHK(hipGraphGetNodes(fg.graph, nodes.data(), &nn));
-            const void* fn = gs::project_kernel(sd.sh_degree);
+            const void* fn_proj = gs::project_kernel(sd.sh_degree);
+            const void* fn_blend = gs::blend_kernel(pend.v.tile_size, pend.v.out_format);
+            hipGraphNode_t proj = nullptr;
             for (hipGraphNode_t node : nodes) {
                 hipGraphNodeType ty;
                 HIPCHK(hipGraphNodeGetType(node, &ty));
                 if (ty != hipGraphNodeTypeKernel) continue;
                 hipKernelNodeParams kp;
                 HIPCHK(hipGraphKernelNodeGetParams(node, &kp));
-                if (kp.func == fn && kp.kernelParams != nullptr) {
-                    const gs::ProjParams p =
-                        frame_proj_params(&pend.v, L, N, pend.tiles_x, pend.tiles_y);
-                    if (gs::graph_project_args_are(node, sd, p)) {
-                        fg.proj = node;
-                        fg.misses = 0;
-                    }
-                    break;
-                }
+                if (kp.kernelParams == nullptr) continue;
+                if (kp.func == fn_proj) proj = node;
+                if (kp.func == fn_blend) fg.blend = node;
+            }
+            if (proj != nullptr && fg.blend != nullptr &&
+                gs::graph_project_args_are(
+                    proj, sd, frame_proj_params(&pend.v, L, N, pend.tiles_x, pend.tiles_y))) {
+                fg.proj = proj;
+                fg.misses = 0;
             }
         }
         return true;

@@ -322,6 +322,11 @@ struct BlendParams {
 };
 hipError_t launch_blend(const float4* brec, const uint32_t* sorted_id, const uint32_t* ranges,
                         BlendParams bp, void* out, hipStream_t st);
+// Captured frames: the k_blend instance launch_blend uses, and an update of a
+// captured k_blend node's image in an instantiated graph (its other arguments
+// are kept).
+const void* blend_kernel(int tile_size, int out_format);
+hipError_t graph_set_blend_out(hipGraphExec_t exec, hipGraphNode_t node, void* out);
 // Counts of the reference's microblock cull over the tile-sorted pairs (ids
 // `sid`, tile ids `stile`, min(p_cap, *p_dev) of them): out[0] += pairs kept by
 // no microblock, out[1] += kept (pair, microblock) pairs.

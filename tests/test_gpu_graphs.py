@@ -192,3 +192,28 @@ def test_graph_odd_pass_count_goes_direct():
         if out is not None:
             ctx.dev_free(out)
         ctx.close()
+
+
+def test_graph_distinct_outputs(orbit):
+    """A camera path into one buffer per view: each slot captures once and replays
+    into its views' own images (eight and, in the odd passes, the buffers swapped)."""
+    scene, cams, cov = orbit
+    ctx = _ctx(scene, cov)
+    outs = []
+    try:
+        views = _views(cams)
+        ref = _direct(ctx, views)
+        outs = [ctx.dev_alloc(ref[0][0].nbytes) for _ in views]
+        for rep in range(4):
+            order = outs if rep % 2 == 0 else outs[::-1]
+            sts = ctx.render_batch(views, order)
+            for i in range(len(views)):
+                img = np.empty_like(ref[i][0])
+                ctx.d2h(img, order[i])
+                _check((img, sts[i]), ref[i], f"outputs {rep} view {i}")
+        caps, reps = ctx.graph_counts()
+        assert caps == 4 and reps == 4 * len(views) - 4, (caps, reps)
+    finally:
+        for o in outs:
+            ctx.dev_free(o)
+        ctx.close()

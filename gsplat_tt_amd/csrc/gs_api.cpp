@@ -257,7 +257,7 @@ struct gs_ctx {
                           &b_dkey, &b_brec, &b_src, &b_valid, &b_offs, &b_bstart, &b_pair_tile, &b_pair_id,
                           &b_ranges, &b_out, &b_kalt, &b_valt, &b_hist, &b_state, &b_lb, &b_cnt,
                           &b_tmp_a, &b_tmp_b, &b_tmp_c, &b_evals, &b_frame, &b_phist_proj,
-                          &b_phist_emit, &b_pchunk, &b_poffs, &b_spec, &b_chunk_box,
+                          &b_phist_emit, &b_bins, &b_pchunk, &b_poffs, &b_spec, &b_chunk_box,
                           &b_skip, &b_tcnt})
             b->release();
         if (h_pin) (void)hipHostFree(h_pin);
@@ -563,7 +563,8 @@ struct gs_ctx {
                                     b_pair_tile.as<uint32_t>(), b_pair_id.as<uint32_t>(), p_pre,
                                     b_lb.as<uint64_t>(), b_cnt.as<uint32_t>() + 10,
                                     b_cnt.as<uint32_t>() + 11, nullptr,
-                                    tile_bits((int64_t)tp.tiles_x * tp.tiles_y), true, st));
+                                    tile_bits((int64_t)tp.tiles_x * tp.tiles_y),
+                                    gs::Emit::kCompact, st));
         HIPCHK(hipMemcpyAsync(h_pin, b_cnt.p, 64 * 4, hipMemcpyDeviceToHost, st));
         sync();
         ctl_check(h_pin[C_CTL], "tile_assign");
@@ -571,18 +572,16 @@ struct gs_ctx {
     }
 
     // --------------------------------------------------------- render
-    // Frame-scratch layout (u32 words): counters, histograms, look-back states.
-    static constexpr size_t kFrCnt = 0;         // 64 counters (below)
-    static constexpr size_t kFrDepthHist = 64;  // [4][256] depth-key digits
-    static constexpr size_t kFrTileHist = 64 + 1024;  // [2 or 4][256] tile-id digits
-    static constexpr size_t kFrLb = 64 + 1024 + 1024;  // look-back states (u64 each)
+    // Frame-scratch layout (u32 words): counters, then what FrameLayout points at.
+    static constexpr size_t kFrCnt = 0;  // 64 counters (below)
     enum : int {
         C_PROJ_TICKET = 0, C_M = 1, C_SKIPPED = 2, C_CTL = 4, C_RECT_TICKET = 8, C_PPRE = 9,
-        C_EMIT_TICKET = 10, C_P = 11, C_DSORT_TICKETS = 16, C_TSORT_TICKETS = 24,
+        C_EMIT_TICKET = 10, C_P = 11, C_RUNS = 12, C_DSORT_TICKETS = 16, C_TSORT_TICKETS = 24,
         C_MBSTAT = 40  // two u64: pairs no microblock keeps, kept (pair, microblock)
     };
     uint64_t pair_cap = 0;  // candidate-pair capacity of the frame buffers
     DevBuf b_frame, b_phist_proj, b_phist_emit;
+    DevBuf b_bins;             // binned frames: pairs per (emit partition, tile)
     DevBuf b_pchunk, b_poffs;  // tile sort's first pass: emit row chunk sums, offsets
     static constexpr size_t kEmitPerSort = gs::kSortPartition32 / gs::kEmitPartition;
     static_assert(gs::kSortPartition32 % gs::kEmitPartition == 0,
@@ -748,6 +747,7 @@ struct gs_ctx {
             s.num_visible = h_pin[C_M];
             s.pairs_pre = h_pin[C_PPRE];
             s.num_entries = h_pin[C_P];
+            plan_seen(sd.n, pend.T, s.num_entries);
             s.chunks_skipped = h_pin[C_SKIPPED];
             if (cull_stats) {
                 uint64_t mb[2];
@@ -1056,13 +1056,47 @@ struct gs_ctx {
         uint32_t* fr;
         uint32_t* cnt;
         uint64_t *lb_proj, *lb_rect, *lb_emit;
-        uint32_t* tcnt;  // pairs per tile (the tile sort's last pass counts them)
-        size_t fwords, pparts, rparts, eparts;
+        uint32_t* tcnt;  // pairs per tile
+        uint32_t *hist_depth, *hist_tile;  // [4][256] depth-key, [2 or 4][256] tile-id digits
+        uint32_t* runs;      // binned: runs of the long tile lists
+        size_t fwords;       // words that a frame clears
+        size_t pparts, rparts, eparts;
         uint32_t pcap;
+        bool binned;
     };
-    FrameLayout frame_prepare(int64_t N, int64_t T) {
+    // Whether frames of N Gaussians and T tiles have their tile lists binned
+    // (launch_binned_lists) or sorted. Binning saves the sorts' launches and passes
+    // but stores each pair at its list's end and sorts each list on its own, so it
+    // wins up to about 2.4M pairs (us a frame alone and in a path, sorted against
+    // binned; 1280x720: 1.1M pairs 331, 219 / 263, 187; 1.7M 390, 250 / 313, 221;
+    // 2.8M 464, 308 / 402, 290; 1237x822: 1.5M 287, 177 / 227, 152; 3.0M 347, 238 /
+    // 348, 254; 5.0M 431, 310 / 515, 398; 400x300, 3100 pairs a tile: 1.5M 388,
+    // 241 / 403, 234). The pairs of a view are not known before it is rendered: a
+    // scene's frames start from the number of Gaussians and go on with the pairs
+    // of the frames that finished, with a gap between the two limits so that a
+    // camera path does not alternate.
+    static constexpr int64_t kBinnedFirst = 1 << 20, kBinnedMost = 2400000,
+                             kBinnedAgain = 1800000;
+    struct TilePlan {
+        int64_t n = -1, T = -1;
+        bool binned = false;
+    } plan;  // of the first slot, for all of them
+    bool binned_frame(int64_t N, int64_t T, bool want_keys) {
+        TilePlan& p = (owner ? owner : this)->plan;
+        if (p.n != N || p.T != T) p = {N, T, N <= kBinnedFirst};
+        // the microblock statistics need the sorted tile keys
+        return p.binned && !want_keys && T <= gs::kBinnedTiles && N < ((int64_t)1 << 28);
+    }
+    void plan_seen(int64_t N, int64_t T, int64_t P) {
+        TilePlan& p = (owner ? owner : this)->plan;
+        if (p.n != N || p.T != T) return;
+        if (P > kBinnedMost) p.binned = false;
+        if (P < kBinnedAgain) p.binned = true;
+    }
+    FrameLayout frame_prepare(int64_t N, int64_t T, bool want_keys) {
         FrameLayout L{};
         L.pcap = (uint32_t)pair_cap;
+        L.binned = binned_frame(N, T, want_keys);
         L.pparts = gs::project_partitions(N);
         L.rparts = gs::rect_scan_partitions(N);
         L.eparts = gs::emit_partitions(L.pcap);
@@ -1076,24 +1110,35 @@ struct gs_ctx {
         b_pair_tile.ensure((size_t)L.pcap * 4);
         b_pair_id.ensure((size_t)L.pcap * 4);
         b_ranges.ensure((size_t)T * 8);
-        b_phist_proj.ensure(L.pparts * 1024 * 4);
-        b_phist_emit.ensure(L.eparts * gs::tile_hist_cols(tile_bits(T)) * 4);
-        b_pchunk.ensure(gs::reduce_chunks((uint32_t)L.eparts) * gs::tile_hist_cols(tile_bits(T)) *
-                        4);
-        b_poffs.ensure(((L.eparts + kEmitPerSort - 1) / kEmitPerSort)
-                       << gs::sort_digit_width(tile_bits(T))
-                       << 2);
-        const size_t lb_words = 2 * (L.pparts + L.rparts + L.eparts);
-        L.fwords = kFrLb + lb_words + (size_t)T;
-        b_frame.ensure(L.fwords * 4);
+        if (L.binned) {
+            b_bins.ensure(gs::binned_scratch_words(L.pcap, T) * 4);
+        } else {
+            b_phist_proj.ensure(L.pparts * 1024 * 4);
+            b_phist_emit.ensure(L.eparts * gs::tile_hist_cols(tile_bits(T)) * 4);
+            b_pchunk.ensure(gs::reduce_chunks((uint32_t)L.eparts) *
+                            gs::tile_hist_cols(tile_bits(T)) * 4);
+            b_poffs.ensure(((L.eparts + kEmitPerSort - 1) / kEmitPerSort)
+                           << gs::sort_digit_width(tile_bits(T))
+                           << 2);
+        }
+        // cleared by every frame: counters, compaction states, pairs per tile; by the
+        // sorted ones also the histograms and the other states
+        const size_t tile_words = ((size_t)T + 1) & ~size_t(1);
+        const size_t binned_words = 64 + 2 * L.pparts + tile_words;
+        const size_t all_words = binned_words + 2048 + 2 * (L.rparts + L.eparts);
+        b_frame.ensure(all_words * 4);
+        L.fwords = L.binned ? binned_words : all_words;
         ensure_sort(std::max<int64_t>(N, L.pcap), 4);
         if (blend_counts) b_evals.ensure(64 * 8 * 8);
         L.fr = b_frame.as<uint32_t>();
-        L.lb_proj = reinterpret_cast<uint64_t*>(L.fr + kFrLb);
-        L.lb_rect = L.lb_proj + L.pparts;
-        L.lb_emit = L.lb_rect + L.rparts;
-        L.tcnt = L.fr + kFrLb + lb_words;
         L.cnt = L.fr + kFrCnt;
+        L.lb_proj = reinterpret_cast<uint64_t*>(L.fr + 64);
+        L.tcnt = L.fr + 64 + 2 * L.pparts;
+        L.hist_depth = L.tcnt + tile_words;
+        L.hist_tile = L.hist_depth + 1024;
+        L.lb_rect = reinterpret_cast<uint64_t*>(L.hist_tile + 1024);
+        L.lb_emit = L.lb_rect + L.rparts;
+        L.runs = reinterpret_cast<uint32_t*>(L.lb_emit);  // a binned frame scans no partitions
         return L;
     }
 
@@ -1107,8 +1152,8 @@ struct gs_ctx {
         // counts the pairs per tile instead of writing them, and the ranges come
         // from the counts
         const bool want_keys = tiles_out != nullptr;
-        uint32_t* fr = L.fr;
         uint32_t* cnt = L.cnt;
+        if (L.binned) return binned_tiles(L, N, T, tp);
         sort.ctl = cnt + C_CTL;
         // depth order of the visible Gaussians (stable: ties keep index order)
         // (values: the projection's packed ones when tp.idx_bits is set, else
@@ -1117,7 +1162,7 @@ struct gs_ctx {
         void* kf = nullptr;
         uint32_t* order = nullptr;
         HIPCHK(gs::radix_sort_pairs_dev(b_dkey.p, b_tmp_a.as<uint32_t>(), N, cnt + C_M, 4, 0, 32,
-                                        fr + kFrDepthHist, cnt + C_DSORT_TICKETS, sort, st,
+                                        L.hist_depth, cnt + C_DSORT_TICKETS, sort, st,
                                         tp.idx_bits == 0, &kf, &order, nullptr, nullptr, nullptr,
                                         0xFFFFFFFFu, false));
         record(2);
@@ -1130,18 +1175,18 @@ struct gs_ctx {
                                     L.pcap, cnt + C_PPRE, tp, b_pair_tile.as<uint32_t>(),
                                     b_pair_id.as<uint32_t>(), L.pcap, L.lb_emit,
                                     cnt + C_EMIT_TICKET, cnt + C_P, b_phist_emit.as<uint32_t>(),
-                                    tile_bits(T), false, st));
+                                    tile_bits(T), gs::Emit::kSlots, st));
         const int hcols = gs::tile_hist_cols(tile_bits(T));
         const int dw = gs::sort_digit_width(tile_bits(T));
         HIPCHK(gs::launch_reduce_rows(b_phist_emit.as<uint32_t>(), hcols, (uint32_t)L.eparts,
                                       cnt + C_PPRE, L.pcap, gs::kEmitPartition, dw,
-                                      fr + kFrTileHist, st, b_pchunk.as<uint32_t>(),
+                                      L.hist_tile, st, b_pchunk.as<uint32_t>(),
                                       cnt + C_CTL));
         // the first tile pass's output positions per partition, from the emit
         // rows (four emit partitions per sort partition): no look-back
         HIPCHK(gs::launch_part_offsets(b_phist_emit.as<uint32_t>(), hcols, (uint32_t)L.eparts,
                                        cnt + C_PPRE, L.pcap, gs::kEmitPartition, kEmitPerSort,
-                                       dw, b_pchunk.as<uint32_t>(), fr + kFrTileHist,
+                                       dw, b_pchunk.as<uint32_t>(), L.hist_tile,
                                        b_poffs.as<uint32_t>(), st, cnt + C_CTL));
         record(3);
         // stable tile sort of the depth-ordered candidate slots; its first pass
@@ -1149,7 +1194,7 @@ struct gs_ctx {
         void* tiles_sorted = nullptr;
         uint32_t* ids_sorted = nullptr;
         HIPCHK(gs::radix_sort_pairs_dev(b_pair_tile.p, b_pair_id.as<uint32_t>(), L.pcap,
-                                        cnt + C_PPRE, 4, 0, tile_bits(T), fr + kFrTileHist,
+                                        cnt + C_PPRE, 4, 0, tile_bits(T), L.hist_tile,
                                         cnt + C_TSORT_TICKETS, sort, st, false, &tiles_sorted,
                                         &ids_sorted, cnt + C_P, want_keys ? nullptr : L.tcnt,
                                         b_poffs.as<uint32_t>(), (uint32_t)T));
@@ -1163,6 +1208,31 @@ struct gs_ctx {
         return ids_sorted;
     }
 
+    // frame_tiles of a binned frame, whose projection scanned the candidates:
+    // pair emission in compact order, then the tiles' lists sorted one by one.
+    uint32_t* binned_tiles(const FrameLayout& L, int64_t N, int64_t T, const gs::TileParams& tp) {
+        uint32_t* cnt = L.cnt;
+        record(2);  // no depth sort of its own
+        HIPCHK(gs::launch_pair_emit(b_rc.as<float4>(), b_rc.as<float4>() + 1, 2, false, nullptr,
+                                    b_offs.as<uint32_t>(), b_bstart.as<uint32_t>(), N, cnt + C_M,
+                                    L.pcap, cnt + C_PPRE, tp, b_pair_tile.as<uint32_t>(),
+                                    b_pair_id.as<uint32_t>(), L.pcap, nullptr, nullptr, cnt + C_P,
+                                    nullptr, tile_bits(T), gs::Emit::kBinned, st,
+                                    b_bins.as<uint32_t>()));
+        record(3);
+        HIPCHK(gs::launch_binned_lists(b_pair_tile.as<uint32_t>(), b_pair_id.as<uint32_t>(),
+                                       L.pcap, cnt + C_PPRE, b_bins.as<uint32_t>(), L.tcnt, T,
+                                       b_dkey.as<uint32_t>(), b_ranges.as<uint32_t>(),
+                                       b_valt.as<uint32_t>(), b_kalt.as<uint32_t>(), L.runs,
+                                       cnt + C_RUNS, b_pair_id.as<uint32_t>(), L.cnt + C_CTL, st));
+        return b_pair_id.as<uint32_t>();
+    }
+    gs::BinnedOut binned_out(const FrameLayout& L) const {
+        if (!L.binned) return gs::BinnedOut{};
+        return gs::BinnedOut{b_offs.as<uint32_t>(), b_bstart.as<uint32_t>(),
+                             (uint32_t)(L.eparts + 1), L.cnt + C_PPRE, L.pcap};
+    }
+
     // The projection's parameters for a frame of view v in layout L.
     gs::ProjParams frame_proj_params(const gs_view* v, const FrameLayout& L, int64_t N,
                                      int tiles_x, int tiles_y) {
@@ -1173,7 +1243,8 @@ struct gs_ctx {
         p.tiles_y = tiles_y;
         p.tile_size = v->tile_size;
         p.idx_bits = dval_idx_bits(N);
-        p.dvals = p.idx_bits ? b_tmp_a.as<uint32_t>() : nullptr;
+        p.dvals = p.idx_bits && !L.binned ? b_tmp_a.as<uint32_t>() : nullptr;
+        p.binned = binned_out(L);
         return p;
     }
 
@@ -1215,6 +1286,7 @@ struct gs_ctx {
         int deg = -2;
         uint64_t pcap = 0, gen = 0;
         uint32_t spin = 0;
+        bool binned = false;
         SortMarks marks{};
         int misses = 0;  // captures of this shape in a row that were not replayable
     } fg;
@@ -1247,7 +1319,7 @@ struct gs_ctx {
         uint64_t h = 1469598103934665603ull;
         for (const DevBuf* b : {&b_rc, &b_dkey, &b_brec, &b_src, &b_tmp_a, &b_offs, &b_bstart,
                                 &b_pair_tile, &b_pair_id, &b_ranges, &b_phist_proj, &b_phist_emit,
-                                &b_pchunk, &b_poffs, &b_frame, &b_kalt, &b_valt, &b_hist,
+                                &b_bins, &b_pchunk, &b_poffs, &b_frame, &b_kalt, &b_valt, &b_hist,
                                 &b_state, &b_out}) {
             h ^= (uint64_t)(uintptr_t)b->p;
             h *= 1099511628211ull;
@@ -1263,11 +1335,12 @@ struct gs_ctx {
             return false;
         if (sd.chunk_box != nullptr && pend.v.k_cap <= 3.0f) return false;
         if (N >= ((int64_t)1 << 30) || pair_cap >= (1ull << 30)) return false;
-        const FrameLayout L = frame_prepare(N, pend.T);  // every allocation before a capture
+        const FrameLayout L = frame_prepare(N, pend.T, false);  // every allocation before a capture
         const gs_view shape = graph_shape(&pend.v);
         const uint64_t gen = buffers_key();
         const bool same_shape = fg.n == N && fg.T == pend.T && fg.deg == sd.sh_degree && fg.pcap == pair_cap && fg.gen == gen &&
-                                fg.spin == spin_limit && same_scene(fg.sd, sd) &&
+                                fg.spin == spin_limit && fg.binned == L.binned &&
+                                same_scene(fg.sd, sd) &&
                                 std::memcmp(&fg.shape, &shape, sizeof(shape)) == 0;
         // a shape whose frames never leave the sort state as they found it (an
         // odd pass count flips its half every frame: above 2^16 tiles the tile
@@ -1298,6 +1371,7 @@ struct gs_ctx {
         g.pcap = pair_cap;
         g.gen = gen;
         g.spin = spin_limit;
+        g.binned = L.binned;
         g.marks = sort_marks();
         auto capture = [&](hipGraph_t* out) {
             HIPCHK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
@@ -1342,7 +1416,7 @@ struct gs_ctx {
             HIPCHK(hipGraphGetNodes(fg.graph, nullptr, &nn));
             std::vector<hipGraphNode_t> nodes(nn);
             if (nn) HIPCHK(hipGraphGetNodes(fg.graph, nodes.data(), &nn));
-            const void* fn_proj = gs::project_kernel(sd.sh_degree);
+            const void* fn_proj = gs::project_kernel(sd.sh_degree, L.binned);
             const void* fn_blend = gs::blend_kernel(pend.v.tile_size, pend.v.out_format);
             hipGraphNode_t proj = nullptr;
             for (hipGraphNode_t node : nodes) {
@@ -1369,7 +1443,7 @@ struct gs_ctx {
     // ranges -> blend) on the stream; no host synchronisation.
     void frame(const gs_view* v, void* dout, int64_t T, int tiles_x, int tiles_y) {
         const int64_t N = sd.n;
-        const FrameLayout L = frame_prepare(N, T);
+        const FrameLayout L = frame_prepare(N, T, cull_stats);
         record(0);
         HIPCHK(gs::launch_fill_u32(L.fr, 0u, L.fwords, st));
         if (spin_limit) HIPCHK(gs::launch_fill_u32(L.cnt + C_CTL + 1, spin_limit, 1, st));
@@ -1387,9 +1461,10 @@ struct gs_ctx {
                       b_brec.as<float4>(), nullptr};
         HIPCHK(gs::launch_project(sd, p, c, nullptr, L.lb_proj, L.cnt + C_PROJ_TICKET,
                                   L.cnt + C_M, b_phist_proj.as<uint32_t>(), st));
-        HIPCHK(gs::launch_reduce_rows(b_phist_proj.as<uint32_t>(), 1024, (uint32_t)L.pparts,
-                                      nullptr, 0, 0, 0, L.fr + kFrDepthHist, st, nullptr,
-                                      L.cnt + C_CTL));
+        if (!L.binned)
+            HIPCHK(gs::launch_reduce_rows(b_phist_proj.as<uint32_t>(), 1024, (uint32_t)L.pparts,
+                                          nullptr, 0, 0, 0, L.hist_depth, st, nullptr,
+                                          L.cnt + C_CTL));
         record(1);
         gs::TileParams tp{tiles_x, tiles_y, v->tile_size, v->cull_disabled ? 0 : 1,
                           L.cnt + C_CTL, p.idx_bits};
@@ -1621,7 +1696,7 @@ struct gs_ctx {
         tr.tiles_y = (H + 15) / 16;
         const int64_t T = (int64_t)tr.tiles_x * tr.tiles_y;
         tr.cam = train_cam(v, c);
-        const FrameLayout L = frame_prepare(std::max<int64_t>(N, 1), T);
+        const FrameLayout L = frame_prepare(std::max<int64_t>(N, 1), T, true);
         const size_t px = (size_t)H * W;
         t_img.ensure(px * 12);
         t_T.ensure(px * 4);
@@ -1643,7 +1718,7 @@ struct gs_ctx {
                                         L.cnt + C_PROJ_TICKET, L.cnt + C_M,
                                         b_phist_proj.as<uint32_t>(), dbg, st));
         HIPCHK(gs::launch_reduce_rows(b_phist_proj.as<uint32_t>(), 1024, (uint32_t)L.pparts,
-                                      nullptr, 0, 0, 0, L.fr + kFrDepthHist, st, nullptr,
+                                      nullptr, 0, 0, 0, L.hist_depth, st, nullptr,
                                       L.cnt + C_CTL));
         gs::TileParams tp{tr.tiles_x, tr.tiles_y, 16, 1, L.cnt + C_CTL};
         tr.ids = frame_tiles(L, std::max<int64_t>(N, 1), T, tp, nullptr);

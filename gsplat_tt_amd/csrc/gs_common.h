@@ -241,6 +241,36 @@ __device__ __forceinline__ uint64_t lookback_exclusive(uint64_t* state, uint32_t
     return lookback_walk(state, vid, aggregate, ctl);
 }
 
+// ---------------------------------------------------------------------------
+// Binned frames: the compaction's look-back carries the visible count and the
+// candidate total together (count above bit 34, candidates below: a binned
+// frame has at most 2^32 of them and fewer than 2^28 Gaussians).
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ uint64_t binned_pack(uint32_t count, uint64_t cands) {
+    return ((uint64_t)count << 34) | cands;
+}
+__device__ __forceinline__ uint64_t binned_count(uint64_t v) { return v >> 34; }
+__device__ __forceinline__ uint64_t binned_cands(uint64_t v) { return v & ((1ull << 34) - 1); }
+
+// The last partition's inclusive prefix: visible count, candidate total
+// (saturated), and kErrCapacity when the candidates do not fit.
+__device__ __forceinline__ void binned_totals(uint64_t v, uint32_t* count_out,
+                                              const BinnedOut& b, uint32_t* ctl) {
+    const uint64_t c = binned_cands(v);
+    *count_out = (uint32_t)binned_count(v);
+    *b.total_out = c > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)c;
+    if (c > b.cap) report_error(ctl, kErrCapacity);
+}
+
+// Gaussian m owns the candidates [o, o + cnt): its offset, and the emission
+// partitions whose first candidate it owns.
+__device__ __forceinline__ void binned_write(const BinnedOut& b, uint64_t m, uint64_t o,
+                                             uint32_t cnt) {
+    b.offs[m] = (uint32_t)o;
+    uint64_t e = (o + kEmitPartition - 1) / kEmitPartition;
+    for (; e * kEmitPartition < o + cnt && e < b.bstart_cap; ++e) b.bstart[e] = (uint32_t)m;
+}
+
 }  // namespace gs
 
 // Host-side launch check: every launcher returns hipError_t.

@@ -44,6 +44,18 @@ struct SceneDev {
     double chunk_k = 1.5;
 };
 
+// Outputs of a binned frame's projection (all null otherwise): exclusive scan of
+// the tile counts in compact order, the compact id owning candidate b *
+// kEmitPartition (b < bstart_cap), the candidate total, and the capacity that it
+// must not exceed (kErrCapacity).
+struct BinnedOut {
+    uint32_t* offs;
+    uint32_t* bstart;
+    uint32_t bstart_cap;
+    uint32_t* total_out;
+    uint32_t cap;
+};
+
 struct ProjParams {
     float r[9];
     float t[3];
@@ -64,6 +76,7 @@ struct ProjParams {
     // (its loads are skipped); nullptr = no partition is skipped
     const uint8_t* skip;
     uint32_t* ctl;             // control words (gs_common.h), may be null
+    BinnedOut binned;
 };
 
 // Compact (visible-only) Gaussian records, index m in [0, M).
@@ -85,7 +98,7 @@ hipError_t launch_project(const SceneDev& s, const ProjParams& p, Compact out,
 // Captured frames (HIP graphs): the k_project instance launch_project uses for
 // an SH degree, and an update of a captured k_project node's view parameters
 // in an instantiated graph (the node's other arguments are kept).
-const void* project_kernel(int sh_degree);
+const void* project_kernel(int sh_degree, bool binned);
 // The captured k_project node's scene and view arguments are s and p (its
 // argument layout is what graph_set_project_params assumes).
 bool graph_project_args_are(hipGraphNode_t node, const SceneDev& s, const ProjParams& p);
@@ -244,6 +257,12 @@ inline int sort_digit_width(int bits) {
 inline int tile_hist_cols(int tile_bits) {
     return (tile_bits > 16 ? 4 : 2) << sort_digit_width(tile_bits);
 }
+// How a frame's kept pairs leave the emission: compacted in candidate order (with
+// a look-back), every candidate slot written (dropped ones as kPairDrop), or
+// every slot written as (tile << 11 | rank), rank counting the partition's kept
+// pairs of the tile in no particular order, and their numbers as the partition's
+// row of bins (bin_words(tiles) words of two 16-bit counts).
+enum class Emit { kCompact, kSlots, kBinned };
 // Rank r's rectangle and conic are rect / cov[e * stride] with e = order[r]
 // when by_order (records in compact order, as the projection writes them),
 // else e = r (records already in rank order); pair ids are order[r] (r when
@@ -256,7 +275,21 @@ hipError_t launch_pair_emit(const float4* rect, const float4* cov, int stride, b
                             const uint32_t* m_dev, uint32_t p_pre, const uint32_t* p_pre_dev,
                             TileParams tp, uint32_t* pair_tile, uint32_t* pair_id, uint32_t cap,
                             uint64_t* lb_state, uint32_t* ticket, uint32_t* total_out,
-                            uint32_t* part_hist, int tile_bits, bool compact, hipStream_t st);
+                            uint32_t* part_hist, int tile_bits, Emit mode, hipStream_t st,
+                            uint32_t* bins = nullptr);
+constexpr int kBinnedTiles = 1 << 14;  // most tiles of a binned frame (32 KB of LDS counters)
+uint32_t bin_words(int64_t num_tiles);
+// The binned tile lists: from the emission's slots (tile and rank, compact id)
+// and bins to the pairs per tile (cleared before), the ranges and the ids of each
+// tile in (depth bits, id) order. bins: binned_scratch_words, the emission's rows
+// first; ids, deps: scratch for p_cap words each; runs: scratch for 2 *
+// emit_partitions(p_cap) words; n_runs: a cleared word.
+size_t binned_scratch_words(uint32_t p_cap, int64_t num_tiles);
+hipError_t launch_binned_lists(const uint32_t* slot, const uint32_t* slot_id, uint32_t p_cap,
+                               const uint32_t* p_pre_dev, uint32_t* bins, uint32_t* tile_count,
+                               int64_t num_tiles, const uint32_t* depth, uint32_t* ranges,
+                               uint32_t* ids, uint32_t* deps, uint32_t* runs, uint32_t* n_runs,
+                               uint32_t* sorted_ids, const uint32_t* ctl, hipStream_t st);
 hipError_t launch_tile_ranges(const uint32_t* sorted_tile, uint32_t p, const uint32_t* p_dev,
                               uint32_t* ranges, int64_t num_tiles, hipStream_t st);
 // ranges[t] = [start, end) from per-tile pair counts (an exclusive scan in tile

@@ -87,15 +87,27 @@ __device__ __forceinline__ void sh_eval(const float* __restrict__ rec, float x, 
     }
 }
 
-template <int DEG>
-__global__ __launch_bounds__(kProjThreads) void k_project(SceneDev s, ProjParams p, Compact out,
+// Tiles of a projected Gaussian's rectangle.
+__device__ __forceinline__ uint32_t rect_tiles(float x, float y, float rx, float ry,
+                                               const ProjParams& p) {
+    const Rect q = tile_rect(make_float4(x, y, rx, ry), p.tiles_x, p.tiles_y, ts_div(p.tile_size));
+    return (uint32_t)(q.x1 - q.x0 + 1) * (uint32_t)(q.y1 - q.y0 + 1);
+}
+
+// BINNED: instead of the depth sort's inputs (dvals, part_hist), the compaction
+// also scans the visible Gaussians' tile counts in compact order: offs[m], the
+// emission's owner table and the candidate total (write_binned), the two prefixes
+// packed into one look-back descriptor.
+template <int DEG, bool BINNED>
+__global__ __launch_bounds__(kProjThreads, BINNED ? 4 : 1) void k_project(SceneDev s, ProjParams p, Compact out,
                                                           uint8_t* __restrict__ valid_mask,
                                                           uint64_t* lb_state, uint32_t* ticket,
                                                           uint32_t* count_out,
                                                           uint32_t* __restrict__ part_hist) {
     __shared__ uint32_t s_vid;
     __shared__ uint32_t s_cnt[kProjItems][kProjThreads / GS_WAVE];
-    __shared__ uint32_t s_hist[4][256];
+    __shared__ uint32_t s_hist[BINNED ? 1 : 4][256];
+    __shared__ uint32_t s_ccnt[kProjItems][kProjThreads / GS_WAVE];
     __shared__ uint64_t s_excl;
     // each item's projected values, held here over the colour evaluation (in
     // registers they would leave one workgroup per CU instead of two)
@@ -104,7 +116,7 @@ __global__ __launch_bounds__(kProjThreads) void k_project(SceneDev s, ProjParams
     const int w = tid / GS_WAVE;
     const int lane = lane_id();
     if (tid == 0) s_vid = atomicAdd(ticket, 1u);
-    if (part_hist != nullptr)
+    if (!BINNED && part_hist != nullptr)
         for (int i = tid; i < 4 * 256; i += kProjThreads) (&s_hist[0][0])[i] = 0;
     __syncthreads();
     const uint32_t vid = s_vid;
@@ -118,6 +130,7 @@ __global__ __launch_bounds__(kProjThreads) void k_project(SceneDev s, ProjParams
     float va[kProjItems], vb[kProjItems], vc[kProjItems], vrx[kProjItems], vry[kProjItems];
     bool valid[kProjItems];
     uint64_t bal[kProjItems];
+    uint32_t coff[kProjItems];  // BINNED: the tile counts' prefix
 
     // loads in two stages over all items: the means and opacities, then the
     // covariance words of the items that pass the depth and opacity tests
@@ -237,7 +250,12 @@ __global__ __launch_bounds__(kProjThreads) void k_project(SceneDev s, ProjParams
         s_iv[1][it][tid] = make_float4(va[it], vb[it], vc[it], vtz[it]);
         bal[it] = __ballot(valid[it]);
         if (lane == 0) s_cnt[it][w] = (uint32_t)__popcll(bal[it]);
-        if (part_hist != nullptr) {
+        if constexpr (BINNED) {
+            const uint32_t c = valid[it] ? rect_tiles(vmx[it], vmy[it], vrx[it], vry[it], p) : 0u;
+            const uint32_t incl = wave_incl_scan(c);
+            coff[it] = incl - c;
+            if (lane == GS_WAVE - 1) s_ccnt[it][w] = incl;
+        } else if (part_hist != nullptr) {
             // digit histograms of the depth keys, for the depth sort's passes
             const uint32_t k = __float_as_uint(vtz[it]);
             hist_add_wave(s_hist[0], k & 255u, valid[it]);
@@ -247,24 +265,37 @@ __global__ __launch_bounds__(kProjThreads) void k_project(SceneDev s, ProjParams
         }
     }
     __syncthreads();
-    if (part_hist != nullptr)
+    if (!BINNED && part_hist != nullptr)
         for (int i = tid; i < 4 * 256; i += kProjThreads)
             part_hist[(size_t)vid * 1024 + i] = (&s_hist[0][0])[i];
 
-    uint32_t total = 0;
-    uint32_t my_off[kProjItems];
+    // exclusive prefixes of the (item, wave) counts in source order: lane
+    // it * waves + w of a wave scan
+    constexpr int kWaves = kProjThreads / GS_WAVE;
+    static_assert(kProjItems * kWaves <= GS_WAVE, "one count per lane");
+    uint32_t total, my_off[kProjItems];
+    uint64_t ctotal = 0;
+    {
+        const uint32_t c = lane < kProjItems * kWaves ? (&s_cnt[0][0])[lane] : 0u;
+        const uint32_t incl = wave_incl_scan(c);
+        total = (uint32_t)__builtin_amdgcn_readlane((int)incl, GS_WAVE - 1);
 #pragma unroll
-    for (int it = 0; it < kProjItems; ++it) {
+        for (int it = 0; it < kProjItems; ++it)
+            my_off[it] = (uint32_t)__builtin_amdgcn_readlane((int)(incl - c), it * kWaves + w);
+        if constexpr (BINNED) {
+            const uint32_t cc = lane < kProjItems * kWaves ? (&s_ccnt[0][0])[lane] : 0u;
+            const uint32_t ci = wave_incl_scan(cc);
+            ctotal = (uint32_t)__builtin_amdgcn_readlane((int)ci, GS_WAVE - 1);
 #pragma unroll
-        for (int ww = 0; ww < kProjThreads / GS_WAVE; ++ww) {
-            if (ww == w) my_off[it] = total;
-            total += s_cnt[it][ww];
+            for (int it = 0; it < kProjItems; ++it)
+                coff[it] += (uint32_t)__builtin_amdgcn_readlane((int)(ci - cc), it * kWaves + w);
         }
     }
+    const uint64_t agg = BINNED ? binned_pack(total, ctotal) : (uint64_t)total;
     // The partition's count goes out first; the colours of the valid items
     // (the SH records, the kernel's largest reads) are evaluated before the
     // walk over the predecessors, so that the walk finds them mostly done.
-    if (w == 0) lookback_publish(lb_state, vid, total);
+    if (w == 0) lookback_publish(lb_state, vid, agg);
     float vr[kProjItems], vg[kProjItems], vbl[kProjItems];
 #pragma unroll
     for (int it = 0; it < kProjItems; ++it) {
@@ -290,14 +321,19 @@ __global__ __launch_bounds__(kProjThreads) void k_project(SceneDev s, ProjParams
         vbl[it] = rgb[2];
     }
     if (w == 0) {
-        const uint64_t excl = lookback_walk(lb_state, vid, total, p.ctl);
+        const uint64_t excl = lookback_walk(lb_state, vid, agg, p.ctl);
         if (lane == 0) {
             s_excl = excl;
-            if (vid == gridDim.x - 1) *count_out = (uint32_t)(excl + total);
+            if (vid == gridDim.x - 1) {
+                if constexpr (BINNED)
+                    binned_totals(excl + agg, count_out, p.binned, p.ctl);
+                else
+                    *count_out = (uint32_t)(excl + agg);
+            }
         }
     }
     __syncthreads();
-    const uint64_t excl = s_excl;
+    const uint64_t excl = BINNED ? binned_count(s_excl) : s_excl;
     const uint64_t lt_mask = lanemask_lt();
 
 #pragma unroll
@@ -318,12 +354,13 @@ __global__ __launch_bounds__(kProjThreads) void k_project(SceneDev s, ProjParams
         out.rc[2 * m + 0] = make_float4(vmx[it], vmy[it], vrx[it], vry[it]);
         out.rc[2 * m + 1] = make_float4(a, b, c, s.m2thr[i]);
         out.dkey[m] = __float_as_uint(vtz[it]);
-        if (p.dvals != nullptr) {
+        if constexpr (BINNED) {
+            binned_write(p.binned, m, binned_cands(s_excl) + coff[it],
+                         rect_tiles(vmx[it], vmy[it], vrx[it], vry[it], p));
+        } else if (p.dvals != nullptr) {
             // the tile count that the candidate scan would read the rectangle for
-            const Rect q = tile_rect(make_float4(vmx[it], vmy[it], vrx[it], vry[it]), p.tiles_x,
-                                     p.tiles_y, ts_div(p.tile_size));
-            const uint32_t cnt = (uint32_t)(q.x1 - q.x0 + 1) * (uint32_t)(q.y1 - q.y0 + 1);
-            p.dvals[m] = dval_pack((uint32_t)m, cnt, p.idx_bits);
+            p.dvals[m] = dval_pack((uint32_t)m,
+                                   rect_tiles(vmx[it], vmy[it], vrx[it], vry[it], p), p.idx_bits);
         }
         // Microblock cull / blend record (cull_and_blend.cpp:723-777).
         const float det = fmax_std(a * c - b * b, 1e-6f);
@@ -492,28 +529,40 @@ hipError_t launch_project(const SceneDev& s, const ProjParams& p, Compact out,
                           uint32_t* count_out, uint32_t* part_hist, hipStream_t st) {
     if (s.n <= 0) return hipSuccess;
     const unsigned grid = (unsigned)((s.n + kProjPart - 1) / kProjPart);
+#define GS_PROJECT(D)                                                                         \
+    if (p.binned.offs != nullptr)                                                             \
+        k_project<D, true><<<grid, kProjThreads, 0, st>>>(s, p, out, valid_mask, lb_state,    \
+                                                          ticket, count_out, part_hist);      \
+    else                                                                                      \
+        k_project<D, false><<<grid, kProjThreads, 0, st>>>(s, p, out, valid_mask, lb_state,   \
+                                                           ticket, count_out, part_hist)
     switch (s.sh_degree) {
-        case -1: k_project<-1><<<grid, kProjThreads, 0, st>>>(s, p, out, valid_mask, lb_state, ticket, count_out, part_hist); break;
-        case 0: k_project<0><<<grid, kProjThreads, 0, st>>>(s, p, out, valid_mask, lb_state, ticket, count_out, part_hist); break;
-        case 1: k_project<1><<<grid, kProjThreads, 0, st>>>(s, p, out, valid_mask, lb_state, ticket, count_out, part_hist); break;
-        case 2: k_project<2><<<grid, kProjThreads, 0, st>>>(s, p, out, valid_mask, lb_state, ticket, count_out, part_hist); break;
-        case 3: k_project<3><<<grid, kProjThreads, 0, st>>>(s, p, out, valid_mask, lb_state, ticket, count_out, part_hist); break;
+        case -1: GS_PROJECT(-1); break;
+        case 0: GS_PROJECT(0); break;
+        case 1: GS_PROJECT(1); break;
+        case 2: GS_PROJECT(2); break;
+        case 3: GS_PROJECT(3); break;
         default: return hipErrorInvalidValue;
     }
+#undef GS_PROJECT
     return hipGetLastError();
 }
 
 size_t project_partitions(int64_t n) { return (size_t)((n + kProjPart - 1) / kProjPart); }
 
-const void* project_kernel(int sh_degree) {
+template <bool BINNED>
+static const void* project_instance(int sh_degree) {
     switch (sh_degree) {
-        case -1: return reinterpret_cast<const void*>(&k_project<-1>);
-        case 0: return reinterpret_cast<const void*>(&k_project<0>);
-        case 1: return reinterpret_cast<const void*>(&k_project<1>);
-        case 2: return reinterpret_cast<const void*>(&k_project<2>);
-        case 3: return reinterpret_cast<const void*>(&k_project<3>);
+        case -1: return reinterpret_cast<const void*>(&k_project<-1, BINNED>);
+        case 0: return reinterpret_cast<const void*>(&k_project<0, BINNED>);
+        case 1: return reinterpret_cast<const void*>(&k_project<1, BINNED>);
+        case 2: return reinterpret_cast<const void*>(&k_project<2, BINNED>);
+        case 3: return reinterpret_cast<const void*>(&k_project<3, BINNED>);
         default: return nullptr;
     }
+}
+const void* project_kernel(int sh_degree, bool binned) {
+    return binned ? project_instance<true>(sh_degree) : project_instance<false>(sh_degree);
 }
 
 bool graph_project_args_are(hipGraphNode_t node, const SceneDev& s, const ProjParams& p) {
@@ -524,7 +573,8 @@ bool graph_project_args_are(hipGraphNode_t node, const SceneDev& s, const ProjPa
     const ProjParams& b = *static_cast<const ProjParams*>(kp.kernelParams[1]);
     bool same = a.n == s.n && a.sh_degree == s.sh_degree && a.sh == s.sh && a.opac == s.opac &&
                 a.mean[0] == s.mean[0] && a.cov[5] == s.cov[5] && a.lthr == s.lthr &&
-                b.ctl == p.ctl && b.dvals == p.dvals && b.skip == p.skip && b.fx == p.fx &&
+                b.ctl == p.ctl && b.dvals == p.dvals && b.skip == p.skip &&
+                b.binned.offs == p.binned.offs && b.binned.cap == p.binned.cap && b.fx == p.fx &&
                 b.fy == p.fy && b.width == p.width && b.height == p.height;
     for (int j = 0; j < 9; ++j) same = same && b.r[j] == p.r[j];
     for (int j = 0; j < 3; ++j) same = same && b.t[j] == p.t[j];

@@ -30,6 +30,13 @@ constexpr int kEmitWaves = kEmitThreads / GS_WAVE;
 constexpr int kEmitPart = 2048;                      // candidates per emit partition
 constexpr int kEmitItems = kEmitPart / kEmitThreads;
 constexpr int kRankCache = 384;
+// Binned frames: rank bits of a slot (a partition's pairs of one tile, at most
+// kEmitPart - 1 before one), partitions per segment of bins (their sums stay
+// below 2^16)
+constexpr int kBinRankBits = 11;
+static_assert((1 << kBinRankBits) == kEmitPart, "a rank is below the partition's size");
+constexpr uint32_t kBinSegment = 31;
+static_assert(kBinSegment * kEmitPart < 65536, "a segment's offsets are held in 16 bits");
 static_assert(kEmitPart == (int)kEmitPartition, "emit partition size is part of the interface");
 static_assert(kEmitPart + 1 <= 65535, "a partition's ranks are held as 16-bit indices");
 
@@ -258,8 +265,12 @@ __global__ __launch_bounds__(kSumThreads) void k_scan_part_sums(uint64_t* __rest
 // pair or kPairDrop for a culled one (the pair id only for kept ones), and the
 // kept count is added to *total_out: the tile sort's first pass drops the
 // culled slots, so no partition waits on another here.
-// NDIG: tile-id digit histograms made (2, or 3 above 16 tile bits).
-template <bool COMPACT, int NDIG>
+// Binned (Emit::kBinned): the slot of a kept pair holds its tile and its rank
+// among the partition's pairs of that tile (LDS counters, two 16-bit ones a word;
+// the order of the ranks does not matter, the lists are sorted after), and the
+// counters become the partition's row of bins.
+// NDIG: tile-id digit histograms made (2, or 3 above 16 tile bits; none binned).
+template <Emit MODE, int NDIG>
 __global__ __launch_bounds__(kEmitThreads) void k_pair_emit(
     const float4* __restrict__ rect, const float4* __restrict__ cov, int stride,
     bool by_order, const uint32_t* __restrict__ order, const uint32_t* __restrict__ offs,
@@ -267,7 +278,10 @@ __global__ __launch_bounds__(kEmitThreads) void k_pair_emit(
     uint32_t p_pre_cap, const uint32_t* __restrict__ p_pre_dev, TileParams tp,
     uint32_t* __restrict__ pair_tile, uint32_t* __restrict__ pair_id, uint32_t cap,
     uint64_t* lb_state, uint32_t* ticket, uint32_t* total_out,
-    uint32_t* __restrict__ part_hist, int dig_bits) {
+    uint32_t* __restrict__ part_hist, int dig_bits, uint32_t* __restrict__ bins,
+    uint32_t bin_words) {
+    extern __shared__ uint32_t s_bin[];  // bin_words counters (binned)
+    constexpr bool COMPACT = MODE == Emit::kCompact, BINNED = MODE == Emit::kBinned;
     __shared__ uint32_t s_vid;
     __shared__ uint32_t s_off[kEmitPart + 1];
     __shared__ uint32_t s_xy[kEmitPart + 1];
@@ -279,7 +293,7 @@ __global__ __launch_bounds__(kEmitThreads) void k_pair_emit(
     __shared__ float4 s_cv[kRankCache];
     __shared__ uint32_t s_wmax[kEmitWaves];
     __shared__ uint32_t s_cnt[kEmitItems][kEmitWaves];
-    __shared__ uint32_t s_th[NDIG][256];
+    __shared__ uint32_t s_th[BINNED ? 1 : NDIG][256];
     __shared__ uint64_t s_excl;
     const int tid = threadIdx.x, w = tid / GS_WAVE, lane = lane_id();
     // The counts and this partition's rank bounds, loaded together (every
@@ -301,7 +315,9 @@ __global__ __launch_bounds__(kEmitThreads) void k_pair_emit(
         s_vid = failed ? 0xFFFFFFFFu : (COMPACT ? atomicAdd(ticket, 1u) : blockIdx.x);
     }
     for (int i = tid; i < kEmitPart; i += kEmitThreads) s_own[i] = 0;
-    if (part_hist != nullptr)
+    if constexpr (BINNED)
+        for (uint32_t i = tid; i < bin_words; i += kEmitThreads) s_bin[i] = 0;
+    else if (part_hist != nullptr)
         for (int i = tid; i < NDIG * 256; i += kEmitThreads) (&s_th[0][0])[i] = 0;
     __syncthreads();
     const uint32_t vid = s_vid;
@@ -425,11 +441,20 @@ __global__ __launch_bounds__(kEmitThreads) void k_pair_emit(
     }
     // bookkeeping after all candidates are evaluated, so the evaluations of the
     // candidates of one thread can overlap
+    uint32_t trank[kEmitItems];
+    if constexpr (BINNED) {
+#pragma unroll
+        for (int it = 0; it < kEmitItems; ++it)
+            if (keep[it]) {
+                const uint32_t sh = 16u * (tile[it] & 1u);
+                trank[it] = (atomicAdd(&s_bin[tile[it] >> 1], 1u << sh) >> sh) & 0xFFFFu;
+            }
+    }
 #pragma unroll
     for (int it = 0; it < kEmitItems; ++it) {
         bal[it] = __ballot(keep[it]);
         if (lane == 0) s_cnt[it][w] = (uint32_t)__popcll(bal[it]);
-        if (part_hist != nullptr && keep[it]) {
+        if (!BINNED && part_hist != nullptr && keep[it]) {
             // digit histograms of the tile keys, for the tile sort's passes: a
             // partition's kept tiles spread over the digits, so one LDS atomic
             // per lane (no aggregation of equal digits)
@@ -442,7 +467,7 @@ __global__ __launch_bounds__(kEmitThreads) void k_pair_emit(
     for (int it = 0; it < kEmitItems; ++it)
         gid[it] = order != nullptr ? dval_index(gid[it], tp.idx_bits) : (uint32_t)(rlo + lo[it]);
     __syncthreads();
-    if (part_hist != nullptr) {
+    if (!BINNED && part_hist != nullptr) {
         // the row holds digit q's 2^dig_bits counts at [q << dig_bits], then zeros
         // up to tile_hist_cols(tile bits) words
         const int cols = (NDIG == 2 ? 2 : 4) << dig_bits;
@@ -450,12 +475,16 @@ __global__ __launch_bounds__(kEmitThreads) void k_pair_emit(
         for (int i = tid; i < cols; i += kEmitThreads)
             part_hist[(size_t)vid * cols + i] = (i >> dig_bits) < NDIG ? s_th[i >> dig_bits][i & dm] : 0u;
     }
+    if constexpr (BINNED)
+        for (uint32_t i = tid; i < bin_words; i += kEmitThreads)
+            bins[(size_t)vid * bin_words + i] = s_bin[i];
     if (!COMPACT) {
 #pragma unroll
         for (int it = 0; it < kEmitItems; ++it) {
             const uint64_t c = c0 + it * kEmitThreads + tid;
             if (c < c1 && c < cap) {
-                pair_tile[c] = keep[it] ? tile[it] : kPairDrop;
+                const uint32_t t = BINNED ? (tile[it] << kBinRankBits) | trank[it] : tile[it];
+                pair_tile[c] = keep[it] ? t : kPairDrop;
                 if (keep[it]) pair_id[c] = gid[it];
             }
         }
@@ -728,6 +757,268 @@ __global__ __launch_bounds__(kRangeThreads) void k_ranges_from_counts(
     }
 }
 
+// ---------------------------------------------------------------------------
+// Binned tile lists. Frames of small scenes have their pairs counted per tile by
+// the emission and put into the tiles' lists in any order; each list is then
+// sorted by (depth bits, compact id) in LDS. This replaces the depth sort, the
+// count scan and the tile sort (twelve launches whose workgroups fill a part of
+// the chip each) by five launches.
+// ---------------------------------------------------------------------------
+
+// Ranges as k_ranges_from_counts, and the runs (kRun pairs) of the tiles with
+// more than one: runs[] = tile << 16 | index, *n_runs of them (any order).
+constexpr int kRunThreads = 256;
+constexpr int kRunItems = 8;  // keys per thread
+constexpr uint32_t kRun = kRunThreads * kRunItems;
+__global__ __launch_bounds__(kRangeThreads) void k_binned_ranges(
+    const uint32_t* __restrict__ counts, uint32_t ntiles, uint32_t* __restrict__ ranges,
+    uint32_t* __restrict__ runs, uint32_t* n_runs) {
+    __shared__ uint32_t s_w[kRangeThreads / GS_WAVE];
+    const int tid = threadIdx.x, w = tid / GS_WAVE, lane = lane_id();
+    const uint32_t per = (ntiles + kRangeThreads - 1) / kRangeThreads;
+    const uint32_t t0 = min(ntiles, (uint32_t)tid * per), t1 = min(ntiles, t0 + per);
+    uint32_t sum = 0;
+    for (uint32_t t = t0; t < t1; ++t) sum += counts[t];
+    const uint32_t inc = wave_incl_scan(sum);
+    if (lane == GS_WAVE - 1) s_w[w] = inc;
+    __syncthreads();
+    uint32_t pre = 0;
+    for (int i = 0; i < w; ++i) pre += s_w[i];
+    uint32_t start = pre + inc - sum;
+    for (uint32_t t = t0; t < t1; ++t) {
+        const uint32_t c = counts[t];
+        ranges[2 * (size_t)t] = c ? start : 0u;
+        ranges[2 * (size_t)t + 1] = c ? start + c : 0u;
+        start += c;
+        if (c > kRun) {
+            const uint32_t k = (c + kRun - 1) / kRun;
+            const uint32_t at = atomicAdd(n_runs, k);
+            for (uint32_t i = 0; i < k; ++i) runs[at + i] = (t << 16) | i;
+        }
+    }
+}
+
+// Bins of kBinSegment partitions turned into exclusive offsets within the segment
+// (in place, 16 bits: 31 * 2048 pairs at most), and the segment's counts added to
+// the pairs per tile, the sum before giving the segment's base. One thread per
+// word of two tiles; a tile's counter gains one atomic per segment (an atomic per
+// pair serialised on the counters: the emission of the 100K view went from 10 to
+// 62 us).
+__global__ __launch_bounds__(256) void k_binned_offsets(
+    uint32_t* __restrict__ bins, uint32_t words, uint32_t p_cap,
+    const uint32_t* __restrict__ p_pre_dev, uint32_t* __restrict__ tile_count,
+    uint32_t* __restrict__ seg_base, const uint32_t* ctl) {
+    if (upstream_failed(ctl)) return;
+    const uint32_t p = min(p_cap, *p_pre_dev);
+    const uint32_t parts = (p + kEmitPart - 1) / kEmitPart;
+    const uint32_t p0 = blockIdx.y * kBinSegment;
+    const uint32_t w = blockIdx.x * 256 + threadIdx.x;
+    if (p0 >= parts || w >= words) return;
+    uint32_t v[kBinSegment];
+#pragma unroll
+    for (uint32_t i = 0; i < kBinSegment; ++i)
+        v[i] = p0 + i < parts ? bins[(size_t)(p0 + i) * words + w] : 0u;
+    uint32_t run = 0;  // two 16-bit sums
+#pragma unroll
+    for (uint32_t i = 0; i < kBinSegment; ++i) {
+        if (p0 + i < parts) bins[(size_t)(p0 + i) * words + w] = run;
+        run += v[i];
+    }
+    uint2 base = make_uint2(0u, 0u);
+    if (run & 0xFFFFu) base.x = atomicAdd(&tile_count[2 * w], run & 0xFFFFu);
+    if (run >> 16) base.y = atomicAdd(&tile_count[2 * w + 1], run >> 16);
+    reinterpret_cast<uint2*>(seg_base)[(size_t)blockIdx.y * words + w] = base;
+}
+
+// Each kept slot's id to its place in its tile's list.
+__global__ __launch_bounds__(256) void k_binned_scatter(
+    const uint32_t* __restrict__ slot, const uint32_t* __restrict__ slot_id, uint32_t p_cap,
+    const uint32_t* __restrict__ p_pre_dev, const uint32_t* __restrict__ bins, uint32_t words,
+    const uint32_t* __restrict__ seg_base, const uint32_t* __restrict__ ranges,
+    uint32_t* __restrict__ ids, const uint32_t* ctl) {
+    if (upstream_failed(ctl)) return;
+    const uint32_t p = min(p_cap, *p_pre_dev);
+    for (uint32_t c = blockIdx.x * 256 + threadIdx.x; c < p; c += gridDim.x * 256) {
+        const uint32_t v = slot[c];
+        if (v == kPairDrop) continue;
+        const uint32_t part = c / kEmitPart, tile = v >> kBinRankBits;
+        const uint32_t off = (bins[(size_t)part * words + (tile >> 1)] >> (16u * (tile & 1u))) & 0xFFFFu;
+        const uint32_t base = seg_base[(size_t)(part / kBinSegment) * 2 * words + tile];
+        ids[ranges[2 * (size_t)tile] + base + off + (v & ((1u << kBinRankBits) - 1u))] = slot_id[c];
+    }
+}
+
+__device__ __forceinline__ void order2(uint64_t& a, uint64_t& b) {
+    const bool s = b < a;
+    const uint64_t lo = s ? b : a, hi = s ? a : b;
+    a = lo;
+    b = hi;
+}
+// Batcher's odd-even merge network on eight keys (19 comparisons).
+__device__ __forceinline__ void sort8(uint64_t (&k)[8]) {
+    constexpr int net[19][2] = {{0, 1}, {2, 3}, {4, 5}, {6, 7}, {0, 2}, {1, 3}, {4, 6},
+                                {5, 7}, {1, 2}, {5, 6}, {0, 4}, {1, 5}, {2, 6}, {3, 7},
+                                {2, 4}, {3, 5}, {1, 2}, {3, 4}, {5, 6}};
+#pragma unroll
+    for (int i = 0; i < 19; ++i) order2(k[net[i][0]], k[net[i][1]]);
+}
+
+// Sorts one run of at most kRun pairs of a tile by (depth bits, id): each thread
+// sorts eight keys in registers, then the threads' runs are merged in LDS, two by
+// two, every thread finding by a search along its diagonal where its eight
+// outputs start in the two inputs (log2 of the list length rounds; a list of at
+// most 512 is one wave's work). Bound by LDS latency, so many lists share a CU:
+// 18 KB of LDS each, with one key of padding per eight against bank conflicts.
+// Workgroup b < ntiles: the list of tile b when it is one run, ids to sorted;
+// the others take the runs of longer lists in turn, sorted in place in ids, their
+// depths to deps, for k_binned_merge.
+__global__ __launch_bounds__(kRunThreads) void k_binned_sort(
+    const uint32_t* __restrict__ ranges, uint32_t ntiles, const uint32_t* __restrict__ depth,
+    uint32_t* __restrict__ ids, uint32_t* __restrict__ deps, const uint32_t* __restrict__ runs,
+    const uint32_t* __restrict__ n_runs, uint32_t* __restrict__ sorted, const uint32_t* ctl) {
+    __shared__ uint64_t s_key[kRun + kRun / 8];
+    if (upstream_failed(ctl)) return;
+    const int tid = threadIdx.x;
+    const auto at = [](uint32_t i) { return i + (i >> 3); };
+    const bool whole = blockIdx.x < ntiles;
+    const uint32_t step = gridDim.x - ntiles;
+    for (uint32_t e = whole ? 0u : blockIdx.x - ntiles;; e += step) {
+        uint32_t tile = blockIdx.x, first = 0;
+        if (!whole) {
+            if (e >= *n_runs) return;
+            tile = runs[e] >> 16;
+            first = (runs[e] & 0xFFFFu) * kRun;
+        }
+        const uint32_t start = ranges[2 * (size_t)tile] + first, end = ranges[2 * (size_t)tile + 1];
+        uint32_t n = end - start;
+        if (whole && (n == 0 || n > kRun)) return;
+        n = min(n, kRun);
+        const uint32_t n8 = (n + 7u) & ~7u;
+        for (uint32_t i = tid; i < n8; i += kRunThreads) {
+            uint64_t k = ~0ull;  // after every key
+            if (i < n) {
+                const uint32_t id = ids[start + i];
+                k = ((uint64_t)depth[id] << 32) | id;
+            }
+            s_key[at(i)] = k;
+        }
+        __syncthreads();
+        const uint32_t o = (uint32_t)tid * kRunItems;  // this thread's outputs [o, o + 8)
+        const bool on = o < n8;
+        uint64_t k[8];
+        if (on) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) k[i] = s_key[at(o + i)];
+            sort8(k);
+        }
+#pragma unroll 1
+        for (uint32_t len = kRunItems; len < n8; len *= 2) {
+            __syncthreads();
+            if (on) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) s_key[at(o + i)] = k[i];
+            }
+            __syncthreads();
+            if (on) {
+                const uint32_t base = o & ~(2 * len - 1);
+                const uint32_t a1 = min(base + len, n8), b1 = min(base + 2 * len, n8);
+                const uint32_t na = a1 - base, nb = b1 - a1, diag = o - base;
+                // how many of the first diag outputs come from the first input
+                uint32_t lo = diag > nb ? diag - nb : 0u, hi = min(diag, na);
+#pragma unroll 1
+                while (lo < hi) {
+                    const uint32_t mid = (lo + hi) / 2;
+                    if (s_key[at(base + mid)] < s_key[at(a1 + diag - 1 - mid)]) lo = mid + 1;
+                    else hi = mid;
+                }
+                uint32_t ia = base + lo, ib = a1 + diag - lo;
+                uint64_t ka = ia < a1 ? s_key[at(ia)] : ~0ull;
+                uint64_t kb = ib < b1 ? s_key[at(ib)] : ~0ull;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    // (a spent input reads as the padding key, which equals the padding)
+                    const bool b = kb < ka;
+                    k[i] = b ? kb : ka;
+                    const uint32_t next = b ? ++ib : ++ia;
+                    const uint64_t v = s_key[at(min(next, n8 - 1))];
+                    const uint64_t got = next < (b ? b1 : a1) ? v : ~0ull;
+                    ka = b ? ka : got;
+                    kb = b ? got : kb;
+                }
+            }
+        }
+        __syncthreads();
+        if (on) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) s_key[at(o + i)] = k[i];
+        }
+        __syncthreads();
+        for (uint32_t i = tid; i < n; i += kRunThreads) {
+            const uint64_t v = s_key[at(i)];
+            if (whole) {
+                sorted[start + i] = (uint32_t)v;
+            } else {
+                ids[start + i] = (uint32_t)v;
+                deps[start + i] = (uint32_t)(v >> 32);
+            }
+        }
+        if (whole) return;
+        __syncthreads();  // the next run overwrites the keys
+    }
+}
+
+// Lists of several sorted runs: a pair's place is its place in its own run plus,
+// for each of the other runs, the number of pairs before it there. A workgroup
+// takes a run, keeps its keys in registers and searches the list's other runs
+// one after the other in LDS (a search in memory, one key after the other, took
+// 178 us for the lists of 13K pairs of a 300x200 view); keys are distinct.
+__global__ __launch_bounds__(kRunThreads) void k_binned_merge(
+    const uint32_t* __restrict__ ranges, const uint32_t* __restrict__ ids,
+    const uint32_t* __restrict__ deps, const uint32_t* __restrict__ runs,
+    const uint32_t* __restrict__ n_runs, uint32_t* __restrict__ sorted, const uint32_t* ctl) {
+    __shared__ uint64_t s_key[kRun];
+    if (upstream_failed(ctl)) return;
+    const int tid = threadIdx.x;
+    const uint32_t total = *n_runs;
+    for (uint32_t e = blockIdx.x; e < total; e += gridDim.x) {
+        const uint32_t tile = runs[e] >> 16, mine = runs[e] & 0xFFFFu;
+        const uint32_t start = ranges[2 * (size_t)tile], end = ranges[2 * (size_t)tile + 1];
+        const uint32_t first = start + mine * kRun, n = min(end - first, kRun);
+        uint64_t k[kRunItems];
+        uint32_t rank[kRunItems];
+#pragma unroll
+        for (int j = 0; j < kRunItems; ++j) {
+            const uint32_t i = tid + j * kRunThreads;
+            rank[j] = i;
+            k[j] = i < n ? ((uint64_t)deps[first + i] << 32) | ids[first + i] : 0ull;
+        }
+        for (uint32_t r0 = start; r0 < end; r0 += kRun) {
+            if (r0 == first) continue;
+            const uint32_t m = min(end - r0, kRun);
+            __syncthreads();  // the searches of the run before are done
+            for (uint32_t i = tid; i < m; i += kRunThreads)
+                s_key[i] = ((uint64_t)deps[r0 + i] << 32) | ids[r0 + i];
+            __syncthreads();
+            // the keys' searches step together: eight reads in flight
+            uint32_t lo[kRunItems];
+#pragma unroll
+            for (int j = 0; j < kRunItems; ++j) lo[j] = 0;
+            for (uint32_t half = kRun; half > 0; half /= 2) {
+#pragma unroll
+                for (int j = 0; j < kRunItems; ++j) {
+                    const uint32_t at = lo[j] + half;
+                    if (at <= m && s_key[at - 1] < k[j]) lo[j] = at;
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < kRunItems; ++j) rank[j] += lo[j];
+        }
+#pragma unroll
+        for (int j = 0; j < kRunItems; ++j)
+            if (tid + j * kRunThreads < n) sorted[start + rank[j]] = (uint32_t)k[j];
+    }
+}
+
 // key = (tile << 32) | fp32 depth bits of the pair's Gaussian (sort.cpp:180-205).
 __global__ void k_make_keys64(const uint32_t* __restrict__ gid, const uint32_t* __restrict__ tid,
                               const float* __restrict__ depths, uint32_t p,
@@ -796,7 +1087,8 @@ hipError_t launch_pair_emit(const float4* rect, const float4* cov, int stride, b
                             const uint32_t* m_dev, uint32_t p_pre, const uint32_t* p_pre_dev,
                             TileParams tp, uint32_t* pair_tile, uint32_t* pair_id, uint32_t cap,
                             uint64_t* lb_state, uint32_t* ticket, uint32_t* total_out,
-                            uint32_t* part_hist, int tile_bits, bool compact, hipStream_t st) {
+                            uint32_t* part_hist, int tile_bits, Emit mode, hipStream_t st,
+                            uint32_t* bins) {
     if (p_pre == 0 || m <= 0) return hipSuccess;
     if (stride < 1 || (by_order && order == nullptr)) return hipErrorInvalidValue;
     const unsigned grid = (unsigned)emit_partitions(p_pre);
@@ -807,17 +1099,55 @@ hipError_t launch_pair_emit(const float4* rect, const float4* cov, int stride, b
         return hipErrorInvalidValue;
     const int dbits = sort_digit_width(tile_bits);
     const bool three = tile_bits > 16;
+    const uint32_t bw = mode == Emit::kBinned ? bin_words((int64_t)tp.tiles_x * tp.tiles_y) : 0u;
 #define GS_EMIT(CP, ND)                                                                    \
-    k_pair_emit<CP, ND><<<grid, kEmitThreads, 0, st>>>(                                    \
+    k_pair_emit<CP, ND><<<grid, kEmitThreads, bw * 4, st>>>(                                    \
         rect, cov, stride, by_order, order, offs, bstart, m, m_dev, p_pre, p_pre_dev, tp,    \
         pair_tile, pair_id,                                                                \
-        cap, lb_state, ticket, total_out, part_hist, dbits)
-    if (compact) {
-        if (three) GS_EMIT(true, 3); else GS_EMIT(true, 2);
-    } else {
-        if (three) GS_EMIT(false, 3); else GS_EMIT(false, 2);
+        cap, lb_state, ticket, total_out, part_hist, dbits, bins, bw)
+    switch (mode) {
+        case Emit::kCompact:
+            if (three) GS_EMIT(Emit::kCompact, 3); else GS_EMIT(Emit::kCompact, 2);
+            break;
+        case Emit::kSlots:
+            if (three) GS_EMIT(Emit::kSlots, 3); else GS_EMIT(Emit::kSlots, 2);
+            break;
+        case Emit::kBinned:
+            if (bins == nullptr || (1 << tile_bits) > kBinnedTiles) return hipErrorInvalidValue;
+            GS_EMIT(Emit::kBinned, 2);
+            break;
     }
 #undef GS_EMIT
+    return hipGetLastError();
+}
+
+uint32_t bin_words(int64_t num_tiles) { return ((uint32_t)num_tiles + 7u) / 8u * 4u; }
+size_t binned_scratch_words(uint32_t p_cap, int64_t num_tiles) {
+    const size_t parts = emit_partitions(p_cap), segs = (parts + kBinSegment - 1) / kBinSegment;
+    return (parts + 2 * segs) * bin_words(num_tiles);
+}
+
+hipError_t launch_binned_lists(const uint32_t* slot, const uint32_t* slot_id, uint32_t p_cap,
+                               const uint32_t* p_pre_dev, uint32_t* bins, uint32_t* tile_count,
+                               int64_t num_tiles, const uint32_t* depth, uint32_t* ranges,
+                               uint32_t* ids, uint32_t* deps, uint32_t* runs, uint32_t* n_runs,
+                               uint32_t* sorted_ids, const uint32_t* ctl, hipStream_t st) {
+    if (num_tiles <= 0 || p_cap == 0) return hipSuccess;
+    if (num_tiles > kBinnedTiles) return hipErrorInvalidValue;
+    const uint32_t T = (uint32_t)num_tiles, words = bin_words(T);
+    const uint32_t parts = (uint32_t)emit_partitions(p_cap);
+    uint32_t* seg_base = bins + (size_t)parts * words;
+    const dim3 og((words + 255) / 256, (parts + kBinSegment - 1) / kBinSegment);
+    k_binned_offsets<<<og, 256, 0, st>>>(bins, words, p_cap, p_pre_dev, tile_count, seg_base, ctl);
+    k_binned_ranges<<<1, kRangeThreads, 0, st>>>(tile_count, T, ranges, runs, n_runs);
+    // persistent grids: the real counts are on the device
+    const unsigned sg = std::max(1u, std::min(1024u, (p_cap + 255) / 256));
+    k_binned_scatter<<<sg, 256, 0, st>>>(slot, slot_id, p_cap, p_pre_dev, bins, words, seg_base,
+                                         ranges, ids, ctl);
+    const unsigned long_runs = std::max(1u, std::min(512u, 2 * (p_cap / kRun)));
+    k_binned_sort<<<T + long_runs, kRunThreads, 0, st>>>(ranges, T, depth, ids, deps, runs,
+                                                         n_runs, sorted_ids, ctl);
+    k_binned_merge<<<long_runs, kRunThreads, 0, st>>>(ranges, ids, deps, runs, n_runs, sorted_ids, ctl);
     return hipGetLastError();
 }
 

@@ -1,0 +1,107 @@
+"""The two ways a frame's tile lists are made: binned (pairs counted per tile, each
+list sorted on its own in runs of 2048) and sorted (depth sort, then tile sort; the
+microblock statistics select it). Both give the stable (tile, depth bits, compact id)
+order, so ids, ranges, counts and images are compared for equality, at list lengths
+around the runs of the list sort, with equal depths, empty views and many tiles."""
+import numpy as np
+import pytest
+
+from gsplat_tt_amd import _lib as L
+from gsplat_tt_amd import scenes
+
+pytestmark = pytest.mark.gpu
+
+
+def _both(ctx, view):
+    """(image, stats, readback) of the view, binned then sorted."""
+    out = []
+    for stats in (False, True):
+        ctx.set_cull_stats(stats)
+        img, st = ctx.render(view)
+        out.append((img, st, ctx.frame_readback() if st["num_visible"] else None))
+    ctx.set_cull_stats(False)
+    return out
+
+
+def _equal(a, b):
+    assert np.array_equal(a[0], b[0])
+    for k in ("num_visible", "num_entries", "pairs_pre"):
+        assert a[1][k] == b[1][k], k
+    if a[2] is not None:
+        assert np.array_equal(a[2]["tile_ranges"], b[2]["tile_ranges"])
+        assert np.array_equal(a[2]["sorted_ids"], b[2]["sorted_ids"])
+
+
+def _stack(n, levels, spread=0.004, seed=0):
+    """n small Gaussians in one column at z of a few levels (many equal depths)."""
+    rng = np.random.default_rng(seed)
+    z = (2.0 + rng.integers(0, levels, n) / 64.0).astype(np.float32)
+    means = np.stack([rng.normal(0, spread, n) * z, rng.normal(0, spread, n) * z, z], 1)
+    q = rng.standard_normal((n, 4))
+    q /= np.linalg.norm(q, axis=1, keepdims=True)
+    cov = scenes.cov3d(np.full((n, 3), 0.004, np.float32), q.astype(np.float32))
+    return (means.astype(np.float32), cov, rng.uniform(0.05, 0.6, n).astype(np.float32),
+            rng.random((n, 3)).astype(np.float32))
+
+
+@pytest.mark.parametrize("n,levels", [(1, 1), (7, 2), (8, 1), (9, 3), (64, 2), (513, 5),
+                                      (2047, 40), (2048, 1), (2049, 7), (4097, 500), (9000, 3)])
+def test_lists_around_the_runs(gpu_ctx, n, levels):
+    print("lists", n, levels, flush=True)
+    gpu_ctx.set_scene(*_stack(n, levels, seed=n))
+    for ts, h, w in ((16, 48, 64), (32, 35, 61)):
+        K = scenes.intrinsics(60, 60, w / 2, h / 2)
+        view = L.make_view(np.eye(4, dtype=np.float32), K, h, w, tile_size=ts, output="f32")
+        a, b = _both(gpu_ctx, view)
+        if n == 9000:
+            r = a[2]["tile_ranges"]
+            assert (r[:, 1] - r[:, 0]).max() > 4096  # a list of several runs
+        _equal(a, b)
+
+
+def test_many_tiles_and_empty_views(gpu_ctx):
+    """Close to the most tiles of a binned frame (127 x 129 = 16383 of 16384), one row of
+    tiles past it (sorted either way), and a view with nothing visible."""
+    print("many tiles", flush=True)
+    scene, cams = scenes.config1(seed=5, n=6_000)
+    cov = scenes.cov3d(scene.scales, scene.quats)
+    gpu_ctx.set_scene(scene.means, cov, scene.opacities, scene.colors)
+    for h, w in ((127 * 16, 129 * 16 - 3), (130 * 16 - 15, 129 * 16)):
+        K = scenes.intrinsics(500 * w / 640, 500 * w / 640, w / 2, h / 2)
+        view = L.make_view(cams[0].w2c, K, h, w, tile_size=16, output="bf16")
+        _equal(*_both(gpu_ctx, view))
+    back = np.diag([-1, 1, -1, 1]).astype(np.float32)
+    view = L.make_view(back, cams[0].K, 100, 120, tile_size=16, output="f32")
+    a, b = _both(gpu_ctx, view)
+    assert a[1]["num_visible"] == b[1]["num_visible"] == 0 and not a[0].any() and not b[0].any()
+
+
+def test_plan_follows_the_pairs():
+    """A scene whose view has more pairs than binning pays for goes on sorted, one with
+    fewer binned again: every frame of the change equals the sorted one."""
+    print("plan", flush=True)
+    scene, cams = scenes.config3(seed=17, n=700_000, views=3)
+    cov = scenes.cov3d(scene.scales, scene.quats)
+    ctx = L.Context(0)
+    try:
+        ctx.set_scene(scene.means, cov, scene.opacities, scene.sh, sh_degree=3)
+        near = [L.make_view(c.w2c, c.K, c.height, c.width, tile_size=16, output="bf16")
+                for c in cams]
+        far_w2c = cams[0].w2c.copy()
+        far_w2c[2, 3] += 60.0  # small on screen: few pairs
+        far = L.make_view(far_w2c, cams[0].K, cams[0].height, cams[0].width, tile_size=16,
+                          output="bf16")
+        pairs = []
+        for view in (near[0], near[1], far, far, near[2], far):
+            a, st = ctx.render(view)
+            rb = ctx.frame_readback()
+            pairs.append(st["num_entries"])
+            _equal((a, st, rb), _both(ctx, view)[1])
+        assert max(pairs) > 2_400_000 and min(pairs) < 1_800_000, pairs
+        outs = [np.empty((822, 1237, 3), np.uint16) for _ in range(6)]
+        views = [near[0], far, near[1], far, near[2], far]
+        ctx.render_batch(views, outs, out_on_device=False)
+        for v, o in zip(views, outs):
+            assert np.array_equal(o, _both(ctx, v)[1][0])
+    finally:
+        ctx.close()

@@ -573,7 +573,9 @@ struct gs_ctx {
 
     // --------------------------------------------------------- render
     // Frame-scratch layout (u32 words): counters, then what FrameLayout points at.
-    static constexpr size_t kFrCnt = 0;  // 64 counters (below)
+    static constexpr size_t kSumBytes = gs::kTrainSumSlots * sizeof(gs::TrainSums);
+    static constexpr size_t kFrCnt = 0;    // 64 counters (below)
+    static constexpr size_t kFrSums = 64;  // a training forward's TrainSums
     enum : int {
         C_PROJ_TICKET = 0, C_M = 1, C_SKIPPED = 2, C_CTL = 4, C_RECT_TICKET = 8, C_PPRE = 9,
         C_EMIT_TICKET = 10, C_P = 11, C_RUNS = 12, C_DSORT_TICKETS = 16, C_TSORT_TICKETS = 24,
@@ -678,7 +680,8 @@ struct gs_ctx {
         if (!graph_frame()) frame(&pend.v, pend.dout, pend.T, pend.tiles_x, pend.tiles_y);
         if (!pend.out_dev)
             HIPCHK(hipMemcpyAsync(pend.out, pend.dout, pend.bytes, hipMemcpyDeviceToHost, st));
-        HIPCHK(hipMemcpyAsync(h_pin, b_frame.p, 64 * 4, hipMemcpyDeviceToHost, st));
+        if (cull_stats)  // counted after the ranges, which report the counters otherwise
+            HIPCHK(hipMemcpyAsync(h_pin, b_frame.p, 64 * 4, hipMemcpyDeviceToHost, st));
         if (blend_counts)
             HIPCHK(hipMemcpyAsync(h_evals.data(), b_evals.p, 64 * 8 * 8, hipMemcpyDeviceToHost, st));
     }
@@ -1055,6 +1058,7 @@ struct gs_ctx {
     struct FrameLayout {
         uint32_t* fr;
         uint32_t* cnt;
+        gs::TrainSums* sums;  // a training forward's, after the counters
         uint64_t *lb_proj, *lb_rect, *lb_emit;
         uint32_t* tcnt;  // pairs per tile
         uint32_t *hist_depth, *hist_tile;  // [4][256] depth-key, [2 or 4][256] tile-id digits
@@ -1124,7 +1128,7 @@ struct gs_ctx {
         // cleared by every frame: counters, compaction states, pairs per tile; by the
         // sorted ones also the histograms and the other states
         const size_t tile_words = ((size_t)T + 1) & ~size_t(1);
-        const size_t binned_words = 64 + 2 * L.pparts + tile_words;
+        const size_t binned_words = kFrSums + kSumBytes / 4 + 2 * L.pparts + tile_words;
         const size_t all_words = binned_words + 2048 + 2 * (L.rparts + L.eparts);
         b_frame.ensure(all_words * 4);
         L.fwords = L.binned ? binned_words : all_words;
@@ -1132,8 +1136,9 @@ struct gs_ctx {
         if (blend_counts) b_evals.ensure(64 * 8 * 8);
         L.fr = b_frame.as<uint32_t>();
         L.cnt = L.fr + kFrCnt;
-        L.lb_proj = reinterpret_cast<uint64_t*>(L.fr + 64);
-        L.tcnt = L.fr + 64 + 2 * L.pparts;
+        L.sums = reinterpret_cast<gs::TrainSums*>(L.fr + kFrSums);
+        L.lb_proj = reinterpret_cast<uint64_t*>(L.fr + kFrSums + kSumBytes / 4);
+        L.tcnt = reinterpret_cast<uint32_t*>(L.lb_proj + L.pparts);
         L.hist_depth = L.tcnt + tile_words;
         L.hist_tile = L.hist_depth + 1024;
         L.lb_rect = reinterpret_cast<uint64_t*>(L.hist_tile + 1024);
@@ -1146,14 +1151,15 @@ struct gs_ctx {
     // cnt[C_M], depth-key histograms reduced) to the tile-sorted compact ids and
     // tile ranges: depth sort, candidate scan, pair emission + cull, tile sort,
     // tile bounds. Returns the sorted compact ids.
+    // report: copied to the host once the counters are final (not with tiles_out).
     uint32_t* frame_tiles(const FrameLayout& L, int64_t N, int64_t T, const gs::TileParams& tp,
-                          uint32_t** tiles_out) {
+                          uint32_t** tiles_out, const gs::HostCopy& report) {
         // without a caller for the tile-sorted keys, the tile sort's last pass
         // counts the pairs per tile instead of writing them, and the ranges come
         // from the counts
         const bool want_keys = tiles_out != nullptr;
         uint32_t* cnt = L.cnt;
-        if (L.binned) return binned_tiles(L, N, T, tp);
+        if (L.binned) return binned_tiles(L, N, T, tp, report);
         sort.ctl = cnt + C_CTL;
         // depth order of the visible Gaussians (stable: ties keep index order)
         // (values: the projection's packed ones when tp.idx_bits is set, else
@@ -1203,14 +1209,15 @@ struct gs_ctx {
                                           b_ranges.as<uint32_t>(), T, st));
             *tiles_out = static_cast<uint32_t*>(tiles_sorted);
         } else {
-            HIPCHK(gs::launch_ranges_from_counts(L.tcnt, T, b_ranges.as<uint32_t>(), st));
+            HIPCHK(gs::launch_ranges_from_counts(L.tcnt, T, b_ranges.as<uint32_t>(), st, report));
         }
         return ids_sorted;
     }
 
     // frame_tiles of a binned frame, whose projection scanned the candidates:
     // pair emission in compact order, then the tiles' lists sorted one by one.
-    uint32_t* binned_tiles(const FrameLayout& L, int64_t N, int64_t T, const gs::TileParams& tp) {
+    uint32_t* binned_tiles(const FrameLayout& L, int64_t N, int64_t T, const gs::TileParams& tp,
+                           const gs::HostCopy& report) {
         uint32_t* cnt = L.cnt;
         record(2);  // no depth sort of its own
         HIPCHK(gs::launch_pair_emit(b_rc.as<float4>(), b_rc.as<float4>() + 1, 2, false, nullptr,
@@ -1224,7 +1231,7 @@ struct gs_ctx {
                                        L.pcap, cnt + C_PPRE, b_bins.as<uint32_t>(), L.tcnt, T,
                                        b_dkey.as<uint32_t>(), b_ranges.as<uint32_t>(),
                                        b_valt.as<uint32_t>(), b_kalt.as<uint32_t>(), L.runs,
-                                       cnt + C_RUNS, b_pair_id.as<uint32_t>(), L.cnt + C_CTL, st));
+                                       cnt + C_RUNS, b_pair_id.as<uint32_t>(), cnt + C_CTL, report, st));
         return b_pair_id.as<uint32_t>();
     }
     gs::BinnedOut binned_out(const FrameLayout& L) const {
@@ -1469,7 +1476,8 @@ struct gs_ctx {
         gs::TileParams tp{tiles_x, tiles_y, v->tile_size, v->cull_disabled ? 0 : 1,
                           L.cnt + C_CTL, p.idx_bits};
         uint32_t* tiles_sorted = nullptr;
-        uint32_t* ids_sorted = frame_tiles(L, N, T, tp, cull_stats ? &tiles_sorted : nullptr);
+        uint32_t* ids_sorted = frame_tiles(L, N, T, tp, cull_stats ? &tiles_sorted : nullptr,
+                                           gs::HostCopy{h_pin, L.cnt, 64});
         record(4);
         gs::BlendParams bp{tiles_x, tiles_y, v->tile_size, v->image_height, v->image_width,
                            v->cull_disabled ? 1 : 0, v->transmittance_threshold, v->out_format,
@@ -1650,8 +1658,7 @@ struct gs_ctx {
                 "train: lambda_dssim must be in [0, 1]");
     }
 
-    // The groups of partial sums of a forward and its loss (t_loss), added up.
-    static constexpr size_t kSumBytes = gs::kTrainSumSlots * sizeof(gs::TrainSums);
+    // The groups of partial sums of a forward and its loss, added up.
     static gs::TrainSums add_sums(const void* p) {
         gs::TrainSums t{}, v;
         for (int k = 0; k < gs::kTrainSumSlots; ++k) {
@@ -1686,8 +1693,9 @@ struct gs_ctx {
     }
 
     // Enqueues projection, tiles and the forward (+ L1 with a device target).
+    // step: the backward follows on the stream (its accumulators are cleared here).
     void train_forward_enqueue(const gs_view* v, const gs_train_cfg* c, const float* tgt_dev,
-                               const gs::TrainDebug& dbg) {
+                               const gs::TrainDebug& dbg, bool step) {
         const int64_t N = tr.n;
         const int H = v->image_height, W = v->image_width;
         tr.H = H;
@@ -1696,13 +1704,12 @@ struct gs_ctx {
         tr.tiles_y = (H + 15) / 16;
         const int64_t T = (int64_t)tr.tiles_x * tr.tiles_y;
         tr.cam = train_cam(v, c);
-        const FrameLayout L = frame_prepare(std::max<int64_t>(N, 1), T, true);
+        const FrameLayout L = frame_prepare(std::max<int64_t>(N, 1), T, false);
         const size_t px = (size_t)H * W;
         t_img.ensure(px * 12);
         t_T.ensure(px * 4);
         t_stop.ensure(px * 4);
         t_dimg.ensure(px * 12);
-        t_loss.ensure(kSumBytes);
         if (timing)
             for (auto& e : tev)
                 if (!e) HIPCHK(hipEventCreate(&e));
@@ -1710,18 +1717,25 @@ struct gs_ctx {
         HIPCHK(gs::launch_fill_u32(L.fr, 0u, L.fwords, st));
         if (spin_limit) HIPCHK(gs::launch_fill_u32(L.cnt + C_CTL + 1, spin_limit, 1, st));
         tr.cam.ctl = L.cnt + C_CTL;
-        HIPCHK(gs::launch_fill_u32(t_loss.as<uint32_t>(), 0u, kSumBytes / 4, st));
+        tr.cam.tiles_x = tr.tiles_x;
+        tr.cam.tiles_y = tr.tiles_y;
+        tr.cam.binned = binned_out(L);
+        if (step) {
+            t_grad2d.ensure((size_t)std::max<int64_t>(N, 1) * 36);
+            tr.cam.grad2d = t_grad2d.as<float>();
+        }
         gs::Compact cpt{b_rc.as<float4>(), b_dkey.as<uint32_t>(),
                         nullptr, b_src.as<uint32_t>()};
         HIPCHK(gs::launch_train_project(train_rows(), tr.cam, cpt, b_brec.as<float4>(),
                                         t_cidx.as<uint32_t>(), t_vis.as<uint8_t>(), L.lb_proj,
                                         L.cnt + C_PROJ_TICKET, L.cnt + C_M,
                                         b_phist_proj.as<uint32_t>(), dbg, st));
-        HIPCHK(gs::launch_reduce_rows(b_phist_proj.as<uint32_t>(), 1024, (uint32_t)L.pparts,
-                                      nullptr, 0, 0, 0, L.hist_depth, st, nullptr,
-                                      L.cnt + C_CTL));
+        if (!L.binned)
+            HIPCHK(gs::launch_reduce_rows(b_phist_proj.as<uint32_t>(), 1024, (uint32_t)L.pparts,
+                                          nullptr, 0, 0, 0, L.hist_depth, st, nullptr,
+                                          L.cnt + C_CTL));
         gs::TileParams tp{tr.tiles_x, tr.tiles_y, 16, 1, L.cnt + C_CTL};
-        tr.ids = frame_tiles(L, std::max<int64_t>(N, 1), T, tp, nullptr);
+        tr.ids = frame_tiles(L, std::max<int64_t>(N, 1), T, tp, nullptr, gs::HostCopy{});
         gs::TrainFwdParams fp{};
         fp.tiles_x = tr.tiles_x;
         fp.tiles_y = tr.tiles_y;
@@ -1738,18 +1752,20 @@ struct gs_ctx {
         fp.dimage = t_dimg.as<float>();
         fp.grad_scale = (float)((double)c->loss_scale * (1.0 - (double)c->lambda_dssim) /
                                 (3.0 * (double)px));
-        fp.sums = t_loss.as<gs::TrainSums>();
+        fp.sums = L.sums;
         fp.ctl = L.cnt + C_CTL;
         HIPCHK(gs::launch_train_fwd(b_brec.as<float4>(), tr.ids, b_ranges.as<uint32_t>(), fp, st));
         if (tgt_dev != nullptr && c->lambda_dssim > 0.0f)
             enqueue_ssim(t_img.as<float>(), tgt_dev, H, W, c->lambda_dssim, c->loss_scale,
-                         t_dimg.as<float>(), t_loss.as<gs::TrainSums>());
+                         t_dimg.as<float>(), L.sums);
         if (timing) HIPCHK(hipEventRecord(tev[1], st));
     }
 
-    // Forward with the pair-capacity retry; one host synchronisation.
+    // Forward with the pair-capacity retry - with step, the whole step: backward and
+    // sparse Adam are enqueued behind it, and their kernels do nothing when the
+    // forward failed or did not fit. One host synchronisation per attempt.
     void train_forward(const gs_view* v, const gs_train_cfg* c, const float* target,
-                       bool target_dev, const gs::TrainDebug& dbg) {
+                       bool target_dev, const gs::TrainDebug& dbg, bool step) {
         const size_t px = (size_t)v->image_height * v->image_width;
         const float* tgt = nullptr;
         if (target != nullptr) {
@@ -1766,10 +1782,13 @@ struct gs_ctx {
         tr.grads_valid = false;
         rb_valid = false;
         if (pair_cap == 0) pair_cap = default_pair_cap(tr.n);
+        constexpr size_t kReport = kFrSums + kSumBytes / 4;
         for (int attempt = 0;; ++attempt) {
-            train_forward_enqueue(v, c, tgt, dbg);
-            HIPCHK(hipMemcpyAsync(h_pin, b_frame.p, 64 * 4, hipMemcpyDeviceToHost, st));
-            HIPCHK(hipMemcpyAsync(h_pin + 64, t_loss.p, kSumBytes, hipMemcpyDeviceToHost, st));
+            train_forward_enqueue(v, c, tgt, dbg, step);
+            if (step) train_backward_enqueue(c, true, gs::HostCopy{h_pin, b_frame.as<uint32_t>(),
+                                                                   (uint32_t)kReport});
+            if (!step || tr.n == 0)  // the last kernel of a step reports otherwise
+                HIPCHK(hipMemcpyAsync(h_pin, b_frame.p, kReport * 4, hipMemcpyDeviceToHost, st));
             sync();
             // The capacity test comes first: an attempt past the capacity has
             // kErrCapacity raised by the count scan, and is re-run (its fill
@@ -1784,10 +1803,12 @@ struct gs_ctx {
             REQUIRE(attempt == 0, "train: pair capacity did not converge");
             pair_cap = std::min<uint64_t>(0xFFFFFFFFull, (uint64_t)p_pre + p_pre / 8 + 4096);
         }
+        if (step) ++tr.step;
         tr.M = h_pin[C_M];
         tr.p_pre = h_pin[C_PPRE];
         tr.P = h_pin[C_P];
-        const gs::TrainSums sum = add_sums(h_pin + 64);
+        plan_seen(std::max<int64_t>(tr.n, 1), (int64_t)tr.tiles_x * tr.tiles_y, tr.P);
+        const gs::TrainSums sum = add_sums(h_pin + kFrSums);
         tr.pixel_pairs = (int64_t)sum.considered;
         tr.pixel_blended = (int64_t)sum.blended;
         const double lam = c->lambda_dssim;
@@ -1801,10 +1822,8 @@ struct gs_ctx {
 
     // Enqueues the blend backward and the gradients of the parameters (in t_g);
     // with adam, the sparse Adam of the step in the same pass.
-    void train_backward_enqueue(const gs_train_cfg* c, bool adam) {
-        t_grad2d.ensure((size_t)std::max<uint32_t>(tr.M, 1) * 36);
+    void train_backward_enqueue(const gs_train_cfg* c, bool adam, const gs::HostCopy& report) {
         if (timing) HIPCHK(hipEventRecord(tev[2], st));
-        HIPCHK(gs::launch_fill_u32(t_grad2d.as<uint32_t>(), 0u, (size_t)tr.M * 9, st));
         gs::TrainBwdParams bp{};
         bp.tiles_x = tr.tiles_x;
         bp.tiles_y = tr.tiles_y;
@@ -1817,8 +1836,8 @@ struct gs_ctx {
         bp.stop = t_stop.as<uint32_t>();
         bp.dimage = t_dimg.as<float>();
         bp.grad2d = t_grad2d.as<float>();
-        if (tr.M > 0 && tr.P > 0)
-            HIPCHK(gs::launch_train_bwd(b_brec.as<float4>(), tr.ids, b_ranges.as<uint32_t>(), bp, st));
+        bp.ctl = tr.cam.ctl;
+        HIPCHK(gs::launch_train_bwd(b_brec.as<float4>(), tr.ids, b_ranges.as<uint32_t>(), bp, st));
         // the device time of a step's Adam is part of its gradient pass
         if (timing && adam) HIPCHK(hipEventRecord(tev[3], st));
         if (timing && adam) HIPCHK(hipEventRecord(tev[4], st));
@@ -1826,9 +1845,8 @@ struct gs_ctx {
         HIPCHK(gs::launch_train_grads(train_rows(), tr.cam, t_cidx.as<uint32_t>(),
                                       t_grad2d.as<float>(), t_g.as<float4>(), t_gnz.as<uint8_t>(),
                                       t_m.p, t_v.p, t_vis.as<uint8_t>(), adam ? &ap : nullptr,
-                                      t_bf16_mom, st));
+                                      t_bf16_mom, report, st));
         if (timing) HIPCHK(hipEventRecord(tev[adam ? 5 : 3], st));
-        if (adam) ++tr.step;
     }
 
     gs::AdamParams adam_params(const gs_train_cfg* c) const {
@@ -2629,7 +2647,7 @@ int gs_train_forward(gs_ctx* ctx, const gs_view* view, const gs_train_cfg* cfg,
             dbg.depth = f + 9 * nn;
             dbg.valid = reinterpret_cast<uint8_t*>(f + 10 * nn);
         }
-        ctx->train_forward(view, cfg, target, false, dbg);
+        ctx->train_forward(view, cfg, target, false, dbg, false);
         const size_t px = (size_t)view->image_height * view->image_width;
         if (image) HIPCHK(hipMemcpyAsync(image, ctx->t_img.p, px * 12, hipMemcpyDeviceToHost, ctx->st));
         if (final_T) HIPCHK(hipMemcpyAsync(final_T, ctx->t_T.p, px * 4, hipMemcpyDeviceToHost, ctx->st));
@@ -2662,7 +2680,10 @@ int gs_train_backward(gs_ctx* ctx, const gs_train_cfg* cfg, const float* dimage,
         const size_t px = (size_t)ctx->tr.H * ctx->tr.W;
         if (dimage)
             HIPCHK(hipMemcpyAsync(ctx->t_dimg.p, dimage, px * 12, hipMemcpyHostToDevice, ctx->st));
-        ctx->train_backward_enqueue(cfg, false);
+        ctx->t_grad2d.ensure((size_t)std::max<uint32_t>(ctx->tr.M, 1) * 36);
+        HIPCHK(gs::launch_fill_u32(ctx->t_grad2d.as<uint32_t>(), 0u, (size_t)ctx->tr.M * 9,
+                                   ctx->st));
+        ctx->train_backward_enqueue(cfg, false, gs::HostCopy{});
         if (g2d != nullptr) {
             const int64_t n = ctx->tr.n;
             const uint32_t M = ctx->tr.M;
@@ -2710,9 +2731,7 @@ int gs_train_step(gs_ctx* ctx, const gs_view* view, const gs_train_cfg* cfg, con
         HIPCHK(hipSetDevice(ctx->device));
         ctx->drain_spec();
         ctx->train_check(view, cfg);
-        ctx->train_forward(view, cfg, target, target_on_device != 0, gs::TrainDebug{});
-        ctx->train_backward_enqueue(cfg, true);
-        ctx->sync();
+        ctx->train_forward(view, cfg, target, target_on_device != 0, gs::TrainDebug{}, true);
         ctx->tr.fwd_valid = false;
         ctx->tr.grads_valid = false;
         ctx->train_stats(stats, true, true, true, t0);

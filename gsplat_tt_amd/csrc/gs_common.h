@@ -241,6 +241,21 @@ __device__ __forceinline__ uint64_t lookback_exclusive(uint64_t* state, uint32_t
     return lookback_walk(state, vid, aggregate, ctl);
 }
 
+// Tiles of a projected Gaussian's rectangle.
+__device__ __forceinline__ uint32_t rect_tiles(float x, float y, float rx, float ry, int tiles_x,
+                                               int tiles_y, int tile_size) {
+    const Rect q = tile_rect(make_float4(x, y, rx, ry), tiles_x, tiles_y, ts_div(tile_size));
+    return (uint32_t)(q.x1 - q.x0 + 1) * (uint32_t)(q.y1 - q.y0 + 1);
+}
+
+// One workgroup's copy of a few words to pinned host memory, which the host reads
+// once it has waited for the stream: a frame or a step ends without a copy of
+// its own (4 us and a gap).
+__device__ __forceinline__ void host_copy(const HostCopy& c, uint32_t tid, uint32_t threads) {
+    for (uint32_t i = tid; i < c.words; i += threads)
+        __hip_atomic_store(&c.dst[i], c.src[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // ---------------------------------------------------------------------------
 // Binned frames: the compaction's look-back carries the visible count and the
 // candidate total together (count above bit 34, candidates below: a binned

@@ -44,6 +44,13 @@ struct SceneDev {
     double chunk_k = 1.5;
 };
 
+// Words that a kernel copies to pinned host memory (words 0: none).
+struct HostCopy {
+    uint32_t* dst = nullptr;
+    const uint32_t* src = nullptr;
+    uint32_t words = 0;
+};
+
 // Outputs of a binned frame's projection (all null otherwise): exclusive scan of
 // the tile counts in compact order, the compact id owning candidate b *
 // kEmitPartition (b < bstart_cap), the candidate total, and the capacity that it
@@ -283,19 +290,22 @@ uint32_t bin_words(int64_t num_tiles);
 // and bins to the pairs per tile (cleared before), the ranges and the ids of each
 // tile in (depth bits, id) order. bins: binned_scratch_words, the emission's rows
 // first; ids, deps: scratch for p_cap words each; runs: scratch for 2 *
-// emit_partitions(p_cap) words; n_runs: a cleared word.
+// emit_partitions(p_cap) words; n_runs: a cleared word; report: the frame's
+// counters, final by then.
 size_t binned_scratch_words(uint32_t p_cap, int64_t num_tiles);
 hipError_t launch_binned_lists(const uint32_t* slot, const uint32_t* slot_id, uint32_t p_cap,
                                const uint32_t* p_pre_dev, uint32_t* bins, uint32_t* tile_count,
                                int64_t num_tiles, const uint32_t* depth, uint32_t* ranges,
                                uint32_t* ids, uint32_t* deps, uint32_t* runs, uint32_t* n_runs,
-                               uint32_t* sorted_ids, const uint32_t* ctl, hipStream_t st);
+                               uint32_t* sorted_ids, const uint32_t* ctl, const HostCopy& report,
+                               hipStream_t st);
 hipError_t launch_tile_ranges(const uint32_t* sorted_tile, uint32_t p, const uint32_t* p_dev,
                               uint32_t* ranges, int64_t num_tiles, hipStream_t st);
 // ranges[t] = [start, end) from per-tile pair counts (an exclusive scan in tile
 // order; (0, 0) for an empty tile), one workgroup.
+// report: the frame's counters, final by then.
 hipError_t launch_ranges_from_counts(const uint32_t* counts, int64_t num_tiles, uint32_t* ranges,
-                                     hipStream_t st);
+                                     hipStream_t st, const HostCopy& report = HostCopy{});
 // Same ranges by per-tile binary search over the sorted tile keys (reads
 // O(tiles * log p) keys instead of all p; no clearing pass).
 hipError_t launch_tile_bounds(const uint32_t* sorted_tile, uint32_t p_cap, const uint32_t* p_dev,
@@ -389,7 +399,10 @@ struct TrainCam {
     float ccx, ccy, ccz;       // camera centre -R^T t
     float near, lowpass, alpha_min;
     int H, W;
+    int tiles_x, tiles_y;      // 16-pixel tiles
     uint32_t* ctl;             // control words (gs_common.h), may be null
+    BinnedOut binned;
+    float* grad2d;             // rows of 9 that the projection clears (a step), may be null
 };
 
 // Optional Gaussian-indexed copies of the projection values (parity tests).
@@ -451,6 +464,7 @@ struct TrainBwdParams {
     const float* final_T;
     const uint32_t* stop;
     const float* dimage;
+    const uint32_t* ctl;   // control words of the forward (nothing is read after an error)
     float* grad2d;         // (M,9) per compact Gaussian: dmx dmy dA dB dC dop dr dg db
 };
 
@@ -474,12 +488,13 @@ hipError_t launch_train_bwd(const float4* trec, const uint32_t* sid, const uint3
 // Gradients (G rows) of every Gaussian from its accumulated 2D gradients; gnz[i]
 // marks the rows of G that are not zero (kept from call to call, so that rows
 // that stay zero are not written again). With adam (optional), the sparse Adam
-// of the visible rows in the same pass, as launch_sparse_adam.
+// of the visible rows in the same pass, as launch_sparse_adam. Nothing is read or
+// written after an error in cam.ctl; report is copied either way.
 // m, v: float rows, or rows of bf16 bits (uint16_t) with bf16_moments.
 hipError_t launch_train_grads(const TrainParamsDev& P, const TrainCam& cam, const uint32_t* cidx,
                               const float* grad2d, float4* G, uint8_t* gnz, void* m, void* v,
                               const uint8_t* visible, const AdamParams* adam, bool bf16_moments,
-                              hipStream_t st);
+                              const HostCopy& report, hipStream_t st);
 hipError_t launch_sparse_adam(const TrainParamsDev& P, void* m, void* v, const float4* G,
                               const uint8_t* visible, const AdamParams& ap, bool bf16_moments,
                               hipStream_t st);

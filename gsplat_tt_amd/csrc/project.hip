@@ -87,13 +87,6 @@ __device__ __forceinline__ void sh_eval(const float* __restrict__ rec, float x, 
     }
 }
 
-// Tiles of a projected Gaussian's rectangle.
-__device__ __forceinline__ uint32_t rect_tiles(float x, float y, float rx, float ry,
-                                               const ProjParams& p) {
-    const Rect q = tile_rect(make_float4(x, y, rx, ry), p.tiles_x, p.tiles_y, ts_div(p.tile_size));
-    return (uint32_t)(q.x1 - q.x0 + 1) * (uint32_t)(q.y1 - q.y0 + 1);
-}
-
 // BINNED: instead of the depth sort's inputs (dvals, part_hist), the compaction
 // also scans the visible Gaussians' tile counts in compact order: offs[m], the
 // emission's owner table and the candidate total (write_binned), the two prefixes
@@ -251,7 +244,8 @@ __global__ __launch_bounds__(kProjThreads, BINNED ? 4 : 1) void k_project(SceneD
         bal[it] = __ballot(valid[it]);
         if (lane == 0) s_cnt[it][w] = (uint32_t)__popcll(bal[it]);
         if constexpr (BINNED) {
-            const uint32_t c = valid[it] ? rect_tiles(vmx[it], vmy[it], vrx[it], vry[it], p) : 0u;
+            const uint32_t c = valid[it] ? rect_tiles(vmx[it], vmy[it], vrx[it], vry[it], p.tiles_x,
+                                                        p.tiles_y, p.tile_size) : 0u;
             const uint32_t incl = wave_incl_scan(c);
             coff[it] = incl - c;
             if (lane == GS_WAVE - 1) s_ccnt[it][w] = incl;
@@ -356,11 +350,13 @@ __global__ __launch_bounds__(kProjThreads, BINNED ? 4 : 1) void k_project(SceneD
         out.dkey[m] = __float_as_uint(vtz[it]);
         if constexpr (BINNED) {
             binned_write(p.binned, m, binned_cands(s_excl) + coff[it],
-                         rect_tiles(vmx[it], vmy[it], vrx[it], vry[it], p));
+                         rect_tiles(vmx[it], vmy[it], vrx[it], vry[it], p.tiles_x,
+                                                        p.tiles_y, p.tile_size));
         } else if (p.dvals != nullptr) {
             // the tile count that the candidate scan would read the rectangle for
             p.dvals[m] = dval_pack((uint32_t)m,
-                                   rect_tiles(vmx[it], vmy[it], vrx[it], vry[it], p), p.idx_bits);
+                                   rect_tiles(vmx[it], vmy[it], vrx[it], vry[it], p.tiles_x,
+                                                        p.tiles_y, p.tile_size), p.idx_bits);
         }
         // Microblock cull / blend record (cull_and_blend.cpp:723-777).
         const float det = fmax_std(a * c - b * b, 1e-6f);

@@ -736,8 +736,10 @@ __global__ __launch_bounds__(kOffsThreads) void k_part_offsets(
 // writes its tiles' [start, end) (sort.cpp:146-165: (0, 0) for an empty tile).
 constexpr int kRangeThreads = 1024;
 __global__ __launch_bounds__(kRangeThreads) void k_ranges_from_counts(
-    const uint32_t* __restrict__ counts, uint32_t ntiles, uint32_t* __restrict__ ranges) {
+    const uint32_t* __restrict__ counts, uint32_t ntiles, uint32_t* __restrict__ ranges,
+    HostCopy report) {
     __shared__ uint32_t s_w[kRangeThreads / GS_WAVE];
+    host_copy(report, threadIdx.x, kRangeThreads);
     const int tid = threadIdx.x, w = tid / GS_WAVE, lane = lane_id();
     const uint32_t per = (ntiles + kRangeThreads - 1) / kRangeThreads;
     const uint32_t t0 = min(ntiles, (uint32_t)tid * per), t1 = min(ntiles, t0 + per);
@@ -772,8 +774,9 @@ constexpr int kRunItems = 8;  // keys per thread
 constexpr uint32_t kRun = kRunThreads * kRunItems;
 __global__ __launch_bounds__(kRangeThreads) void k_binned_ranges(
     const uint32_t* __restrict__ counts, uint32_t ntiles, uint32_t* __restrict__ ranges,
-    uint32_t* __restrict__ runs, uint32_t* n_runs) {
+    uint32_t* __restrict__ runs, uint32_t* n_runs, HostCopy report) {
     __shared__ uint32_t s_w[kRangeThreads / GS_WAVE];
+    host_copy(report, threadIdx.x, kRangeThreads);
     const int tid = threadIdx.x, w = tid / GS_WAVE, lane = lane_id();
     const uint32_t per = (ntiles + kRangeThreads - 1) / kRangeThreads;
     const uint32_t t0 = min(ntiles, (uint32_t)tid * per), t1 = min(ntiles, t0 + per);
@@ -1131,7 +1134,8 @@ hipError_t launch_binned_lists(const uint32_t* slot, const uint32_t* slot_id, ui
                                const uint32_t* p_pre_dev, uint32_t* bins, uint32_t* tile_count,
                                int64_t num_tiles, const uint32_t* depth, uint32_t* ranges,
                                uint32_t* ids, uint32_t* deps, uint32_t* runs, uint32_t* n_runs,
-                               uint32_t* sorted_ids, const uint32_t* ctl, hipStream_t st) {
+                               uint32_t* sorted_ids, const uint32_t* ctl, const HostCopy& report,
+                               hipStream_t st) {
     if (num_tiles <= 0 || p_cap == 0) return hipSuccess;
     if (num_tiles > kBinnedTiles) return hipErrorInvalidValue;
     const uint32_t T = (uint32_t)num_tiles, words = bin_words(T);
@@ -1139,7 +1143,7 @@ hipError_t launch_binned_lists(const uint32_t* slot, const uint32_t* slot_id, ui
     uint32_t* seg_base = bins + (size_t)parts * words;
     const dim3 og((words + 255) / 256, (parts + kBinSegment - 1) / kBinSegment);
     k_binned_offsets<<<og, 256, 0, st>>>(bins, words, p_cap, p_pre_dev, tile_count, seg_base, ctl);
-    k_binned_ranges<<<1, kRangeThreads, 0, st>>>(tile_count, T, ranges, runs, n_runs);
+    k_binned_ranges<<<1, kRangeThreads, 0, st>>>(tile_count, T, ranges, runs, n_runs, report);
     // persistent grids: the real counts are on the device
     const unsigned sg = std::max(1u, std::min(1024u, (p_cap + 255) / 256));
     k_binned_scatter<<<sg, 256, 0, st>>>(slot, slot_id, p_cap, p_pre_dev, bins, words, seg_base,
@@ -1161,10 +1165,10 @@ hipError_t launch_tile_ranges(const uint32_t* sorted_tile, uint32_t p, const uin
 }
 
 hipError_t launch_ranges_from_counts(const uint32_t* counts, int64_t num_tiles, uint32_t* ranges,
-                                     hipStream_t st) {
+                                     hipStream_t st, const HostCopy& report) {
     if (num_tiles <= 0) return hipSuccess;
     if (num_tiles > ((int64_t)1 << 24)) return hipErrorInvalidValue;
-    k_ranges_from_counts<<<1, kRangeThreads, 0, st>>>(counts, (uint32_t)num_tiles, ranges);
+    k_ranges_from_counts<<<1, kRangeThreads, 0, st>>>(counts, (uint32_t)num_tiles, ranges, report);
     return hipGetLastError();
 }
 

@@ -193,154 +193,202 @@ __device__ __forceinline__ void geometry(const Head& h, const TrainCam& cam, Geo
     g.C = g.a / det;
 }
 
+// SH colour + 0.5 of a row's Gaussian; the coefficients are read as they are used.
 template <int DEG>
-__device__ __forceinline__ void colour(const Head& h, const float* sh, const TrainCam& cam,
+__device__ __forceinline__ void colour(const Head& h, const float4* row, const TrainCam& cam,
                                        float* raw, float* dir, float& dnorm) {
-    constexpr int K = Row<DEG>::K;
     const float dx = h.a.x - cam.ccx, dy = h.a.y - cam.ccy, dz = h.a.z - cam.ccz;
     dnorm = sqrtf(dx * dx + dy * dy + dz * dz);
     dir[0] = dx / dnorm; dir[1] = dy / dnorm; dir[2] = dz / dnorm;
     float b[16];
     sh_basis<DEG, false>(dir[0], dir[1], dir[2], b, nullptr);
+    float acc[3] = {0.0f, 0.0f, 0.0f};
+    acc[0] += b[0] * h.c.w;
 #pragma unroll
-    for (int ch = 0; ch < 3; ++ch) {
-        float acc = 0.0f;
+    for (int q = 3; q < Row<DEG>::V; ++q) {
+        const float4 f = row[q];
+        const float t[4] = {f.x, f.y, f.z, f.w};
 #pragma unroll
-        for (int k = 0; k < K; ++k) acc += b[k] * sh[3 * k + ch];
-        raw[ch] = acc + 0.5f;
+        for (int e = 0; e < 4; ++e) {
+            const int j = 4 * (q - 3) + 1 + e;  // SH value 3k + channel
+            if (j < 3 * Row<DEG>::K) acc[j % 3] += b[j / 3] * t[e];
+        }
     }
+#pragma unroll
+    for (int ch = 0; ch < 3; ++ch) raw[ch] = acc[ch] + 0.5f;
 }
 
 __device__ __forceinline__ float sigmoidf(float x) { return 1.0f / (1.0f + expf(-x)); }
 
 // Projection of the optimizer-space parameters; stable compaction of the
-// Gaussians that can reach alpha_min somewhere in the image.
-template <int DEG>
-__global__ __launch_bounds__(kTThreads) void k_train_project(
+// Gaussians that can reach alpha_min somewhere in the image. As the render's
+// projection: the geometry of a thread's four rows first, held in LDS (in
+// registers, with the colours, it left one workgroup on a CU), the partition's
+// count published, then the colours of the kept rows, which are the largest
+// reads, then the walk over the predecessors. BINNED as there.
+// (1M Gaussians, SH1: 48.5 -> 40.3 us; with the tile counts' scan.)
+template <int DEG, bool BINNED>
+__global__ __launch_bounds__(kTThreads, 4) void k_train_project(
     TrainParamsDev P, TrainCam cam, Compact out, float4* __restrict__ trec,
     uint32_t* __restrict__ cidx, uint8_t* __restrict__ visible, uint64_t* lb_state,
     uint32_t* ticket, uint32_t* count_out, uint32_t* __restrict__ part_hist, TrainDebug dbg) {
+    constexpr int V = Row<DEG>::V, kWaves = kTThreads / GS_WAVE;
     __shared__ uint32_t s_vid;
-    __shared__ uint32_t s_cnt[kTItems][kTThreads / GS_WAVE];
-    __shared__ uint32_t s_hist[4][256];
+    __shared__ uint32_t s_cnt[kTItems][kWaves], s_ccnt[kTItems][kWaves];
+    __shared__ uint32_t s_hist[BINNED ? 1 : 4][256];
+    __shared__ float4 s_iv[2][kTItems][kTThreads];
     __shared__ uint64_t s_excl;
     const int tid = threadIdx.x, w = tid / GS_WAVE, lane = lane_id();
     if (tid == 0) s_vid = atomicAdd(ticket, 1u);
-    for (int k = tid; k < 1024; k += kTThreads) (&s_hist[0][0])[k] = 0;
+    if (!BINNED)
+        for (int k = tid; k < 1024; k += kTThreads) (&s_hist[0][0])[k] = 0;
     __syncthreads();
     const uint32_t vid = s_vid;
     const int64_t base = (int64_t)vid * kTPart;
     const int64_t n = P.n;
     bool keep[kTItems];
-    float4 rect[kTItems], cov[kTItems], r0[kTItems], r1[kTItems], r2[kTItems];
-    float depth[kTItems];
+    float ops[kTItems], m2[kTItems];
+    uint32_t coff[kTItems];
     uint64_t bal[kTItems];
     // the heads of a thread's rows together (past the end: the last row's)
     Head head[kTItems];
 #pragma unroll
     for (int it = 0; it < kTItems; ++it)
-        head[it] = load_head(P.rows + min(base + it * kTThreads + tid, n - 1) * Row<DEG>::V);
+        head[it] = load_head(P.rows + min(base + it * kTThreads + tid, n - 1) * V);
 #pragma unroll
     for (int it = 0; it < kTItems; ++it) {
         const int64_t i = base + it * kTThreads + tid;
-        keep[it] = false;
-        depth[it] = 0.0f;
+        Geo g;
+        geometry(head[it], cam, g);
+        const float op = sigmoidf(head[it].c.z);
+        // sparse-Adam rows: 3-sigma box overlaps the image (train_oracle.py:175-181)
+        const float rx3 = ceilf(3.0f * sqrtf(fmaxf(g.a, 0.0f)));
+        const float ry3 = ceilf(3.0f * sqrtf(fmaxf(g.c, 0.0f)));
+        const bool vis = g.valid && (g.u + rx3 > 0.0f) && (g.u - rx3 < (float)cam.W) &&
+                         (g.v + ry3 > 0.0f) && (g.v - ry3 < (float)cam.H);
+        // blendable: alpha = op exp(power) >= alpha_min somewhere in the image
+        bool k = i < n && g.valid && op >= cam.alpha_min && g.a * g.c - g.b * g.b > 0.0f;
+        float m2thr = 0.0f, rx = 0.0f, ry = 0.0f;
+        if (k) {
+            m2thr = 2.0f * logf(op / cam.alpha_min);
+            const float kk = sqrtf(m2thr);
+            rx = ceilf(kk * sqrtf(fmaxf(g.a, 0.0f)));
+            ry = ceilf(kk * sqrtf(fmaxf(g.c, 0.0f)));
+            k = rx > 0.0f && ry > 0.0f && (g.u + rx > 0.0f) && (g.u - rx < (float)cam.W) &&
+                (g.v + ry > 0.0f) && (g.v - ry < (float)cam.H);
+        }
+        keep[it] = k;
+        ops[it] = op;
+        m2[it] = m2thr;
         if (i < n) {
-            Geo g;
-            geometry(head[it], cam, g);
-            const float op = sigmoidf(head[it].c.z);
-            // sparse-Adam rows: 3-sigma box overlaps the image (train_oracle.py:175-181)
-            const float rx3 = ceilf(3.0f * sqrtf(fmaxf(g.a, 0.0f)));
-            const float ry3 = ceilf(3.0f * sqrtf(fmaxf(g.c, 0.0f)));
-            const bool vis = g.valid && (g.u + rx3 > 0.0f) && (g.u - rx3 < (float)cam.W) &&
-                             (g.v + ry3 > 0.0f) && (g.v - ry3 < (float)cam.H);
             visible[i] = vis ? 1 : 0;
-            // blendable: alpha = op exp(power) >= alpha_min somewhere in the image
-            bool k = g.valid && op >= cam.alpha_min && g.a * g.c - g.b * g.b > 0.0f;
-            float m2thr = 0.0f, rx = 0.0f, ry = 0.0f;
-            if (k) {
-                m2thr = 2.0f * logf(op / cam.alpha_min);
-                const float kk = sqrtf(m2thr);
-                rx = ceilf(kk * sqrtf(fmaxf(g.a, 0.0f)));
-                ry = ceilf(kk * sqrtf(fmaxf(g.c, 0.0f)));
-                k = rx > 0.0f && ry > 0.0f && (g.u + rx > 0.0f) && (g.u - rx < (float)cam.W) &&
-                    (g.v + ry > 0.0f) && (g.v - ry < (float)cam.H);
-            }
-            keep[it] = k;
-            // the colour of the rest is needed by the parity outputs only
-            float raw[3] = {0.0f, 0.0f, 0.0f};
-            if (k || dbg.means2d != nullptr) {
-                float sh[3 * Row<DEG>::K], dir[3], dn;
-                load_sh<DEG>(P.rows + i * Row<DEG>::V, head[it], sh);
-                colour<DEG>(head[it], sh, cam, raw, dir, dn);
-            }
-            const float col[3] = {raw[0] < 0.0f ? 0.0f : raw[0], raw[1] < 0.0f ? 0.0f : raw[1],
-                                  raw[2] < 0.0f ? 0.0f : raw[2]};
-            rect[it] = make_float4(g.u, g.v, rx, ry);
-            cov[it] = make_float4(g.a, g.b, g.c, m2thr);
-            r0[it] = make_float4(g.u, g.v, op, m2thr);
-            r1[it] = make_float4(g.A, g.B, g.C, 0.0f);
-            r2[it] = make_float4(col[0], col[1], col[2], 0.0f);
-            depth[it] = g.z;
-            if (dbg.means2d != nullptr) {
+            if (!k) cidx[i] = 0xFFFFFFFFu;
+            if (dbg.means2d != nullptr) {  // parity outputs, the colours of all
+                float raw[3], dir[3], dn;
+                colour<DEG>(head[it], P.rows + i * V, cam, raw, dir, dn);
                 dbg.means2d[2 * i] = g.u;
                 dbg.means2d[2 * i + 1] = g.v;
                 dbg.conic[3 * i] = g.A;
                 dbg.conic[3 * i + 1] = g.B;
                 dbg.conic[3 * i + 2] = g.C;
                 dbg.opacity[i] = op;
-                dbg.colors[3 * i] = col[0];
-                dbg.colors[3 * i + 1] = col[1];
-                dbg.colors[3 * i + 2] = col[2];
+                for (int ch = 0; ch < 3; ++ch)
+                    dbg.colors[3 * i + ch] = raw[ch] < 0.0f ? 0.0f : raw[ch];
                 dbg.depth[i] = g.z;
                 dbg.valid[i] = g.valid ? 1 : 0;
             }
-            if (!k) cidx[i] = 0xFFFFFFFFu;
         }
-        {
-            const uint32_t key = __float_as_uint(depth[it]);
-            hist_add_wave(s_hist[0], key & 255u, keep[it]);
-            hist_add_wave(s_hist[1], (key >> 8) & 255u, keep[it]);
-            hist_add_wave(s_hist[2], (key >> 16) & 255u, keep[it]);
-            hist_add_wave(s_hist[3], key >> 24, keep[it]);
-        }
-        bal[it] = __ballot(keep[it]);
+        s_iv[0][it][tid] = make_float4(g.u, g.v, rx, ry);
+        s_iv[1][it][tid] = make_float4(g.a, g.b, g.c, g.z);
+        bal[it] = __ballot(k);
         if (lane == 0) s_cnt[it][w] = (uint32_t)__popcll(bal[it]);
+        if constexpr (BINNED) {
+            const uint32_t c = k ? rect_tiles(g.u, g.v, rx, ry, cam.tiles_x, cam.tiles_y, 16) : 0u;
+            const uint32_t incl = wave_incl_scan(c);
+            coff[it] = incl - c;
+            if (lane == GS_WAVE - 1) s_ccnt[it][w] = incl;
+        } else {
+            const uint32_t key = __float_as_uint(g.z);
+            hist_add_wave(s_hist[0], key & 255u, k);
+            hist_add_wave(s_hist[1], (key >> 8) & 255u, k);
+            hist_add_wave(s_hist[2], (key >> 16) & 255u, k);
+            hist_add_wave(s_hist[3], key >> 24, k);
+        }
     }
     __syncthreads();
-    for (int k = tid; k < 1024; k += kTThreads)
-        part_hist[(size_t)vid * 1024 + k] = (&s_hist[0][0])[k];
-    uint32_t total = 0, my_off[kTItems];
+    if (!BINNED)
+        for (int k = tid; k < 1024; k += kTThreads)
+            part_hist[(size_t)vid * 1024 + k] = (&s_hist[0][0])[k];
+    // exclusive prefixes of the (item, wave) counts in source order: lane
+    // it * waves + w of a wave scan
+    static_assert(kTItems * kWaves <= GS_WAVE, "one count per lane");
+    uint32_t total, my_off[kTItems];
+    uint64_t ctotal = 0;
+    {
+        const uint32_t c = lane < kTItems * kWaves ? (&s_cnt[0][0])[lane] : 0u;
+        const uint32_t incl = wave_incl_scan(c);
+        total = (uint32_t)__builtin_amdgcn_readlane((int)incl, GS_WAVE - 1);
 #pragma unroll
-    for (int it = 0; it < kTItems; ++it)
+        for (int it = 0; it < kTItems; ++it)
+            my_off[it] = (uint32_t)__builtin_amdgcn_readlane((int)(incl - c), it * kWaves + w);
+        if constexpr (BINNED) {
+            const uint32_t cc = lane < kTItems * kWaves ? (&s_ccnt[0][0])[lane] : 0u;
+            const uint32_t ci = wave_incl_scan(cc);
+            ctotal = (uint32_t)__builtin_amdgcn_readlane((int)ci, GS_WAVE - 1);
 #pragma unroll
-        for (int ww = 0; ww < kTThreads / GS_WAVE; ++ww) {
-            if (ww == w) my_off[it] = total;
-            total += s_cnt[it][ww];
+            for (int it = 0; it < kTItems; ++it)
+                coff[it] += (uint32_t)__builtin_amdgcn_readlane((int)(ci - cc), it * kWaves + w);
         }
+    }
+    const uint64_t agg = BINNED ? binned_pack(total, ctotal) : (uint64_t)total;
+    if (w == 0) lookback_publish(lb_state, vid, agg);
+    float col[kTItems][3];
+#pragma unroll
+    for (int it = 0; it < kTItems; ++it) {
+        if (!keep[it]) continue;
+        const float4* row = P.rows + (base + it * kTThreads + tid) * V;
+        float dir[3], dn;
+        colour<DEG>(load_head(row), row, cam, col[it], dir, dn);
+    }
     if (w == 0) {
-        const uint64_t excl = lookback_exclusive(lb_state, vid, total, cam.ctl);
+        const uint64_t excl = lookback_walk(lb_state, vid, agg, cam.ctl);
         if (lane == 0) {
             s_excl = excl;
-            if (vid == gridDim.x - 1) *count_out = (uint32_t)(excl + total);
+            if (vid == gridDim.x - 1) {
+                if constexpr (BINNED)
+                    binned_totals(excl + agg, count_out, cam.binned, cam.ctl);
+                else
+                    *count_out = (uint32_t)(excl + agg);
+            }
         }
     }
     __syncthreads();
-    const uint64_t excl = s_excl;
+    const uint64_t excl = BINNED ? binned_count(s_excl) : s_excl;
     const uint64_t ltm = lanemask_lt();
 #pragma unroll
     for (int it = 0; it < kTItems; ++it) {
         if (!keep[it]) continue;
         const int64_t i = base + it * kTThreads + tid;
         const uint64_t m = excl + my_off[it] + (uint64_t)__popcll(bal[it] & ltm);
-        out.rc[2 * m + 0] = rect[it];
-        out.rc[2 * m + 1] = cov[it];
-        out.dkey[m] = __float_as_uint(depth[it]);
-        trec[3 * m + 0] = r0[it];
-        trec[3 * m + 1] = r1[it];
-        trec[3 * m + 2] = r2[it];
+        const float4 q0 = s_iv[0][it][tid], q1 = s_iv[1][it][tid];
+        const float a = q1.x, b = q1.y, c = q1.z, det = a * c - b * b;
+        out.rc[2 * m + 0] = q0;
+        out.rc[2 * m + 1] = make_float4(a, b, c, m2[it]);
+        out.dkey[m] = __float_as_uint(q1.w);
+        trec[3 * m + 0] = make_float4(q0.x, q0.y, ops[it], m2[it]);
+        trec[3 * m + 1] = make_float4(c / det, -b / det, a / det, 0.0f);
+        trec[3 * m + 2] = make_float4(col[it][0] < 0.0f ? 0.0f : col[it][0],
+                                      col[it][1] < 0.0f ? 0.0f : col[it][1],
+                                      col[it][2] < 0.0f ? 0.0f : col[it][2], 0.0f);
         out.src[m] = (uint32_t)i;
         cidx[i] = (uint32_t)m;
+        if constexpr (BINNED)
+            binned_write(cam.binned, m, binned_cands(s_excl) + coff[it],
+                         rect_tiles(q0.x, q0.y, q0.z, q0.w, cam.tiles_x, cam.tiles_y, 16));
+        if (cam.grad2d != nullptr) {  // the step's backward adds into these
+#pragma unroll
+            for (int k = 0; k < 9; ++k) cam.grad2d[9 * m + k] = 0.0f;
+        }
     }
 }
 
@@ -760,6 +808,7 @@ __global__ __launch_bounds__(GS_WAVE) void k_train_bwd(const float4* __restrict_
                                                        const uint32_t* __restrict__ ranges,
                                                        TrainBwdParams bp) {
     __shared__ float4 s0[GS_WAVE], s1[GS_WAVE], s2[GS_WAVE];
+    if (upstream_failed(bp.ctl)) return;
     const int lane = threadIdx.x;
     const int tile = blockIdx.x / kBandsPerTile, band = blockIdx.x % kBandsPerTile;
     const int tx = tile % bp.tiles_x, ty = tile / bp.tiles_x;
@@ -955,7 +1004,7 @@ __device__ __forceinline__ void row_gradient(const float4* row, const TrainCam& 
     float sh[3 * K];
     load_sh<DEG>(row, head, sh);
     float raw[3], dir[3], dn;
-    colour<DEG>(head, sh, cam, raw, dir, dn);
+    colour<DEG>(head, row, cam, raw, dir, dn);
     float gcol[3];
 #pragma unroll
     for (int ch = 0; ch < 3; ++ch) gcol[ch] = raw[ch] >= 0.0f ? gg[6 + ch] : 0.0f;
@@ -1043,13 +1092,16 @@ template <int DEG, bool ADAM, typename MOM>
 __global__ __launch_bounds__(kGradThreads) void k_train_grads(
     TrainParamsDev P, TrainCam cam, const uint32_t* __restrict__ cidx,
     const float* __restrict__ grad2d, float4* __restrict__ G, uint8_t* __restrict__ gnz,
-    MOM* __restrict__ m, MOM* __restrict__ v, const uint8_t* __restrict__ visible, AdamParams ap) {
+    MOM* __restrict__ m, MOM* __restrict__ v, const uint8_t* __restrict__ visible, AdamParams ap,
+    HostCopy report) {
     constexpr int V = Row<DEG>::V;
     constexpr int R = DEG < 2 ? kGradThreads : kGradThreads / 2;  // rows: 16 to 30 KB of LDS
     __shared__ float4 s_g[R][V];
     __shared__ float4 s_step[V];
     __shared__ uint32_t s_list[R];
     __shared__ uint32_t s_count;
+    // the step's counters and sums are final by now, whether it failed or not
+    if (blockIdx.x == 0) host_copy(report, threadIdx.x, kGradThreads);
     if (upstream_failed(cam.ctl)) return;
     const int tid = threadIdx.x;
     const int64_t row0 = (int64_t)blockIdx.x * R;
@@ -1125,9 +1177,15 @@ hipError_t launch_train_project(const TrainParamsDev& P, const TrainCam& cam, Co
                                 uint32_t* part_hist, const TrainDebug& dbg, hipStream_t st) {
     if (P.n <= 0) return hipSuccess;
     const unsigned grid = (unsigned)((P.n + kTPart - 1) / kTPart);
-#define GS_TP(D)                                                                            \
-    k_train_project<D><<<grid, kTThreads, 0, st>>>(P, cam, out, trec, cidx, visible, lb_state, \
-                                                   ticket, count_out, part_hist, dbg)
+#define GS_TP(D)                                                                           \
+    if (cam.binned.offs != nullptr)                                                        \
+        k_train_project<D, true><<<grid, kTThreads, 0, st>>>(P, cam, out, trec, cidx,      \
+                                                             visible, lb_state, ticket,    \
+                                                             count_out, part_hist, dbg);   \
+    else                                                                                   \
+        k_train_project<D, false><<<grid, kTThreads, 0, st>>>(P, cam, out, trec, cidx,     \
+                                                              visible, lb_state, ticket,   \
+                                                              count_out, part_hist, dbg)
     switch (P.sh_degree) {
         case 0: GS_TP(0); break;
         case 1: GS_TP(1); break;
@@ -1179,20 +1237,20 @@ template <int DEG>
 hipError_t train_grads_deg(const TrainParamsDev& P, const TrainCam& cam, const uint32_t* cidx,
                            const float* grad2d, float4* G, uint8_t* gnz, void* m, void* v,
                            const uint8_t* visible, const AdamParams* adam, bool bf16_moments,
-                           hipStream_t st) {
+                           const HostCopy& report, hipStream_t st) {
     constexpr int R = DEG < 2 ? kGradThreads : kGradThreads / 2;
     const unsigned grid = (unsigned)((P.n + R - 1) / R);
     if (adam == nullptr)
         k_train_grads<DEG, false, float><<<grid, kGradThreads, 0, st>>>(
-            P, cam, cidx, grad2d, G, gnz, nullptr, nullptr, nullptr, AdamParams{});
+            P, cam, cidx, grad2d, G, gnz, nullptr, nullptr, nullptr, AdamParams{}, report);
     else if (bf16_moments)
         k_train_grads<DEG, true, uint16_t><<<grid, kGradThreads, 0, st>>>(
             P, cam, cidx, grad2d, G, gnz, static_cast<uint16_t*>(m), static_cast<uint16_t*>(v),
-            visible, *adam);
+            visible, *adam, report);
     else
         k_train_grads<DEG, true, float><<<grid, kGradThreads, 0, st>>>(
             P, cam, cidx, grad2d, G, gnz, static_cast<float*>(m), static_cast<float*>(v), visible,
-            *adam);
+            *adam, report);
     return hipGetLastError();
 }
 
@@ -1214,10 +1272,10 @@ hipError_t sparse_adam_deg(const TrainParamsDev& P, void* m, void* v, const floa
 hipError_t launch_train_grads(const TrainParamsDev& P, const TrainCam& cam, const uint32_t* cidx,
                               const float* grad2d, float4* G, uint8_t* gnz, void* m, void* v,
                               const uint8_t* visible, const AdamParams* adam, bool bf16_moments,
-                              hipStream_t st) {
+                              const HostCopy& report, hipStream_t st) {
     if (P.n <= 0) return hipSuccess;
 #define GS_TG(D) \
-    train_grads_deg<D>(P, cam, cidx, grad2d, G, gnz, m, v, visible, adam, bf16_moments, st)
+    train_grads_deg<D>(P, cam, cidx, grad2d, G, gnz, m, v, visible, adam, bf16_moments, report, st)
     switch (P.sh_degree) {
         case 0: return GS_TG(0);
         case 1: return GS_TG(1);

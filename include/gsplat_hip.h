@@ -344,8 +344,8 @@ typedef struct gs_train_stats {
     int64_t step;           /* Adam steps taken so far */
     double loss;            /* the loss of cfg (with a target) */
     float ms_forward;       /* device time: projection + tiles + forward + L1 */
-    float ms_backward;      /* blend backward + projection backward */
-    float ms_adam;
+    float ms_backward;      /* blend backward + projection backward (a step: the blend's) */
+    float ms_adam;          /* a step: parameter gradients and Adam, one pass */
     float ms_total;         /* host wall clock of the call */
     double l1;              /* mean |image - target| */
     double ssim;            /* mean SSIM (computed when lambda_dssim > 0) */

@@ -388,3 +388,30 @@ def test_train_step_rows(gpu_ctx, n, deg, bf16):
         assert all(np.all(a == 0) for a in tr.read(3).values())
     finally:
         tr.set_moments(False)
+
+
+def test_train_step_capacity_rerun():
+    """A first step whose candidate pairs exceed the starting capacity (2000 Gaussians over
+    most of 3600 tiles) is run again whole: the attempt that did not fit leaves
+    parameters, moments and the step count alone, so one Adam step has been taken."""
+    print("train step capacity", flush=True)
+    rng = np.random.default_rng(4)
+    n, H, W = 2000, 720, 1280
+    p = {"means": np.stack([rng.uniform(-1, 1, n), rng.uniform(-1, 1, n),
+                            rng.uniform(3, 5, n)], 1),
+         "log_scales": rng.normal(0.3, 0.1, (n, 3)), "quats": rng.standard_normal((n, 4)),
+         "opacity_logits": rng.normal(-3, 0.3, n), "sh": rng.uniform(-0.5, 0.5, (n, 1, 3))}
+    p = {k: v.astype(np.float32) for k, v in p.items()}
+    K = scenes.intrinsics(1000.0, 1000.0, W / 2, H / 2)
+    view = L.make_view(np.eye(4, dtype=np.float32), K, H, W, tile_size=16)
+    ctx = L.Context(0)
+    try:
+        tr = L.Trainer(ctx, p, 0)
+        st = tr.step(view, L.make_train_cfg(), np.zeros((H, W, 3), np.float32))
+        assert st["pairs_pre"] > (1 << 20) and st["step"] == 1, st
+        assert st["pair_capacity"] >= st["pairs_pre"]
+        g, m = tr.read(3), tr.read(1)
+        for k in TO.PARAM_NAMES:
+            assert np.array_equal(m[k], np.float32(1.0 - 0.9) * g[k]), k
+    finally:
+        ctx.close()

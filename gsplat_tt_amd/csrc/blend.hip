@@ -66,6 +66,13 @@ __device__ __forceinline__ uint8_t bf16_to_u8(uint32_t b) {
     return (uint8_t)(((sig << 8) - sig) >> (134u - e));
 }
 
+// A record's words as one register tuple (a HIP float4 carried over the batch loop
+// went through scratch memory, and its store waited for the load).
+using vec4 = __attribute__((ext_vector_type(4))) float;
+__device__ __forceinline__ vec4 load_vec4(const float4* p) {
+    return *reinterpret_cast<const vec4*>(p);
+}
+
 // Per-wave geometry of one 16x4 band (two microblocks).
 struct Band {
     int tile, tile_x, tile_y, mbx, mby;
@@ -123,9 +130,46 @@ __device__ __forceinline__ Band make_band(const BlendParams& bp, int lane) {
     return g;
 }
 
+// The same of one 8x4 microblock, both halves of the wave on its pixels.
+template <int TS>
+__device__ __forceinline__ Band make_microblock(const BlendParams& bp, int lane) {
+    constexpr int MX = TS / 8, MY = TS / 4;
+    Band g{};
+    const int mb = blockIdx.x % (MX * MY);
+    g.tile = blockIdx.x / (MX * MY);
+    g.mbx = mb % MX;
+    g.mby = mb / MX;
+    g.tile_x = g.tile % bp.tiles_x;
+    g.tile_y = g.tile / bp.tiles_x;
+    const int q = lane & 31, pi = q >> 3, pj = q & 7;
+    const int px_tile = g.tile_x * TS, py_tile = g.tile_y * TS;
+    g.px_start = px_tile + g.mbx * 8;
+    g.py0 = py_tile + g.mby * 4;
+    const int px_end = min(g.px_start + 8, min(px_tile + TS, bp.width));
+    const int py_end = min(g.py0 + 4, min(py_tile + TS, bp.height));
+    g.emptyA = g.py0 >= py_end || g.px_start >= px_end;
+    g.full = !g.emptyA && px_end - g.px_start == 8 && py_end - g.py0 == 4;
+    g.pix_valid = g.px_start + pj < px_end && g.py0 + pi < py_end;
+    g.tx_tile = (float)px_tile;
+    g.ty_tile = (float)py_tile;
+    g.pxs = (float)g.px_start;
+    g.offx = (float)pj + 0.5f;
+    g.pxc = (float)(g.px_start + pj) + 0.5f;
+    g.pyc = (float)(g.py0 + pi) + 0.5f;
+    g.pyr0 = (float)g.py0 + 0.5f;
+    g.mb_oy = g.ty_tile + (float)(g.mby * 4);
+    g.mb_ox = g.tx_tile + (float)(g.mbx * 8);
+    g.ext_x0 = (float)(8 * g.mbx);
+    g.ext_x1 = (float)(8 * g.mbx + 8);
+    g.ext_y0 = (float)(4 * g.mby);
+    g.ext_y1 = (float)(4 * g.mby + 4);
+    return g;
+}
+
 // Constrained-minimum cull of one entry against the lane's microblock
 // (cull_and_blend.cpp:447-498).
-__device__ __forceinline__ bool mb_keep(const Band& g, float4 r0, float4 r1, int cull_disabled) {
+template <typename V>  // float4 or vec4
+__device__ __forceinline__ bool mb_keep(const Band& g, V r0, V r1, int cull_disabled) {
     const float lt = r1.w;
     const float mx = r0.x, my = r0.y;
     // The reference's microblock range of the extent, mx_lo = max(0, floor(ax / 8)),
@@ -434,6 +478,276 @@ __device__ __forceinline__ void blend_band_edge(const Band& g, const float4* __r
     }
 }
 
+template <int OUT>
+__device__ __forceinline__ void store_pixel(void* out, size_t o, float cr, float cg, float cb) {
+    if (OUT == 2) {
+        float* img = static_cast<float*>(out);
+        img[o + 0] = cr;
+        img[o + 1] = cg;
+        img[o + 2] = cb;
+    } else if (OUT == 1) {
+        uint16_t* img = static_cast<uint16_t*>(out);
+        img[o + 0] = f32_to_bf16_rne(cr);
+        img[o + 1] = f32_to_bf16_rne(cg);
+        img[o + 2] = f32_to_bf16_rne(cb);
+    } else {
+        // the bf16 image packed to u8, as the reference's render_view does
+        uint8_t* img = static_cast<uint8_t*>(out);
+        img[o + 0] = bf16_to_u8(f32_to_bf16_rne(cr));
+        img[o + 1] = bf16_to_u8(f32_to_bf16_rne(cg));
+        img[o + 2] = bf16_to_u8(f32_to_bf16_rne(cb));
+    }
+}
+
+// Alpha of an entry at the lane's pixel. A full microblock: AVX2 rule (power clamp
+// [-30, 0], degree-4 exp, alpha <= 0.99) from the staged terms.
+__device__ __forceinline__ float alpha_full(float2 row, float dx, float2 aop) {
+    float pwr = __builtin_fmaf(row.y, dx, row.x);
+    pwr = __builtin_fmaf(aop.x, dx * dx, pwr);
+    pwr = __builtin_amdgcn_fmed3f(pwr, -30.0f, 0.0f);
+    const float al = aop.y * exp4(pwr);
+    return (al < 0.99f) ? al : 0.99f;
+}
+// By the scalar rule, of a microblock that the image edge cuts, from the entry:
+// (mx, my, op), (ci_a, ci_b, ci_c).
+__device__ __forceinline__ float alpha_cut(float4 e0, float4 e1, const Band& g) {
+    const float dx = g.pxc - e0.x;
+    const float dy = g.pyc - e0.y;
+    const float power = -0.5f * (e1.x * dx * dx + 2.0f * e1.y * dx * dy + e1.z * dy * dy);
+    return fmin_std(e0.z * expf(fmin_std(power, 0.0f)), 0.99f);
+}
+
+// One kept entry blended: T and two of the pixel's channels.
+template <bool EDGE>
+__device__ __forceinline__ void blend_channels(float al, float2 e2, float& T,
+                                               float& c0, float& c1) {
+    const float at = al * T;
+    if (!EDGE) {
+        c0 = __builtin_fmaf(at, e2.x, c0);
+        c1 = __builtin_fmaf(at, e2.y, c1);
+        T = T - at;
+    } else {
+        c0 += at * e2.x;
+        c1 += at * e2.y;
+        T = T * (1.0f - al);
+    }
+}
+
+// ---------------------------------------------------------------------------
+// One wave per microblock: lanes 0-31 are its pixels, lanes 32-63 the same
+// pixels again. 64 entries at a time are tested against the microblock (one per
+// lane) and the kept ones packed into LDS; they are walked in groups of four,
+// lanes 0-31 evaluating a pair's first alpha, lanes 32-63 its second, exchanged
+// by one permlane swap; T's chain runs in both halves, the first accumulating
+// (r, g), the second b. Groups hold exactly the four kept entries between two
+// early-out tests: a batch's last one to three wait for the next batch. An entry
+// costs 12.5 vector instructions a microblock against 21 for both of a band's,
+// and only the entries this microblock keeps: it wins where few are kept by
+// both neighbours (small Gaussians) and where too few bands run to hide a wave's
+// latencies (a band's wave walks entry by entry, 440 clocks each when alone).
+// Kernel time, band against microblock: 20K Gaussians at 320x240 41 -> 17 us,
+// 100K at 640x480 78 -> 50, 1M at 1280x720 108 -> 91.
+// ---------------------------------------------------------------------------
+struct MbStage {
+    float2 rows[68][4];   // (y_term, xy_coef) of the 4 rows
+    float dx[68][8];      // columns
+    float2 aop[68];       // -ci_a/2, opacity
+    float4 rgb[68];       // r, g, b, 0
+};
+struct MbEdgeStage {
+    float4 p0[68], p1[68], rgb[68];
+};
+union MbLds {
+    MbStage full;
+    MbEdgeStage edge;
+};
+constexpr int kMbBatch = GS_WAVE;
+
+__device__ __forceinline__ float swap_halves(float mine, float& first) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(mine), __float_as_uint(mine),
+                                                    false, false);
+    // r[0]: lanes 0-31's value in both halves, r[1]: lanes 32-63's
+    first = __uint_as_float(r[0]);
+    return __uint_as_float(r[1]);
+}
+
+// Entries [from, from + count), count <= 3, to the first slots.
+template <bool EDGE>
+__device__ __forceinline__ void move_slots(MbLds* lds, int from, int count, int lane) {
+    if (lane >= count) return;
+    if constexpr (EDGE) {
+        MbEdgeStage& st = lds->edge;
+        st.p0[lane] = st.p0[from + lane];
+        st.p1[lane] = st.p1[from + lane];
+        st.rgb[lane] = st.rgb[from + lane];
+    } else {
+        MbStage& st = lds->full;
+        const float4* r = reinterpret_cast<const float4*>(&st.rows[from + lane][0]);
+        const float4* d = reinterpret_cast<const float4*>(&st.dx[from + lane][0]);
+        const float4 r0 = r[0], r1 = r[1], d0 = d[0], d1 = d[1];
+        float4* rw = reinterpret_cast<float4*>(&st.rows[lane][0]);
+        float4* dw = reinterpret_cast<float4*>(&st.dx[lane][0]);
+        rw[0] = r0;
+        rw[1] = r1;
+        dw[0] = d0;
+        dw[1] = d1;
+        st.aop[lane] = st.aop[from + lane];
+        st.rgb[lane] = st.rgb[from + lane];
+    }
+}
+
+template <bool EDGE>
+__device__ __forceinline__ void blend_mb(const Band& g, const float4* __restrict__ brec,
+                                         const uint32_t* __restrict__ sid, uint32_t start,
+                                         uint32_t end, const BlendParams& bp, int lane, MbLds* lds,
+                                         float& c0, float& c1, uint32_t& cnt, uint32_t& n_batch,
+                                         uint32_t& n_iter) {
+    if (start >= end) return;
+    const int s = lane >> 5, q = lane & 31, pi = q >> 3, pj = q & 7;
+    const float thr = bp.thr;
+    float T = 1.0f;
+    uint32_t gi = sid[min(start + (uint32_t)lane, end - 1)];
+    vec4 r0 = load_vec4(brec + 3 * (size_t)gi), r1 = load_vec4(brec + 3 * (size_t)gi + 1),
+         r2 = load_vec4(brec + 3 * (size_t)gi + 2);
+    gi = sid[min(start + kMbBatch + (uint32_t)lane, end - 1)];
+    int carry = 0;  // entries of the batches before that wait in slots 0 .. carry-1
+    for (uint32_t base = start; base < end; base += kMbBatch) {
+        const bool keep = base + (uint32_t)lane < end && mb_keep(g, r0, r1, bp.cull_disabled);
+        const uint64_t mask = __ballot(keep);
+        ++n_batch;
+        const int have = carry + __popcll(mask);
+        const bool last = base + kMbBatch >= end;
+        // whole groups, and at the list's end the rest padded with opacity 0
+        const int n = last ? (have + 3) & ~3 : have & ~3;
+        __syncthreads();  // one wave per workgroup: orders the reads of the batch before
+        const int k = carry + __popcll(mask & lanemask_lt());
+        if (keep) {
+            if constexpr (EDGE) {
+                lds->edge.p0[k] = make_float4(r0.x, r0.y, r2.w, 0.0f);
+                lds->edge.p1[k] = make_float4(r1.x, r1.y, r1.z, 0.0f);
+                lds->edge.rgb[k] = make_float4(r2.x, r2.y, r2.z, 0.0f);
+            } else {
+                MbStage* st = &lds->full;
+                const float Bq = -r1.y, Cq = -0.5f * r1.z;
+#pragma unroll
+                for (int r = 0; r < 4; r += 2) {
+                    const float da = g.pyr0 + (float)r - r0.y, db = g.pyr0 + (float)(r + 1) - r0.y;
+                    *reinterpret_cast<float4*>(&st->rows[k][r]) =
+                        make_float4(Cq * da * da, Bq * da, Cq * db * db, Bq * db);
+                }
+                const float pb = g.pxs - r0.x;
+                float4* dx = reinterpret_cast<float4*>(&st->dx[k][0]);
+                dx[0] = make_float4(pb + 0.5f, pb + 1.5f, pb + 2.5f, pb + 3.5f);
+                dx[1] = make_float4(pb + 4.5f, pb + 5.5f, pb + 6.5f, pb + 7.5f);
+                st->aop[k] = make_float2(-0.5f * r1.x, r2.w);
+                st->rgb[k] = make_float4(r2.x, r2.y, r2.z, 0.0f);
+            }
+        }
+        if (lane < n - have) {
+            const int e = have + lane;
+            if constexpr (EDGE) {
+                lds->edge.p0[e] = lds->edge.p1[e] = lds->edge.rgb[e] = make_float4(0, 0, 0, 0);
+            } else {
+                for (int r = 0; r < 4; ++r) lds->full.rows[e][r] = make_float2(0, 0);
+                for (int r = 0; r < 8; ++r) lds->full.dx[e][r] = 0.0f;
+                lds->full.aop[e] = make_float2(0, 0);
+                lds->full.rgb[e] = make_float4(0, 0, 0, 0);
+            }
+        }
+        r0 = load_vec4(brec + 3 * (size_t)gi);
+        r1 = load_vec4(brec + 3 * (size_t)gi + 1);
+        r2 = load_vec4(brec + 3 * (size_t)gi + 2);
+        gi = sid[min(base + 2 * kMbBatch + (uint32_t)lane, end - 1)];
+        __syncthreads();
+        for (int j = 0; j < n; j += 4) {
+            ++n_iter;
+            float al[4];
+#pragma unroll
+            for (int p = 0; p < 2; ++p) {
+                const int e = j + 2 * p + s;
+                float a;
+                if constexpr (EDGE) {
+                    a = alpha_cut(lds->edge.p0[e], lds->edge.p1[e], g);
+                } else {
+                    const MbStage& st = lds->full;
+                    a = alpha_full(st.rows[e][pi], st.dx[e][pj], st.aop[e]);
+                }
+                al[2 * p + 1] = swap_halves(a, al[2 * p]);
+            }
+            float T0 = T, a0 = c0, a1 = c1;
+#pragma unroll
+            for (int p = 0; p < 4; ++p) {
+                const float2 col = *reinterpret_cast<const float2*>(
+                    &(EDGE ? lds->edge.rgb[j + p] : lds->full.rgb[j + p]).x + 2 * s);
+                blend_channels<EDGE>(al[p], col, T, c0, c1);
+            }
+            cnt += (uint32_t)min(4, have - j);
+            const uint64_t live = __ballot((!EDGE || g.pix_valid) && !(T < thr));
+            if (live != 0ull) continue;
+            if constexpr (EDGE) {
+                // the scalar rule tests after every entry: the group again, one by one
+                T = T0;
+                c0 = a0;
+                c1 = a1;
+                cnt -= (uint32_t)min(4, have - j);
+                for (int p = 0; p < 4 && j + p < have; ++p) {
+                    ++cnt;
+                    const float2 col = *reinterpret_cast<const float2*>(
+                        &lds->edge.rgb[j + p].x + 2 * s);
+                    blend_channels<EDGE>(al[p], col, T, c0, c1);
+                    if (__ballot(g.pix_valid && !(T < thr)) == 0ull) break;
+                }
+            }
+            return;
+        }
+        carry = have - min(n, have);
+        if (carry > 0 && !last) {
+            // the waiting entries move to the first slots (n >= 4 > carry, or they are there)
+            if (n > 0) {
+                __syncthreads();
+                move_slots<EDGE>(lds, n, carry, lane);
+            }
+        }
+    }
+}
+
+template <int TS, int OUT>
+__global__ __launch_bounds__(GS_WAVE) void k_blend_mb(const float4* __restrict__ brec,
+                                                      const uint32_t* __restrict__ sid,
+                                                      const uint32_t* __restrict__ ranges,
+                                                      BlendParams bp, void* __restrict__ out) {
+    const int lane = threadIdx.x;
+    // after an earlier give-up the sorted ids may be wrong: read nothing
+    if (__builtin_amdgcn_readfirstlane(upstream_failed(bp.ctl) ? 1 : 0)) return;
+    const Band g = make_microblock<TS>(bp, lane);
+    if (g.emptyA) return;
+    float c0 = 0.0f, c1 = 0.0f;
+    uint32_t cnt = 0, n_batch = 0, n_iter = 0;
+    const uint32_t start = ranges[2 * g.tile], end = ranges[2 * g.tile + 1];
+    __shared__ MbLds lds;
+    if (g.full)
+        blend_mb<false>(g, brec, sid, start, end, bp, lane, &lds, c0, c1, cnt, n_batch, n_iter);
+    else
+        blend_mb<true>(g, brec, sid, start, end, bp, lane, &lds, c0, c1, cnt, n_batch, n_iter);
+    if (bp.evals != nullptr) {
+        const uint32_t px = (uint32_t)__popcll(__ballot(g.pix_valid)) / 2u;
+        if (lane == 0) {
+            unsigned long long* slot = bp.evals + (size_t)(blockIdx.x & 63u) * 8;
+            atomicAdd(slot + 0, (unsigned long long)cnt * px);
+            atomicAdd(slot + 1, (unsigned long long)n_batch);
+            atomicAdd(slot + 2, (unsigned long long)n_iter * 4);
+            atomicAdd(slot + 3, (unsigned long long)cnt);
+            atomicMax(slot + 4, (unsigned long long)n_iter * 4);
+        }
+    }
+    // blue from the second half's lane of the pixel
+    const float blue = __shfl(c0, (lane & 31) + 32, GS_WAVE);
+    if (!g.pix_valid || lane >= 32) return;
+    const int pi = lane >> 3, pj = lane & 7;
+    store_pixel<OUT>(out, ((size_t)(g.py0 + pi) * bp.width + (size_t)(g.px_start + pj)) * 3, c0, c1,
+                     blue);
+}
+
 template <int TS, int OUT>
 __global__ __launch_bounds__(GS_WAVE) void k_blend(const float4* __restrict__ brec,
                                                    const uint32_t* __restrict__ sid,
@@ -471,24 +785,8 @@ __global__ __launch_bounds__(GS_WAVE) void k_blend(const float4* __restrict__ br
     }
     if (!g.pix_valid) return;
     const int q = lane & 31, pi = q >> 3, pj = q & 7;
-    const size_t o = ((size_t)(g.py0 + pi) * bp.width + (size_t)(g.px_start + pj)) * 3;
-    if (OUT == 2) {
-        float* img = static_cast<float*>(out);
-        img[o + 0] = cr;
-        img[o + 1] = cg;
-        img[o + 2] = cb;
-    } else if (OUT == 1) {
-        uint16_t* img = static_cast<uint16_t*>(out);
-        img[o + 0] = f32_to_bf16_rne(cr);
-        img[o + 1] = f32_to_bf16_rne(cg);
-        img[o + 2] = f32_to_bf16_rne(cb);
-    } else {
-        // the bf16 image packed to u8, as the reference's render_view does
-        uint8_t* img = static_cast<uint8_t*>(out);
-        img[o + 0] = bf16_to_u8(f32_to_bf16_rne(cr));
-        img[o + 1] = bf16_to_u8(f32_to_bf16_rne(cg));
-        img[o + 2] = bf16_to_u8(f32_to_bf16_rne(cb));
-    }
+    store_pixel<OUT>(out, ((size_t)(g.py0 + pi) * bp.width + (size_t)(g.px_start + pj)) * 3, cr, cg,
+                     cb);
 }
 
 // Statistics of the reference's per-microblock cull (cull_and_blend.cpp:
@@ -572,11 +870,14 @@ __global__ __launch_bounds__(kStatThreads) void k_mb_stats(
 }
 
 template <int TS>
-const void* blend_ts(int out_format) {
-    switch (out_format) {
+const void* blend_ts(int out_format, bool by_mb) {
+    switch (out_format * 2 + (by_mb ? 1 : 0)) {
         case 0: return reinterpret_cast<const void*>(&k_blend<TS, 0>);
-        case 1: return reinterpret_cast<const void*>(&k_blend<TS, 1>);
-        case 2: return reinterpret_cast<const void*>(&k_blend<TS, 2>);
+        case 1: return reinterpret_cast<const void*>(&k_blend_mb<TS, 0>);
+        case 2: return reinterpret_cast<const void*>(&k_blend<TS, 1>);
+        case 3: return reinterpret_cast<const void*>(&k_blend_mb<TS, 1>);
+        case 4: return reinterpret_cast<const void*>(&k_blend<TS, 2>);
+        case 5: return reinterpret_cast<const void*>(&k_blend_mb<TS, 2>);
         default: return nullptr;
     }
 }
@@ -584,11 +885,14 @@ const void* blend_ts(int out_format) {
 template <int TS>
 hipError_t launch_ts(const float4* brec, const uint32_t* sid, const uint32_t* ranges,
                      BlendParams bp, void* out, hipStream_t st) {
-    const unsigned grid = (unsigned)(bp.tiles_x * bp.tiles_y * (TS / 16) * (TS / 4));
-    switch (bp.out_format) {
-        case 0: k_blend<TS, 0><<<grid, GS_WAVE, 0, st>>>(brec, sid, ranges, bp, out); break;
-        case 1: k_blend<TS, 1><<<grid, GS_WAVE, 0, st>>>(brec, sid, ranges, bp, out); break;
-        case 2: k_blend<TS, 2><<<grid, GS_WAVE, 0, st>>>(brec, sid, ranges, bp, out); break;
+    const unsigned bands = (unsigned)(bp.tiles_x * bp.tiles_y * (TS / 16) * (TS / 4));
+    switch (bp.out_format * 2 + (bp.by_microblock ? 1 : 0)) {
+        case 0: k_blend<TS, 0><<<bands, GS_WAVE, 0, st>>>(brec, sid, ranges, bp, out); break;
+        case 1: k_blend_mb<TS, 0><<<2 * bands, GS_WAVE, 0, st>>>(brec, sid, ranges, bp, out); break;
+        case 2: k_blend<TS, 1><<<bands, GS_WAVE, 0, st>>>(brec, sid, ranges, bp, out); break;
+        case 3: k_blend_mb<TS, 1><<<2 * bands, GS_WAVE, 0, st>>>(brec, sid, ranges, bp, out); break;
+        case 4: k_blend<TS, 2><<<bands, GS_WAVE, 0, st>>>(brec, sid, ranges, bp, out); break;
+        case 5: k_blend_mb<TS, 2><<<2 * bands, GS_WAVE, 0, st>>>(brec, sid, ranges, bp, out); break;
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
@@ -615,9 +919,9 @@ hipError_t launch_blend(const float4* brec, const uint32_t* sid, const uint32_t*
     return hipErrorInvalidValue;
 }
 
-const void* blend_kernel(int tile_size, int out_format) {
-    if (tile_size == 16) return blend_ts<16>(out_format);
-    if (tile_size == 32) return blend_ts<32>(out_format);
+const void* blend_kernel(int tile_size, int out_format, bool by_microblock) {
+    if (tile_size == 16) return blend_ts<16>(out_format, by_microblock);
+    if (tile_size == 32) return blend_ts<32>(out_format, by_microblock);
     return nullptr;
 }
 

@@ -1424,7 +1424,8 @@ struct gs_ctx {
             std::vector<hipGraphNode_t> nodes(nn);
             if (nn) HIPCHK(hipGraphGetNodes(fg.graph, nodes.data(), &nn));
             const void* fn_proj = gs::project_kernel(sd.sh_degree, L.binned);
-            const void* fn_blend = gs::blend_kernel(pend.v.tile_size, pend.v.out_format);
+            const void* fn_blend = gs::blend_kernel(pend.v.tile_size, pend.v.out_format,
+                                                    blend_by_microblock(L));
             hipGraphNode_t proj = nullptr;
             for (hipGraphNode_t node : nodes) {
                 hipGraphNodeType ty;
@@ -1445,6 +1446,15 @@ struct gs_ctx {
         }
         return true;
     }
+
+    // A wave per microblock blends every frame that runs alone faster, and every
+    // binned one; a wave per band takes 15 % fewer instructions where most entries
+    // are kept by both of its microblocks, which is what counts for a large frame
+    // among others in flight (us a frame alone and in a path, band against
+    // microblock; 1237x822 slab scenes: 300K 228, 154 / 200, 154; 1.5M 545, 380 /
+    // 495, 387; 6M 1264, 1022 / 1223, 1046; 300x200, 3300 pairs a tile: 696, 364 /
+    // 280, 153).
+    bool blend_by_microblock(const FrameLayout& L) const { return L.binned || !batch_frame; }
 
     // Enqueues one frame (project -> depth sort -> tile assign -> tile sort ->
     // ranges -> blend) on the stream; no host synchronisation.
@@ -1482,7 +1492,7 @@ struct gs_ctx {
         gs::BlendParams bp{tiles_x, tiles_y, v->tile_size, v->image_height, v->image_width,
                            v->cull_disabled ? 1 : 0, v->transmittance_threshold, v->out_format,
                            blend_counts ? b_evals.as<unsigned long long>() : nullptr,
-                           L.cnt + C_CTL};
+                           L.cnt + C_CTL, blend_by_microblock(L)};
         HIPCHK(gs::launch_blend(b_brec.as<float4>(), ids_sorted, b_ranges.as<uint32_t>(), bp,
                                 dout, st));
         record(5);

@@ -362,13 +362,14 @@ struct BlendParams {
     // pairs, max apply iterations of one wave
     unsigned long long* evals;
     const uint32_t* ctl;  // control words of the frame (nothing is read after an error)
+    bool by_microblock;   // a wave per microblock (k_blend_mb) instead of per band
 };
 hipError_t launch_blend(const float4* brec, const uint32_t* sorted_id, const uint32_t* ranges,
                         BlendParams bp, void* out, hipStream_t st);
 // Captured frames: the k_blend instance launch_blend uses, and an update of a
 // captured k_blend node's image in an instantiated graph (its other arguments
 // are kept).
-const void* blend_kernel(int tile_size, int out_format);
+const void* blend_kernel(int tile_size, int out_format, bool by_microblock);
 hipError_t graph_set_blend_out(hipGraphExec_t exec, hipGraphNode_t node, void* out);
 // Counts of the reference's microblock cull over the tile-sorted pairs (ids
 // `sid`, tile ids `stile`, min(p_cap, *p_dev) of them): out[0] += pairs kept by

@@ -105,3 +105,39 @@ def test_plan_follows_the_pairs():
             assert np.array_equal(o, _both(ctx, v)[1][0])
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("h,w,ts", [(1, 1, 16), (4, 8, 16), (5, 9, 32), (3, 7, 16), (17, 33, 16),
+                                    (35, 61, 32), (64, 48, 16)])
+@pytest.mark.parametrize("n,op", [(3, 0.9), (70, 0.03), (67, 0.5), (400, 0.15), (400, 0.98)])
+def test_blend_by_microblock_equals_by_band(gpu_ctx, h, w, ts, n, op):
+    """render() blends with a wave per microblock, gs_cull_and_blend with one per band:
+    the same image bit for bit, for whole and cut microblocks, lists whose kept entries
+    leave every remainder of four, faint entries (no early-out) and opaque ones."""
+    print("blend", h, w, ts, n, op, flush=True)
+    rng = np.random.default_rng(n + h)
+    f = 0.7 * max(h, w)
+    z = rng.uniform(2, 4, n)
+    means = np.stack([rng.uniform(-0.6, 0.6, n) * w / f * z, rng.uniform(-0.6, 0.6, n) * h / f * z,
+                      z], 1).astype(np.float32)
+    q = rng.standard_normal((n, 4))
+    q /= np.linalg.norm(q, axis=1, keepdims=True)
+    cov = scenes.cov3d(np.exp(rng.normal(-1.5, 0.8, (n, 3))).astype(np.float32),
+                       q.astype(np.float32))
+    opac = np.full(n, op, np.float32)
+    col = rng.random((n, 3)).astype(np.float32)
+    view = L.make_view(np.eye(4, dtype=np.float32), scenes.intrinsics(f, f, w / 2, h / 2), h, w,
+                       tile_size=ts, output="f32", max_radius=10_000)
+    gpu_ctx.set_scene(means, cov, opac, col)
+    img, st = gpu_ctx.render(view)
+    p = gpu_ctx.project(means, cov, opac, col, view)
+    g, t, _ = gpu_ctx.tile_assign(p["means2d"], p["radii"], h, w, ts, p["covs2d"],
+                                  p["opacities"])
+    assert g.shape[0] == st["num_entries"]
+    if g.shape[0] == 0:
+        assert not img.any()
+        return
+    ids, ranges = gpu_ctx.sort_and_bin(g, t, p["depths"], -(-w // ts), -(-h // ts))
+    ref = gpu_ctx.cull_and_blend(p["means2d"], p["covs2d"], p["colors"], p["opacities"], ids,
+                                 ranges, view)
+    assert np.array_equal(img.view(np.uint32), ref.view(np.uint32))

@@ -394,6 +394,13 @@ struct TrainParamsDev {
     int sh_degree;
 };
 
+// Rows [row0, row0 + count) split into (split) or joined from the caller's arrays,
+// one after the other in `arrays`: means, log-scales, quaternions, opacity logits,
+// SH, float32; bf16: the rows hold bf16 bits (rounded to nearest even when
+// joined). The padding of a joined row is zero.
+hipError_t launch_train_rows(void* rows, int64_t row0, int64_t count, int sh_degree, float* arrays,
+                             bool split, bool bf16, hipStream_t st);
+
 struct TrainCam {
     float r[9], t[3];          // world-to-camera rotation (row-major) and translation
     float fx, fy, cx, cy;

@@ -1169,7 +1169,58 @@ __global__ __launch_bounds__(256) void k_sparse_adam(TrainParamsDev P, MOM* __re
     adam_float4(P.rows, m, v, f, G[f], s_step[f % V], ap);
 }
 
+// Rows <-> the caller's arrays: a thread per value, the arrays' side contiguous,
+// the rows' side within a few lines (bound by HBM, 8 MB of either in a few us).
+__device__ __forceinline__ float row_get(const float* r, size_t k) { return r[k]; }
+__device__ __forceinline__ float row_get(const uint16_t* r, size_t k) { return bf16_to_f32(r[k]); }
+__device__ __forceinline__ void row_put(float* r, size_t k, float x) { r[k] = x; }
+__device__ __forceinline__ void row_put(uint16_t* r, size_t k, float x) {
+    r[k] = f32_to_bf16_rne(x);
+}
+template <typename T, bool SPLIT>
+__global__ __launch_bounds__(256) void k_train_rows(T* __restrict__ rows, int64_t row0,
+                                                    int64_t count, int vals, int stride,
+                                                    float* __restrict__ arrays) {
+    const int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (k >= count * vals) {
+        // a joined row's padding
+        const int64_t e = k - count * vals, pad = stride - vals;
+        if (!SPLIT && e < count * pad)
+            row_put(rows, (size_t)(row0 + e / pad) * stride + vals + e % pad, 0.0f);
+        return;
+    }
+    const int start[6] = {0, 3, 6, 10, 11, vals};
+    int q = 0;
+    while (k >= count * start[q + 1]) ++q;
+    const int w = start[q + 1] - start[q];
+    const int64_t j = k - count * start[q];
+    const size_t r = (size_t)(row0 + j / w) * stride + start[q] + j % w;
+    if (SPLIT) arrays[k] = row_get(rows, r);
+    else row_put(rows, r, arrays[k]);
+}
+
 }  // namespace
+
+hipError_t launch_train_rows(void* rows, int64_t row0, int64_t count, int sh_degree, float* arrays,
+                             bool split, bool bf16, hipStream_t st) {
+    if (count <= 0) return hipSuccess;
+    if (sh_degree < 0 || sh_degree > 3) return hipErrorInvalidValue;
+    const int vals = train_row_values(sh_degree), stride = train_row_floats(sh_degree);
+    const unsigned grid = (unsigned)((count * stride + 255) / 256);
+    if (split && bf16)
+        k_train_rows<uint16_t, true><<<grid, 256, 0, st>>>(static_cast<uint16_t*>(rows), row0,
+                                                           count, vals, stride, arrays);
+    else if (split)
+        k_train_rows<float, true><<<grid, 256, 0, st>>>(static_cast<float*>(rows), row0, count,
+                                                        vals, stride, arrays);
+    else if (bf16)
+        k_train_rows<uint16_t, false><<<grid, 256, 0, st>>>(static_cast<uint16_t*>(rows), row0,
+                                                            count, vals, stride, arrays);
+    else
+        k_train_rows<float, false><<<grid, 256, 0, st>>>(static_cast<float*>(rows), row0, count,
+                                                         vals, stride, arrays);
+    return hipGetLastError();
+}
 
 hipError_t launch_train_project(const TrainParamsDev& P, const TrainCam& cam, Compact out,
                                 float4* trec, uint32_t* cidx, uint8_t* visible,

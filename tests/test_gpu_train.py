@@ -415,3 +415,33 @@ def test_train_step_capacity_rerun():
             assert np.array_equal(m[k], np.float32(1.0 - 0.9) * g[k]), k
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("n,deg", [(1, 0), (3, 3), (5001, 2), (35_544, 3), (35_545, 3),
+                                   (95_000, 3), (91_181, 1)])
+def test_train_arrays_round_trip(gpu_ctx, n, deg):
+    """Parameters, moments (fp32 and bf16) and gradients come back as they were written:
+    one chunk of the staged transfer, its edge (35544 rows of degree 3 fill 8 MiB), several."""
+    print("train arrays", n, deg, flush=True)
+    rng = np.random.default_rng(n)
+    shp = {"means": (n, 3), "log_scales": (n, 3), "quats": (n, 4), "opacity_logits": (n,),
+           "sh": (n, (deg + 1) ** 2, 3)}
+    arrs = [{k: rng.standard_normal(s, dtype=np.float32) for k, s in shp.items()}
+            for _ in range(4)]
+    tr = L.Trainer(gpu_ctx, arrs[0], deg)
+    try:
+        for which in (1, 2, 3):
+            tr.write(which, arrs[which])
+        for which in range(4):
+            got = tr.read(which)
+            assert all(np.array_equal(got[k], arrs[which][k]) for k in shp), which
+        tr.set_moments(True)
+        got = tr.read(2)
+        assert all(np.array_equal(got[k], TO.bf16_round(arrs[2][k])) for k in shp)
+        tr.write(1, arrs[3])
+        got = tr.read(1)
+        assert all(np.array_equal(got[k], TO.bf16_round(arrs[3][k])) for k in shp)
+        got = tr.read(0)
+        assert all(np.array_equal(got[k], arrs[0][k]) for k in shp)
+    finally:
+        tr.set_moments(False)

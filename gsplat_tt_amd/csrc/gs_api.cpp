@@ -1128,7 +1128,8 @@ struct gs_ctx {
         // cleared by every frame: counters, compaction states, pairs per tile; by the
         // sorted ones also the histograms and the other states
         const size_t tile_words = ((size_t)T + 1) & ~size_t(1);
-        const size_t binned_words = kFrSums + kSumBytes / 4 + 2 * L.pparts + tile_words;
+        const size_t states = L.binned ? gs::project_states(N) : L.pparts;
+        const size_t binned_words = kFrSums + kSumBytes / 4 + 2 * states + tile_words;
         const size_t all_words = binned_words + 2048 + 2 * (L.rparts + L.eparts);
         b_frame.ensure(all_words * 4);
         L.fwords = L.binned ? binned_words : all_words;
@@ -1138,7 +1139,7 @@ struct gs_ctx {
         L.cnt = L.fr + kFrCnt;
         L.sums = reinterpret_cast<gs::TrainSums*>(L.fr + kFrSums);
         L.lb_proj = reinterpret_cast<uint64_t*>(L.fr + kFrSums + kSumBytes / 4);
-        L.tcnt = reinterpret_cast<uint32_t*>(L.lb_proj + L.pparts);
+        L.tcnt = reinterpret_cast<uint32_t*>(L.lb_proj + states);
         L.hist_depth = L.tcnt + tile_words;
         L.hist_tile = L.hist_depth + 1024;
         L.lb_rect = reinterpret_cast<uint64_t*>(L.hist_tile + 1024);
@@ -1423,7 +1424,7 @@ struct gs_ctx {
             HIPCHK(hipGraphGetNodes(fg.graph, nullptr, &nn));
             std::vector<hipGraphNode_t> nodes(nn);
             if (nn) HIPCHK(hipGraphGetNodes(fg.graph, nodes.data(), &nn));
-            const void* fn_proj = gs::project_kernel(sd.sh_degree, L.binned);
+            const void* fn_proj = gs::project_kernel(sd.sh_degree, L.binned, N);
             const void* fn_blend = gs::blend_kernel(pend.v.tile_size, pend.v.out_format,
                                                     blend_by_microblock(L));
             hipGraphNode_t proj = nullptr;

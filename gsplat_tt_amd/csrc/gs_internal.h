@@ -105,7 +105,7 @@ hipError_t launch_project(const SceneDev& s, const ProjParams& p, Compact out,
 // Captured frames (HIP graphs): the k_project instance launch_project uses for
 // an SH degree, and an update of a captured k_project node's view parameters
 // in an instantiated graph (the node's other arguments are kept).
-const void* project_kernel(int sh_degree, bool binned);
+const void* project_kernel(int sh_degree, bool binned, int64_t n);
 // The captured k_project node's scene and view arguments are s and p (its
 // argument layout is what graph_set_project_params assumes).
 bool graph_project_args_are(hipGraphNode_t node, const SceneDev& s, const ProjParams& p);
@@ -121,6 +121,10 @@ hipError_t launch_chunk_cull(const double* box, int64_t n, const ProjParams& p, 
 hipError_t launch_soa_transpose(const float* aos, int64_t n, int cols, const int* col_map,
                                 int planes, float* soa, hipStream_t st);
 size_t project_partitions(int64_t n);
+// Compaction states that a binned projection of n Gaussians may need.
+size_t project_states(int64_t n);
+// Gaussians per thread of a binned projection (the training's too).
+int project_items(int64_t n);
 hipError_t launch_brec_from_arrays(const float* means2d, const float* covs2d,
                                    const float* colors, const float* opac, const float* lthr,
                                    int64_t m, float4* brec, hipStream_t st);

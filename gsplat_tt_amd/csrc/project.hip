@@ -91,20 +91,21 @@ __device__ __forceinline__ void sh_eval(const float* __restrict__ rec, float x, 
 // also scans the visible Gaussians' tile counts in compact order: offs[m], the
 // emission's owner table and the candidate total (write_binned), the two prefixes
 // packed into one look-back descriptor.
-template <int DEG, bool BINNED>
+// ITEMS: Gaussians per thread, one for a small scene's binned frame (project_items).
+template <int DEG, bool BINNED, int ITEMS>
 __global__ __launch_bounds__(kProjThreads, BINNED ? 4 : 1) void k_project(SceneDev s, ProjParams p, Compact out,
                                                           uint8_t* __restrict__ valid_mask,
                                                           uint64_t* lb_state, uint32_t* ticket,
                                                           uint32_t* count_out,
                                                           uint32_t* __restrict__ part_hist) {
     __shared__ uint32_t s_vid;
-    __shared__ uint32_t s_cnt[kProjItems][kProjThreads / GS_WAVE];
+    __shared__ uint32_t s_cnt[ITEMS][kProjThreads / GS_WAVE];
     __shared__ uint32_t s_hist[BINNED ? 1 : 4][256];
-    __shared__ uint32_t s_ccnt[kProjItems][kProjThreads / GS_WAVE];
+    __shared__ uint32_t s_ccnt[ITEMS][kProjThreads / GS_WAVE];
     __shared__ uint64_t s_excl;
     // each item's projected values, held here over the colour evaluation (in
     // registers they would leave one workgroup per CU instead of two)
-    __shared__ float4 s_iv[2][kProjItems][kProjThreads];
+    __shared__ float4 s_iv[2][ITEMS][kProjThreads];
     const int tid = threadIdx.x;
     const int w = tid / GS_WAVE;
     const int lane = lane_id();
@@ -113,26 +114,26 @@ __global__ __launch_bounds__(kProjThreads, BINNED ? 4 : 1) void k_project(SceneD
         for (int i = tid; i < 4 * 256; i += kProjThreads) (&s_hist[0][0])[i] = 0;
     __syncthreads();
     const uint32_t vid = s_vid;
-    const int64_t base = (int64_t)vid * kProjPart;
+    const int64_t base = (int64_t)vid * (kProjThreads * ITEMS);
     const int64_t n = s.n;
     // a partition the view's frustum test rules out reads nothing: its Gaussians
     // are all invalid (it still publishes its zero count to the compaction)
-    const bool skipped = p.skip != nullptr && p.skip[vid] != 0;
+    const bool skipped = p.skip != nullptr && p.skip[base / kProjPart] != 0;
 
-    float vmx[kProjItems], vmy[kProjItems], vtz[kProjItems];
-    float va[kProjItems], vb[kProjItems], vc[kProjItems], vrx[kProjItems], vry[kProjItems];
-    bool valid[kProjItems];
-    uint64_t bal[kProjItems];
-    uint32_t coff[kProjItems];  // BINNED: the tile counts' prefix
+    float vmx[ITEMS], vmy[ITEMS], vtz[ITEMS];
+    float va[ITEMS], vb[ITEMS], vc[ITEMS], vrx[ITEMS], vry[ITEMS];
+    bool valid[ITEMS];
+    uint64_t bal[ITEMS];
+    uint32_t coff[ITEMS];  // BINNED: the tile counts' prefix
 
     // loads in two stages over all items: the means and opacities, then the
     // covariance words of the items that pass the depth and opacity tests
-    float ltx[kProjItems], lty[kProjItems], ltz[kProjItems];
-    bool lok[kProjItems];
+    float ltx[ITEMS], lty[ITEMS], ltz[ITEMS];
+    bool lok[ITEMS];
     {
-        float lmx[kProjItems], lmy[kProjItems], lmz[kProjItems], lop[kProjItems];
+        float lmx[ITEMS], lmy[ITEMS], lmz[ITEMS], lop[ITEMS];
 #pragma unroll
-        for (int it = 0; it < kProjItems; ++it) {
+        for (int it = 0; it < ITEMS; ++it) {
             const int64_t i = base + it * kProjThreads + tid;
             const bool in = i < n && !skipped;
             lmx[it] = in ? s.mean[0][i] : 0.0f;
@@ -141,7 +142,7 @@ __global__ __launch_bounds__(kProjThreads, BINNED ? 4 : 1) void k_project(SceneD
             lop[it] = (in && p.has_opac) ? s.opac[i] : 1.0f;
         }
 #pragma unroll
-        for (int it = 0; it < kProjItems; ++it) {
+        for (int it = 0; it < ITEMS; ++it) {
             const int64_t i = base + it * kProjThreads + tid;
             const float mx = lmx[it], my = lmy[it], mz = lmz[it];
             const float rmx = mx * p.r[0] + my * p.r[1] + mz * p.r[2];
@@ -155,9 +156,9 @@ __global__ __launch_bounds__(kProjThreads, BINNED ? 4 : 1) void k_project(SceneD
             lok[it] = ok;
         }
     }
-    float lc[6][kProjItems], lk[kProjItems];
+    float lc[6][ITEMS], lk[ITEMS];
 #pragma unroll
-    for (int it = 0; it < kProjItems; ++it) {
+    for (int it = 0; it < ITEMS; ++it) {
         const int64_t i = base + it * kProjThreads + tid;
 #pragma unroll
         for (int q = 0; q < 6; ++q) lc[q][it] = lok[it] ? s.cov[q][i] : 0.0f;
@@ -165,7 +166,7 @@ __global__ __launch_bounds__(kProjThreads, BINNED ? 4 : 1) void k_project(SceneD
     }
 
 #pragma unroll
-    for (int it = 0; it < kProjItems; ++it) {
+    for (int it = 0; it < ITEMS; ++it) {
         const int64_t i = base + it * kProjThreads + tid;
         valid[it] = false;
         vmx[it] = vmy[it] = vtz[it] = va[it] = vb[it] = vc[it] = vrx[it] = vry[it] = 0.0f;
@@ -266,22 +267,22 @@ __global__ __launch_bounds__(kProjThreads, BINNED ? 4 : 1) void k_project(SceneD
     // exclusive prefixes of the (item, wave) counts in source order: lane
     // it * waves + w of a wave scan
     constexpr int kWaves = kProjThreads / GS_WAVE;
-    static_assert(kProjItems * kWaves <= GS_WAVE, "one count per lane");
-    uint32_t total, my_off[kProjItems];
+    static_assert(ITEMS * kWaves <= GS_WAVE, "one count per lane");
+    uint32_t total, my_off[ITEMS];
     uint64_t ctotal = 0;
     {
-        const uint32_t c = lane < kProjItems * kWaves ? (&s_cnt[0][0])[lane] : 0u;
+        const uint32_t c = lane < ITEMS * kWaves ? (&s_cnt[0][0])[lane] : 0u;
         const uint32_t incl = wave_incl_scan(c);
         total = (uint32_t)__builtin_amdgcn_readlane((int)incl, GS_WAVE - 1);
 #pragma unroll
-        for (int it = 0; it < kProjItems; ++it)
+        for (int it = 0; it < ITEMS; ++it)
             my_off[it] = (uint32_t)__builtin_amdgcn_readlane((int)(incl - c), it * kWaves + w);
         if constexpr (BINNED) {
-            const uint32_t cc = lane < kProjItems * kWaves ? (&s_ccnt[0][0])[lane] : 0u;
+            const uint32_t cc = lane < ITEMS * kWaves ? (&s_ccnt[0][0])[lane] : 0u;
             const uint32_t ci = wave_incl_scan(cc);
             ctotal = (uint32_t)__builtin_amdgcn_readlane((int)ci, GS_WAVE - 1);
 #pragma unroll
-            for (int it = 0; it < kProjItems; ++it)
+            for (int it = 0; it < ITEMS; ++it)
                 coff[it] += (uint32_t)__builtin_amdgcn_readlane((int)(ci - cc), it * kWaves + w);
         }
     }
@@ -290,9 +291,9 @@ __global__ __launch_bounds__(kProjThreads, BINNED ? 4 : 1) void k_project(SceneD
     // (the SH records, the kernel's largest reads) are evaluated before the
     // walk over the predecessors, so that the walk finds them mostly done.
     if (w == 0) lookback_publish(lb_state, vid, agg);
-    float vr[kProjItems], vg[kProjItems], vbl[kProjItems];
+    float vr[ITEMS], vg[ITEMS], vbl[ITEMS];
 #pragma unroll
-    for (int it = 0; it < kProjItems; ++it) {
+    for (int it = 0; it < ITEMS; ++it) {
         vr[it] = vg[it] = vbl[it] = 0.0f;
         if (!valid[it]) continue;
         const int64_t i = base + it * kProjThreads + tid;
@@ -331,7 +332,7 @@ __global__ __launch_bounds__(kProjThreads, BINNED ? 4 : 1) void k_project(SceneD
     const uint64_t lt_mask = lanemask_lt();
 
 #pragma unroll
-    for (int it = 0; it < kProjItems; ++it) {
+    for (int it = 0; it < ITEMS; ++it) {
         if (!valid[it]) continue;
         const int64_t i = base + it * kProjThreads + tid;
         const uint64_t m = excl + my_off[it] + (uint64_t)__popcll(bal[it] & lt_mask);
@@ -524,14 +525,15 @@ hipError_t launch_project(const SceneDev& s, const ProjParams& p, Compact out,
                           uint8_t* valid_mask, uint64_t* lb_state, uint32_t* ticket,
                           uint32_t* count_out, uint32_t* part_hist, hipStream_t st) {
     if (s.n <= 0) return hipSuccess;
-    const unsigned grid = (unsigned)((s.n + kProjPart - 1) / kProjPart);
-#define GS_PROJECT(D)                                                                         \
-    if (p.binned.offs != nullptr)                                                             \
-        k_project<D, true><<<grid, kProjThreads, 0, st>>>(s, p, out, valid_mask, lb_state,    \
-                                                          ticket, count_out, part_hist);      \
-    else                                                                                      \
-        k_project<D, false><<<grid, kProjThreads, 0, st>>>(s, p, out, valid_mask, lb_state,   \
-                                                           ticket, count_out, part_hist)
+    const int items = p.binned.offs != nullptr ? project_items(s.n) : kProjItems;
+    const unsigned grid = (unsigned)((s.n + kProjThreads * items - 1) / (kProjThreads * items));
+#define GS_PROJECT_I(D, B, I)                                                               \
+    k_project<D, B, I><<<grid, kProjThreads, 0, st>>>(s, p, out, valid_mask, lb_state,      \
+                                                      ticket, count_out, part_hist)
+#define GS_PROJECT(D)                                                                       \
+    if (p.binned.offs == nullptr) GS_PROJECT_I(D, false, kProjItems);                       \
+    else if (items == 1) GS_PROJECT_I(D, true, 1);                                          \
+    else GS_PROJECT_I(D, true, kProjItems)
     switch (s.sh_degree) {
         case -1: GS_PROJECT(-1); break;
         case 0: GS_PROJECT(0); break;
@@ -541,24 +543,37 @@ hipError_t launch_project(const SceneDev& s, const ProjParams& p, Compact out,
         default: return hipErrorInvalidValue;
     }
 #undef GS_PROJECT
+#undef GS_PROJECT_I
     return hipGetLastError();
 }
 
 size_t project_partitions(int64_t n) { return (size_t)((n + kProjPart - 1) / kProjPart); }
+// One Gaussian per thread up to 256K, where partitions of four leave most CUs idle
+// (20K: 10 workgroups) and a thread's four in a row are the kernel's latency: a 20K
+// frame 79 -> 74 us, 100K 195 -> 188, a 100K path 1263 -> 1218. At 300K the two are
+// equal (800 us a stream), at 1M the longer look-back costs 9% (220 -> 240 us a frame).
+// Sorted frames keep four: their digit counts are one row per partition.
+int project_items(int64_t n) { return n <= (1 << 18) ? 1 : kProjItems; }
+size_t project_states(int64_t n) {
+    const int64_t part = (int64_t)kProjThreads * project_items(n);
+    return (size_t)((n + part - 1) / part);
+}
 
-template <bool BINNED>
+template <bool BINNED, int ITEMS>
 static const void* project_instance(int sh_degree) {
     switch (sh_degree) {
-        case -1: return reinterpret_cast<const void*>(&k_project<-1, BINNED>);
-        case 0: return reinterpret_cast<const void*>(&k_project<0, BINNED>);
-        case 1: return reinterpret_cast<const void*>(&k_project<1, BINNED>);
-        case 2: return reinterpret_cast<const void*>(&k_project<2, BINNED>);
-        case 3: return reinterpret_cast<const void*>(&k_project<3, BINNED>);
+        case -1: return reinterpret_cast<const void*>(&k_project<-1, BINNED, ITEMS>);
+        case 0: return reinterpret_cast<const void*>(&k_project<0, BINNED, ITEMS>);
+        case 1: return reinterpret_cast<const void*>(&k_project<1, BINNED, ITEMS>);
+        case 2: return reinterpret_cast<const void*>(&k_project<2, BINNED, ITEMS>);
+        case 3: return reinterpret_cast<const void*>(&k_project<3, BINNED, ITEMS>);
         default: return nullptr;
     }
 }
-const void* project_kernel(int sh_degree, bool binned) {
-    return binned ? project_instance<true>(sh_degree) : project_instance<false>(sh_degree);
+const void* project_kernel(int sh_degree, bool binned, int64_t n) {
+    if (!binned) return project_instance<false, kProjItems>(sh_degree);
+    return project_items(n) == 1 ? project_instance<true, 1>(sh_degree)
+                                 : project_instance<true, kProjItems>(sh_degree);
 }
 
 bool graph_project_args_are(hipGraphNode_t node, const SceneDev& s, const ProjParams& p) {

@@ -22,7 +22,7 @@ namespace {
 constexpr int kTThreads = 512;
 constexpr int kTItems = 4;
 constexpr int kTPart = kTThreads * kTItems;
-static_assert(kTPart == (int)kProjPartition, "projection partition size");
+static_assert(kTPart == (int)kProjPartition && kTThreads == 512, "projection partition size");
 
 constexpr float kC0 = 0.28209479177387814f;
 constexpr float kC1 = 0.4886025119029199f;
@@ -227,16 +227,17 @@ __device__ __forceinline__ float sigmoidf(float x) { return 1.0f / (1.0f + expf(
 // count published, then the colours of the kept rows, which are the largest
 // reads, then the walk over the predecessors. BINNED as there.
 // (1M Gaussians, SH1: 48.5 -> 40.3 us; with the tile counts' scan.)
-template <int DEG, bool BINNED>
+// ITEMS as there too (a 20K step's loop 1263 -> 1235 us, a 50K gradient call 722 -> 713).
+template <int DEG, bool BINNED, int ITEMS>
 __global__ __launch_bounds__(kTThreads, 4) void k_train_project(
     TrainParamsDev P, TrainCam cam, Compact out, float4* __restrict__ trec,
     uint32_t* __restrict__ cidx, uint8_t* __restrict__ visible, uint64_t* lb_state,
     uint32_t* ticket, uint32_t* count_out, uint32_t* __restrict__ part_hist, TrainDebug dbg) {
     constexpr int V = Row<DEG>::V, kWaves = kTThreads / GS_WAVE;
     __shared__ uint32_t s_vid;
-    __shared__ uint32_t s_cnt[kTItems][kWaves], s_ccnt[kTItems][kWaves];
+    __shared__ uint32_t s_cnt[ITEMS][kWaves], s_ccnt[ITEMS][kWaves];
     __shared__ uint32_t s_hist[BINNED ? 1 : 4][256];
-    __shared__ float4 s_iv[2][kTItems][kTThreads];
+    __shared__ float4 s_iv[2][ITEMS][kTThreads];
     __shared__ uint64_t s_excl;
     const int tid = threadIdx.x, w = tid / GS_WAVE, lane = lane_id();
     if (tid == 0) s_vid = atomicAdd(ticket, 1u);
@@ -244,19 +245,19 @@ __global__ __launch_bounds__(kTThreads, 4) void k_train_project(
         for (int k = tid; k < 1024; k += kTThreads) (&s_hist[0][0])[k] = 0;
     __syncthreads();
     const uint32_t vid = s_vid;
-    const int64_t base = (int64_t)vid * kTPart;
+    const int64_t base = (int64_t)vid * (kTThreads * ITEMS);
     const int64_t n = P.n;
-    bool keep[kTItems];
-    float ops[kTItems], m2[kTItems];
-    uint32_t coff[kTItems];
-    uint64_t bal[kTItems];
+    bool keep[ITEMS];
+    float ops[ITEMS], m2[ITEMS];
+    uint32_t coff[ITEMS];
+    uint64_t bal[ITEMS];
     // the heads of a thread's rows together (past the end: the last row's)
-    Head head[kTItems];
+    Head head[ITEMS];
 #pragma unroll
-    for (int it = 0; it < kTItems; ++it)
+    for (int it = 0; it < ITEMS; ++it)
         head[it] = load_head(P.rows + min(base + it * kTThreads + tid, n - 1) * V);
 #pragma unroll
-    for (int it = 0; it < kTItems; ++it) {
+    for (int it = 0; it < ITEMS; ++it) {
         const int64_t i = base + it * kTThreads + tid;
         Geo g;
         geometry(head[it], cam, g);
@@ -321,30 +322,30 @@ __global__ __launch_bounds__(kTThreads, 4) void k_train_project(
             part_hist[(size_t)vid * 1024 + k] = (&s_hist[0][0])[k];
     // exclusive prefixes of the (item, wave) counts in source order: lane
     // it * waves + w of a wave scan
-    static_assert(kTItems * kWaves <= GS_WAVE, "one count per lane");
-    uint32_t total, my_off[kTItems];
+    static_assert(ITEMS * kWaves <= GS_WAVE, "one count per lane");
+    uint32_t total, my_off[ITEMS];
     uint64_t ctotal = 0;
     {
-        const uint32_t c = lane < kTItems * kWaves ? (&s_cnt[0][0])[lane] : 0u;
+        const uint32_t c = lane < ITEMS * kWaves ? (&s_cnt[0][0])[lane] : 0u;
         const uint32_t incl = wave_incl_scan(c);
         total = (uint32_t)__builtin_amdgcn_readlane((int)incl, GS_WAVE - 1);
 #pragma unroll
-        for (int it = 0; it < kTItems; ++it)
+        for (int it = 0; it < ITEMS; ++it)
             my_off[it] = (uint32_t)__builtin_amdgcn_readlane((int)(incl - c), it * kWaves + w);
         if constexpr (BINNED) {
-            const uint32_t cc = lane < kTItems * kWaves ? (&s_ccnt[0][0])[lane] : 0u;
+            const uint32_t cc = lane < ITEMS * kWaves ? (&s_ccnt[0][0])[lane] : 0u;
             const uint32_t ci = wave_incl_scan(cc);
             ctotal = (uint32_t)__builtin_amdgcn_readlane((int)ci, GS_WAVE - 1);
 #pragma unroll
-            for (int it = 0; it < kTItems; ++it)
+            for (int it = 0; it < ITEMS; ++it)
                 coff[it] += (uint32_t)__builtin_amdgcn_readlane((int)(ci - cc), it * kWaves + w);
         }
     }
     const uint64_t agg = BINNED ? binned_pack(total, ctotal) : (uint64_t)total;
     if (w == 0) lookback_publish(lb_state, vid, agg);
-    float col[kTItems][3];
+    float col[ITEMS][3];
 #pragma unroll
-    for (int it = 0; it < kTItems; ++it) {
+    for (int it = 0; it < ITEMS; ++it) {
         if (!keep[it]) continue;
         const float4* row = P.rows + (base + it * kTThreads + tid) * V;
         float dir[3], dn;
@@ -366,7 +367,7 @@ __global__ __launch_bounds__(kTThreads, 4) void k_train_project(
     const uint64_t excl = BINNED ? binned_count(s_excl) : s_excl;
     const uint64_t ltm = lanemask_lt();
 #pragma unroll
-    for (int it = 0; it < kTItems; ++it) {
+    for (int it = 0; it < ITEMS; ++it) {
         if (!keep[it]) continue;
         const int64_t i = base + it * kTThreads + tid;
         const uint64_t m = excl + my_off[it] + (uint64_t)__popcll(bal[it] & ltm);
@@ -1227,16 +1228,16 @@ hipError_t launch_train_project(const TrainParamsDev& P, const TrainCam& cam, Co
                                 uint64_t* lb_state, uint32_t* ticket, uint32_t* count_out,
                                 uint32_t* part_hist, const TrainDebug& dbg, hipStream_t st) {
     if (P.n <= 0) return hipSuccess;
-    const unsigned grid = (unsigned)((P.n + kTPart - 1) / kTPart);
+    const int items = cam.binned.offs != nullptr ? project_items(P.n) : kTItems;
+    const unsigned grid = (unsigned)((P.n + kTThreads * items - 1) / (kTThreads * items));
+#define GS_TP_I(D, B, I)                                                                   \
+    k_train_project<D, B, I><<<grid, kTThreads, 0, st>>>(P, cam, out, trec, cidx, visible,  \
+                                                         lb_state, ticket, count_out,      \
+                                                         part_hist, dbg)
 #define GS_TP(D)                                                                           \
-    if (cam.binned.offs != nullptr)                                                        \
-        k_train_project<D, true><<<grid, kTThreads, 0, st>>>(P, cam, out, trec, cidx,      \
-                                                             visible, lb_state, ticket,    \
-                                                             count_out, part_hist, dbg);   \
-    else                                                                                   \
-        k_train_project<D, false><<<grid, kTThreads, 0, st>>>(P, cam, out, trec, cidx,     \
-                                                              visible, lb_state, ticket,   \
-                                                              count_out, part_hist, dbg)
+    if (cam.binned.offs == nullptr) GS_TP_I(D, false, kTItems);                            \
+    else if (items == 1) GS_TP_I(D, true, 1);                                              \
+    else GS_TP_I(D, true, kTItems)
     switch (P.sh_degree) {
         case 0: GS_TP(0); break;
         case 1: GS_TP(1); break;
@@ -1245,6 +1246,7 @@ hipError_t launch_train_project(const TrainParamsDev& P, const TrainCam& cam, Co
         default: return hipErrorInvalidValue;
     }
 #undef GS_TP
+#undef GS_TP_I
     return hipGetLastError();
 }
 

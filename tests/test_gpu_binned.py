@@ -59,6 +59,25 @@ def test_lists_around_the_runs(gpu_ctx, n, levels):
         _equal(a, b)
 
 
+@pytest.mark.parametrize("n,deg", [(511, 0), (512, 1), (1025, 2), (1 << 18, 3), (1 << 18, -1),
+                                   ((1 << 18) + 1, 2)])
+def test_projection_partitions(gpu_ctx, n, deg):
+    """Binned projection by one and by four Gaussians a thread (the line is at 2^18)
+    against the sorted frames', at whole and ragged partitions and every colour form."""
+    print("partitions", n, deg, flush=True)
+    rng = np.random.default_rng(n)
+    means, cov, op, col = _stack(n, 300, spread=0.3, seed=n)
+    means[:, 2] *= np.where(rng.random(n) < 0.2, -1, 1)  # a fifth behind the camera
+    if deg >= 0:
+        col = rng.uniform(-0.5, 0.5, (n, (deg + 1) ** 2, 3)).astype(np.float32)
+    gpu_ctx.set_scene(means, cov, op, col, sh_degree=deg)
+    K = scenes.intrinsics(200, 200, 120, 67)
+    view = L.make_view(np.eye(4, dtype=np.float32), K, 135, 241, tile_size=16, output="f32")
+    a, b = _both(gpu_ctx, view)
+    assert a[1]["num_visible"] > n // 2
+    _equal(a, b)
+
+
 def test_many_tiles_and_empty_views(gpu_ctx):
     """Close to the most tiles of a binned frame (127 x 129 = 16383 of 16384), one row of
     tiles past it (sorted either way), and a view with nothing visible."""

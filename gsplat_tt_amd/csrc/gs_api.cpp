@@ -578,7 +578,7 @@ struct gs_ctx {
     static constexpr size_t kFrSums = 64;  // a training forward's TrainSums
     enum : int {
         C_PROJ_TICKET = 0, C_M = 1, C_SKIPPED = 2, C_CTL = 4, C_RECT_TICKET = 8, C_PPRE = 9,
-        C_EMIT_TICKET = 10, C_P = 11, C_RUNS = 12, C_DSORT_TICKETS = 16, C_TSORT_TICKETS = 24,
+        C_EMIT_TICKET = 10, C_P = 11, C_RUNS = 12, C_ITEMS = 13, C_KITEMS = 14, C_SEGS = 15, C_DSORT_TICKETS = 16, C_TSORT_TICKETS = 24,
         C_MBSTAT = 40  // two u64: pairs no microblock keeps, kept (pair, microblock)
     };
     uint64_t pair_cap = 0;  // candidate-pair capacity of the frame buffers
@@ -1061,24 +1061,34 @@ struct gs_ctx {
         gs::TrainSums* sums;  // a training forward's, after the counters
         uint64_t *lb_proj, *lb_rect, *lb_emit;
         uint32_t* tcnt;  // pairs per tile
+        uint32_t* bcnt;  // blocks: items per block
         uint32_t *hist_depth, *hist_tile;  // [4][256] depth-key, [2 or 4][256] tile-id digits
         uint32_t* runs;      // binned: runs of the long tile lists
         size_t fwords;       // words that a frame clears
         size_t pparts, rparts, eparts;
         uint32_t pcap;
         bool binned;
+        bool blocks;   // sorted by blocks of tiles (not the microblock statistics' frames)
+        int key_bits;  // of the sorted tile (block) ids
     };
     // Whether frames of N Gaussians and T tiles have their tile lists binned
-    // (launch_binned_lists) or sorted. Binning saves the sorts' launches and passes
-    // but stores each pair at its list's end and sorts each list on its own, so it
-    // wins up to about 2.4M pairs (us a frame alone and in a path, sorted against
-    // binned; 1280x720: 1.1M pairs 331, 219 / 263, 187; 1.7M 390, 250 / 313, 221;
-    // 2.8M 464, 308 / 402, 290; 1237x822: 1.5M 287, 177 / 227, 152; 3.0M 347, 238 /
-    // 348, 254; 5.0M 431, 310 / 515, 398; 400x300, 3100 pairs a tile: 1.5M 388,
-    // 241 / 403, 234). The pairs of a view are not known before it is rendered: a
-    // scene's frames start from the number of Gaussians and go on with the pairs
-    // of the frames that finished, with a gap between the two limits so that a
-    // camera path does not alternate.
+    // (launch_binned_lists) or made by blocks of tiles (block_tiles). Binning needs
+    // no depth sort and fewer launches but stores each pair at its list's end and
+    // sorts each list on its own, so it wins up to about 2.4M pairs (us a frame
+    // alone and in a path, blocks against binned; 1280x720: 1.1M pairs 317, 213 /
+    // 243, 186; 1.7M 366, 246 / 294, 227; 2.8M 434, 295 / 380, 291; 1237x822: 1.5M
+    // 263, 173 / 201, 156; 3.0M 314, 221 / 320, 255; 5.0M 367, 276 / 477, 407;
+    // 400x300, 3100 pairs a tile: 1.5M 283, 234 / 294, 186). The pairs of a view are
+    // not known before it is rendered: a scene's frames start from the number of
+    // Gaussians and go on with the pairs of the frames that finished, with a gap
+    // between the two limits so that a camera path does not alternate.
+    // Frames that are not binned sort every pair by its tile only for the microblock
+    // statistics, which read the sorted keys, and above 2^16 tiles, where few pairs
+    // share a tile (us a frame alone and in a path, pairs against blocks; 1237x822:
+    // 3.0M pairs 318, 237 / 314, 221; 15M 723, 582 / 623, 475; 30M 1264, 985 / 990,
+    // 775; 1920x1080, 54M 1727, 1467 / 1208, 961; Gaussians of about one tile,
+    // 300x200 in tiles of 32, 4.6M: 1197, 1546 / 1119, 1448).
+    static constexpr int64_t kBlockTilesMost = 1 << 16;
     static constexpr int64_t kBinnedFirst = 1 << 20, kBinnedMost = 2400000,
                              kBinnedAgain = 1800000;
     struct TilePlan {
@@ -1097,10 +1107,14 @@ struct gs_ctx {
         if (P > kBinnedMost) p.binned = false;
         if (P < kBinnedAgain) p.binned = true;
     }
-    FrameLayout frame_prepare(int64_t N, int64_t T, bool want_keys) {
+    FrameLayout frame_prepare(int64_t N, int tiles_x, int tiles_y, bool want_keys) {
         FrameLayout L{};
+        const int64_t T = (int64_t)tiles_x * tiles_y;
         L.pcap = (uint32_t)pair_cap;
         L.binned = binned_frame(N, T, want_keys);
+        const int64_t nb = ((int64_t)tiles_x + 3) / 4 * (((int64_t)tiles_y + 3) / 4);
+        L.blocks = !L.binned && !want_keys && T <= kBlockTilesMost;
+        L.key_bits = tile_bits(L.blocks ? nb : T);
         L.pparts = gs::project_partitions(N);
         L.rparts = gs::rect_scan_partitions(N);
         L.eparts = gs::emit_partitions(L.pcap);
@@ -1118,19 +1132,22 @@ struct gs_ctx {
             b_bins.ensure(gs::binned_scratch_words(L.pcap, T) * 4);
         } else {
             b_phist_proj.ensure(L.pparts * 1024 * 4);
-            b_phist_emit.ensure(L.eparts * gs::tile_hist_cols(tile_bits(T)) * 4);
+            b_phist_emit.ensure(L.eparts * gs::tile_hist_cols(L.key_bits) * 4);
             b_pchunk.ensure(gs::reduce_chunks((uint32_t)L.eparts) *
-                            gs::tile_hist_cols(tile_bits(T)) * 4);
+                            gs::tile_hist_cols(L.key_bits) * 4);
             b_poffs.ensure(((L.eparts + kEmitPerSort - 1) / kEmitPerSort)
-                           << gs::sort_digit_width(tile_bits(T))
+                           << gs::sort_digit_width(L.key_bits)
                            << 2);
+            if (L.blocks) b_bins.ensure(gs::block_scratch_words(L.pcap, (uint32_t)nb) * 4);
         }
         // cleared by every frame: counters, compaction states, pairs per tile; by the
         // sorted ones also the histograms and the other states
         const size_t tile_words = ((size_t)T + 1) & ~size_t(1);
         const size_t states = L.binned ? gs::project_states(N) : L.pparts;
         const size_t binned_words = kFrSums + kSumBytes / 4 + 2 * states + tile_words;
-        const size_t all_words = binned_words + 2048 + 2 * (L.rparts + L.eparts);
+        const size_t block_words = L.blocks ? ((size_t)nb + 1) & ~size_t(1) : 0;
+        const size_t all_words = binned_words + block_words + 2048 +
+                                 2 * (L.rparts + std::max({L.rparts, L.pparts, L.eparts}));
         b_frame.ensure(all_words * 4);
         L.fwords = L.binned ? binned_words : all_words;
         ensure_sort(std::max<int64_t>(N, L.pcap), 4);
@@ -1140,12 +1157,29 @@ struct gs_ctx {
         L.sums = reinterpret_cast<gs::TrainSums*>(L.fr + kFrSums);
         L.lb_proj = reinterpret_cast<uint64_t*>(L.fr + kFrSums + kSumBytes / 4);
         L.tcnt = reinterpret_cast<uint32_t*>(L.lb_proj + states);
-        L.hist_depth = L.tcnt + tile_words;
+        L.bcnt = L.tcnt + tile_words;
+        L.hist_depth = L.bcnt + block_words;
         L.hist_tile = L.hist_depth + 1024;
         L.lb_rect = reinterpret_cast<uint64_t*>(L.hist_tile + 1024);
         L.lb_emit = L.lb_rect + L.rparts;
         L.runs = reinterpret_cast<uint32_t*>(L.lb_emit);  // a binned frame scans no partitions
         return L;
+    }
+
+    // Depth order of the visible Gaussians (stable: ties keep index order). The
+    // values are the projection's packed ones when tp.idx_bits is set, else the
+    // compact indices 0..M-1; the sorted depth keys are not needed, so the last
+    // pass writes the values only.
+    uint32_t* depth_order(const FrameLayout& L, int64_t N, const gs::TileParams& tp) {
+        uint32_t* cnt = L.cnt;
+        sort.ctl = cnt + C_CTL;
+        void* kf = nullptr;
+        uint32_t* order = nullptr;
+        HIPCHK(gs::radix_sort_pairs_dev(b_dkey.p, b_tmp_a.as<uint32_t>(), N, cnt + C_M, 4, 0, 32,
+                                        L.hist_depth, cnt + C_DSORT_TICKETS, sort, st,
+                                        tp.idx_bits == 0, &kf, &order, nullptr, nullptr, nullptr,
+                                        0xFFFFFFFFu, false));
+        return order;
     }
 
     // From the compact records of the M visible Gaussians (count on the device at
@@ -1161,17 +1195,8 @@ struct gs_ctx {
         const bool want_keys = tiles_out != nullptr;
         uint32_t* cnt = L.cnt;
         if (L.binned) return binned_tiles(L, N, T, tp, report);
-        sort.ctl = cnt + C_CTL;
-        // depth order of the visible Gaussians (stable: ties keep index order)
-        // (values: the projection's packed ones when tp.idx_bits is set, else
-        // the compact indices 0..M-1); the sorted depth keys are not needed, so
-        // the last pass writes the values only
-        void* kf = nullptr;
-        uint32_t* order = nullptr;
-        HIPCHK(gs::radix_sort_pairs_dev(b_dkey.p, b_tmp_a.as<uint32_t>(), N, cnt + C_M, 4, 0, 32,
-                                        L.hist_depth, cnt + C_DSORT_TICKETS, sort, st,
-                                        tp.idx_bits == 0, &kf, &order, nullptr, nullptr, nullptr,
-                                        0xFFFFFFFFu, false));
+        if (L.blocks) return block_tiles(L, N, tp, report);
+        uint32_t* order = depth_order(L, N, tp);
         record(2);
         HIPCHK(gs::launch_rect_count_scan(b_rc.as<float4>(), 2, order, N, cnt + C_M, tp,
                                           b_offs.as<uint32_t>(), b_bstart.as<uint32_t>(),
@@ -1215,6 +1240,47 @@ struct gs_ctx {
         return ids_sorted;
     }
 
+    // frame_tiles of a sorted frame without a caller for the keys: Gaussians emitted
+    // by blocks of tiles in depth order, sorted by block, split into the tiles' lists.
+    uint32_t* block_tiles(const FrameLayout& L, int64_t N, const gs::TileParams& tp,
+                          const gs::HostCopy& report) {
+        uint32_t* cnt = L.cnt;
+        const uint32_t nb = gs::num_blocks(tp.tiles_x, tp.tiles_y);
+        uint32_t* order = depth_order(L, N, tp);
+        record(2);
+        HIPCHK(gs::launch_block_scan(b_rc.as<float4>(), order, N, cnt + C_M, tp,
+                                     b_offs.as<uint32_t>(), b_bstart.as<uint32_t>(),
+                                     (uint32_t)(L.eparts + 1), L.lb_rect, L.lb_emit,
+                                     tp.idx_bits ? (uint32_t)L.pparts : 0u, cnt + C_ITEMS, cnt + C_PPRE, L.pcap, st));
+        HIPCHK(gs::launch_block_emit(b_rc.as<float4>(), order, b_offs.as<uint32_t>(),
+                                     b_bstart.as<uint32_t>(), N, cnt + C_M, L.pcap, cnt + C_ITEMS,
+                                     tp, b_pair_tile.as<uint32_t>(), b_pair_id.as<uint32_t>(),
+                                     cnt + C_KITEMS, cnt + C_P, b_phist_emit.as<uint32_t>(),
+                                     L.key_bits, st));
+        const int hcols = gs::tile_hist_cols(L.key_bits), dw = gs::sort_digit_width(L.key_bits);
+        HIPCHK(gs::launch_reduce_rows(b_phist_emit.as<uint32_t>(), hcols, (uint32_t)L.eparts,
+                                      cnt + C_ITEMS, L.pcap, gs::kEmitPartition, dw, L.hist_tile,
+                                      st, b_pchunk.as<uint32_t>(), cnt + C_CTL));
+        HIPCHK(gs::launch_part_offsets(b_phist_emit.as<uint32_t>(), hcols, (uint32_t)L.eparts,
+                                       cnt + C_ITEMS, L.pcap, gs::kEmitPartition, kEmitPerSort,
+                                       dw, b_pchunk.as<uint32_t>(), L.hist_tile,
+                                       b_poffs.as<uint32_t>(), st, cnt + C_CTL));
+        record(3);
+        void* keys = nullptr;
+        uint32_t* ids = nullptr;
+        HIPCHK(gs::radix_sort_pairs_dev(b_pair_tile.p, b_pair_id.as<uint32_t>(), L.pcap,
+                                        cnt + C_ITEMS, 4, 16, 16 + L.key_bits, L.hist_tile,
+                                        cnt + C_TSORT_TICKETS, sort, st, false, &keys, &ids,
+                                        cnt + C_KITEMS, L.bcnt,
+                                        b_poffs.as<uint32_t>(), nb, true, 16));
+        uint32_t* out = ids == b_pair_id.as<uint32_t>() ? b_valt.as<uint32_t>()
+                                                        : b_pair_id.as<uint32_t>();
+        HIPCHK(gs::launch_block_lists(static_cast<uint32_t*>(keys), ids, L.pcap,
+                                      L.bcnt, b_bins.as<uint32_t>(), cnt + C_SEGS, tp, L.tcnt,
+                                      b_ranges.as<uint32_t>(), out, report, st));
+        return out;
+    }
+
     // frame_tiles of a binned frame, whose projection scanned the candidates:
     // pair emission in compact order, then the tiles' lists sorted one by one.
     uint32_t* binned_tiles(const FrameLayout& L, int64_t N, int64_t T, const gs::TileParams& tp,
@@ -1252,6 +1318,7 @@ struct gs_ctx {
         p.tile_size = v->tile_size;
         p.idx_bits = dval_idx_bits(N);
         p.dvals = p.idx_bits && !L.binned ? b_tmp_a.as<uint32_t>() : nullptr;
+        p.tile_sums = L.blocks && p.dvals ? L.lb_emit : nullptr;
         p.binned = binned_out(L);
         return p;
     }
@@ -1343,7 +1410,7 @@ struct gs_ctx {
             return false;
         if (sd.chunk_box != nullptr && pend.v.k_cap <= 3.0f) return false;
         if (N >= ((int64_t)1 << 30) || pair_cap >= (1ull << 30)) return false;
-        const FrameLayout L = frame_prepare(N, pend.T, false);  // every allocation before a capture
+        const FrameLayout L = frame_prepare(N, pend.tiles_x, pend.tiles_y, false);  // every allocation before a capture
         const gs_view shape = graph_shape(&pend.v);
         const uint64_t gen = buffers_key();
         const bool same_shape = fg.n == N && fg.T == pend.T && fg.deg == sd.sh_degree && fg.pcap == pair_cap && fg.gen == gen &&
@@ -1461,7 +1528,7 @@ struct gs_ctx {
     // ranges -> blend) on the stream; no host synchronisation.
     void frame(const gs_view* v, void* dout, int64_t T, int tiles_x, int tiles_y) {
         const int64_t N = sd.n;
-        const FrameLayout L = frame_prepare(N, T, cull_stats);
+        const FrameLayout L = frame_prepare(N, tiles_x, tiles_y, cull_stats);
         record(0);
         HIPCHK(gs::launch_fill_u32(L.fr, 0u, L.fwords, st));
         if (spin_limit) HIPCHK(gs::launch_fill_u32(L.cnt + C_CTL + 1, spin_limit, 1, st));
@@ -1778,7 +1845,7 @@ struct gs_ctx {
         tr.tiles_y = (H + 15) / 16;
         const int64_t T = (int64_t)tr.tiles_x * tr.tiles_y;
         tr.cam = train_cam(v, c);
-        const FrameLayout L = frame_prepare(std::max<int64_t>(N, 1), T, false);
+        const FrameLayout L = frame_prepare(std::max<int64_t>(N, 1), tr.tiles_x, tr.tiles_y, false);
         const size_t px = (size_t)H * W;
         t_img.ensure(px * 12);
         t_T.ensure(px * 4);

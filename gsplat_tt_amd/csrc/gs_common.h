@@ -101,8 +101,14 @@ __device__ __forceinline__ Rect tile_rect(float4 r, int tiles_x, int tiles_y, co
     return o;
 }
 
+// Blocks of 4 x 4 tiles that a rectangle of tiles touches.
+constexpr int kBlk = 4;
+__device__ __forceinline__ uint32_t block_cells(const Rect& q) {
+    return (uint32_t)(q.x1 / kBlk - q.x0 / kBlk + 1) * (uint32_t)(q.y1 / kBlk - q.y0 / kBlk + 1);
+}
+
 // Depth-sort values of the frame: compact index in the low idx_bits bits, the
-// Gaussian's tile count above them, saturated at the field's largest value
+// Gaussian's tile count (its blocks' in a frame sorted by blocks) above them, saturated at the field's largest value
 // (which, like a zero field, means "not held: read the rectangle").
 // idx_bits 0: plain compact indices.
 __device__ __forceinline__ uint32_t dval_index(uint32_t v, int idx_bits) {

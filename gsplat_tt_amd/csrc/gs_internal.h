@@ -79,6 +79,9 @@ struct ProjParams {
     // the frame's tile grid, written when dvals is set (idx_bits > 0)
     int tiles_x, tiles_y, tile_size, idx_bits;
     uint32_t* dvals;
+    // a frame sorted by blocks (with dvals, which then hold the blocks): the
+    // candidate tiles per projection partition, else null
+    uint64_t* tile_sums;
     // per projection partition: nonzero = no Gaussian of it can reach the image
     // (its loads are skipped); nullptr = no partition is skipped
     const uint8_t* skip;
@@ -175,6 +178,8 @@ hipError_t radix_sort_pairs(void* keys, uint32_t* vals, int64_t n, int key_bytes
 // passes sort min(n_cap, *n_kept_dev) keys, and `hist` counts kept keys only.
 // run_cnt (u32 keys only, optional): the sorted keys are not written (*keys_final = nullptr); run_cnt[k] (cleared by the caller) gains
 // the number of keys equal to k, for launch_ranges_from_counts.
+// With run_shift, run_cnt counts the runs of key >> run_shift (the sorted bits:
+// begin_bit = run_shift), and the sorted keys are written too.
 // keys_out = false (u32 keys): the last pass writes the sorted values only
 // (*keys_final = nullptr).
 // first_offs (u32 keys only, optional): the first pass's output positions per
@@ -189,7 +194,8 @@ hipError_t radix_sort_pairs_dev(void* keys, uint32_t* vals, int64_t n_cap, const
                                 const uint32_t* n_kept_dev = nullptr,
                                 uint32_t* run_cnt = nullptr,
                                 const uint32_t* first_offs = nullptr,
-                                uint32_t run_limit = 0xFFFFFFFFu, bool keys_out = true);
+                                uint32_t run_limit = 0xFFFFFFFFu, bool keys_out = true,
+                                int run_shift = 0);
 
 // The 64-bit-key sort of radix_sort_pairs_dev over exactly n keys, with no
 // producer histogram: a histogram kernel counts the first pass's digits and
@@ -254,6 +260,33 @@ hipError_t launch_rect_count_scan(const float4* rect, int stride, const uint32_t
                                   uint32_t* bstart, uint32_t bstart_cap, uint64_t* lb_state,
                                   uint32_t* ticket, uint32_t* total_out, uint32_t cap,
                                   bool reduce_scan, hipStream_t st);
+// Tile lists by blocks of 4 x 4 tiles (tiles.hip). The scan: offs = exclusive scan
+// of the Gaussians' blocks in rank order, bstart over the items, the item total and
+// the candidate total, which the capacity bounds (sums: rect_scan_partitions(m)
+// words; tile_sums: the projection's n_tile_sums partition sums, or 0 and as many
+// words for a plain rank order). The emission: an item per slot, key = block
+// << 16 | mask of kept tiles or kPairDrop, digit counts of the block bits per
+// emit partition. The lists: from the items sorted by block (block_items of them
+// per block) to the pairs per tile, the ranges and the ids; scratch:
+// block_scratch_words. rc: (rectangle, conic) records; n_segs: a word.
+constexpr uint32_t kBlocksMost = 65535;
+uint32_t num_blocks(int tiles_x, int tiles_y);
+size_t block_scratch_words(uint32_t cap, uint32_t nb);
+hipError_t launch_block_scan(const float4* rc, const uint32_t* order, int64_t m,
+                             const uint32_t* m_dev, TileParams tp, uint32_t* offs,
+                             uint32_t* bstart, uint32_t bstart_cap, uint64_t* sums,
+                             uint64_t* tile_sums, uint32_t n_tile_sums, uint32_t* items_out,
+                             uint32_t* cands_out, uint32_t cap, hipStream_t st);
+hipError_t launch_block_emit(const float4* rc, const uint32_t* order, const uint32_t* offs,
+                             const uint32_t* bstart, int64_t m, const uint32_t* m_dev,
+                             uint32_t cap, const uint32_t* items_dev, TileParams tp,
+                             uint32_t* keys, uint32_t* ids, uint32_t* items_kept,
+                             uint32_t* pairs_kept, uint32_t* part_hist, int block_bits,
+                             hipStream_t st);
+hipError_t launch_block_lists(const uint32_t* keys, const uint32_t* ids, uint32_t cap,
+                              const uint32_t* block_items, uint32_t* scratch, uint32_t* n_segs, TileParams tp,
+                              uint32_t* tile_count, uint32_t* ranges, uint32_t* sorted_ids,
+                              const HostCopy& report, hipStream_t st);
 // Digit width of a device sort over `bits` key bits: the fewest 8-bit-or-less
 // passes, with the bits spread evenly over them (12 tile bits: two passes of 6,
 // whose 64 digits give longer runs per digit than 256 would).

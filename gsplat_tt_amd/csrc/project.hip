@@ -330,6 +330,7 @@ __global__ __launch_bounds__(kProjThreads, BINNED ? 4 : 1) void k_project(SceneD
     __syncthreads();
     const uint64_t excl = BINNED ? binned_count(s_excl) : s_excl;
     const uint64_t lt_mask = lanemask_lt();
+    uint64_t tiles = 0;  // this thread's candidate tiles (with dvals)
 
 #pragma unroll
     for (int it = 0; it < ITEMS; ++it) {
@@ -354,10 +355,13 @@ __global__ __launch_bounds__(kProjThreads, BINNED ? 4 : 1) void k_project(SceneD
                          rect_tiles(vmx[it], vmy[it], vrx[it], vry[it], p.tiles_x,
                                                         p.tiles_y, p.tile_size));
         } else if (p.dvals != nullptr) {
-            // the tile count that the candidate scan would read the rectangle for
-            p.dvals[m] = dval_pack((uint32_t)m,
-                                   rect_tiles(vmx[it], vmy[it], vrx[it], vry[it], p.tiles_x,
-                                                        p.tiles_y, p.tile_size), p.idx_bits);
+            // the count that the candidate scan would read the rectangle for
+            const Rect q = tile_rect(make_float4(vmx[it], vmy[it], vrx[it], vry[it]), p.tiles_x,
+                                     p.tiles_y, ts_div(p.tile_size));
+            const uint32_t t = (uint32_t)(q.x1 - q.x0 + 1) * (uint32_t)(q.y1 - q.y0 + 1);
+            tiles += t;
+            p.dvals[m] = dval_pack((uint32_t)m, p.tile_sums != nullptr ? block_cells(q) : t,
+                                   p.idx_bits);
         }
         // Microblock cull / blend record (cull_and_blend.cpp:723-777).
         const float det = fmax_std(a * c - b * b, 1e-6f);
@@ -376,6 +380,17 @@ __global__ __launch_bounds__(kProjThreads, BINNED ? 4 : 1) void k_project(SceneD
         out.brec[m * 3 + 1] = make_float4(ci_a, ci_b, ci_c, lt);
         out.brec[m * 3 + 2] = make_float4(vr[it], vg[it], vbl[it], op);
         if (out.src != nullptr) out.src[m] = (uint32_t)i;
+    }
+    if (!BINNED && p.tile_sums != nullptr) {  // uniform
+        __shared__ uint64_t s_tiles[kProjThreads / GS_WAVE];
+        const uint64_t inc = wave_incl_scan64(tiles);
+        if (lane == GS_WAVE - 1) s_tiles[w] = inc;
+        __syncthreads();
+        if (tid == 0) {
+            uint64_t t = 0;
+            for (int ww = 0; ww < kProjThreads / GS_WAVE; ++ww) t += s_tiles[ww];
+            p.tile_sums[vid] = t;
+        }
     }
 }
 
@@ -584,7 +599,7 @@ bool graph_project_args_are(hipGraphNode_t node, const SceneDev& s, const ProjPa
     const ProjParams& b = *static_cast<const ProjParams*>(kp.kernelParams[1]);
     bool same = a.n == s.n && a.sh_degree == s.sh_degree && a.sh == s.sh && a.opac == s.opac &&
                 a.mean[0] == s.mean[0] && a.cov[5] == s.cov[5] && a.lthr == s.lthr &&
-                b.ctl == p.ctl && b.dvals == p.dvals && b.skip == p.skip &&
+                b.ctl == p.ctl && b.dvals == p.dvals && b.tile_sums == p.tile_sums && b.skip == p.skip &&
                 b.binned.offs == p.binned.offs && b.binned.cap == p.binned.cap && b.fx == p.fx &&
                 b.fy == p.fy && b.width == p.width && b.height == p.height;
     for (int j = 0; j < 9; ++j) same = same && b.r[j] == p.r[j];

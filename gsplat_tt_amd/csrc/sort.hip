@@ -207,7 +207,7 @@ __device__ __forceinline__ uint32_t digit_walk(DT* state, uint32_t vid, int digi
 // in the same LDS space, so a partition holds only its keys in LDS (larger
 // partitions, fewer look-back links).
 // RUNS (the last pass of a sort whose keys' high bits index run_cnt): the
-// sorted keys are not written; instead every run of equal key >> run_shift in
+// sorted keys are written only if wanted (kout); every run of equal key >> run_shift in
 // the partition (the last pass leaves a partition sorted by all the key bits
 // in LDS) adds its length to run_cnt[key >> run_shift], with at most two
 // atomics per run.
@@ -272,9 +272,13 @@ __global__ __launch_bounds__(THREADS) void k_onesweep(
     const int lane = lane_id();
     const uint32_t mask = (1u << bits) - 1u;
 
-    if (tid == 0) s_vid = atomicAdd(ticket, 1u);
     // this workgroup's row of the descriptors that the next pass uses
     if (clear_next != nullptr && tid < 256) clear_next[(size_t)blockIdx.x * 256 + tid] = 0u;
+    // grid sized for a capacity; the key count may be known only on the device.
+    // The workgroups past it take no ticket: as many as there are partitions do.
+    const int64_t n = n_dev ? min(n_cap, (int64_t)*n_dev) : n_cap;
+    if ((int64_t)blockIdx.x * PART >= n) return;
+    if (tid == 0) s_vid = atomicAdd(ticket, 1u);
     for (int i = tid; i < WAVES * 256; i += THREADS) (&s_wcnt[0][0])[i] = 0;
     if (next_hist != nullptr && tid < 256) s_nh[tid] = 0u;
     // A pass whose digit is the same for all n keys (one histogram bin holds
@@ -287,9 +291,8 @@ __global__ __launch_bounds__(THREADS) void k_onesweep(
     __shared__ uint32_t s_vote[kIdentityOk ? 4 : 1];
     if constexpr (kIdentityOk) {
         if (tid < 256) {
-            const int64_t nn = n_dev ? min(n_cap, (int64_t)*n_dev) : n_cap;
             const bool v = next_hist == nullptr && part_offs == nullptr &&
-                           (int64_t)g_hist_pass[tid] == nn;
+                           (int64_t)g_hist_pass[tid] == n;
             const uint64_t b = __ballot(v);
             if (lane == 0) s_vote[w] = b != 0ull ? 1u : 0u;
         }
@@ -303,9 +306,7 @@ __global__ __launch_bounds__(THREADS) void k_onesweep(
     // cleared above all the same)
     if (__builtin_amdgcn_readfirstlane(upstream_failed(ctl) ? 1 : 0)) return;
     const int64_t part_base = (int64_t)vid * PART;
-    // grid sized for a capacity; the key count may be known only on the device
-    const int64_t n = n_dev ? min(n_cap, (int64_t)*n_dev) : n_cap;
-    if (part_base >= n) return;  // tickets are in order: no later partition has keys
+    if (part_base >= n) return;
     const int64_t wave_base = part_base + (int64_t)w * (ITEMS * GS_WAVE);
     if (identity) {
 #pragma unroll
@@ -463,7 +464,7 @@ __global__ __launch_bounds__(THREADS) void k_onesweep(
             const uint32_t d = digit_of(k, shift, mask);
             const uint32_t g = s_gpos[d] + (uint32_t)j;
             if ((int64_t)g < n) {
-                if (!RUNS && kout != nullptr) kout[g] = k;
+                if (kout != nullptr) kout[g] = k;
                 vout[g] = s_vals[j];
             }
             if (RUNS) {
@@ -497,7 +498,7 @@ __global__ __launch_bounds__(THREADS) void k_onesweep(
                 }
                 const uint32_t g = s_gpos[d] + (uint32_t)j;
                 gq[q] = g;
-                if (!RUNS && kout != nullptr && (int64_t)g < n) kout[g] = k;
+                if (kout != nullptr && (int64_t)g < n) kout[g] = k;
                 if (KONLY && RUNS && (int64_t)g < n)
                     vout[g] = (uint32_t)k & (uint32_t)(0xFFFFFFFFull >> (32 - val_bits));
                 if (RUNS) {
@@ -588,6 +589,9 @@ struct PassOut {
     uint32_t* key_err = nullptr;  // kErrKeyRange of narrowing and run counting
     int val_bits = 32;            // the value field of the joined words
     uint32_t val_limit = 0u;      // values must be below it (0: any)
+    // a sort of one pass whose output positions are given: it uses no look-back, and
+    // a frame whose depth sort takes four passes leaves the state as it found it
+    bool no_state = false;
 };
 
 // A digit pass with partition shape CFG.
@@ -603,7 +607,9 @@ hipError_t launch_cfg(bool iota, const K* kin, const uint32_t* vin, K* kout, uin
     const bool d32 = n_cap < ((int64_t)1 << 30);
     uint32_t* state = reinterpret_cast<uint32_t*>(tmp.state);
     uint32_t* clear_next = nullptr;
-    if (d32 && tmp.state_parts >= grid) {
+    if (po.no_state) {
+        // nothing is published or walked: the descriptors stay as they are
+    } else if (d32 && tmp.state_parts >= grid) {
         const int h = tmp.half;
         const size_t half_words = tmp.state_parts * 256;
         uint32_t* cur = state + (size_t)h * half_words;
@@ -765,7 +771,8 @@ hipError_t sort_dev_impl(K* keys, uint32_t* vals, int64_t n_cap, const uint32_t*
                          uint32_t** vals_final, const uint32_t* n_kept_dev,
                          uint32_t* chain_hist = nullptr, bool pass_events = false,
                          uint32_t* run_cnt = nullptr, const uint32_t* first_offs = nullptr,
-                         uint32_t run_limit = 0xFFFFFFFFu, bool keys_out = true) {
+                         uint32_t run_limit = 0xFFFFFFFFu, bool keys_out = true,
+                         int run_shift = 0) {
     *keys_final = keys;
     *vals_final = vals;
     if (n_cap <= 0) return hipSuccess;
@@ -779,6 +786,9 @@ hipError_t sort_dev_impl(K* keys, uint32_t* vals, int64_t n_cap, const uint32_t*
     const int dw = sort_digit_width(end_bit - begin_bit);
     PassOut po;
     po.run_limit = run_limit;
+    po.run_shift = run_shift;
+    po.no_state = npass == 1 && first_offs != nullptr;
+    if (run_cnt != nullptr && run_shift == 0) keys_out = false;
     for (int p = 0; p < npass; ++p) {
         const int shift = begin_bit + dw * p;
         const int bits = std::min(dw, end_bit - shift);
@@ -812,14 +822,16 @@ hipError_t radix_sort_pairs_dev(void* keys, uint32_t* vals, int64_t n_cap, const
                                 uint32_t* tickets, SortTemp& tmp, hipStream_t st, bool vals_iota,
                                 void** keys_final, uint32_t** vals_final,
                                 const uint32_t* n_kept_dev, uint32_t* run_cnt,
-                                const uint32_t* first_offs, uint32_t run_limit, bool keys_out) {
+                                const uint32_t* first_offs, uint32_t run_limit, bool keys_out,
+                                int run_shift) {
     if (key_bytes == 4) {
         uint32_t* kf = nullptr;
         hipError_t e = sort_dev_impl<uint32_t>(static_cast<uint32_t*>(keys), vals, n_cap, n_dev,
                                                begin_bit, end_bit, hist, tickets, tmp, st,
                                                vals_iota, &kf, vals_final, n_kept_dev, nullptr,
-                                               false, run_cnt, first_offs, run_limit, keys_out);
-        *keys_final = run_cnt != nullptr ? nullptr : kf;
+                                               false, run_cnt, first_offs, run_limit, keys_out,
+                                               run_shift);
+        *keys_final = kf;
         return e;
     }
     if (key_bytes == 8) {
@@ -923,7 +935,7 @@ hipError_t radix_sort_ids_dev_chain(uint64_t* keys, uint32_t* vals, int64_t n, i
             po.konly = true;
             po.run_shift = 32 + at;  // the tile field of the joined word
             po.run_limit = num_tiles;
-            e = launch_pass<uint64_t>(false, k64[ki], nullptr, k64[ki ^ 1],
+            e = launch_pass<uint64_t>(false, k64[ki], nullptr, last ? nullptr : k64[ki ^ 1],
                                       last ? vals : nullptr, n, nullptr, shift, bits,
                                       hist + p * 256, tmp, tickets + p, st, false, nh,
                                       next_shift, next_bits, last ? run_cnt : nullptr, nullptr,

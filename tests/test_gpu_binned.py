@@ -1,6 +1,7 @@
-"""The two ways a frame's tile lists are made: binned (pairs counted per tile, each
-list sorted on its own in runs of 2048) and sorted (depth sort, then tile sort; the
-microblock statistics select it). Both give the stable (tile, depth bits, compact id)
+"""The ways a frame's tile lists are made: binned (pairs counted per tile, each
+list sorted on its own in runs of 2048), by blocks (depth sort, items of 4 x 4 tiles
+sorted by block and split) and sorted (depth sort, then tile sort; the microblock
+statistics select it). All give the stable (tile, depth bits, compact id)
 order, so ids, ranges, counts and images are compared for equality, at list lengths
 around the runs of the list sort, with equal depths, empty views and many tiles."""
 import numpy as np
@@ -76,6 +77,70 @@ def test_projection_partitions(gpu_ctx, n, deg):
     a, b = _both(gpu_ctx, view)
     assert a[1]["num_visible"] > n // 2
     _equal(a, b)
+
+
+@pytest.mark.parametrize("h,w,ts,n,spread", [
+    (129 * 16, 128 * 16 + 1, 16, 9000, 0.004),   # a block's list of five segments
+    (203 * 16 - 7, 131 * 16, 16, 3000, 0.3), (16, 16390 * 16 - 9, 16, 700, 0.3),
+    (16390 * 16 - 9, 5, 16, 2049, 0.3), (129 * 32 - 31, 130 * 32, 32, 2000, 0.2),
+    (200, 299, 16, (1 << 20) + 1, 0.1), (33, 17, 32, (1 << 20) + 7, 0.002)])  # one sort pass
+@pytest.mark.parametrize("cull", [True, False])
+def test_lists_by_blocks(gpu_ctx, h, w, ts, n, spread, cull):
+    """Frames of more than 2^14 tiles, and first frames of more than 2^20 Gaussians,
+    are made by blocks: whole and cut blocks, one row or column of them, one block
+    and thousands, lists of several segments, with and without the tile cull."""
+    print("blocks", h, w, ts, n, cull, flush=True)
+    if not cull and n > 9000:
+        n = (1 << 20) + 3
+    gpu_ctx.set_scene(*_stack(n, 300, spread=spread, seed=n))
+    K = scenes.intrinsics(0.5 * w, 0.5 * h, w / 2, h / 2)
+    view = L.make_view(np.eye(4, dtype=np.float32), K, h, w, tile_size=ts, output="u8",
+                       cull_disabled=not cull, max_radius=-1)
+    a, b = _both(gpu_ctx, view)
+    assert a[1]["num_visible"] > n // 3
+    _equal(a, b)
+
+
+def test_blocks_pair_limit():
+    """The pair limit counts candidate tiles, not items: the same floor, retries and
+    image by blocks as sorted."""
+    print("block limit", flush=True)
+    scene, cams = scenes.config1(seed=5, n=6_000)
+    cov = scenes.cov3d(scene.scales, scene.quats)
+    h, w = 130 * 16 - 15, 129 * 16
+    K = scenes.intrinsics(500 * w / 640, 500 * w / 640, w / 2, h / 2)
+    ctx = L.Context(0)
+    try:
+        ctx.set_scene(scene.means, cov, scene.opacities, scene.colors)
+        view = L.make_view(cams[0].w2c, K, h, w, tile_size=16, output="bf16")
+        full = ctx.render(view)[1]["pairs_pre"]
+        ctx.set_pair_limit(int(full * 0.9))
+        a, b = _both(ctx, view)
+        assert a[1]["floor_retries"] == b[1]["floor_retries"] > 0
+        assert a[1]["contrib_floor"] == b[1]["contrib_floor"]
+        _equal(a, b)
+    finally:
+        ctx.close()
+
+
+def test_training_forward_by_blocks(gpu_ctx):
+    """A training image of more than 2^14 tiles (by blocks) against the same view two
+    rows of tiles shorter (binned): the shared rows are the same bit for bit."""
+    print("train blocks", flush=True)
+    n, w = 4000, 129 * 16 - 3
+    rng = np.random.default_rng(3)
+    z = rng.uniform(2, 4, n)
+    p = {"means": np.stack([rng.uniform(-0.5, 0.5, n) * z, rng.uniform(-0.5, 0.5, n) * z, z], 1),
+         "log_scales": rng.normal(-3.5, 0.5, (n, 3)), "quats": rng.standard_normal((n, 4)),
+         "opacity_logits": rng.normal(0, 1.0, n), "sh": rng.uniform(-0.5, 0.5, (n, 4, 3))}
+    p = {k: v.astype(np.float32) for k, v in p.items()}
+    K = scenes.intrinsics(0.9 * w, 0.9 * w, w / 2, 64 * 16)
+    tr = L.Trainer(gpu_ctx, p, 1)
+    imgs = []
+    for rows in (127, 129):
+        view = L.make_view(np.eye(4, dtype=np.float32), K, rows * 16, w, tile_size=16)
+        imgs.append(tr.forward(view, L.make_train_cfg())[0])
+    assert imgs[0].any() and np.array_equal(imgs[1][:127 * 16], imgs[0])
 
 
 def test_many_tiles_and_empty_views(gpu_ctx):

@@ -492,7 +492,7 @@ struct SsimParams {
     float w;               // -lambda * loss_scale / (3HW): scale of the SSIM terms
     const float* image;    // (H,W,3)
     const float* target;   // (H,W,3)
-    float* maps;           // 3 x (H,W,3): w dS/dmu_x, w dS/dE_xx, w dS/dE_xy
+    float* maps;           // 3 x (3,H,W): w dS/dmu_x, w dS/dE_xx, w dS/dE_xy
     float* dimage;         // (H,W,3): the SSIM gradient is added
     TrainSums* sums;       // kTrainSumSlots groups: the sum of S over the 3HW values
 };

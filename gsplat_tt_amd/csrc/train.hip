@@ -569,88 +569,126 @@ __global__ __launch_bounds__(GS_WAVE) void k_train_fwd(const float4* __restrict_
 // ---------------------------------------------------------------------------
 // Full 3DGS loss (train_oracle.py:253-279): SSIM with an 11-tap Gaussian window
 // (sigma 1.5), zero padding, S = A B / (C D); the image gradient in the
-// fused-SSIM form of train_loss.py:5-19. One workgroup per 16x16 tile and
-// channel loop; a 26x26 halo in LDS, row pass then column pass.
+// fused-SSIM form of train_loss.py:5-19. A workgroup takes one channel of 32 x 22
+// pixels: 32 halo rows are one row-pass unit of four adjacent outputs per thread
+// (14 values read for four of 11 taps each), the column pass gives each thread
+// three outputs of a column from 13 rows, and products go into fused adds (which
+// also drop a rounding): a quarter of the LDS reads and half of the VALU issue of
+// one output per thread on 16 x 16 tiles. Bound by both still, and by the terms'
+// seven divisions a pixel (960x720, forward and backward: 35.3 -> 25.1 and 38.6 ->
+// 23.3 us; 501x333: 16.0 -> 10.8 and 13.6 -> 9.9).
 // ---------------------------------------------------------------------------
-constexpr int kSsimT = 16, kSsimR = 5, kSsimE = kSsimT + 2 * kSsimR;
+constexpr int kSsimW = 32, kSsimH = 22, kSsimR = 5;
+constexpr int kSsimEW = kSsimW + 2 * kSsimR, kSsimEH = kSsimH + 2 * kSsimR;  // with the halo
+constexpr int kSsimX = 44, kSsimHs = 36;  // row strides in LDS, whole float4
+constexpr int kSsimCol = 3;               // outputs of a column per thread
+constexpr int kSsimHRows = 256 / kSsimW * kSsimCol + 2 * kSsimR;  // rows that the column pass reads
+static_assert(kSsimEH * (kSsimW / 4) == 256, "one row-pass unit per thread");
+static_assert(256 / kSsimW * kSsimCol >= kSsimH && kSsimHRows >= kSsimEH, "the columns are covered");
+
+// Sixteen values of an LDS row: the taps of four adjacent outputs.
+__device__ __forceinline__ void load14(const float* row, float (&v)[16]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float4 q = reinterpret_cast<const float4*>(row)[i];
+        v[4 * i] = q.x;
+        v[4 * i + 1] = q.y;
+        v[4 * i + 2] = q.z;
+        v[4 * i + 3] = q.w;
+    }
+}
+// The column filter of Q planes at kSsimCol outputs from row r0 of column c.
+template <int Q>
+__device__ __forceinline__ void ssim_columns(const float (*h)[kSsimHRows][kSsimHs], int r0, int c,
+                                             const float* g, float (&acc)[kSsimCol][Q]) {
+#pragma unroll
+    for (int j = 0; j < kSsimCol; ++j)
+#pragma unroll
+        for (int q = 0; q < Q; ++q) acc[j][q] = 0.0f;
+#pragma unroll
+    for (int r = 0; r < kSsimCol + 2 * kSsimR; ++r) {
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            const float v = h[q][r0 + r][c];
+#pragma unroll
+            for (int j = 0; j < kSsimCol; ++j)
+                if (r >= j && r - j <= 2 * kSsimR) acc[j][q] = fmaf(g[r - j], v, acc[j][q]);
+        }
+    }
+}
 
 // Forward: mu_x, mu_y, E_xx, E_yy, E_xy -> S and the three per-pixel terms
-// w dS/dmu_x, w dS/dE_xx, w dS/dE_xy (zero outside the image), sum of S.
+// w dS/dmu_x, w dS/dE_xx, w dS/dE_xy (planes by term and channel), sum of S.
 __global__ __launch_bounds__(256) void k_ssim_fwd(SsimParams sp) {
-    __shared__ float s_x[kSsimE][kSsimE + 1], s_y[kSsimE][kSsimE + 1];
-    __shared__ float s_h[5][kSsimE][kSsimT + 1];
+    __shared__ __attribute__((aligned(16))) float s_x[kSsimEH][kSsimX], s_y[kSsimEH][kSsimX];
+    __shared__ __attribute__((aligned(16))) float s_h[5][kSsimHRows][kSsimHs];
     __shared__ double s_sum[4];
     const int tid = threadIdx.x;
-    const int tiles_x = (sp.width + kSsimT - 1) / kSsimT;
-    const int tx = blockIdx.x % tiles_x, ty = blockIdx.x / tiles_x;
-    const int x0 = tx * kSsimT - kSsimR, y0 = ty * kSsimT - kSsimR;
-    const int lx = tid & 15, ly = tid >> 4;
-    const int px = tx * kSsimT + lx, py = ty * kSsimT + ly;
-    const bool inside = px < sp.width && py < sp.height;
+    const int tiles_x = (sp.width + kSsimW - 1) / kSsimW;
+    const int tiles = tiles_x * ((sp.height + kSsimH - 1) / kSsimH);
+    const int ch = blockIdx.x / tiles, t = blockIdx.x % tiles;
+    const int x0 = t % tiles_x * kSsimW, y0 = t / tiles_x * kSsimH;
     const size_t npx = (size_t)sp.width * sp.height;
+    for (int i = tid; i < kSsimEH * kSsimEW; i += 256) {
+        const int r = i / kSsimEW, c = i % kSsimEW;
+        const int gx = x0 - kSsimR + c, gy = y0 - kSsimR + r;
+        float xv = 0.0f, yv = 0.0f;
+        if (gx >= 0 && gx < sp.width && gy >= 0 && gy < sp.height) {
+            const size_t q = ((size_t)gy * sp.width + gx) * 3 + ch;
+            xv = sp.image[q];
+            yv = sp.target[q];
+        }
+        s_x[r][c] = xv;
+        s_y[r][c] = yv;
+    }
+    __syncthreads();
+    {
+        const int r = tid / (kSsimW / 4), c = tid % (kSsimW / 4) * 4;
+        float v[5][16], h[5][4] = {};
+        load14(&s_x[r][c], v[0]);
+        load14(&s_y[r][c], v[1]);
+#pragma unroll
+        for (int i = 0; i < kSsimR * 2 + 4; ++i) {
+            v[2][i] = v[0][i] * v[0][i];
+            v[3][i] = v[1][i] * v[1][i];
+            v[4][i] = v[0][i] * v[1][i];
+        }
+#pragma unroll
+        for (int q = 0; q < 5; ++q)
+#pragma unroll
+            for (int k = 0; k < 2 * kSsimR + 1; ++k)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) h[q][j] = fmaf(sp.g[k], v[q][j + k], h[q][j]);
+#pragma unroll
+        for (int q = 0; q < 5; ++q)
+            *reinterpret_cast<float4*>(&s_h[q][r][c]) = make_float4(h[q][0], h[q][1], h[q][2], h[q][3]);
+    }
+    __syncthreads();
+    const int lx = tid % kSsimW, r0 = tid / kSsimW * kSsimCol;
+    float m[kSsimCol][5];
+    ssim_columns<5>(s_h, r0, lx, sp.g, m);
     double ssum = 0.0;
-    for (int ch = 0; ch < 3; ++ch) {
-        for (int i = tid; i < kSsimE * kSsimE; i += 256) {
-            const int r = i / kSsimE, c = i % kSsimE;
-            const int gx = x0 + c, gy = y0 + r;
-            float xv = 0.0f, yv = 0.0f;
-            if (gx >= 0 && gx < sp.width && gy >= 0 && gy < sp.height) {
-                const size_t q = ((size_t)gy * sp.width + gx) * 3 + ch;
-                xv = sp.image[q];
-                yv = sp.target[q];
-            }
-            s_x[r][c] = xv;
-            s_y[r][c] = yv;
-        }
-        __syncthreads();
-        // row pass over all 26 halo rows, 16 output columns
-        for (int i = tid; i < kSsimE * kSsimT; i += 256) {
-            const int r = i / kSsimT, c = i % kSsimT;
-            float hx = 0.0f, hy = 0.0f, hxx = 0.0f, hyy = 0.0f, hxy = 0.0f;
 #pragma unroll
-            for (int k = 0; k < 11; ++k) {
-                const float xv = s_x[r][c + k], yv = s_y[r][c + k], g = sp.g[k];
-                hx += g * xv;
-                hy += g * yv;
-                hxx += g * (xv * xv);
-                hyy += g * (yv * yv);
-                hxy += g * (xv * yv);
-            }
-            s_h[0][r][c] = hx;
-            s_h[1][r][c] = hy;
-            s_h[2][r][c] = hxx;
-            s_h[3][r][c] = hyy;
-            s_h[4][r][c] = hxy;
-        }
-        __syncthreads();
-        float mu_x = 0.0f, mu_y = 0.0f, e_xx = 0.0f, e_yy = 0.0f, e_xy = 0.0f;
-#pragma unroll
-        for (int k = 0; k < 11; ++k) {
-            const float g = sp.g[k];
-            mu_x += g * s_h[0][ly + k][lx];
-            mu_y += g * s_h[1][ly + k][lx];
-            e_xx += g * s_h[2][ly + k][lx];
-            e_yy += g * s_h[3][ly + k][lx];
-            e_xy += g * s_h[4][ly + k][lx];
-        }
-        if (inside) {
+    for (int j = 0; j < kSsimCol; ++j) {
+        const int px = x0 + lx, py = y0 + r0 + j;
+        if (r0 + j < kSsimH && px < sp.width && py < sp.height) {
+            const float mu_x = m[j][0], mu_y = m[j][1], e_xx = m[j][2], e_yy = m[j][3];
             const float c1 = 0.01f * 0.01f, c2 = 0.03f * 0.03f;
             const float mxy = mu_x * mu_y;
             const float A = 2.0f * mxy + c1;
-            const float B = 2.0f * (e_xy - mxy) + c2;
+            const float B = 2.0f * fmaf(-mu_x, mu_y, m[j][4]) + c2;
             const float C = mu_x * mu_x + mu_y * mu_y + c1;
-            const float D = (e_xx - mu_x * mu_x) + (e_yy - mu_y * mu_y) + c2;
+            const float D = fmaf(-mu_x, mu_x, e_xx) + fmaf(-mu_y, mu_y, e_yy) + c2;
             const float S = (A * B) / (C * D);
             const float Sw = S * sp.w;
             const float d_mu = Sw * (2.0f * mu_y / A - 2.0f * mu_y / B - 2.0f * mu_x / C +
                                      2.0f * mu_x / D);
-            const size_t q = ((size_t)py * sp.width + px) * 3 + ch;
-            sp.maps[q] = d_mu;
-            sp.maps[3 * npx + q] = -Sw / D;
-            sp.maps[6 * npx + q] = 2.0f * Sw / B;
+            float* map = sp.maps + (size_t)ch * npx + (size_t)py * sp.width + px;
+            map[0] = d_mu;
+            map[3 * npx] = -Sw / D;
+            map[6 * npx] = 2.0f * Sw / B;
             ssum += (double)S;
         }
-        __syncthreads();  // the next channel overwrites the LDS planes
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) ssum += __shfl_xor(ssum, o, GS_WAVE);
@@ -664,60 +702,48 @@ __global__ __launch_bounds__(256) void k_ssim_fwd(SsimParams sp) {
 // Backward: dimage += G*(w dS/dmu_x) + 2 x G*(w dS/dE_xx) + y G*(w dS/dE_xy)
 // (G symmetric, so its adjoint is the same zero-padded filter).
 __global__ __launch_bounds__(256) void k_ssim_bwd(SsimParams sp) {
-    __shared__ float s_m[3][kSsimE][kSsimE + 1];
-    __shared__ float s_h[3][kSsimE][kSsimT + 1];
+    __shared__ __attribute__((aligned(16))) float s_m[3][kSsimEH][kSsimX];
+    __shared__ __attribute__((aligned(16))) float s_h[3][kSsimHRows][kSsimHs];
     const int tid = threadIdx.x;
-    const int tiles_x = (sp.width + kSsimT - 1) / kSsimT;
-    const int tx = blockIdx.x % tiles_x, ty = blockIdx.x / tiles_x;
-    const int x0 = tx * kSsimT - kSsimR, y0 = ty * kSsimT - kSsimR;
-    const int lx = tid & 15, ly = tid >> 4;
-    const int px = tx * kSsimT + lx, py = ty * kSsimT + ly;
-    const bool inside = px < sp.width && py < sp.height;
+    const int tiles_x = (sp.width + kSsimW - 1) / kSsimW;
+    const int tiles = tiles_x * ((sp.height + kSsimH - 1) / kSsimH);
+    const int ch = blockIdx.x / tiles, t = blockIdx.x % tiles;
+    const int x0 = t % tiles_x * kSsimW, y0 = t / tiles_x * kSsimH;
     const size_t npx = (size_t)sp.width * sp.height;
-    for (int ch = 0; ch < 3; ++ch) {
-        for (int i = tid; i < kSsimE * kSsimE; i += 256) {
-            const int r = i / kSsimE, c = i % kSsimE;
-            const int gx = x0 + c, gy = y0 + r;
-            float a = 0.0f, b = 0.0f, d = 0.0f;
-            if (gx >= 0 && gx < sp.width && gy >= 0 && gy < sp.height) {
-                const size_t q = ((size_t)gy * sp.width + gx) * 3 + ch;
-                a = sp.maps[q];
-                b = sp.maps[3 * npx + q];
-                d = sp.maps[6 * npx + q];
-            }
-            s_m[0][r][c] = a;
-            s_m[1][r][c] = b;
-            s_m[2][r][c] = d;
-        }
-        __syncthreads();
-        for (int i = tid; i < kSsimE * kSsimT; i += 256) {
-            const int r = i / kSsimT, c = i % kSsimT;
-            float h0 = 0.0f, h1 = 0.0f, h2 = 0.0f;
+    const float* map = sp.maps + (size_t)ch * npx;
+    for (int i = tid; i < kSsimEH * kSsimEW; i += 256) {
+        const int r = i / kSsimEW, c = i % kSsimEW;
+        const int gx = x0 - kSsimR + c, gy = y0 - kSsimR + r;
+        const bool in = gx >= 0 && gx < sp.width && gy >= 0 && gy < sp.height;
+        const size_t q = in ? (size_t)gy * sp.width + gx : 0;
 #pragma unroll
-            for (int k = 0; k < 11; ++k) {
-                const float g = sp.g[k];
-                h0 += g * s_m[0][r][c + k];
-                h1 += g * s_m[1][r][c + k];
-                h2 += g * s_m[2][r][c + k];
-            }
-            s_h[0][r][c] = h0;
-            s_h[1][r][c] = h1;
-            s_h[2][r][c] = h2;
-        }
-        __syncthreads();
-        if (inside) {
-            float P = 0.0f, Q = 0.0f, R = 0.0f;
+        for (int p = 0; p < 3; ++p) s_m[p][r][c] = in ? map[(size_t)(3 * p) * npx + q] : 0.0f;
+    }
+    __syncthreads();
+    {
+        const int r = tid / (kSsimW / 4), c = tid % (kSsimW / 4) * 4;
 #pragma unroll
-            for (int k = 0; k < 11; ++k) {
-                const float g = sp.g[k];
-                P += g * s_h[0][ly + k][lx];
-                Q += g * s_h[1][ly + k][lx];
-                R += g * s_h[2][ly + k][lx];
-            }
+        for (int p = 0; p < 3; ++p) {
+            float v[16], h[4] = {};
+            load14(&s_m[p][r][c], v);
+#pragma unroll
+            for (int k = 0; k < 2 * kSsimR + 1; ++k)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) h[j] = fmaf(sp.g[k], v[j + k], h[j]);
+            *reinterpret_cast<float4*>(&s_h[p][r][c]) = make_float4(h[0], h[1], h[2], h[3]);
+        }
+    }
+    __syncthreads();
+    const int lx = tid % kSsimW, r0 = tid / kSsimW * kSsimCol;
+    float m[kSsimCol][3];
+    ssim_columns<3>(s_h, r0, lx, sp.g, m);
+#pragma unroll
+    for (int j = 0; j < kSsimCol; ++j) {
+        const int px = x0 + lx, py = y0 + r0 + j;
+        if (r0 + j < kSsimH && px < sp.width && py < sp.height) {
             const size_t q = ((size_t)py * sp.width + px) * 3 + ch;
-            sp.dimage[q] += P + 2.0f * sp.image[q] * Q + sp.target[q] * R;
+            sp.dimage[q] += m[j][0] + 2.0f * sp.image[q] * m[j][1] + sp.target[q] * m[j][2];
         }
-        __syncthreads();
     }
 }
 
@@ -1260,12 +1286,12 @@ hipError_t launch_train_fwd(const float4* trec, const uint32_t* sid, const uint3
 
 hipError_t launch_ssim(const SsimParams& sp, hipStream_t st) {
     if (sp.width <= 0 || sp.height <= 0) return hipSuccess;
-    const unsigned tiles = (unsigned)(((sp.width + kSsimT - 1) / kSsimT) *
-                                      ((sp.height + kSsimT - 1) / kSsimT));
-    k_ssim_fwd<<<tiles, 256, 0, st>>>(sp);
+    const unsigned grid = 3u * (unsigned)(((sp.width + kSsimW - 1) / kSsimW) *
+                                          ((sp.height + kSsimH - 1) / kSsimH));
+    k_ssim_fwd<<<grid, 256, 0, st>>>(sp);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    k_ssim_bwd<<<tiles, 256, 0, st>>>(sp);
+    k_ssim_bwd<<<grid, 256, 0, st>>>(sp);
     return hipGetLastError();
 }
 

@@ -198,6 +198,22 @@ def test_train_loss_ssim_full_size(gpu_ctx):
     assert np.array_equal(g0, (np.sign(d) * (2.0 / d.size)).astype(np.float32))
 
 
+@pytest.mark.parametrize("h,w", [(1, 1), (1, 70), (50, 1), (21, 31), (22, 32), (23, 33), (45, 65)])
+def test_train_loss_ssim_tiles(gpu_ctx, h, w):
+    """Whole, cut and one-pixel tiles (32 x 22) of the SSIM filters against the fp64
+    oracle. Each filter value is 121 fp32 terms of one sign (relative error below
+    ~1e-6); the variances in D and B are at least 9e-4, against which the moments'
+    error of 1e-6 is 1e-3, the gradient test's bound."""
+    print("ssim tiles", h, w, flush=True)
+    rng = np.random.default_rng(h + w)
+    tgt = rng.uniform(0, 1, (h, w, 3)).astype(np.float32)
+    img = np.clip(tgt + rng.normal(0, 0.05, tgt.shape), 0, 1).astype(np.float32)
+    loss, l1, ssim, grad = gpu_ctx.train_loss(img, tgt, 0.2)
+    lo, l1o, so, go = TO.ssim_loss_grad(img, tgt, 0.2)
+    assert abs(loss - lo) <= 1e-6 * lo and abs(ssim - so) <= 1e-6
+    assert rel_err(grad, go) < 1e-3
+
+
 def test_train_step_ssim_loss_matches_oracle(gpu_ctx):
     """One whole step with the full 3DGS loss (lambda 0.2) of a C5-shaped scene
     against the oracle's forward, SSIM loss gradient, backward and Adam."""

@@ -575,7 +575,7 @@ __global__ __launch_bounds__(GS_WAVE) void k_train_fwd(const float4* __restrict_
 // three outputs of a column from 13 rows, and products go into fused adds (which
 // also drop a rounding): a quarter of the LDS reads and half of the VALU issue of
 // one output per thread on 16 x 16 tiles. Bound by both still, and by the terms'
-// seven divisions a pixel (960x720, forward and backward: 35.3 -> 25.1 and 38.6 ->
+// seven divisions a pixel (800x600, forward and backward: 35.3 -> 25.1 and 38.6 ->
 // 23.3 us; 501x333: 16.0 -> 10.8 and 13.6 -> 9.9).
 // ---------------------------------------------------------------------------
 constexpr int kSsimW = 32, kSsimH = 22, kSsimR = 5;

@@ -272,13 +272,15 @@ __global__ __launch_bounds__(THREADS) void k_onesweep(
     const int lane = lane_id();
     const uint32_t mask = (1u << bits) - 1u;
 
-    // this workgroup's row of the descriptors that the next pass uses
-    if (clear_next != nullptr && tid < 256) clear_next[(size_t)blockIdx.x * 256 + tid] = 0u;
     // grid sized for a capacity; the key count may be known only on the device.
     // The workgroups past it take no ticket: as many as there are partitions do.
     const int64_t n = n_dev ? min(n_cap, (int64_t)*n_dev) : n_cap;
-    if ((int64_t)blockIdx.x * PART >= n) return;
-    if (tid == 0) s_vid = atomicAdd(ticket, 1u);
+    const bool past = (int64_t)blockIdx.x * PART >= n;
+    // (the ticket before the clearing stores: its wait would include theirs)
+    if (tid == 0 && !past) s_vid = atomicAdd(ticket, 1u);
+    // this workgroup's row of the descriptors that the next pass uses
+    if (clear_next != nullptr && tid < 256) clear_next[(size_t)blockIdx.x * 256 + tid] = 0u;
+    if (past) return;
     for (int i = tid; i < WAVES * 256; i += THREADS) (&s_wcnt[0][0])[i] = 0;
     if (next_hist != nullptr && tid < 256) s_nh[tid] = 0u;
     // A pass whose digit is the same for all n keys (one histogram bin holds

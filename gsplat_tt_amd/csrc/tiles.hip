@@ -96,8 +96,8 @@ __device__ __forceinline__ bool pair_keep(float px, float py, float4 cv, int til
 // is then split into its tiles' lists in order, by ballots: the words that the
 // sort moves and ranks are a sixth of those of a sort of every pair by its tile
 // (30M pairs of 3M Gaussians at 1237x822, each frame alone: the two tile passes
-// 605 -> 79 us, emission 226 -> 128, counts and offsets 44 -> 38, and 70 us for the
-// split). Four tiles a side: larger blocks would need masks past half a word, and
+// 267 -> 76 us on one scene and 605 -> 79 on another, emission 227 -> 127, counts
+// and offsets 44 -> 40, and 69 us for the split). Four tiles a side: larger blocks would need masks past half a word, and
 // two halve nothing of the items of Gaussians of three or four tiles a side.
 // ---------------------------------------------------------------------------
 constexpr int kBlkTiles = kBlk * kBlk;

@@ -273,9 +273,10 @@ __global__ __launch_bounds__(THREADS) void k_onesweep(
     const uint32_t mask = (1u << bits) - 1u;
 
     // grid sized for a capacity; the key count may be known only on the device.
-    // The workgroups past it take no ticket: as many as there are partitions do.
+    // The workgroups past it take no ticket: as many as there are partitions do (u64
+    // keys come with their exact count).
     const int64_t n = n_dev ? min(n_cap, (int64_t)*n_dev) : n_cap;
-    const bool past = (int64_t)blockIdx.x * PART >= n;
+    const bool past = sizeof(K) == 4 && (int64_t)blockIdx.x * PART >= n;
     // (the ticket before the clearing stores: its wait would include theirs)
     if (tid == 0 && !past) s_vid = atomicAdd(ticket, 1u);
     // this workgroup's row of the descriptors that the next pass uses

@@ -1099,7 +1099,7 @@ struct gs_ctx {
         TilePlan& p = (owner ? owner : this)->plan;
         if (p.n != N || p.T != T) p = {N, T, N <= kBinnedFirst};
         // the microblock statistics need the sorted tile keys
-        return p.binned && !want_keys && T <= gs::kBinnedTiles && N < ((int64_t)1 << 28);
+        return p.binned && !want_keys && gs::binned_fits(N, T);
     }
     void plan_seen(int64_t N, int64_t T, int64_t P) {
         TilePlan& p = (owner ? owner : this)->plan;

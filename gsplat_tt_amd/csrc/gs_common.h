@@ -262,17 +262,6 @@ __device__ __forceinline__ void host_copy(const HostCopy& c, uint32_t tid, uint3
         __hip_atomic_store(&c.dst[i], c.src[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// ---------------------------------------------------------------------------
-// Binned frames: the compaction's look-back carries the visible count and the
-// candidate total together (count above bit 34, candidates below: a binned
-// frame has at most 2^32 of them and fewer than 2^28 Gaussians).
-// ---------------------------------------------------------------------------
-__device__ __forceinline__ uint64_t binned_pack(uint32_t count, uint64_t cands) {
-    return ((uint64_t)count << 34) | cands;
-}
-__device__ __forceinline__ uint64_t binned_count(uint64_t v) { return v >> 34; }
-__device__ __forceinline__ uint64_t binned_cands(uint64_t v) { return v & ((1ull << 34) - 1); }
-
 // The last partition's inclusive prefix: visible count, candidate total
 // (saturated), and kErrCapacity when the candidates do not fit.
 __device__ __forceinline__ void binned_totals(uint64_t v, uint32_t* count_out,

@@ -6,6 +6,8 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include "tile_plan.h"
+
 struct gs_ctx;  // include/gsplat_hip.h
 
 namespace gs {
@@ -321,7 +323,6 @@ hipError_t launch_pair_emit(const float4* rect, const float4* cov, int stride, b
                             uint64_t* lb_state, uint32_t* ticket, uint32_t* total_out,
                             uint32_t* part_hist, int tile_bits, Emit mode, hipStream_t st,
                             uint32_t* bins = nullptr);
-constexpr int kBinnedTiles = 1 << 14;  // most tiles of a binned frame (32 KB of LDS counters)
 uint32_t bin_words(int64_t num_tiles);
 // The binned tile lists: from the emission's slots (tile and rank, compact id)
 // and bins to the pairs per tile (cleared before), the ranges and the ids of each

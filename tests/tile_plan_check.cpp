@@ -1,0 +1,53 @@
+// Host-only checks of the tile-list rules (gsplat_tt_amd/csrc/tile_plan.h), built with
+// g++ by tests/test_tile_plan.py.
+#include <cstdint>
+#include <cstdio>
+#include <initializer_list>
+
+#include "tile_plan.h"
+
+static int fails = 0;
+#define CHECK(c)                                                              \
+    do {                                                                      \
+        if (!(c)) {                                                           \
+            std::fprintf(stderr, "FAIL line %d: %s\n", __LINE__, #c);         \
+            ++fails;                                                          \
+        }                                                                     \
+    } while (0)
+
+// The compaction's sums over partitions of `part` Gaussians that each cover every
+// tile, as the look-back forms them: what the last partition reports must be the
+// count and the total, and the flag bits above must stay free.
+static void full_cover(int64_t n, int64_t tiles, int64_t part) {
+    uint64_t v = 0;
+    for (int64_t at = 0; at < n; at += part) {
+        const int64_t c = n - at < part ? n - at : part;
+        v += gs::binned_pack((uint32_t)c, (uint64_t)c * (uint64_t)tiles);
+    }
+    CHECK(gs::binned_count(v) == (uint64_t)n);
+    CHECK(gs::binned_cands(v) == (uint64_t)n * (uint64_t)tiles);
+    CHECK((v >> 62) == 0);
+}
+
+static void fields() {
+    const int64_t most = gs::kBinnedTiles;
+    // one Gaussian fewer than 2^34 candidates fits, 2^34 does not (and a first frame of
+    // 2^20 Gaussians over 2^14 tiles is exactly that)
+    CHECK(gs::binned_fits((1 << 20) - 1, most));
+    CHECK(!gs::binned_fits(1 << 20, most));
+    CHECK(!gs::binned_fits(4000000, most));
+    CHECK(gs::binned_fits(4000000, 4000));
+    CHECK(!gs::binned_fits(1, most + 1));
+    CHECK(!gs::binned_fits((int64_t)1 << 28, 1));
+    CHECK(gs::binned_fits(((int64_t)1 << 28) - 1, 1));
+    for (const int64_t n : {1ll, 511ll, 513ll, 1ll << 18, (1ll << 20) - 1, 1ll << 20, 1ll << 22,
+                            6000000ll, (1ll << 28) - 1, 1ll << 28})
+        for (const int64_t t : {1ll, 63ll, 64ll, 65ll, 3600ll, 16383ll, 16384ll, 16385ll})
+            if (gs::binned_fits(n, t)) full_cover(n, t, n > (1 << 18) ? 2048 : 512);
+}
+
+int main() {
+    fields();
+    if (fails == 0) std::puts("ok");
+    return fails ? 1 : 0;
+}

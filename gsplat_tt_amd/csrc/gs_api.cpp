@@ -241,7 +241,6 @@ struct gs_ctx {
     // tile-sorted compact ids and tile ids live in the frame buffers until the
     // next call that reuses them.
     bool rb_valid = false, rb_empty = false;
-    uint32_t* rb_ids = nullptr;
     int64_t rb_T = 0, rb_M = 0, rb_ppre = 0, rb_P = 0;
     int64_t rb_batch = -1;     // its index in the last gs_render_batch (-1: another call)
     bool rb_replayed = false;  // it was replayed from a captured graph
@@ -490,9 +489,15 @@ struct gs_ctx {
         return ms;
     }
 
+    // A training forward's buffers (b_brec, b_ranges, b_pair_id, the image) are about
+    // to be overwritten: no backward may follow it. (The standalone sorts leave
+    // them alone.)
+    void drop_forward() { tr.fwd_valid = false; }
+
     // Project + compaction. Returns M; compact arrays in b_rc/b_dkey/b_brec.
     int64_t run_project(const gs_view* v, bool want_valid, bool want_src) {
         const int64_t n = sd.n;
+        if (n > 0) drop_forward();
         ensure_counters();
         b_rc.ensure(std::max<int64_t>(n, 1) * 32);
         b_dkey.ensure(std::max<int64_t>(n, 1) * 4);
@@ -553,6 +558,7 @@ struct gs_ctx {
         }
         *p_pre_out = p_pre;
         if (p_pre == 0) return 0;
+        drop_forward();
         b_pair_tile.ensure((size_t)p_pre * 4);
         b_pair_id.ensure((size_t)p_pre * 4);
         const size_t eparts = gs::emit_partitions(p_pre);
@@ -635,7 +641,7 @@ struct gs_ctx {
         }
         pend = Pending{};
         pend.t0 = std::chrono::steady_clock::now();
-        tr.fwd_valid = false;  // the frame buffers are about to be reused
+        drop_forward();
         rb_valid = false;
         check_view(v);
         pend.asked = *v;
@@ -1182,12 +1188,30 @@ struct gs_ctx {
         return order;
     }
 
+    // The buffers that a sort of pairs or items over `bits` key bits starts from, of the
+    // pair buffers and the sort's scratch (the other two become its alternates), so
+    // that its last pass ends in the pair buffers, or with `in_scratch` in the scratch.
+    struct SortStart {
+        uint32_t *keys, *vals;
+    };
+    SortStart sort_start(int bits, bool in_scratch) {
+        const bool odd = ((bits + 7) / 8) % 2 != 0;
+        uint32_t* keys[2] = {b_pair_tile.as<uint32_t>(), b_kalt.as<uint32_t>()};
+        uint32_t* vals[2] = {b_pair_id.as<uint32_t>(), b_valt.as<uint32_t>()};
+        const int at = odd != in_scratch ? 1 : 0;
+        sort.keys_alt = keys[at ^ 1];  // (as the next ensure_sort sets them again)
+        sort.vals_alt = vals[at ^ 1];
+        return SortStart{keys[at], vals[at]};
+    }
+
     // From the compact records of the M visible Gaussians (count on the device at
-    // cnt[C_M], depth-key histograms reduced) to the tile-sorted compact ids and
-    // tile ranges: depth sort, candidate scan, pair emission + cull, tile sort,
-    // tile bounds. Returns the sorted compact ids.
+    // cnt[C_M], depth-key histograms reduced) to the tile-sorted compact ids in
+    // b_pair_id and the tile ranges: depth sort, candidate scan, pair emission + cull,
+    // tile sort, tile bounds. The ids end in b_pair_id whichever way the lists are
+    // made: a training forward's backward reads them later, and the standalone sorts
+    // between the two overwrite (or move) the sort's scratch.
     // report: copied to the host once the counters are final (not with tiles_out).
-    uint32_t* frame_tiles(const FrameLayout& L, int64_t N, int64_t T, const gs::TileParams& tp,
+    void frame_tiles(const FrameLayout& L, int64_t N, int64_t T, const gs::TileParams& tp,
                           uint32_t** tiles_out, const gs::HostCopy& report) {
         // without a caller for the tile-sorted keys, the tile sort's last pass
         // counts the pairs per tile instead of writing them, and the ranges come
@@ -1197,6 +1221,7 @@ struct gs_ctx {
         if (L.binned) return binned_tiles(L, N, T, tp, report);
         if (L.blocks) return block_tiles(L, N, tp, report);
         uint32_t* order = depth_order(L, N, tp);
+        const SortStart at = sort_start(tile_bits(T), false);
         record(2);
         HIPCHK(gs::launch_rect_count_scan(b_rc.as<float4>(), 2, order, N, cnt + C_M, tp,
                                           b_offs.as<uint32_t>(), b_bstart.as<uint32_t>(),
@@ -1204,8 +1229,7 @@ struct gs_ctx {
                                           cnt + C_RECT_TICKET, cnt + C_PPRE, L.pcap, true, st));
         HIPCHK(gs::launch_pair_emit(b_rc.as<float4>(), b_rc.as<float4>() + 1, 2, true, order,
                                     b_offs.as<uint32_t>(), b_bstart.as<uint32_t>(), N, cnt + C_M,
-                                    L.pcap, cnt + C_PPRE, tp, b_pair_tile.as<uint32_t>(),
-                                    b_pair_id.as<uint32_t>(), L.pcap, L.lb_emit,
+                                    L.pcap, cnt + C_PPRE, tp, at.keys, at.vals, L.pcap, L.lb_emit,
                                     cnt + C_EMIT_TICKET, cnt + C_P, b_phist_emit.as<uint32_t>(),
                                     tile_bits(T), gs::Emit::kSlots, st));
         const int hcols = gs::tile_hist_cols(tile_bits(T));
@@ -1225,7 +1249,7 @@ struct gs_ctx {
         // drops the culled ones (kPairDrop), so the kept pairs come out compact
         void* tiles_sorted = nullptr;
         uint32_t* ids_sorted = nullptr;
-        HIPCHK(gs::radix_sort_pairs_dev(b_pair_tile.p, b_pair_id.as<uint32_t>(), L.pcap,
+        HIPCHK(gs::radix_sort_pairs_dev(at.keys, at.vals, L.pcap,
                                         cnt + C_PPRE, 4, 0, tile_bits(T), L.hist_tile,
                                         cnt + C_TSORT_TICKETS, sort, st, false, &tiles_sorted,
                                         &ids_sorted, cnt + C_P, want_keys ? nullptr : L.tcnt,
@@ -1237,16 +1261,17 @@ struct gs_ctx {
         } else {
             HIPCHK(gs::launch_ranges_from_counts(L.tcnt, T, b_ranges.as<uint32_t>(), st, report));
         }
-        return ids_sorted;
     }
 
     // frame_tiles of a sorted frame without a caller for the keys: Gaussians emitted
     // by blocks of tiles in depth order, sorted by block, split into the tiles' lists.
-    uint32_t* block_tiles(const FrameLayout& L, int64_t N, const gs::TileParams& tp,
-                          const gs::HostCopy& report) {
+    void block_tiles(const FrameLayout& L, int64_t N, const gs::TileParams& tp,
+                     const gs::HostCopy& report) {
         uint32_t* cnt = L.cnt;
         const uint32_t nb = gs::num_blocks(tp.tiles_x, tp.tiles_y);
         uint32_t* order = depth_order(L, N, tp);
+        // the sorted items in the scratch, the tiles' lists in b_pair_id
+        const SortStart at = sort_start(L.key_bits, true);
         record(2);
         HIPCHK(gs::launch_block_scan(b_rc.as<float4>(), order, N, cnt + C_M, tp,
                                      b_offs.as<uint32_t>(), b_bstart.as<uint32_t>(),
@@ -1254,9 +1279,8 @@ struct gs_ctx {
                                      tp.idx_bits ? (uint32_t)L.pparts : 0u, cnt + C_ITEMS, cnt + C_PPRE, L.pcap, st));
         HIPCHK(gs::launch_block_emit(b_rc.as<float4>(), order, b_offs.as<uint32_t>(),
                                      b_bstart.as<uint32_t>(), N, cnt + C_M, L.pcap, cnt + C_ITEMS,
-                                     tp, b_pair_tile.as<uint32_t>(), b_pair_id.as<uint32_t>(),
-                                     cnt + C_KITEMS, cnt + C_P, b_phist_emit.as<uint32_t>(),
-                                     L.key_bits, st));
+                                     tp, at.keys, at.vals, cnt + C_KITEMS, cnt + C_P,
+                                     b_phist_emit.as<uint32_t>(), L.key_bits, st));
         const int hcols = gs::tile_hist_cols(L.key_bits), dw = gs::sort_digit_width(L.key_bits);
         HIPCHK(gs::launch_reduce_rows(b_phist_emit.as<uint32_t>(), hcols, (uint32_t)L.eparts,
                                       cnt + C_ITEMS, L.pcap, gs::kEmitPartition, dw, L.hist_tile,
@@ -1268,23 +1292,21 @@ struct gs_ctx {
         record(3);
         void* keys = nullptr;
         uint32_t* ids = nullptr;
-        HIPCHK(gs::radix_sort_pairs_dev(b_pair_tile.p, b_pair_id.as<uint32_t>(), L.pcap,
+        HIPCHK(gs::radix_sort_pairs_dev(at.keys, at.vals, L.pcap,
                                         cnt + C_ITEMS, 4, 16, 16 + L.key_bits, L.hist_tile,
                                         cnt + C_TSORT_TICKETS, sort, st, false, &keys, &ids,
                                         cnt + C_KITEMS, L.bcnt,
                                         b_poffs.as<uint32_t>(), nb, true, 16));
-        uint32_t* out = ids == b_pair_id.as<uint32_t>() ? b_valt.as<uint32_t>()
-                                                        : b_pair_id.as<uint32_t>();
         HIPCHK(gs::launch_block_lists(static_cast<uint32_t*>(keys), ids, L.pcap,
                                       L.bcnt, b_bins.as<uint32_t>(), cnt + C_SEGS, tp, L.tcnt,
-                                      b_ranges.as<uint32_t>(), out, report, st));
-        return out;
+                                      b_ranges.as<uint32_t>(), b_pair_id.as<uint32_t>(), report,
+                                      st));
     }
 
     // frame_tiles of a binned frame, whose projection scanned the candidates:
     // pair emission in compact order, then the tiles' lists sorted one by one.
-    uint32_t* binned_tiles(const FrameLayout& L, int64_t N, int64_t T, const gs::TileParams& tp,
-                           const gs::HostCopy& report) {
+    void binned_tiles(const FrameLayout& L, int64_t N, int64_t T, const gs::TileParams& tp,
+                      const gs::HostCopy& report) {
         uint32_t* cnt = L.cnt;
         record(2);  // no depth sort of its own
         HIPCHK(gs::launch_pair_emit(b_rc.as<float4>(), b_rc.as<float4>() + 1, 2, false, nullptr,
@@ -1299,7 +1321,6 @@ struct gs_ctx {
                                        b_dkey.as<uint32_t>(), b_ranges.as<uint32_t>(),
                                        b_valt.as<uint32_t>(), b_kalt.as<uint32_t>(), L.runs,
                                        cnt + C_RUNS, b_pair_id.as<uint32_t>(), cnt + C_CTL, report, st));
-        return b_pair_id.as<uint32_t>();
     }
     gs::BinnedOut binned_out(const FrameLayout& L) const {
         if (!L.binned) return gs::BinnedOut{};
@@ -1554,8 +1575,9 @@ struct gs_ctx {
         gs::TileParams tp{tiles_x, tiles_y, v->tile_size, v->cull_disabled ? 0 : 1,
                           L.cnt + C_CTL, p.idx_bits};
         uint32_t* tiles_sorted = nullptr;
-        uint32_t* ids_sorted = frame_tiles(L, N, T, tp, cull_stats ? &tiles_sorted : nullptr,
-                                           gs::HostCopy{h_pin, L.cnt, 64});
+        frame_tiles(L, N, T, tp, cull_stats ? &tiles_sorted : nullptr,
+                    gs::HostCopy{h_pin, L.cnt, 64});
+        const uint32_t* ids_sorted = b_pair_id.as<uint32_t>();
         record(4);
         gs::BlendParams bp{tiles_x, tiles_y, v->tile_size, v->image_height, v->image_width,
                            v->cull_disabled ? 1 : 0, v->transmittance_threshold, v->out_format,
@@ -1569,7 +1591,6 @@ struct gs_ctx {
                                        L.cnt + C_P, tiles_x, v->tile_size, v->cull_disabled,
                                        reinterpret_cast<unsigned long long*>(L.cnt + C_MBSTAT),
                                        L.cnt + C_CTL, st));
-        rb_ids = ids_sorted;
     }
 
     // ------------------------------------------------------------ training
@@ -1586,7 +1607,6 @@ struct gs_ctx {
         gs::TrainCam cam{};
         uint32_t M = 0, P = 0, p_pre = 0;
         int64_t pixel_pairs = 0, pixel_blended = 0;
-        uint32_t* ids = nullptr;  // tile-sorted compact ids of the last forward
         double loss = 0.0, l1 = 0.0, ssim = 0.0;
     } tr;
     // Adam moments stored as bf16 bits (gs_train_set_moments), kept across
@@ -1876,7 +1896,7 @@ struct gs_ctx {
                                           nullptr, 0, 0, 0, L.hist_depth, st, nullptr,
                                           L.cnt + C_CTL));
         gs::TileParams tp{tr.tiles_x, tr.tiles_y, 16, 1, L.cnt + C_CTL};
-        tr.ids = frame_tiles(L, std::max<int64_t>(N, 1), T, tp, nullptr, gs::HostCopy{});
+        frame_tiles(L, std::max<int64_t>(N, 1), T, tp, nullptr, gs::HostCopy{});
         gs::TrainFwdParams fp{};
         fp.tiles_x = tr.tiles_x;
         fp.tiles_y = tr.tiles_y;
@@ -1895,7 +1915,7 @@ struct gs_ctx {
                                 (3.0 * (double)px));
         fp.sums = L.sums;
         fp.ctl = L.cnt + C_CTL;
-        HIPCHK(gs::launch_train_fwd(b_brec.as<float4>(), tr.ids, b_ranges.as<uint32_t>(), fp, st));
+        HIPCHK(gs::launch_train_fwd(b_brec.as<float4>(), b_pair_id.as<uint32_t>(), b_ranges.as<uint32_t>(), fp, st));
         if (tgt_dev != nullptr && c->lambda_dssim > 0.0f)
             enqueue_ssim(t_img.as<float>(), tgt_dev, H, W, c->lambda_dssim, c->loss_scale,
                          t_dimg.as<float>(), L.sums);
@@ -1978,7 +1998,7 @@ struct gs_ctx {
         bp.dimage = t_dimg.as<float>();
         bp.grad2d = t_grad2d.as<float>();
         bp.ctl = tr.cam.ctl;
-        HIPCHK(gs::launch_train_bwd(b_brec.as<float4>(), tr.ids, b_ranges.as<uint32_t>(), bp, st));
+        HIPCHK(gs::launch_train_bwd(b_brec.as<float4>(), b_pair_id.as<uint32_t>(), b_ranges.as<uint32_t>(), bp, st));
         // the device time of a step's Adam is part of its gradient pass
         if (timing && adam) HIPCHK(hipEventRecord(tev[3], st));
         if (timing && adam) HIPCHK(hipEventRecord(tev[4], st));
@@ -2146,7 +2166,7 @@ int gs_frame_readback(gs_ctx* ctx, int64_t* counts, int64_t* sorted_ids, int64_t
         std::vector<uint32_t> ids(sorted_ids && P > 0 ? (size_t)P : 0), rg(tile_ranges ? (size_t)T * 2 : 0);
         if (!ctx->rb_empty) {
             if (!ids.empty())
-                HIPCHK(hipMemcpyAsync(ids.data(), ctx->rb_ids, (size_t)P * 4, hipMemcpyDeviceToHost,
+                HIPCHK(hipMemcpyAsync(ids.data(), ctx->b_pair_id.p, (size_t)P * 4, hipMemcpyDeviceToHost,
                                       ctx->st));
             if (!rg.empty())
                 HIPCHK(hipMemcpyAsync(rg.data(), ctx->b_ranges.p, (size_t)T * 8,
@@ -2428,6 +2448,7 @@ int gs_sort_and_bin(gs_ctx* ctx, const int64_t* gids, const int64_t* tids, const
             return;
         }
         ctx->sync();
+        ctx->drop_forward();
         ctx->ensure_counters();
         ctx->b_tmp_a.ensure((size_t)p * 4);
         ctx->b_tmp_b.ensure((size_t)p * 4);
@@ -2497,6 +2518,7 @@ int gs_cull_and_blend(gs_ctx* ctx, const float* means2d, const float* covs2d,
             lthr[i] = (o <= view->mb_contrib_floor) ? 0.0f : std::log(view->mb_contrib_floor / o);
         }
         ctx->sync();
+        ctx->drop_forward();
         const size_t mm = (size_t)std::max<int64_t>(m, 1);
         ctx->b_tmp_a.ensure(mm * 4 * 11);
         float* base = ctx->b_tmp_a.as<float>();
@@ -2890,6 +2912,7 @@ int gs_train_loss(gs_ctx* ctx, const float* image, const float* target, int heig
         HIPCHK(hipSetDevice(ctx->device));
         ctx->drain_spec();
         const size_t px = (size_t)height * width;
+        ctx->drop_forward();  // t_dimg and t_img are this call's
         ctx->t_img.ensure(px * 12);
         ctx->t_tgt.ensure(px * 12);
         ctx->t_dimg.ensure(px * 12);
@@ -2910,7 +2933,6 @@ int gs_train_loss(gs_ctx* ctx, const float* image, const float* target, int heig
         HIPCHK(hipMemcpyAsync(dimage, ctx->t_dimg.p, px * 12, hipMemcpyDeviceToHost, st));
         HIPCHK(hipMemcpyAsync(h, sums, sizeof(h), hipMemcpyDeviceToHost, st));
         ctx->sync();
-        ctx->tr.fwd_valid = false;  // t_dimg / t_img no longer hold a training forward
         if (loss3) {
             const double n = 3.0 * (double)px, lam = lambda_dssim;
             const gs::TrainSums sum = gs_ctx::add_sums(h);

@@ -461,3 +461,98 @@ def test_train_arrays_round_trip(gpu_ctx, n, deg):
         assert all(np.array_equal(got[k], arrs[0][k]) for k in shp)
     finally:
         tr.set_moments(False)
+
+
+def _spread_params(rng, n, W, H, f):
+    z = rng.uniform(2, 4, n)
+    p = {"means": np.stack([rng.uniform(-0.5, 0.5, n) * W / f * z,
+                            rng.uniform(-0.5, 0.5, n) * H / f * z, z], 1),
+         "log_scales": rng.normal(np.log(18.0 / f), 0.3, (n, 3)),  # about 6 pixels
+         "quats": rng.standard_normal((n, 4)), "opacity_logits": rng.normal(0, 1.0, n),
+         "sh": rng.uniform(-0.5, 0.5, (n, 1, 3))}
+    return {k: v.astype(np.float32) for k, v in p.items()}
+
+
+@pytest.mark.parametrize("h,w", [(40, 56), (129 * 16, 128 * 16 + 1), (32, 33_000 * 16)])
+def test_train_backward_after_a_sort(h, w):
+    """A standalone sort between a forward and its backward (binned; by blocks, two sort
+    passes; sorted by tile, three) leaves the forward's ids, records and ranges alone:
+    the gradients are those of a backward right after the forward, but for the order
+    of the atomic adds: float32 sums of some 50 band terms, 50 x 2^-24 = 3e-6 of the
+    terms' magnitude, of which a mean's gradient keeps a tenth or more in the 2-norm
+    (single elements may cancel to nothing, so not element by element): 1e-4."""
+    print("train sort between", h, w, flush=True)
+    rng = np.random.default_rng(h)
+    f = 0.9 * w
+    p = _spread_params(rng, 3000, w, h, f)
+    view = L.make_view(np.eye(4, dtype=np.float32), scenes.intrinsics(f, f, w / 2, h / 2), h, w,
+                       tile_size=16)
+    cfg = L.make_train_cfg()
+    target = np.zeros((h, w, 3), np.float32)
+    n, tiles = 100_003, 500
+    keys = (rng.integers(0, tiles, n).astype(np.uint64) << np.uint64(32)) | \
+        rng.uniform(1, 2, n).astype(np.float32).view(np.uint32).astype(np.uint64)
+    ctx = L.Context(0)
+    ptrs = []
+    try:
+        tr = L.Trainer(ctx, p, 0)
+        tr.forward(view, cfg, target)
+        tr.backward(cfg)
+        ref = tr.read(3)
+        ptrs = [ctx.dev_alloc(8 * n), ctx.dev_alloc(4 * n), ctx.dev_alloc(8 * tiles)]
+        for ids in (False, True):
+            tr.forward(view, cfg, target)
+            ctx.h2d(ptrs[0], keys)
+            ctx.h2d(ptrs[1], np.arange(n, dtype=np.uint32))
+            sort = ctx.sort_tile_depth_ids_dev if ids else ctx.sort_tile_depth_dev
+            sort(ptrs[0], ptrs[1], n, tiles, ptrs[2])
+            tr.backward(cfg)
+            got = tr.read(3)
+            for k in TO.PARAM_NAMES:
+                assert np.abs(ref[k]).max() > 0, k
+                assert np.linalg.norm(got[k] - ref[k]) < 1e-4 * np.linalg.norm(ref[k]), (k, ids)
+    finally:
+        for q in ptrs:
+            ctx.dev_free(q)
+        ctx.close()
+
+
+def test_train_backward_needs_its_buffers(gpu_ctx):
+    """Calls that overwrite what a forward left (projection, tile assignment, binning,
+    blending, a loss, a frame) make its backward an error; with nothing to do they
+    leave it."""
+    print("train buffers", flush=True)
+    rng = np.random.default_rng(2)
+    h, w, n = 40, 56, 200
+    p = _spread_params(rng, n, w, h, 50.0)
+    view = L.make_view(np.eye(4, dtype=np.float32), scenes.intrinsics(50.0, 50.0, w / 2, h / 2),
+                       h, w, tile_size=16, output="f32")
+    cfg = L.make_train_cfg()
+    cov = scenes.cov3d(np.exp(p["log_scales"]), p["quats"] /
+                       np.linalg.norm(p["quats"], axis=1, keepdims=True))
+    op, col = np.full(n, 0.5, np.float32), rng.random((n, 3)).astype(np.float32)
+    pr = gpu_ctx.project(p["means"], cov, op, col, view)
+    assign = (pr["means2d"], pr["radii"], h, w, 16, pr["covs2d"], pr["opacities"])
+    g, t, _ = gpu_ctx.tile_assign(*assign)
+    ids, ranges = gpu_ctx.sort_and_bin(g, t, pr["depths"], 4, 3)
+    img = np.zeros((h, w, 3), np.float32)
+    calls = {
+        "project": lambda: gpu_ctx.project(p["means"], cov, op, col, view),
+        "tile_assign": lambda: gpu_ctx.tile_assign(*assign),
+        "sort_and_bin": lambda: gpu_ctx.sort_and_bin(g, t, pr["depths"], 4, 3),
+        "cull_and_blend": lambda: gpu_ctx.cull_and_blend(
+            pr["means2d"], pr["covs2d"], pr["colors"], pr["opacities"], ids, ranges, view),
+        "loss": lambda: gpu_ctx.train_loss(img, img + 0.5, 0.2),
+        "render": lambda: (gpu_ctx.set_scene(p["means"], cov, op, col), gpu_ctx.render(view)),
+    }
+    tr = L.Trainer(gpu_ctx, p, 0)
+    for name, call in calls.items():
+        tr.forward(view, cfg, img)
+        call()
+        with pytest.raises(ValueError, match="no current forward"):
+            tr.backward(cfg)
+    tr.forward(view, cfg, img)
+    gpu_ctx.tile_assign(*(a[:0] for a in assign[:2]), h, w, 16)
+    gpu_ctx.sort_and_bin(g[:0], t[:0], pr["depths"], 4, 3)
+    tr.backward(cfg)
+    assert any(np.abs(a).max() > 0 for a in tr.read(3).values())

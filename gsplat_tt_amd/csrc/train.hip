@@ -13,6 +13,8 @@
 // radius k = sqrt(2 ln(op / alpha_min)) (uncapped) and the per-pair tile cull at
 // the same floor, so the tiled forward blends exactly the pairs the per-pixel
 // oracle blends.
+#include <type_traits>
+
 #include "gs_common.h"
 #include "gs_internal.h"
 
@@ -486,6 +488,9 @@ __global__ __launch_bounds__(GS_WAVE) void k_train_fwd(const float4* __restrict_
         for (uint32_t base = start; base < end; base += GS_WAVE) {
             const bool keep = base + lane < end && band_keeps(r0, r1, bx0, by0);
             const uint64_t mask = __ballot(keep);
+            // kept entries whose colours are not finite (or past the range when added up)
+            const uint64_t odd = __ballot(
+                keep && !(fabsf(r2.x) + fabsf(r2.y) + fabsf(r2.z) < __builtin_inff()));
             const int cnt = __popcll(mask);
             __syncthreads();  // one wave: orders the LDS reads of the batch before
             if (keep) {
@@ -504,28 +509,42 @@ __global__ __launch_bounds__(GS_WAVE) void k_train_fwd(const float4* __restrict_
             r2 = trec[3 * (size_t)gi + 2];
             gi = sid[min(base + 2 * GS_WAVE + lane, end - 1)];
             __syncthreads();
-            for (int k = 0; k < cnt; k += 4) {
+            // An entry that the pixel does not blend adds 0 times its colour, but where a
+            // colour of the batch is not finite the sums are selected instead (1M Gaussians
+            // at 1280x720: 117 us without the second walk, 119 with it, 123.5 with
+            // selects in every batch).
+            const auto walk = [&](auto select) {
+                for (int k = 0; k < cnt; k += 4) {
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const float4 e0 = s0[k + j], e1 = s1[k + j];
-                    const float2 e2 = s2[k + j];
-                    const Splat s = splat_at(pxc, pyc, e0.x, e0.y, e0.w, e1.x, e1.y, e0.z);
-                    const float alpha = fminf(s.raw, fp.alpha_max);
-                    const bool live = alpha >= fp.alpha_min && !done;
-                    const float tn = T * (1.0f - alpha);
-                    const bool hit = live && tn < fp.t_min;
-                    const bool bl = live && !hit;
-                    done = done || hit;
-                    stop = hit ? __float_as_uint(e2.y) : stop;
-                    const float at = bl ? alpha * T : 0.0f;
-                    cr += at * e1.z;
-                    cg += at * e1.w;
-                    cb += at * e2.x;
-                    T = bl ? tn : T;
-                    blended += (uint32_t)__popcll(__ballot(bl));
+                    for (int j = 0; j < 4; ++j) {
+                        const float4 e0 = s0[k + j], e1 = s1[k + j];
+                        const float2 e2 = s2[k + j];
+                        const Splat s = splat_at(pxc, pyc, e0.x, e0.y, e0.w, e1.x, e1.y, e0.z);
+                        const float alpha = fminf(s.raw, fp.alpha_max);
+                        const bool live = alpha >= fp.alpha_min && !done;
+                        const float tn = T * (1.0f - alpha);
+                        const bool hit = live && tn < fp.t_min;
+                        const bool bl = live && !hit;
+                        done = done || hit;
+                        stop = hit ? __float_as_uint(e2.y) : stop;
+                        const float at = bl ? alpha * T : 0.0f;
+                        if constexpr (decltype(select)::value) {
+                            cr = bl ? cr + at * e1.z : cr;
+                            cg = bl ? cg + at * e1.w : cg;
+                            cb = bl ? cb + at * e2.x : cb;
+                        } else {
+                            cr += at * e1.z;
+                            cg += at * e1.w;
+                            cb += at * e2.x;
+                        }
+                        T = bl ? tn : T;
+                        blended += (uint32_t)__popcll(__ballot(bl));
+                    }
+                    if (__ballot(!done) == 0ull) break;
                 }
-                if (__ballot(!done) == 0ull) break;
-            }
+            };
+            if (odd == 0ull) walk(std::false_type{});
+            else walk(std::true_type{});
             if (__ballot(!done) == 0ull) break;
         }
     }
@@ -825,7 +844,8 @@ __device__ __forceinline__ int term_of_lane(int l) {
 // behind_{i+1}) starting from the background's bg . g (the colours behind an
 // entry are only ever needed through their product with the pixel's gradient),
 // dL/dalpha_i = T_i (s_i - behind_i). A lane that does not blend the entry has
-// alpha 0, which leaves T and behind as they are, and contributes exact zeros.
+// alpha 0, which leaves T as it is, keeps its behind (by a select: the entry's colour
+// may not be finite) and contributes exact zeros.
 // The nine per-pair terms (dmx dmy dA dB dC dop dr dg db) of two entries at a
 // time are summed over the wave (sum_terms) and 18 lanes add them to the
 // Gaussians' accumulators, one atomic each. 1/(1 - alpha) is one reciprocal
@@ -909,7 +929,7 @@ __global__ __launch_bounds__(GS_WAVE) void k_train_bwd(const float4* __restrict_
                 const float Tn = T * __builtin_amdgcn_rcpf(1.0f - a);
                 const float d = __builtin_fmaf(e1.z, g0, __builtin_fmaf(e1.w, g1, e2.x * g2)) -
                                 behind;
-                behind = __builtin_fmaf(a, d, behind);
+                behind = live ? __builtin_fmaf(a, d, behind) : behind;
                 T = Tn;
                 const float at = a * Tn;
                 // no gradient through the clamps

@@ -15,7 +15,6 @@
 
 #include <algorithm>
 #include <array>
-#include <atomic>
 #include <chrono>
 #include <climits>
 #include <cmath>
@@ -23,11 +22,11 @@
 #include <memory>
 #include <stdexcept>
 #include <string>
-#include <thread>
 #include <vector>
 
 #include "../../include/gsplat_hip.h"
 #include "gs_internal.h"
+#include "host_threads.h"
 #include "out_ring.h"
 
 namespace {
@@ -90,28 +89,11 @@ struct DevBuf {
     T* as() const { return static_cast<T*>(p); }
 };
 
-template <class F>
-void parallel_for(int64_t n, F&& f) {
-    const int64_t hw = std::max(1u, std::thread::hardware_concurrency());
-    const int64_t workers = std::min<int64_t>(hw, std::max<int64_t>(1, n / 65536));
-    if (workers <= 1) {
-        f(0, n);
-        return;
-    }
-    std::vector<std::thread> ts;
-    const int64_t chunk = (n + workers - 1) / workers;
-    for (int64_t w = 0; w < workers; ++w) {
-        const int64_t lo = w * chunk, hi = std::min(n, lo + chunk);
-        if (lo < hi) ts.emplace_back([&f, lo, hi] { f(lo, hi); });
-    }
-    for (auto& t : ts) t.join();
-}
-
 // Per-Gaussian opacity terms with the C library's logf (types.h:141-176,
 // tile_assign.cpp:171-197, cull_and_blend.cpp:743-753).
 void opacity_terms(const float* op, int64_t n, bool has_opac, float cf, float mbf, float k_cap,
                    float* kfac, float* m2thr, float* lthr) {
-    parallel_for(n, [&](int64_t lo, int64_t hi) {
+    gs::parallel_for(n, [&](int64_t lo, int64_t hi) {
         for (int64_t i = lo; i < hi; ++i) {
             float k = 3.0f;
             if (has_opac) {
@@ -1642,61 +1624,6 @@ struct gs_ctx {
                 if (e) (void)hipEventDestroy(e);
         }
     } stage;
-    // One of a chunk's arrays: `bytes` at `off` of the chunk, and in the caller's memory.
-    struct Piece {
-        char* host;
-        size_t off, bytes;
-    };
-    // Threads that copy each announced chunk together with the calling one.
-    class ChunkCopy {
-    public:
-        ChunkCopy(int workers, bool down) : w_(workers), down_(down) {
-            for (int i = 1; i < w_; ++i) ts_.emplace_back([this, i] { work(i); });
-        }
-        ~ChunkCopy() {
-            stop_.store(true, std::memory_order_release);
-            for (auto& t : ts_) t.join();
-        }
-        // Copies a chunk at `pin`; returns when all of it is copied.
-        void chunk(char* pin, const std::array<Piece, 5>& p) {
-            pin_ = pin;
-            p_ = p;
-            left_.store(w_ - 1, std::memory_order_relaxed);
-            seq_.fetch_add(1, std::memory_order_release);
-            share(0);
-            while (left_.load(std::memory_order_acquire) > 0) std::this_thread::yield();
-        }
-
-    private:
-        void share(int i) const {
-            for (const Piece& q : p_) {
-                const size_t lo = q.bytes * (size_t)i / (size_t)w_ & ~size_t(63);
-                const size_t hi = i + 1 == w_ ? q.bytes
-                                              : q.bytes * (size_t)(i + 1) / (size_t)w_ & ~size_t(63);
-                if (down_) std::memcpy(q.host + lo, pin_ + q.off + lo, hi - lo);
-                else std::memcpy(pin_ + q.off + lo, q.host + lo, hi - lo);
-            }
-        }
-        void work(int i) {
-            for (int seen = 0;;) {
-                while (seq_.load(std::memory_order_acquire) == seen) {
-                    if (stop_.load(std::memory_order_acquire)) return;
-                    std::this_thread::yield();
-                }
-                ++seen;
-                share(i);
-                left_.fetch_sub(1, std::memory_order_release);
-            }
-        }
-        const int w_;
-        const bool down_;
-        std::vector<std::thread> ts_;
-        std::atomic<bool> stop_{false};
-        std::atomic<int> seq_{0}, left_{0};
-        char* pin_ = nullptr;
-        std::array<Piece, 5> p_{};
-    };
-
     void train_move(DevBuf& b, const gs_train_arrays* a, bool down) {
         REQUIRE(a && a->means && a->log_scales && a->quats && a->opacity_logits && a->sh,
                 down ? "train: null output array" : "train: null parameter array");
@@ -1718,7 +1645,7 @@ struct gs_ctx {
         const size_t wide[5] = {12, 12, 16, 4, (size_t)K * 12};  // bytes per Gaussian
         auto count = [&](int64_t c) { return std::min(rows, n - c * rows); };
         auto pieces = [&](int64_t c) {
-            std::array<Piece, 5> p;
+            std::array<gs::Piece, 5> p;
             size_t off = 0;
             for (int q = 0; q < 5; ++q) {
                 p[q] = {host[q] + (size_t)(c * rows) * wide[q], off, (size_t)count(c) * wide[q]};
@@ -1742,7 +1669,7 @@ struct gs_ctx {
             HIPCHK(hipEventRecord(stage.done[c & 1], st));
         };
         const size_t total = (size_t)n * vals * 4;
-        ChunkCopy copy((int)std::max<size_t>(1, std::min<size_t>(8, total >> 21)), down);
+        gs::ChunkCopy copy(gs::host_threads(std::min<int64_t>(8, (int64_t)(total >> 21))), down);
         try {
             if (down)
                 for (int64_t c = 0; c < std::min<int64_t>(2, chunks); ++c) transfer(c);

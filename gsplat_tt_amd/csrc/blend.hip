@@ -21,8 +21,8 @@
 // T *= 1-alpha, test after every entry) (cull_and_blend.cpp:506-670,
 // simd_exp_avx2.h:12-32), a lane evaluating only what its half keeps. The wave
 // exits when both microblocks are done. (k_blend. k_blend_mb, below it, gives a
-// microblock its own wave, two lanes per pixel: frames that run alone or are
-// binned.)
+// microblock its own wave, two lanes per pixel: frames that run alone, and small
+// ones in flight.)
 #include <algorithm>
 
 #include "gs_common.h"

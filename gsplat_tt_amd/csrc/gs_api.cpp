@@ -1039,8 +1039,6 @@ struct gs_ctx {
         }
     }
 
-    // Enqueues one frame (project -> depth sort -> tile assign -> tile sort ->
-    // ranges -> blend) on the stream; no host synchronisation.
     // Frame buffers for N Gaussians, T tiles and the current pair capacity, all
     // allocated before the first launch of a frame.
     struct FrameLayout {
@@ -1496,7 +1494,8 @@ struct gs_ctx {
             if (nn) HIPCHK(hipGraphGetNodes(fg.graph, nodes.data(), &nn));
             const void* fn_proj = gs::project_kernel(sd.sh_degree, L.binned, N);
             const void* fn_blend = gs::blend_kernel(pend.v.tile_size, pend.v.out_format,
-                                                    blend_by_microblock(L));
+                                                    blend_by_microblock(L, pend.T,
+                                                                        pend.v.tile_size));
             hipGraphNode_t proj = nullptr;
             for (hipGraphNode_t node : nodes) {
                 hipGraphNodeType ty;
@@ -1518,14 +1517,21 @@ struct gs_ctx {
         return true;
     }
 
-    // A wave per microblock blends every frame that runs alone faster, and every
-    // binned one; a wave per band takes 15 % fewer instructions where most entries
-    // are kept by both of its microblocks, which is what counts for a large frame
-    // among others in flight (us a frame alone and in a path, band against
-    // microblock; 1237x822 slab scenes: 300K 228, 154 / 200, 154; 1.5M 545, 380 /
-    // 495, 387; 6M 1264, 1022 / 1223, 1046; 300x200, 3300 pairs a tile: 696, 364 /
-    // 280, 153).
-    bool blend_by_microblock(const FrameLayout& L) const { return L.binned || !batch_frame; }
+    // A wave per microblock blends every frame that runs alone faster. Among frames in
+    // flight it wins where a frame's bands are too few to fill the chip four at a time;
+    // larger frames take the wave per band, which needs 15 % fewer instructions and half
+    // of the record reads where most entries are kept by both of its microblocks (us a
+    // frame in a path, band against microblock. Binned: 640x480 0.62M pairs in tiles of
+    // 32 (4800 bands) 211 / 182, 1280x720 (14720) 186 / 172, 1237x822 (16224) 271 / 268,
+    // 1280x960 (19200) 168 / 171, 1920x1080 0.09M (33120) 74 / 84, 1.8M 199 / 220,
+    // 2560x1440 0.9M 202 / 230. Others: 640x480 3.5M 240 / 237, 2.9M in tiles of 32
+    // 372 / 318, 1280x720 6.6M 454 / 451, 1237x822 10M 372 / 381, 30M 1022 / 1046,
+    // 1280x960 5.3M 243 / 251).
+    static constexpr int64_t kMicroblockBands = 15360, kMicroblockBandsBinned = 16384;
+    bool blend_by_microblock(const FrameLayout& L, int64_t T, int tile_size) const {
+        const int64_t bands = T * (tile_size * tile_size / 64);
+        return !batch_frame || bands <= (L.binned ? kMicroblockBandsBinned : kMicroblockBands);
+    }
 
     // Enqueues one frame (project -> depth sort -> tile assign -> tile sort ->
     // ranges -> blend) on the stream; no host synchronisation.
@@ -1564,7 +1570,7 @@ struct gs_ctx {
         gs::BlendParams bp{tiles_x, tiles_y, v->tile_size, v->image_height, v->image_width,
                            v->cull_disabled ? 1 : 0, v->transmittance_threshold, v->out_format,
                            blend_counts ? b_evals.as<unsigned long long>() : nullptr,
-                           L.cnt + C_CTL, blend_by_microblock(L)};
+                           L.cnt + C_CTL, blend_by_microblock(L, T, v->tile_size)};
         HIPCHK(gs::launch_blend(b_brec.as<float4>(), ids_sorted, b_ranges.as<uint32_t>(), bp,
                                 dout, st));
         record(5);

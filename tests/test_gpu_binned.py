@@ -225,3 +225,30 @@ def test_blend_by_microblock_equals_by_band(gpu_ctx, h, w, ts, n, op):
     ref = gpu_ctx.cull_and_blend(p["means2d"], p["covs2d"], p["colors"], p["opacities"], ids,
                                  ranges, view)
     assert np.array_equal(img.view(np.uint32), ref.view(np.uint32))
+
+
+@pytest.mark.parametrize("h,w,ts", [(48, 64, 16), (64 * 16, 64 * 16 - 3, 16), (65 * 16 - 5, 64 * 16, 16),
+                                    (480, 640, 32), (31 * 32, 32 * 32, 32), (33 * 32, 32 * 32, 32)])
+def test_blend_of_frames_in_flight(h, w, ts):
+    """Frames in flight blend with a wave per microblock up to 15360 or 16384 bands of
+    16 x 4 pixels and with one per band above: the images of a path are those of single
+    frames on both sides of the line, binned and not (more than 2^20 Gaussians), through
+    captures and replays."""
+    print("blend in flight", h, w, ts, flush=True)
+    for n in (3000, (1 << 20) + 5):
+        ctx = L.Context(0)
+        try:
+            ctx.set_scene(*_stack(n, 300, spread=0.25, seed=n + h))
+            views = []
+            for k in range(6):
+                w2c = np.eye(4, dtype=np.float32)
+                w2c[0, 3] = 0.03 * k
+                views.append(L.make_view(w2c, scenes.intrinsics(0.7 * w, 0.7 * w, w / 2, h / 2),
+                                         h, w, tile_size=ts, output="bf16"))
+            ref = [ctx.render(v)[0].copy() for v in views]
+            for _ in range(2):
+                outs = [np.empty((h, w, 3), np.uint16) for _ in views]
+                ctx.render_batch(views, outs, out_on_device=False)
+                assert all(np.array_equal(a, b) for a, b in zip(ref, outs))
+        finally:
+            ctx.close()

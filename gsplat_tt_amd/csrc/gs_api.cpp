@@ -738,7 +738,7 @@ struct gs_ctx {
             s.num_visible = h_pin[C_M];
             s.pairs_pre = h_pin[C_PPRE];
             s.num_entries = h_pin[C_P];
-            plan_seen(sd.n, pend.T, s.num_entries);
+            tile_plans().seen(gs::TilePlans::kFrame, sd.n, pend.T, s.num_entries);
             s.chunks_skipped = h_pin[C_SKIPPED];
             if (cull_stats) {
                 uint64_t mb[2];
@@ -1039,8 +1039,6 @@ struct gs_ctx {
         }
     }
 
-    // Frame buffers for N Gaussians, T tiles and the current pair capacity, all
-    // allocated before the first launch of a frame.
     struct FrameLayout {
         uint32_t* fr;
         uint32_t* cnt;
@@ -1057,17 +1055,6 @@ struct gs_ctx {
         bool blocks;   // sorted by blocks of tiles (not the microblock statistics' frames)
         int key_bits;  // of the sorted tile (block) ids
     };
-    // Whether frames of N Gaussians and T tiles have their tile lists binned
-    // (launch_binned_lists) or made by blocks of tiles (block_tiles). Binning needs
-    // no depth sort and fewer launches but stores each pair at its list's end and
-    // sorts each list on its own, so it wins up to about 2.4M pairs (us a frame
-    // alone and in a path, blocks against binned; 1280x720: 1.1M pairs 317, 213 /
-    // 243, 186; 1.7M 366, 246 / 294, 227; 2.8M 434, 295 / 380, 291; 1237x822: 1.5M
-    // 263, 173 / 201, 156; 3.0M 314, 221 / 320, 255; 5.0M 367, 276 / 477, 407;
-    // 400x300, 3100 pairs a tile: 1.5M 283, 234 / 294, 186). The pairs of a view are
-    // not known before it is rendered: a scene's frames start from the number of
-    // Gaussians and go on with the pairs of the frames that finished, with a gap
-    // between the two limits so that a camera path does not alternate.
     // Frames that are not binned sort every pair by its tile only for the microblock
     // statistics, which read the sorted keys, and above 2^16 tiles, where few pairs
     // share a tile (us a frame alone and in a path, pairs against blocks; 1237x822:
@@ -1075,29 +1062,17 @@ struct gs_ctx {
     // 775; 1920x1080, 54M 1727, 1467 / 1208, 961; Gaussians of about one tile,
     // 300x200 in tiles of 32, 4.6M: 1197, 1546 / 1119, 1448).
     static constexpr int64_t kBlockTilesMost = 1 << 16;
-    static constexpr int64_t kBinnedFirst = 1 << 20, kBinnedMost = 2400000,
-                             kBinnedAgain = 1800000;
-    struct TilePlan {
-        int64_t n = -1, T = -1;
-        bool binned = false;
-    } plan;  // of the first slot, for all of them
-    bool binned_frame(int64_t N, int64_t T, bool want_keys) {
-        TilePlan& p = (owner ? owner : this)->plan;
-        if (p.n != N || p.T != T) p = {N, T, N <= kBinnedFirst};
-        // the microblock statistics need the sorted tile keys
-        return p.binned && !want_keys && gs::binned_fits(N, T);
-    }
-    void plan_seen(int64_t N, int64_t T, int64_t P) {
-        TilePlan& p = (owner ? owner : this)->plan;
-        if (p.n != N || p.T != T) return;
-        if (P > kBinnedMost) p.binned = false;
-        if (P < kBinnedAgain) p.binned = true;
-    }
-    FrameLayout frame_prepare(int64_t N, int tiles_x, int tiles_y, bool want_keys) {
+    gs::TilePlans plans;  // the first slot's, for all of them
+    gs::TilePlans& tile_plans() { return (owner ? owner : this)->plans; }
+    // Frame buffers for N Gaussians, T tiles and the current pair capacity, all
+    // allocated before the first launch of a frame.
+    FrameLayout frame_prepare(gs::TilePlans::Kind kind, int64_t N, int tiles_x, int tiles_y,
+                              bool want_keys) {
         FrameLayout L{};
         const int64_t T = (int64_t)tiles_x * tiles_y;
         L.pcap = (uint32_t)pair_cap;
-        L.binned = binned_frame(N, T, want_keys);
+        // the microblock statistics need the sorted tile keys
+        L.binned = !want_keys && tile_plans().binned(kind, N, T);
         const int64_t nb = ((int64_t)tiles_x + 3) / 4 * (((int64_t)tiles_y + 3) / 4);
         L.blocks = !L.binned && !want_keys && T <= kBlockTilesMost;
         L.key_bits = tile_bits(L.blocks ? nb : T);
@@ -1411,7 +1386,8 @@ struct gs_ctx {
             return false;
         if (sd.chunk_box != nullptr && pend.v.k_cap <= 3.0f) return false;
         if (N >= ((int64_t)1 << 30) || pair_cap >= (1ull << 30)) return false;
-        const FrameLayout L = frame_prepare(N, pend.tiles_x, pend.tiles_y, false);  // every allocation before a capture
+        const FrameLayout L = frame_prepare(gs::TilePlans::kFrame, N, pend.tiles_x, pend.tiles_y,
+                                            false);  // every allocation before a capture
         const gs_view shape = graph_shape(&pend.v);
         const uint64_t gen = buffers_key();
         const bool same_shape = fg.n == N && fg.T == pend.T && fg.deg == sd.sh_degree && fg.pcap == pair_cap && fg.gen == gen &&
@@ -1537,7 +1513,7 @@ struct gs_ctx {
     // ranges -> blend) on the stream; no host synchronisation.
     void frame(const gs_view* v, void* dout, int64_t T, int tiles_x, int tiles_y) {
         const int64_t N = sd.n;
-        const FrameLayout L = frame_prepare(N, tiles_x, tiles_y, cull_stats);
+        const FrameLayout L = frame_prepare(gs::TilePlans::kFrame, N, tiles_x, tiles_y, cull_stats);
         record(0);
         HIPCHK(gs::launch_fill_u32(L.fr, 0u, L.fwords, st));
         if (spin_limit) HIPCHK(gs::launch_fill_u32(L.cnt + C_CTL + 1, spin_limit, 1, st));
@@ -1798,7 +1774,8 @@ struct gs_ctx {
         tr.tiles_y = (H + 15) / 16;
         const int64_t T = (int64_t)tr.tiles_x * tr.tiles_y;
         tr.cam = train_cam(v, c);
-        const FrameLayout L = frame_prepare(std::max<int64_t>(N, 1), tr.tiles_x, tr.tiles_y, false);
+        const FrameLayout L = frame_prepare(gs::TilePlans::kTrain, std::max<int64_t>(N, 1), tr.tiles_x,
+                                            tr.tiles_y, false);
         const size_t px = (size_t)H * W;
         t_img.ensure(px * 12);
         t_T.ensure(px * 4);
@@ -1901,7 +1878,8 @@ struct gs_ctx {
         tr.M = h_pin[C_M];
         tr.p_pre = h_pin[C_PPRE];
         tr.P = h_pin[C_P];
-        plan_seen(std::max<int64_t>(tr.n, 1), (int64_t)tr.tiles_x * tr.tiles_y, tr.P);
+        tile_plans().seen(gs::TilePlans::kTrain, std::max<int64_t>(tr.n, 1),
+                          (int64_t)tr.tiles_x * tr.tiles_y, tr.P);
         const gs::TrainSums sum = add_sums(h_pin + kFrSums);
         tr.pixel_pairs = (int64_t)sum.considered;
         tr.pixel_blended = (int64_t)sum.blended;

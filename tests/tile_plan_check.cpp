@@ -46,8 +46,48 @@ static void fields() {
             if (gs::binned_fits(n, t)) full_cover(n, t, n > (1 << 18) ? 2048 : 512);
 }
 
+// Sizes that alternate keep what each of them found, up to as many as are remembered.
+static void sizes() {
+    using P = gs::TilePlans;
+    const int64_t n = 1000000, full = 3600, thumb = 300;
+    {
+        P p;  // few Gaussians start binned, many do not
+        CHECK(p.binned(P::kFrame, P::kFirst, full) && !p.binned(P::kFrame, P::kFirst + 1, full));
+        CHECK(!p.binned(P::kFrame, 1000, gs::kBinnedTiles + 1));
+    }
+    {
+        P p;
+        for (int k = 0; k < 4; ++k) {
+            p.binned(P::kFrame, n, full);
+            p.seen(P::kFrame, n, full, 5000000);
+            p.binned(P::kFrame, n, thumb);
+            p.seen(P::kFrame, n, thumb, 700000);
+            CHECK(!p.binned(P::kFrame, n, full) && p.binned(P::kFrame, n, thumb));
+            CHECK(p.binned(P::kTrain, n, full));  // a training forward's pairs are its own
+        }
+        p.seen(P::kFrame, n, full, P::kAgain);  // between the limits: as it was
+        CHECK(!p.binned(P::kFrame, n, full));
+        p.seen(P::kFrame, n, full, P::kAgain - 1);
+        CHECK(p.binned(P::kFrame, n, full));
+        p.seen(P::kFrame, n, full, P::kMost);
+        CHECK(p.binned(P::kFrame, n, full));
+    }
+    {
+        P p;  // many Gaussians, few pairs: binned from the second frame, also between others
+        for (int k = 0; k < P::kEntries; ++k) {
+            CHECK(!p.binned(P::kFrame, 3000000, 100 + k));
+            p.seen(P::kFrame, 3000000, 100 + k, 500000);
+        }
+        for (int k = 0; k < P::kEntries; ++k) CHECK(p.binned(P::kFrame, 3000000, 100 + k));
+        CHECK(!p.binned(P::kFrame, 3000000, 99));  // one more size: the oldest is given up
+        CHECK(p.binned(P::kFrame, 3000000, 100 + P::kEntries - 1));
+        CHECK(!p.binned(P::kFrame, 3000000, 100));
+    }
+}
+
 int main() {
     fields();
+    sizes();
     if (fails == 0) std::puts("ok");
     return fails ? 1 : 0;
 }

@@ -427,8 +427,10 @@ struct gs_ctx {
 
     void ensure_counters() {
         b_cnt.ensure(64 * 4);
-        if (!h_pin) HIPCHK(hipHostMalloc((void**)&h_pin, (gs::sort_hist_words() + 64) * 4));
+        if (!h_pin) HIPCHK(hipHostMalloc((void**)&h_pin, (gs::sort_hist_words() + 128) * 4));
     }
+    // Where the kernels report the longest tile list of a frame.
+    uint32_t* longest_word() { return h_pin + gs::sort_hist_words() + 64; }
 
     void ensure_sort(int64_t n, int key_bytes) {
         b_kalt.ensure(std::max<int64_t>(n, 1) * key_bytes);
@@ -738,7 +740,9 @@ struct gs_ctx {
             s.num_visible = h_pin[C_M];
             s.pairs_pre = h_pin[C_PPRE];
             s.num_entries = h_pin[C_P];
-            tile_plans().seen(gs::TilePlans::kFrame, sd.n, pend.T, s.num_entries);
+            if (!cull_stats)  // (whose lists are made another way, their longest not known)
+                tile_plans().seen(gs::TilePlans::kFrame, sd.n, pend.T, s.num_entries,
+                                  *longest_word());
             s.chunks_skipped = h_pin[C_SKIPPED];
             if (cull_stats) {
                 uint64_t mb[2];
@@ -1214,7 +1218,8 @@ struct gs_ctx {
                                           b_ranges.as<uint32_t>(), T, st));
             *tiles_out = static_cast<uint32_t*>(tiles_sorted);
         } else {
-            HIPCHK(gs::launch_ranges_from_counts(L.tcnt, T, b_ranges.as<uint32_t>(), st, report));
+            HIPCHK(gs::launch_ranges_from_counts(L.tcnt, T, b_ranges.as<uint32_t>(), st, report,
+                                                 longest_word()));
         }
     }
 
@@ -1255,7 +1260,7 @@ struct gs_ctx {
         HIPCHK(gs::launch_block_lists(static_cast<uint32_t*>(keys), ids, L.pcap,
                                       L.bcnt, b_bins.as<uint32_t>(), cnt + C_SEGS, tp, L.tcnt,
                                       b_ranges.as<uint32_t>(), b_pair_id.as<uint32_t>(), report,
-                                      st));
+                                      longest_word(), st));
     }
 
     // frame_tiles of a binned frame, whose projection scanned the candidates:
@@ -1275,7 +1280,8 @@ struct gs_ctx {
                                        L.pcap, cnt + C_PPRE, b_bins.as<uint32_t>(), L.tcnt, T,
                                        b_dkey.as<uint32_t>(), b_ranges.as<uint32_t>(),
                                        b_valt.as<uint32_t>(), b_kalt.as<uint32_t>(), L.runs,
-                                       cnt + C_RUNS, b_pair_id.as<uint32_t>(), cnt + C_CTL, report, st));
+                                       cnt + C_RUNS, b_pair_id.as<uint32_t>(), cnt + C_CTL, report,
+                                       longest_word(), st));
     }
     gs::BinnedOut binned_out(const FrameLayout& L) const {
         if (!L.binned) return gs::BinnedOut{};
@@ -1879,7 +1885,7 @@ struct gs_ctx {
         tr.p_pre = h_pin[C_PPRE];
         tr.P = h_pin[C_P];
         tile_plans().seen(gs::TilePlans::kTrain, std::max<int64_t>(tr.n, 1),
-                          (int64_t)tr.tiles_x * tr.tiles_y, tr.P);
+                          (int64_t)tr.tiles_x * tr.tiles_y, tr.P, *longest_word());
         const gs::TrainSums sum = add_sums(h_pin + kFrSums);
         tr.pixel_pairs = (int64_t)sum.considered;
         tr.pixel_blended = (int64_t)sum.blended;

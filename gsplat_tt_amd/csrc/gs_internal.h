@@ -288,7 +288,7 @@ hipError_t launch_block_emit(const float4* rc, const uint32_t* order, const uint
 hipError_t launch_block_lists(const uint32_t* keys, const uint32_t* ids, uint32_t cap,
                               const uint32_t* block_items, uint32_t* scratch, uint32_t* n_segs, TileParams tp,
                               uint32_t* tile_count, uint32_t* ranges, uint32_t* sorted_ids,
-                              const HostCopy& report, hipStream_t st);
+                              const HostCopy& report, uint32_t* longest, hipStream_t st);
 // Digit width of a device sort over `bits` key bits: the fewest 8-bit-or-less
 // passes, with the bits spread evenly over them (12 tile bits: two passes of 6,
 // whose 64 digits give longer runs per digit than 256 would).
@@ -328,22 +328,24 @@ uint32_t bin_words(int64_t num_tiles);
 // and bins to the pairs per tile (cleared before), the ranges and the ids of each
 // tile in (depth bits, id) order. bins: binned_scratch_words, the emission's rows
 // first; ids, deps: scratch for p_cap words each; runs: scratch for 2 *
-// emit_partitions(p_cap) words; n_runs: a cleared word; report: the frame's
-// counters, final by then.
+// emit_partitions(p_cap) words; n_runs: a cleared word; report, longest: as
+// launch_ranges_from_counts.
 size_t binned_scratch_words(uint32_t p_cap, int64_t num_tiles);
 hipError_t launch_binned_lists(const uint32_t* slot, const uint32_t* slot_id, uint32_t p_cap,
                                const uint32_t* p_pre_dev, uint32_t* bins, uint32_t* tile_count,
                                int64_t num_tiles, const uint32_t* depth, uint32_t* ranges,
                                uint32_t* ids, uint32_t* deps, uint32_t* runs, uint32_t* n_runs,
                                uint32_t* sorted_ids, const uint32_t* ctl, const HostCopy& report,
-                               hipStream_t st);
+                               uint32_t* longest, hipStream_t st);
 hipError_t launch_tile_ranges(const uint32_t* sorted_tile, uint32_t p, const uint32_t* p_dev,
                               uint32_t* ranges, int64_t num_tiles, hipStream_t st);
 // ranges[t] = [start, end) from per-tile pair counts (an exclusive scan in tile
 // order; (0, 0) for an empty tile), one workgroup.
-// report: the frame's counters, final by then.
+// report: the frame's counters, final by then. longest (pinned host memory, optional):
+// the most pairs of one tile.
 hipError_t launch_ranges_from_counts(const uint32_t* counts, int64_t num_tiles, uint32_t* ranges,
-                                     hipStream_t st, const HostCopy& report = HostCopy{});
+                                     hipStream_t st, const HostCopy& report = HostCopy{},
+                                     uint32_t* longest = nullptr);
 // Same ranges by per-tile binary search over the sorted tile keys (reads
 // O(tiles * log p) keys instead of all p; no clearing pass).
 hipError_t launch_tile_bounds(const uint32_t* sorted_tile, uint32_t p_cap, const uint32_t* p_dev,

@@ -36,10 +36,17 @@ constexpr bool binned_fits(int64_t n, int64_t tiles) {
 // 2.4M pairs (us a frame alone and in a path, blocks against binned; 1280x720: 1.1M
 // pairs 317, 213 / 243, 186; 1.7M 366, 246 / 294, 227; 2.8M 434, 295 / 380, 291;
 // 1237x822: 1.5M 263, 173 / 201, 156; 3.0M 314, 221 / 320, 255; 5.0M 367, 276 / 477,
-// 407; 400x300, 3100 pairs a tile: 1.5M 283, 234 / 294, 186). The pairs of a view are
-// not known before it is rendered: frames start from the number of Gaussians and go
-// on with the pairs of the frames that finished, with a gap between the two limits so
-// that a camera path does not alternate.
+// 407; 400x300, 3100 pairs a tile: 1.5M 283, 234 / 294, 186). A list past two runs of 2048
+// is searched run by run in all its others, while the other ways take as long however
+// the pairs lie: every run past two of the longest list costs a frame 6 us, as 0.3M
+// pairs do (binned against pairs sorted by tile, the longest list in brackets: 320x240
+// 0.44M pairs [9.4K] 168, 100 / 204, 122; 640x480 in tiles of 32 0.99M [7.3K] 189, 127 /
+// 229, 149; 320x240 0.87M [19K] 248, 143 / 250, 146; 640x480 in tiles of 32 1.14M [25K]
+// 325, 195 / 291, 194; 160x120 in tiles of 32 0.48M [64K] 749, 301 / 599, 259; one tile
+// 0.05M 790, 216 / 708, 198 and 1M 4082, 1607 / 635, 224).
+// The lists of a view are not known before it is rendered: the first frame goes by the
+// number of Gaussians, later ones by the lists of the frames that finished, with a gap
+// between the two limits so that a camera path does not alternate.
 // What was found is kept for several sizes (a trainer's photographs, a thumbnail beside
 // the full view), frames and training forwards apart, the least recently used given up.
 // A scene set anew with as many Gaussians goes on from what the last one found: a wrong
@@ -51,22 +58,34 @@ public:
     bool binned(Kind kind, int64_t n, int64_t tiles) {
         return entry(kind, n, tiles).binned && binned_fits(n, tiles);
     }
-    // A frame of these sizes has finished with `pairs` pairs.
-    void seen(Kind kind, int64_t n, int64_t tiles, int64_t pairs) {
+    // A frame of these sizes has finished with `pairs` pairs, `longest` in one tile.
+    void seen(Kind kind, int64_t n, int64_t tiles, int64_t pairs, int64_t longest) {
         Entry& e = entry(kind, n, tiles);
-        if (pairs > kMost) e.binned = false;
-        if (pairs < kAgain) e.binned = true;
+        const int64_t c = cost(pairs, longest);
+        if (c > kMost) e.binned = false;
+        if (c < kAgain || (!e.known && c <= kMost)) e.binned = true;
+        e.known = true;
     }
 
     static constexpr int kEntries = 16;
+    // (2 pairs a Gaussian reach kMost: 0.6 to 5 in the views measured)
     static constexpr int64_t kFirst = 1 << 20, kMost = 2400000, kAgain = 1800000;
 
 private:
+    // In pairs: those there are, and what merging the longest list takes.
+    static constexpr int64_t cost(int64_t pairs, int64_t longest) {
+        return pairs + 150 * (longest > 4096 ? longest - 4096 : 0);
+    }
+    // A size not seen before: two pairs a Gaussian, four times the mean in one tile.
+    static constexpr bool first(int64_t n, int64_t tiles) {
+        return n <= kFirst && cost(2 * n, 4 * n / (tiles > 0 ? tiles : 1)) <= kMost;
+    }
     struct Entry {
         Kind kind = kFrame;
         int64_t n = -1, tiles = -1;
         uint64_t used = 0;
         bool binned = false;
+        bool known = false;  // a frame has finished
     };
     Entry& entry(Kind kind, int64_t n, int64_t tiles) {
         Entry* at = &e_[0];
@@ -77,7 +96,7 @@ private:
             }
             if (e.used < at->used) at = &e;
         }
-        *at = Entry{kind, n, tiles, ++clock_, n <= kFirst};
+        *at = Entry{kind, n, tiles, ++clock_, first(n, tiles), false};
         return *at;
     }
     Entry e_[kEntries];

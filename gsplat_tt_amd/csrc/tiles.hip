@@ -1143,20 +1143,42 @@ __global__ __launch_bounds__(kOffsThreads) void k_part_offsets(
 // Tile ranges from per-tile pair counts in one workgroup: each thread sums a
 // block of consecutive tiles, the block sums are scanned, and each thread
 // writes its tiles' [start, end) (sort.cpp:146-165: (0, 0) for an empty tile).
+// longest (pinned host memory, may be null): the most pairs of one tile.
 constexpr int kRangeThreads = 1024;
+__device__ __forceinline__ uint32_t wave_max(uint32_t v) {
+#pragma unroll
+    for (int o = GS_WAVE / 2; o > 0; o >>= 1) v = max(v, (uint32_t)__shfl_xor((int)v, o, GS_WAVE));
+    return v;
+}
+__device__ __forceinline__ void report_longest(uint32_t* longest, const uint32_t* waves) {
+    if (longest == nullptr || threadIdx.x >= GS_WAVE) return;
+    constexpr int n = kRangeThreads / GS_WAVE;
+    const uint32_t m = wave_max(threadIdx.x < n ? waves[threadIdx.x] : 0u);
+    if (threadIdx.x == 0)
+        __hip_atomic_store(longest, m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 __global__ __launch_bounds__(kRangeThreads) void k_ranges_from_counts(
     const uint32_t* __restrict__ counts, uint32_t ntiles, uint32_t* __restrict__ ranges,
-    HostCopy report) {
-    __shared__ uint32_t s_w[kRangeThreads / GS_WAVE];
+    HostCopy report, uint32_t* longest) {
+    __shared__ uint32_t s_w[kRangeThreads / GS_WAVE], s_m[kRangeThreads / GS_WAVE];
     host_copy(report, threadIdx.x, kRangeThreads);
     const int tid = threadIdx.x, w = tid / GS_WAVE, lane = lane_id();
     const uint32_t per = (ntiles + kRangeThreads - 1) / kRangeThreads;
     const uint32_t t0 = min(ntiles, (uint32_t)tid * per), t1 = min(ntiles, t0 + per);
-    uint32_t sum = 0;
-    for (uint32_t t = t0; t < t1; ++t) sum += counts[t];
+    uint32_t sum = 0, most = 0;
+    for (uint32_t t = t0; t < t1; ++t) {
+        const uint32_t c = counts[t];
+        sum += c;
+        most = max(most, c);
+    }
     const uint32_t inc = wave_incl_scan(sum);
-    if (lane == GS_WAVE - 1) s_w[w] = inc;
+    most = wave_max(most);
+    if (lane == GS_WAVE - 1) {
+        s_w[w] = inc;
+        s_m[w] = most;
+    }
     __syncthreads();
+    report_longest(longest, s_m);
     uint32_t pre = 0;
     for (int i = 0; i < w; ++i) pre += s_w[i];
     uint32_t start = pre + inc - sum;
@@ -1183,17 +1205,26 @@ constexpr int kRunItems = 8;  // keys per thread
 constexpr uint32_t kRun = kRunThreads * kRunItems;
 __global__ __launch_bounds__(kRangeThreads) void k_binned_ranges(
     const uint32_t* __restrict__ counts, uint32_t ntiles, uint32_t* __restrict__ ranges,
-    uint32_t* __restrict__ runs, uint32_t* n_runs, HostCopy report) {
-    __shared__ uint32_t s_w[kRangeThreads / GS_WAVE];
+    uint32_t* __restrict__ runs, uint32_t* n_runs, HostCopy report, uint32_t* longest) {
+    __shared__ uint32_t s_w[kRangeThreads / GS_WAVE], s_m[kRangeThreads / GS_WAVE];
     host_copy(report, threadIdx.x, kRangeThreads);
     const int tid = threadIdx.x, w = tid / GS_WAVE, lane = lane_id();
     const uint32_t per = (ntiles + kRangeThreads - 1) / kRangeThreads;
     const uint32_t t0 = min(ntiles, (uint32_t)tid * per), t1 = min(ntiles, t0 + per);
-    uint32_t sum = 0;
-    for (uint32_t t = t0; t < t1; ++t) sum += counts[t];
+    uint32_t sum = 0, most = 0;
+    for (uint32_t t = t0; t < t1; ++t) {
+        const uint32_t c = counts[t];
+        sum += c;
+        most = max(most, c);
+    }
     const uint32_t inc = wave_incl_scan(sum);
-    if (lane == GS_WAVE - 1) s_w[w] = inc;
+    most = wave_max(most);
+    if (lane == GS_WAVE - 1) {
+        s_w[w] = inc;
+        s_m[w] = most;
+    }
     __syncthreads();
+    report_longest(longest, s_m);
     uint32_t pre = 0;
     for (int i = 0; i < w; ++i) pre += s_w[i];
     uint32_t start = pre + inc - sum;
@@ -1542,7 +1573,7 @@ hipError_t launch_block_emit(const float4* rc, const uint32_t* order, const uint
 hipError_t launch_block_lists(const uint32_t* keys, const uint32_t* ids, uint32_t cap,
                               const uint32_t* block_items, uint32_t* scratch, uint32_t* n_segs, TileParams tp,
                               uint32_t* tile_count, uint32_t* ranges, uint32_t* sorted_ids,
-                              const HostCopy& report, hipStream_t st) {
+                              const HostCopy& report, uint32_t* longest, hipStream_t st) {
     const uint32_t nb = num_blocks(tp.tiles_x, tp.tiles_y);
     if (nb == 0 || cap == 0) return hipSuccess;
     if (nb > kMostBlocks) return hipErrorInvalidValue;
@@ -1555,7 +1586,7 @@ hipError_t launch_block_lists(const uint32_t* keys, const uint32_t* ids, uint32_
     k_block_count<<<grid, kSegThreads, 0, st>>>(keys, seg, n_segs, cnt, tp.ctl);
     k_block_tiles<<<nb, 256, 0, st>>>(first, tp.tiles_x, tp.tiles_y, cnt, tile_count, tp.ctl);
     k_ranges_from_counts<<<1, kRangeThreads, 0, st>>>(
-        tile_count, (uint32_t)(tp.tiles_x * tp.tiles_y), ranges, report);
+        tile_count, (uint32_t)(tp.tiles_x * tp.tiles_y), ranges, report, longest);
     k_block_write<<<grid, kSegThreads, 0, st>>>(keys, ids, seg, n_segs, cnt, ranges, tp.tiles_x,
                                                 tp.tiles_y, sorted_ids, tp.ctl);
     return hipGetLastError();
@@ -1612,7 +1643,7 @@ hipError_t launch_binned_lists(const uint32_t* slot, const uint32_t* slot_id, ui
                                int64_t num_tiles, const uint32_t* depth, uint32_t* ranges,
                                uint32_t* ids, uint32_t* deps, uint32_t* runs, uint32_t* n_runs,
                                uint32_t* sorted_ids, const uint32_t* ctl, const HostCopy& report,
-                               hipStream_t st) {
+                               uint32_t* longest, hipStream_t st) {
     if (num_tiles <= 0 || p_cap == 0) return hipSuccess;
     if (num_tiles > kBinnedTiles) return hipErrorInvalidValue;
     const uint32_t T = (uint32_t)num_tiles, words = bin_words(T);
@@ -1620,7 +1651,7 @@ hipError_t launch_binned_lists(const uint32_t* slot, const uint32_t* slot_id, ui
     uint32_t* seg_base = bins + (size_t)parts * words;
     const dim3 og((words + 255) / 256, (parts + kBinSegment - 1) / kBinSegment);
     k_binned_offsets<<<og, 256, 0, st>>>(bins, words, p_cap, p_pre_dev, tile_count, seg_base, ctl);
-    k_binned_ranges<<<1, kRangeThreads, 0, st>>>(tile_count, T, ranges, runs, n_runs, report);
+    k_binned_ranges<<<1, kRangeThreads, 0, st>>>(tile_count, T, ranges, runs, n_runs, report, longest);
     // persistent grids: the real counts are on the device
     const unsigned sg = std::max(1u, std::min(1024u, (p_cap + 255) / 256));
     k_binned_scatter<<<sg, 256, 0, st>>>(slot, slot_id, p_cap, p_pre_dev, bins, words, seg_base,
@@ -1642,10 +1673,11 @@ hipError_t launch_tile_ranges(const uint32_t* sorted_tile, uint32_t p, const uin
 }
 
 hipError_t launch_ranges_from_counts(const uint32_t* counts, int64_t num_tiles, uint32_t* ranges,
-                                     hipStream_t st, const HostCopy& report) {
+                                     hipStream_t st, const HostCopy& report, uint32_t* longest) {
     if (num_tiles <= 0) return hipSuccess;
     if (num_tiles > ((int64_t)1 << 24)) return hipErrorInvalidValue;
-    k_ranges_from_counts<<<1, kRangeThreads, 0, st>>>(counts, (uint32_t)num_tiles, ranges, report);
+    k_ranges_from_counts<<<1, kRangeThreads, 0, st>>>(counts, (uint32_t)num_tiles, ranges, report,
+                                                      longest);
     return hipGetLastError();
 }
 

@@ -252,3 +252,27 @@ def test_blend_of_frames_in_flight(h, w, ts):
                 assert all(np.array_equal(a, b) for a, b in zip(ref, outs))
         finally:
             ctx.close()
+
+
+@pytest.mark.parametrize("n", [12_000, 30_000, 120_000])
+@pytest.mark.parametrize("h,w,ts", [(16, 16, 16), (33, 17, 16), (40, 60, 32)])
+def test_long_lists(n, h, w, ts):
+    """Lists of many runs, in one tile or a few: the frames on the way from the first
+    guess to the way that the longest list asks for equal the sorted ones, also after a
+    view of the same size with short lists."""
+    print("long lists", n, h, w, ts, flush=True)
+    ctx = L.Context(0)
+    try:
+        ctx.set_scene(*_stack(n, 500, spread=0.02, seed=n))
+        K = scenes.intrinsics(60, 60, w / 2, h / 2)
+        near = L.make_view(np.eye(4, dtype=np.float32), K, h, w, tile_size=ts, output="f32")
+        aside = np.eye(4, dtype=np.float32)
+        aside[0, 3] = -50.0  # nothing in view
+        away = L.make_view(aside, K, h, w, tile_size=ts, output="f32")
+        for view in (near, near, away, away, near, near):
+            a, st = ctx.render(view)
+            rb = ctx.frame_readback() if st["num_visible"] else None
+            _equal((a, st, rb), _both(ctx, view)[1])
+        assert (rb["tile_ranges"][:, 1] - rb["tile_ranges"][:, 0]).max() > 2 * 2048
+    finally:
+        ctx.close()

@@ -1499,20 +1499,28 @@ struct gs_ctx {
         return true;
     }
 
-    // A wave per microblock blends every frame that runs alone faster. Among frames in
-    // flight it wins where a frame's bands are too few to fill the chip four at a time;
-    // larger frames take the wave per band, which needs 15 % fewer instructions and half
-    // of the record reads where most entries are kept by both of its microblocks (us a
-    // frame in a path, band against microblock. Binned: 640x480 0.62M pairs in tiles of
-    // 32 (4800 bands) 211 / 182, 1280x720 (14720) 186 / 172, 1237x822 (16224) 271 / 268,
-    // 1280x960 (19200) 168 / 171, 1920x1080 0.09M (33120) 74 / 84, 1.8M 199 / 220,
-    // 2560x1440 0.9M 202 / 230. Others: 640x480 3.5M 240 / 237, 2.9M in tiles of 32
-    // 372 / 318, 1280x720 6.6M 454 / 451, 1237x822 10M 372 / 381, 30M 1022 / 1046,
-    // 1280x960 5.3M 243 / 251).
-    static constexpr int64_t kMicroblockBands = 15360, kMicroblockBandsBinned = 16384;
+    // A wave per microblock has twice the waves of a wave per band and shorter chains: it
+    // wins where a frame's bands are too few to fill the chip - alone, or four frames at
+    // a time in a path. The wave per band needs 15 % fewer instructions and half of the
+    // record reads where most entries are kept by both of its microblocks, and wins for
+    // larger images (us a frame, band against microblock.
+    // Alone: 640x480 3.5M pairs (4800 bands) 304 / 291, 1280x720 2.2M (14400) 352 / 325,
+    // 1237x822 10M (16224) 514 / 482, 1280x960 (19200) 1.1M 278 / 255, 1.6M 199 / 212,
+    // 5.3M 338 / 346; 1920x1080 (32640) 1.2M 306 / 298, 1.8M 262 / 276, 3.6M 336 / 360,
+    // 6.3M in tiles of 32 613 / 667; 2560x1440 (57600) 0.9M 261 / 293, 1.9M in tiles of 32
+    // 379 / 444, 4.7M 585 / 666.
+    // In a path, binned: 640x480 0.62M in tiles of 32 230 / 181, 1280x720 2.2M 249 / 248,
+    // in tiles of 32 0.6M 189 / 176, 1237x822 2.0M 268 / 270, 1280x960 1.0M 162 / 172,
+    // 1920x1080 1.8M 200 / 222, 2560x1440 0.9M 204 / 235; others: 640x480 3.5M 224 / 220, in
+    // tiles of 32 2.9M 388 / 330, 800x600 4.4M (7600) 244 / 238, 960x640 7M (9600) 328 /
+    // 340, 1237x822 30M 1022 / 1046, 1280x960 5.3M 246 / 256).
+    static constexpr int64_t kMicroblockBands = 8192, kMicroblockBandsBinned = 16384,
+                             kMicroblockBandsAlone = 24576;
     bool blend_by_microblock(const FrameLayout& L, int64_t T, int tile_size) const {
         const int64_t bands = T * (tile_size * tile_size / 64);
-        return !batch_frame || bands <= (L.binned ? kMicroblockBandsBinned : kMicroblockBands);
+        return bands <= (!batch_frame ? kMicroblockBandsAlone
+                         : L.binned   ? kMicroblockBandsBinned
+                                      : kMicroblockBands);
     }
 
     // Enqueues one frame (project -> depth sort -> tile assign -> tile sort ->

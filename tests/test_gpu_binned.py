@@ -227,13 +227,15 @@ def test_blend_by_microblock_equals_by_band(gpu_ctx, h, w, ts, n, op):
     assert np.array_equal(img.view(np.uint32), ref.view(np.uint32))
 
 
-@pytest.mark.parametrize("h,w,ts", [(48, 64, 16), (64 * 16, 64 * 16 - 3, 16), (65 * 16 - 5, 64 * 16, 16),
-                                    (480, 640, 32), (31 * 32, 32 * 32, 32), (33 * 32, 32 * 32, 32)])
+@pytest.mark.parametrize("h,w,ts", [(48, 64, 16), (32 * 16, 64 * 16, 16), (33 * 16, 64 * 16, 16),
+                                    (64 * 16, 64 * 16 - 3, 16), (65 * 16 - 5, 64 * 16, 16),
+                                    (480, 640, 32), (32 * 32, 32 * 32, 32), (33 * 32, 32 * 32, 32),
+                                    (96 * 16, 64 * 16, 16), (97 * 16, 64 * 16, 16)])
 def test_blend_of_frames_in_flight(h, w, ts):
-    """Frames in flight blend with a wave per microblock up to 15360 or 16384 bands of
-    16 x 4 pixels and with one per band above: the images of a path are those of single
-    frames on both sides of the line, binned and not (more than 2^20 Gaussians), through
-    captures and replays."""
+    """A wave per microblock blends up to 8192 bands of 16 x 4 pixels (frames in flight,
+    16384 binned ones) or 24576 (alone), a wave per band above: the images of a path are
+    those of single frames on both sides of each line, binned and not (more than 2^20
+    Gaussians), through captures and replays."""
     print("blend in flight", h, w, ts, flush=True)
     for n in (3000, (1 << 20) + 5):
         ctx = L.Context(0)

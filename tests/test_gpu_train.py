@@ -214,6 +214,29 @@ def test_train_loss_ssim_tiles(gpu_ctx, h, w):
     assert rel_err(grad, go) < 1e-3
 
 
+@pytest.mark.parametrize("term", ["A", "B"])
+def test_train_loss_ssim_zero_terms(gpu_ctx, term):
+    """SSIM = A B / (C D) where A or B passes through 0: pairs of lone pixels, 12 apart, the
+    target's stepping through the 400 floats around the one that makes the term 0 (an ulp
+    of the term a step, so some step has it exactly 0 in fp32). Loss and gradient are
+    finite and the oracle's, whose 64-bit quotients by terms of 1e-12 and more hold to
+    1e-8. Bound as in the tiles' test."""
+    print("ssim zero terms", term, flush=True)
+    g = np.exp(-np.arange(-5, 6) ** 2 / 4.5)
+    g2 = (g[5] / g.sum()) ** 2  # the window's middle
+    # A = 2 g2^2 a b + c1, B = 2 g2 a b (1 - g2) + c2, with a = 1
+    root = -TO.SSIM_C1 / (2 * g2 * g2) if term == "A" else -TO.SSIM_C2 / (2 * g2 * (1 - g2))
+    first = np.float32(root).view(np.uint32) - np.uint32(200)
+    steps = (first + np.arange(400, dtype=np.uint32)).view(np.float32).reshape(20, 20)
+    img, tgt = np.zeros((240, 240, 3), np.float32), np.zeros((240, 240, 3), np.float32)
+    img[6::12, 6::12], tgt[6::12, 6::12] = 1.0, steps[..., None]
+    loss, l1, ssim, grad = gpu_ctx.train_loss(img, tgt, 0.2)
+    lo, l1o, so, go = TO.ssim_loss_grad(img, tgt, 0.2)
+    assert np.isfinite(go).all() and np.isfinite(grad).all()
+    assert abs(loss - lo) <= 1e-6 * lo and abs(ssim - so) <= 1e-6
+    assert rel_err(grad, go) < 1e-3
+
+
 def test_train_step_ssim_loss_matches_oracle(gpu_ctx):
     """One whole step with the full 3DGS loss (lambda 0.2) of a C5-shaped scene
     against the oracle's forward, SSIM loss gradient, backward and Adam."""

@@ -638,3 +638,47 @@ def test_train_nonfinite_colour_stays_where_it_blends(gpu_ctx, bad):
             assert np.linalg.norm(a - b) <= 1e-4 * np.linalg.norm(b), (name, k)
             if name == "hidden":
                 assert not got[k][-1].any(), k
+
+
+@pytest.mark.parametrize("bad", [np.inf, -np.inf, np.nan])
+def test_train_nonfinite_pixel_gradient_stays_where_it_blends(gpu_ctx, bad):
+    """A non-finite gradient of one pixel reaches the Gaussians that this pixel blends and
+    no other: not those that only other pixels of the band blend, nor what is summed
+    beside them (the entries go in twos, an odd last one with padding that carries the
+    id 0). The others' gradients are those with that pixel's gradient at 0, but for the
+    order of the atomic adds (20 x 2^-24 of the terms, a tenth of which is left: 1e-4)."""
+    print("train nonfinite pixel", bad, flush=True)
+    h, w, f = 33, 48, 40.0
+    view = L.make_view(np.eye(4, dtype=np.float32), scenes.intrinsics(f, f, w / 2, h / 2), h, w,
+                       tile_size=16)
+    cfg = L.make_train_cfg(background=(0.2, 0.4, 0.6))
+    rng = np.random.default_rng(11)
+    dimage = rng.standard_normal((h, w, 3)).astype(np.float32)
+    for count in (2, 3, 4, 5):  # entries of the pixel's band, even and odd
+        # the first far from the band, then a column of one pixel's width in it
+        at = [(40.5, 28.5)] + [(4.5 + 2.5 * k, 9.5) for k in range(count)]
+        z = 3.0 + 0.25 * np.arange(len(at))
+        p = {"means": np.stack([(np.array([a[0] for a in at]) - w / 2) / f * z,
+                                (np.array([a[1] for a in at]) - h / 2) / f * z, z], 1),
+             "log_scales": np.log(0.3 * z / f)[:, None].repeat(3, 1) +
+             rng.normal(0, 0.05, (len(at), 3)),
+             "quats": rng.standard_normal((len(at), 4)), "opacity_logits": np.full(len(at), 1.0),
+             "sh": rng.uniform(0.2, 1.0, (len(at), 1, 3))}
+        p = {k: np.ascontiguousarray(v, np.float32) for k, v in p.items()}
+        tr = L.Trainer(gpu_ctx, p, 0)
+
+        def gradients(value):
+            tr.forward(view, cfg)
+            d = dimage.copy()
+            d[9, 4] = value
+            tr.backward(cfg, dimage=d)
+            return tr.read(3)
+
+        ref, got = gradients(0.0), gradients(bad)
+        assert not np.isfinite(got["sh"][1]).any()  # the pixel blends it
+        others = [0] + list(range(3, len(at)))  # 5 pixels and more from it
+        for k in TO.PARAM_NAMES:
+            a, b = got[k][others], ref[k][others]
+            assert np.isfinite(a).all(), (count, k)
+            assert np.abs(b[0]).max() > 0 or k == "quats", (count, k)
+            assert np.linalg.norm(a - b) <= 1e-4 * np.linalg.norm(b), (count, k)

@@ -429,7 +429,8 @@ struct gs_ctx {
         b_cnt.ensure(64 * 4);
         if (!h_pin) HIPCHK(hipHostMalloc((void**)&h_pin, (gs::sort_hist_words() + 128) * 4));
     }
-    // Where the kernels report the longest tile list of a frame.
+    // Where the kernels report the longest tile list of a frame: cleared before each, as
+    // binned ones report only lists of several runs.
     uint32_t* longest_word() { return h_pin + gs::sort_hist_words() + 64; }
 
     void ensure_sort(int64_t n, int key_bytes) {
@@ -667,6 +668,7 @@ struct gs_ctx {
 
     void enqueue_attempt() {
         pend.replayed = false;
+        *longest_word() = 0;
         if (!graph_frame()) frame(&pend.v, pend.dout, pend.T, pend.tiles_x, pend.tiles_y);
         if (!pend.out_dev)
             HIPCHK(hipMemcpyAsync(pend.out, pend.dout, pend.bytes, hipMemcpyDeviceToHost, st));
@@ -1799,6 +1801,7 @@ struct gs_ctx {
             for (auto& e : tev)
                 if (!e) HIPCHK(hipEventCreate(&e));
         if (timing) HIPCHK(hipEventRecord(tev[0], st));
+        *longest_word() = 0;
         HIPCHK(gs::launch_fill_u32(L.fr, 0u, L.fwords, st));
         if (spin_limit) HIPCHK(gs::launch_fill_u32(L.cnt + C_CTL + 1, spin_limit, 1, st));
         tr.cam.ctl = L.cnt + C_CTL;

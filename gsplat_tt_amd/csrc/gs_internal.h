@@ -328,8 +328,9 @@ uint32_t bin_words(int64_t num_tiles);
 // and bins to the pairs per tile (cleared before), the ranges and the ids of each
 // tile in (depth bits, id) order. bins: binned_scratch_words, the emission's rows
 // first; ids, deps: scratch for p_cap words each; runs: scratch for 2 *
-// emit_partitions(p_cap) words; n_runs: a cleared word; report, longest: as
-// launch_ranges_from_counts.
+// emit_partitions(p_cap) words; n_runs: a cleared word; report: as
+// launch_ranges_from_counts; longest (pinned host memory, optional): the pairs of the
+// longest list of more than one run, left alone when there is none.
 size_t binned_scratch_words(uint32_t p_cap, int64_t num_tiles);
 hipError_t launch_binned_lists(const uint32_t* slot, const uint32_t* slot_id, uint32_t p_cap,
                                const uint32_t* p_pre_dev, uint32_t* bins, uint32_t* tile_count,

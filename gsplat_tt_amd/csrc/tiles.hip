@@ -1150,10 +1150,10 @@ __device__ __forceinline__ uint32_t wave_max(uint32_t v) {
     for (int o = GS_WAVE / 2; o > 0; o >>= 1) v = max(v, (uint32_t)__shfl_xor((int)v, o, GS_WAVE));
     return v;
 }
-__device__ __forceinline__ void report_longest(uint32_t* longest, const uint32_t* waves) {
+__device__ __forceinline__ void report_longest(uint32_t* longest, const uint32_t* waves,
+                                               int n) {
     if (longest == nullptr || threadIdx.x >= GS_WAVE) return;
-    constexpr int n = kRangeThreads / GS_WAVE;
-    const uint32_t m = wave_max(threadIdx.x < n ? waves[threadIdx.x] : 0u);
+    const uint32_t m = wave_max((int)threadIdx.x < n ? waves[threadIdx.x] : 0u);
     if (threadIdx.x == 0)
         __hip_atomic_store(longest, m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
@@ -1178,7 +1178,7 @@ __global__ __launch_bounds__(kRangeThreads) void k_ranges_from_counts(
         s_m[w] = most;
     }
     __syncthreads();
-    report_longest(longest, s_m);
+    report_longest(longest, s_m, kRangeThreads / GS_WAVE);
     uint32_t pre = 0;
     for (int i = 0; i < w; ++i) pre += s_w[i];
     uint32_t start = pre + inc - sum;
@@ -1205,26 +1205,17 @@ constexpr int kRunItems = 8;  // keys per thread
 constexpr uint32_t kRun = kRunThreads * kRunItems;
 __global__ __launch_bounds__(kRangeThreads) void k_binned_ranges(
     const uint32_t* __restrict__ counts, uint32_t ntiles, uint32_t* __restrict__ ranges,
-    uint32_t* __restrict__ runs, uint32_t* n_runs, HostCopy report, uint32_t* longest) {
-    __shared__ uint32_t s_w[kRangeThreads / GS_WAVE], s_m[kRangeThreads / GS_WAVE];
+    uint32_t* __restrict__ runs, uint32_t* n_runs, HostCopy report) {
+    __shared__ uint32_t s_w[kRangeThreads / GS_WAVE];
     host_copy(report, threadIdx.x, kRangeThreads);
     const int tid = threadIdx.x, w = tid / GS_WAVE, lane = lane_id();
     const uint32_t per = (ntiles + kRangeThreads - 1) / kRangeThreads;
     const uint32_t t0 = min(ntiles, (uint32_t)tid * per), t1 = min(ntiles, t0 + per);
-    uint32_t sum = 0, most = 0;
-    for (uint32_t t = t0; t < t1; ++t) {
-        const uint32_t c = counts[t];
-        sum += c;
-        most = max(most, c);
-    }
+    uint32_t sum = 0;
+    for (uint32_t t = t0; t < t1; ++t) sum += counts[t];
     const uint32_t inc = wave_incl_scan(sum);
-    most = wave_max(most);
-    if (lane == GS_WAVE - 1) {
-        s_w[w] = inc;
-        s_m[w] = most;
-    }
+    if (lane == GS_WAVE - 1) s_w[w] = inc;
     __syncthreads();
-    report_longest(longest, s_m);
     uint32_t pre = 0;
     for (int i = 0; i < w; ++i) pre += s_w[i];
     uint32_t start = pre + inc - sum;
@@ -1415,14 +1406,30 @@ __global__ __launch_bounds__(kRunThreads) void k_binned_sort(
 // takes a run, keeps its keys in registers and searches the list's other runs
 // one after the other in LDS (a search in memory, one key after the other, took
 // 178 us for the lists of 13K pairs of a 300x200 view); keys are distinct.
+// The first workgroup also reports the longest of these lists (in pinned host memory;
+// nothing when there is none): in k_binned_ranges, which finds all the lengths, that
+// cost every frame 0.6 us.
 __global__ __launch_bounds__(kRunThreads) void k_binned_merge(
     const uint32_t* __restrict__ ranges, const uint32_t* __restrict__ ids,
     const uint32_t* __restrict__ deps, const uint32_t* __restrict__ runs,
-    const uint32_t* __restrict__ n_runs, uint32_t* __restrict__ sorted, const uint32_t* ctl) {
+    const uint32_t* __restrict__ n_runs, uint32_t* __restrict__ sorted, const uint32_t* ctl,
+    uint32_t* longest) {
     __shared__ uint64_t s_key[kRun];
+    __shared__ uint32_t s_m[kRunThreads / GS_WAVE];
     if (upstream_failed(ctl)) return;
     const int tid = threadIdx.x;
     const uint32_t total = *n_runs;
+    if (longest != nullptr && blockIdx.x == 0 && total > 0) {
+        uint32_t most = 0;
+        for (uint32_t e = tid; e < total; e += kRunThreads) {
+            const size_t tile = runs[e] >> 16;
+            most = max(most, ranges[2 * tile + 1] - ranges[2 * tile]);
+        }
+        most = wave_max(most);
+        if (lane_id() == 0) s_m[tid / GS_WAVE] = most;
+        __syncthreads();
+        report_longest(longest, s_m, kRunThreads / GS_WAVE);
+    }
     for (uint32_t e = blockIdx.x; e < total; e += gridDim.x) {
         const uint32_t tile = runs[e] >> 16, mine = runs[e] & 0xFFFFu;
         const uint32_t start = ranges[2 * (size_t)tile], end = ranges[2 * (size_t)tile + 1];
@@ -1651,7 +1658,7 @@ hipError_t launch_binned_lists(const uint32_t* slot, const uint32_t* slot_id, ui
     uint32_t* seg_base = bins + (size_t)parts * words;
     const dim3 og((words + 255) / 256, (parts + kBinSegment - 1) / kBinSegment);
     k_binned_offsets<<<og, 256, 0, st>>>(bins, words, p_cap, p_pre_dev, tile_count, seg_base, ctl);
-    k_binned_ranges<<<1, kRangeThreads, 0, st>>>(tile_count, T, ranges, runs, n_runs, report, longest);
+    k_binned_ranges<<<1, kRangeThreads, 0, st>>>(tile_count, T, ranges, runs, n_runs, report);
     // persistent grids: the real counts are on the device
     const unsigned sg = std::max(1u, std::min(1024u, (p_cap + 255) / 256));
     k_binned_scatter<<<sg, 256, 0, st>>>(slot, slot_id, p_cap, p_pre_dev, bins, words, seg_base,
@@ -1659,7 +1666,8 @@ hipError_t launch_binned_lists(const uint32_t* slot, const uint32_t* slot_id, ui
     const unsigned long_runs = std::max(1u, std::min(512u, 2 * (p_cap / kRun)));
     k_binned_sort<<<T + long_runs, kRunThreads, 0, st>>>(ranges, T, depth, ids, deps, runs,
                                                          n_runs, sorted_ids, ctl);
-    k_binned_merge<<<long_runs, kRunThreads, 0, st>>>(ranges, ids, deps, runs, n_runs, sorted_ids, ctl);
+    k_binned_merge<<<long_runs, kRunThreads, 0, st>>>(ranges, ids, deps, runs, n_runs, sorted_ids,
+                                                      ctl, longest);
     return hipGetLastError();
 }
 

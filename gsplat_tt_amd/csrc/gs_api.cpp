@@ -573,6 +573,7 @@ struct gs_ctx {
         C_MBSTAT = 40  // two u64: pairs no microblock keeps, kept (pair, microblock)
     };
     uint64_t pair_cap = 0;  // candidate-pair capacity of the frame buffers
+    uint32_t frame_cap = 0; // of the last frame: less when it was binned (kBinnedCands)
     DevBuf b_frame, b_phist_proj, b_phist_emit;
     DevBuf b_bins;             // binned frames: pairs per (emit partition, tile)
     DevBuf b_pchunk, b_poffs;  // tile sort's first pass: emit row chunk sums, offsets
@@ -700,10 +701,15 @@ struct gs_ctx {
             if (pend.empty) break;
             // candidates of the last attempt (0xFFFFFFFF: more than 2^32-2)
             const uint32_t p_pre = h_pin[C_PPRE];
-            if (p_pre != 0xFFFFFFFFu && p_pre <= pair_cap) break;
-            if (pend.attempt > 2 * kFloorRetries + 2)
+            if (p_pre != 0xFFFFFFFFu && p_pre <= frame_cap) break;
+            if (pend.attempt > 2 * kFloorRetries + 3)
                 throw GsError(GS_E_INVALID, "render: pair capacity did not converge");
             ++pend.attempt;
+            if (p_pre > gs::kBinnedCands) tile_plans().past(gs::TilePlans::kFrame, sd.n, pend.T);
+            if (p_pre != 0xFFFFFFFFu && p_pre <= pair_cap) {  // a binned frame's room is less
+                enqueue_attempt();
+                continue;
+            }
             if (p_pre != 0xFFFFFFFFu && p_pre <= pair_limit) {
                 // the same frame again with room for its pairs
                 pair_cap = std::min<uint64_t>(pair_limit, (uint64_t)p_pre + p_pre / 8 + 4096);
@@ -743,8 +749,8 @@ struct gs_ctx {
             s.pairs_pre = h_pin[C_PPRE];
             s.num_entries = h_pin[C_P];
             if (!cull_stats)  // (whose lists are made another way, their longest not known)
-                tile_plans().seen(gs::TilePlans::kFrame, sd.n, pend.T, s.num_entries,
-                                  *longest_word());
+                tile_plans().seen(gs::TilePlans::kFrame, sd.n, pend.T, s.pairs_pre,
+                                  s.num_entries, *longest_word());
             s.chunks_skipped = h_pin[C_SKIPPED];
             if (cull_stats) {
                 uint64_t mb[2];
@@ -1076,9 +1082,10 @@ struct gs_ctx {
                               bool want_keys) {
         FrameLayout L{};
         const int64_t T = (int64_t)tiles_x * tiles_y;
-        L.pcap = (uint32_t)pair_cap;
         // the microblock statistics need the sorted tile keys
         L.binned = !want_keys && tile_plans().binned(kind, N, T);
+        L.pcap = (uint32_t)(L.binned ? std::min<uint64_t>(pair_cap, gs::kBinnedCands) : pair_cap);
+        frame_cap = L.pcap;
         const int64_t nb = ((int64_t)tiles_x + 3) / 4 * (((int64_t)tiles_y + 3) / 4);
         L.blocks = !L.binned && !want_keys && T <= kBlockTilesMost;
         L.key_bits = tile_bits(L.blocks ? nb : T);
@@ -1117,7 +1124,12 @@ struct gs_ctx {
                                  2 * (L.rparts + std::max({L.rparts, L.pparts, L.eparts}));
         b_frame.ensure(all_words * 4);
         L.fwords = L.binned ? binned_words : all_words;
-        ensure_sort(std::max<int64_t>(N, L.pcap), 4);
+        if (L.binned) {  // scratch for its lists; it has no use for the sort's other state
+            b_kalt.ensure((size_t)L.pcap * 4);
+            b_valt.ensure((size_t)L.pcap * 4);
+        } else {
+            ensure_sort(std::max<int64_t>(N, L.pcap), 4);
+        }
         if (blend_counts) b_evals.ensure(64 * 8 * 8);
         L.fr = b_frame.as<uint32_t>();
         L.cnt = L.fr + kFrCnt;
@@ -1884,19 +1896,24 @@ struct gs_ctx {
             const uint32_t p_pre = h_pin[C_PPRE];
             if (p_pre == 0xFFFFFFFFu)
                 throw GsError(GS_E_CAPACITY, "train: more than 2^32-1 candidate pairs");
-            if (p_pre <= pair_cap) {
+            if (p_pre <= frame_cap) {
                 ctl_check(h_pin[C_CTL], "train forward");
                 break;
             }
             REQUIRE(attempt == 0, "train: pair capacity did not converge");
-            pair_cap = std::min<uint64_t>(0xFFFFFFFFull, (uint64_t)p_pre + p_pre / 8 + 4096);
+            if (p_pre > gs::kBinnedCands)
+                tile_plans().past(gs::TilePlans::kTrain, std::max<int64_t>(tr.n, 1),
+                                  (int64_t)tr.tiles_x * tr.tiles_y);
+            if (p_pre > pair_cap)
+                pair_cap = std::min<uint64_t>(0xFFFFFFFFull, (uint64_t)p_pre + p_pre / 8 + 4096);
         }
         if (step) ++tr.step;
         tr.M = h_pin[C_M];
         tr.p_pre = h_pin[C_PPRE];
         tr.P = h_pin[C_P];
         tile_plans().seen(gs::TilePlans::kTrain, std::max<int64_t>(tr.n, 1),
-                          (int64_t)tr.tiles_x * tr.tiles_y, tr.P, *longest_word());
+                          (int64_t)tr.tiles_x * tr.tiles_y, tr.p_pre, tr.P,
+                          *longest_word());
         const gs::TrainSums sum = add_sums(h_pin + kFrSums);
         tr.pixel_pairs = (int64_t)sum.considered;
         tr.pixel_blended = (int64_t)sum.blended;

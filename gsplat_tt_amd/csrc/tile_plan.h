@@ -30,6 +30,12 @@ constexpr bool binned_fits(int64_t n, int64_t tiles) {
            (uint64_t)n * (uint64_t)tiles < (1ull << kBinnedCandBits);
 }
 
+// Most candidates of a binned frame, for which its buffers are sized: the bins take a word
+// per two tiles and 2048 of them (64 MB at 2^14 tiles; for a context's whole pair
+// capacity, which only grows, gigabytes). Views with 2.4M pairs have 2.5M to 3M of them. A
+// frame that has more is made again another way, which takes no longer there.
+constexpr uint32_t kBinnedCands = 1u << 22;
+
 // How frames make their tile lists, from what the finished frames of the same sizes
 // found. Binning (launch_binned_lists) needs no depth sort and fewer launches but stores
 // each pair at its list's end and sorts each list on its own, so it wins up to about
@@ -58,14 +64,20 @@ public:
     bool binned(Kind kind, int64_t n, int64_t tiles) {
         return entry(kind, n, tiles).binned && binned_fits(n, tiles);
     }
-    // A frame of these sizes has finished with `pairs` pairs, `longest` in one tile.
-    void seen(Kind kind, int64_t n, int64_t tiles, int64_t pairs, int64_t longest) {
+    // A frame of these sizes has finished: it had `cands` candidates, of which `pairs` are
+    // left, `longest` in one tile.
+    void seen(Kind kind, int64_t n, int64_t tiles, int64_t cands, int64_t pairs,
+              int64_t longest) {
         Entry& e = entry(kind, n, tiles);
         const int64_t c = cost(pairs, longest);
-        if (c > kMost) e.binned = false;
-        if (c < kAgain || (!e.known && c <= kMost)) e.binned = true;
+        if (c > kMost || cands > kBinnedCands) e.binned = false;
+        if ((c < kAgain && cands < kBinnedCands / 4 * 3) ||
+            (!e.known && c <= kMost && cands <= kBinnedCands))
+            e.binned = true;
         e.known = true;
     }
+    // A binned frame of these sizes did not fit kBinnedCands: it is made again, not binned.
+    void past(Kind kind, int64_t n, int64_t tiles) { entry(kind, n, tiles).binned = false; }
 
     static constexpr int kEntries = 16;
     // (2 pairs a Gaussian reach kMost: 0.6 to 5 in the views measured)

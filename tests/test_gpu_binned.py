@@ -4,6 +4,8 @@ sorted by block and split) and sorted (depth sort, then tile sort; the microbloc
 statistics select it). All give the stable (tile, depth bits, compact id)
 order, so ids, ranges, counts and images are compared for equality, at list lengths
 around the runs of the list sort, with equal depths, empty views and many tiles."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -276,5 +278,69 @@ def test_long_lists(n, h, w, ts):
             rb = ctx.frame_readback() if st["num_visible"] else None
             _equal((a, st, rb), _both(ctx, view)[1])
         assert (rb["tile_ranges"][:, 1] - rb["tile_ranges"][:, 0]).max() > 2 * 2048
+    finally:
+        ctx.close()
+
+
+def _free_bytes(ctx):
+    """Free device memory, by the HIP runtime that the library is linked to."""
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert ctx._L.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
+
+
+def test_more_candidates_than_a_binned_frame_holds():
+    """A view of 29M candidates over 14400 tiles and an empty one by turns, alone, in paths and
+    in training: a binned frame that has no room for its candidates is made again and
+    equals the sorted one, and its bins are allocated for 2^22 candidates (about 64 MB), not
+    for the pair capacity (460 MB): the context takes four buffers of that capacity
+    (32.4M, 4 bytes), 64 MB of bins and some 70 MB of others, below 800 MB."""
+    print("binned room", flush=True)
+    rng = np.random.default_rng(8)
+    n, h, w, f = 2000, 1440, 2560, 2000.0
+    means = np.concatenate([rng.normal(0, 0.01, (n, 2)), rng.uniform(2, 3, (n, 1))], 1)
+    q = np.tile(np.float32([1, 0, 0, 0]), (n, 1))
+    scale = np.full((n, 3), 2.0, np.float32)
+    views = []
+    for turn in (1, -1):  # the second looks away
+        w2c = np.diag([turn, 1, turn, 1]).astype(np.float32)
+        views.append(L.make_view(w2c, scenes.intrinsics(f, f, w / 2, h / 2), h, w, tile_size=16,
+                                 output="bf16", max_radius=100_000))
+    near, away = views
+    ctx = L.Context(0)
+    try:
+        ctx.set_scene(means.astype(np.float32), scenes.cov3d(scale, q),
+                      rng.uniform(0.01, 0.05, n).astype(np.float32),
+                      rng.random((n, 3)).astype(np.float32))
+        free = _free_bytes(ctx)
+        a, b = _both(ctx, near)
+        assert a[1]["pairs_pre"] == n * 14400
+        _equal(a, b)
+        away_img = ctx.render(away)[0].copy()
+        for _ in range(3):
+            assert np.array_equal(ctx.render(away)[0], away_img)
+            img, st = ctx.render(near)
+            assert np.array_equal(img, a[0]) and st["pairs_pre"] == a[1]["pairs_pre"]
+            ctx.render(away)
+        used = free - _free_bytes(ctx)
+        print("device MB", used >> 20, flush=True)
+        assert used < 800 << 20
+        path = [away, away, near, away, near, near]
+        outs = [np.empty((h, w, 3), np.uint16) for _ in path]
+        for _ in range(2):
+            ctx.render_batch(path, outs, out_on_device=False)
+            for v, o in zip(path, outs):
+                assert np.array_equal(o, a[0] if v is near else away_img)
+        p = {"means": means, "log_scales": np.log(scale), "quats": q,
+             "opacity_logits": rng.uniform(-4.0, -3.0, n), "sh": rng.uniform(0, 0.5, (n, 1, 3))}
+        tr = L.Trainer(ctx, {k: np.ascontiguousarray(v, np.float32) for k, v in p.items()}, 0)
+        cfg = L.make_train_cfg()
+        first = tr.forward(near, cfg)
+        for _ in range(2):
+            assert not tr.forward(away, cfg)[0].any()
+            assert not tr.forward(away, cfg)[0].any()
+            got = tr.forward(near, cfg)
+            assert np.array_equal(got[0], first[0]) and np.array_equal(got[1], first[1])
+            assert got[3]["pairs_pre"] == first[3]["pairs_pre"] > 1 << 22
     finally:
         ctx.close()

@@ -59,24 +59,24 @@ static void sizes() {
         P p;
         for (int k = 0; k < 4; ++k) {
             p.binned(P::kFrame, n, full);
-            p.seen(P::kFrame, n, full, 5000000, 3000);
+            p.seen(P::kFrame, n, full, 5000000, 5000000, 3000);
             p.binned(P::kFrame, n, thumb);
-            p.seen(P::kFrame, n, thumb, 700000, 4096);
+            p.seen(P::kFrame, n, thumb, 700000, 700000, 4096);
             CHECK(!p.binned(P::kFrame, n, full) && p.binned(P::kFrame, n, thumb));
             CHECK(p.binned(P::kTrain, n, full));  // a training forward's pairs are its own
         }
-        p.seen(P::kFrame, n, full, P::kAgain, 0);  // between the limits: as it was
+        p.seen(P::kFrame, n, full, P::kAgain, P::kAgain, 0);  // between the limits: as it was
         CHECK(!p.binned(P::kFrame, n, full));
-        p.seen(P::kFrame, n, full, P::kAgain - 1, 0);
+        p.seen(P::kFrame, n, full, P::kAgain - 1, P::kAgain - 1, 0);
         CHECK(p.binned(P::kFrame, n, full));
-        p.seen(P::kFrame, n, full, P::kMost, 0);
+        p.seen(P::kFrame, n, full, P::kMost, P::kMost, 0);
         CHECK(p.binned(P::kFrame, n, full));
     }
     {
         P p;  // many Gaussians, few pairs: binned from the second frame, also between others
         for (int k = 0; k < P::kEntries; ++k) {
             CHECK(!p.binned(P::kFrame, 3000000, 100 + k));
-            p.seen(P::kFrame, 3000000, 100 + k, 500000, 0);
+            p.seen(P::kFrame, 3000000, 100 + k, 500000, 500000, 0);
         }
         for (int k = 0; k < P::kEntries; ++k) CHECK(p.binned(P::kFrame, 3000000, 100 + k));
         CHECK(!p.binned(P::kFrame, 3000000, 99));  // one more size: the oldest is given up
@@ -92,20 +92,20 @@ static void lists() {
     {   // the first frame that finishes decides by the upper limit, whatever was guessed
         P q;
         CHECK(!q.binned(P::kFrame, 300000, 70) && !q.binned(P::kFrame, 3000000, 3600));
-        q.seen(P::kFrame, 300000, 70, 414000, 14914);  // 2.04M
-        q.seen(P::kFrame, 3000000, 3600, P::kMost, 0);
+        q.seen(P::kFrame, 300000, 70, 414000, 414000, 14914);  // 2.04M
+        q.seen(P::kFrame, 3000000, 3600, P::kMost, P::kMost, 0);
         CHECK(q.binned(P::kFrame, 300000, 70) && q.binned(P::kFrame, 3000000, 3600));
     }
     P p;
-    p.seen(P::kFrame, 100000, 3600, 500000, 4096);
+    p.seen(P::kFrame, 100000, 3600, 500000, 500000, 4096);
     CHECK(p.binned(P::kFrame, 100000, 3600));
-    p.seen(P::kFrame, 100000, 3600, 500000, 18000);  // 2.59M
+    p.seen(P::kFrame, 100000, 3600, 500000, 500000, 18000);  // 2.59M
     CHECK(!p.binned(P::kFrame, 100000, 3600));
-    p.seen(P::kFrame, 100000, 3600, 500000, 14000);  // 1.99M: as it was
+    p.seen(P::kFrame, 100000, 3600, 500000, 500000, 14000);  // 1.99M: as it was
     CHECK(!p.binned(P::kFrame, 100000, 3600));
-    p.seen(P::kFrame, 100000, 3600, 500000, 12000);  // 1.69M
+    p.seen(P::kFrame, 100000, 3600, 500000, 500000, 12000);  // 1.69M
     CHECK(p.binned(P::kFrame, 100000, 3600));
-    p.seen(P::kFrame, 100000, 3600, 500000, 16000);  // 2.29M: as it was
+    p.seen(P::kFrame, 100000, 3600, 500000, 500000, 16000);  // 2.29M: as it was
     CHECK(p.binned(P::kFrame, 100000, 3600));
     // first frames: a scene over a few tiles has long lists, over many it has not
     CHECK(!p.binned(P::kFrame, 1 << 20, 1) && !p.binned(P::kFrame, 1 << 20, 63));
@@ -113,8 +113,33 @@ static void lists() {
     CHECK(p.binned(P::kFrame, 1000000, 3600) && p.binned(P::kFrame, 100000, 300));
 }
 
+// A frame of more candidates than a binned one has room for is not binned, and the bins
+// stay small whatever the pair capacity is.
+static void room() {
+    using P = gs::TilePlans;
+    const int64_t most = gs::kBinnedCands, pairs = 1000000;
+    P p;
+    CHECK(p.binned(P::kFrame, 500000, 3600));
+    p.past(P::kFrame, 500000, 3600);
+    CHECK(!p.binned(P::kFrame, 500000, 3600));
+    p.seen(P::kFrame, 500000, 3600, most + 1, pairs, 0);
+    CHECK(!p.binned(P::kFrame, 500000, 3600));
+    p.seen(P::kFrame, 500000, 3600, most, pairs, 0);  // near its room: as it was
+    CHECK(!p.binned(P::kFrame, 500000, 3600));
+    p.seen(P::kFrame, 500000, 3600, most / 2, pairs, 0);
+    CHECK(p.binned(P::kFrame, 500000, 3600));
+    p.seen(P::kFrame, 500000, 3600, most, pairs, 0);
+    CHECK(p.binned(P::kFrame, 500000, 3600));
+    p.seen(P::kFrame, 500000, 3600, most + 1, pairs, 0);
+    CHECK(!p.binned(P::kFrame, 500000, 3600));
+    // a first frame that was not binned and had too many
+    p.seen(P::kFrame, 3000000, 3600, most + 1, pairs, 0);
+    CHECK(!p.binned(P::kFrame, 3000000, 3600));
+}
+
 int main() {
     fields();
+    room();
     sizes();
     lists();
     if (fails == 0) std::puts("ok");

@@ -175,12 +175,13 @@ def stage_summary(n, sh_degree, tiles, stats):
 def dominant_roofline(st, tag, deg, out):
     """The roofline object of the frame's dominant kernel: k_project (the project
     stage is that one kernel plus a small histogram reduction, HBM-bound) or
-    k_blend (FP32 VALU-bound; no MFMA on this path), whichever takes longer.
+    the blend (FP32 VALU-bound; no MFMA on this path), whichever takes longer.
     `traffic` is the kernel's PMC-measured HBM bytes per dispatch for this
-    workload (profiles/frame_<tag>_pmc_traffic.md), for the kernel instance the
-    workload runs (k_project<sh degree>, k_blend<tile, output format>)."""
-    proj_k = f"k_project<{deg}>"
-    blend_k = f"k_blend<16, {ORDER_OUT.index(out)}>"
+    workload's frames rendered alone, as the stage times are
+    (profiles/frame_<tag>_pmc_traffic.md), for the kernel instance that they
+    run (k_project<sh degree, binned, items>, k_blend or k_blend_mb<tile, output format>)."""
+    proj_k = rf"k_project<{deg}, \w+, \d>"
+    blend_k = rf"k_blend(?:_mb)?<16, {ORDER_OUT.index(out)}>"
     r = st["roofline"]
     proj_ms, blend_ms = r["project"]["ms"], r["blend"]["ms"]
     if blend_ms >= proj_ms:
@@ -202,14 +203,14 @@ ORDER_OUT = ("u8", "bf16", "f32")  # k_blend's output-format template argument
 
 
 def pmc_traffic(kernel, tag):
-    """HBM bytes per dispatch of `kernel` in workload `tag` from the committed
+    """HBM bytes per dispatch of the kernel that the pattern matches in workload `tag` from the committed
     rocprofv3 PMC summary (FETCH_SIZE and WRITE_SIZE scaled by a copy-kernel
     calibration), or None when no summary holds it."""
     import re
     path = os.path.join(ROOT, "profiles", f"frame_{tag}_pmc_traffic.md")
     if not os.path.exists(path):
         return None
-    m = re.search(r"traffic_bytes_per_dispatch\[" + re.escape(kernel) + r"\]\s*=\s*([0-9]+)",
+    m = re.search(r"traffic_bytes_per_dispatch\[" + kernel + r"\]\s*=\s*([0-9]+)",
                   open(path).read())
     return int(m.group(1)) if m else None
 

@@ -89,7 +89,7 @@ __device__ __forceinline__ void sh_eval(const float* __restrict__ rec, float x, 
 
 // BINNED: instead of the depth sort's inputs (dvals, part_hist), the compaction
 // also scans the visible Gaussians' tile counts in compact order: offs[m], the
-// emission's owner table and the candidate total (write_binned), the two prefixes
+// emission's owner table and the candidate total (binned_write), the two prefixes
 // packed into one look-back descriptor.
 // ITEMS: Gaussians per thread, one for a small scene's binned frame (project_items).
 template <int DEG, bool BINNED, int ITEMS>

@@ -568,7 +568,7 @@ struct gs_ctx {
     static constexpr size_t kFrCnt = 0;    // 64 counters (below)
     static constexpr size_t kFrSums = 64;  // a training forward's TrainSums
     enum : int {
-        C_PROJ_TICKET = 0, C_M = 1, C_SKIPPED = 2, C_CTL = 4, C_RECT_TICKET = 8, C_PPRE = 9,
+        C_PROJ_TICKET = 0, C_M = 1, C_SKIPPED = 2, C_CTL = 4, C_ODD = 6, C_RECT_TICKET = 8, C_PPRE = 9,
         C_EMIT_TICKET = 10, C_P = 11, C_RUNS = 12, C_ITEMS = 13, C_KITEMS = 14, C_SEGS = 15, C_DSORT_TICKETS = 16, C_TSORT_TICKETS = 24,
         C_MBSTAT = 40  // two u64: pairs no microblock keeps, kept (pair, microblock)
     };
@@ -1817,6 +1817,7 @@ struct gs_ctx {
         HIPCHK(gs::launch_fill_u32(L.fr, 0u, L.fwords, st));
         if (spin_limit) HIPCHK(gs::launch_fill_u32(L.cnt + C_CTL + 1, spin_limit, 1, st));
         tr.cam.ctl = L.cnt + C_CTL;
+        tr.cam.odd = L.cnt + C_ODD;
         tr.cam.tiles_x = tr.tiles_x;
         tr.cam.tiles_y = tr.tiles_y;
         tr.cam.binned = binned_out(L);
@@ -1853,6 +1854,7 @@ struct gs_ctx {
         fp.grad_scale = (float)((double)c->loss_scale * (1.0 - (double)c->lambda_dssim) /
                                 (3.0 * (double)px));
         fp.sums = L.sums;
+        fp.odd = tr.cam.odd;
         fp.ctl = L.cnt + C_CTL;
         HIPCHK(gs::launch_train_fwd(b_brec.as<float4>(), b_pair_id.as<uint32_t>(), b_ranges.as<uint32_t>(), fp, st));
         if (tgt_dev != nullptr && c->lambda_dssim > 0.0f)
@@ -1943,6 +1945,8 @@ struct gs_ctx {
         bp.dimage = t_dimg.as<float>();
         bp.grad2d = t_grad2d.as<float>();
         bp.ctl = tr.cam.ctl;
+        bp.odd = tr.cam.odd;
+        bp.image = t_img.as<float>();
         HIPCHK(gs::launch_train_bwd(b_brec.as<float4>(), b_pair_id.as<uint32_t>(), b_ranges.as<uint32_t>(), bp, st));
         // the device time of a step's Adam is part of its gradient pass
         if (timing && adam) HIPCHK(hipEventRecord(tev[3], st));

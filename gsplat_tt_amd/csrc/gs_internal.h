@@ -450,6 +450,7 @@ struct TrainCam {
     int H, W;
     int tiles_x, tiles_y;      // 16-pixel tiles
     uint32_t* ctl;             // control words (gs_common.h), may be null
+    uint32_t* odd;             // set when a kept Gaussian's colour is not finite (cleared before)
     BinnedOut binned;
     float* grad2d;             // rows of 9 that the projection clears (a step), may be null
 };
@@ -487,6 +488,7 @@ struct TrainFwdParams {
     float grad_scale;      // loss_scale / (3HW)
     TrainSums* sums;       // kTrainSumSlots groups of partial sums, cleared before
     const uint32_t* ctl;   // control words of the forward (nothing is read after an error)
+    const uint32_t* odd;   // the projection's (TrainCam)
 };
 
 // Full 3DGS loss terms (1 - lambda) L1 + lambda (1 - SSIM) on an (H,W,3) image.
@@ -513,7 +515,9 @@ struct TrainBwdParams {
     const float* final_T;
     const uint32_t* stop;
     const float* dimage;
+    const float* image;    // the forward's
     const uint32_t* ctl;   // control words of the forward (nothing is read after an error)
+    const uint32_t* odd;   // the projection's (TrainCam)
     float* grad2d;         // (M,9) per compact Gaussian: dmx dmy dA dB dC dop dr dg db
 };
 

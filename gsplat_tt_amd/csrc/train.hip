@@ -220,6 +220,11 @@ __device__ __forceinline__ void colour(const Head& h, const float4* row, const T
     for (int ch = 0; ch < 3; ++ch) raw[ch] = acc[ch] + 0.5f;
 }
 
+__device__ __forceinline__ bool finite3(float x, float y, float z) {
+    const float inf = __builtin_inff();
+    return fabsf(x) < inf && fabsf(y) < inf && fabsf(z) < inf;
+}
+
 __device__ __forceinline__ float sigmoidf(float x) { return 1.0f / (1.0f + expf(-x)); }
 
 // Projection of the optimizer-space parameters; stable compaction of the
@@ -352,6 +357,7 @@ __global__ __launch_bounds__(kTThreads, 4) void k_train_project(
         const float4* row = P.rows + (base + it * kTThreads + tid) * V;
         float dir[3], dn;
         colour<DEG>(load_head(row), row, cam, col[it], dir, dn);
+        if (!finite3(col[it][0], col[it][1], col[it][2])) *cam.odd = 1u;
     }
     if (w == 0) {
         const uint64_t excl = lookback_walk(lb_state, vid, agg, cam.ctl);
@@ -468,6 +474,7 @@ __global__ __launch_bounds__(GS_WAVE) void k_train_fwd(const float4* __restrict_
     // after an earlier give-up the sorted ids may be wrong: read nothing (the
     // flag was raised by an earlier launch, so every thread sees the same value)
     if (upstream_failed(fp.ctl)) return;
+    const bool any_odd = __builtin_amdgcn_readfirstlane((int)*fp.odd) != 0;
     const int lane = threadIdx.x;
     const int tile = blockIdx.x / kBandsPerTile, band = blockIdx.x % kBandsPerTile;
     const int tx = tile % fp.tiles_x, ty = tile / fp.tiles_x;
@@ -488,9 +495,8 @@ __global__ __launch_bounds__(GS_WAVE) void k_train_fwd(const float4* __restrict_
         for (uint32_t base = start; base < end; base += GS_WAVE) {
             const bool keep = base + lane < end && band_keeps(r0, r1, bx0, by0);
             const uint64_t mask = __ballot(keep);
-            // kept entries whose colours are not finite (or past the range when added up)
-            const uint64_t odd = __ballot(
-                keep && !(fabsf(r2.x) + fabsf(r2.y) + fabsf(r2.z) < __builtin_inff()));
+            // kept entries whose colours are not finite
+            const uint64_t odd = any_odd ? __ballot(keep && !finite3(r2.x, r2.y, r2.z)) : 0ull;
             const int cnt = __popcll(mask);
             __syncthreads();  // one wave: orders the LDS reads of the batch before
             if (keep) {
@@ -512,7 +518,7 @@ __global__ __launch_bounds__(GS_WAVE) void k_train_fwd(const float4* __restrict_
             // An entry that the pixel does not blend adds 0 times its colour, but where a
             // colour of the batch is not finite the sums are selected instead (1M Gaussians
             // at 1280x720: 117 us with and without that walk, 119 when it is unrolled as the
-            // other, 123.5 with selects in every batch).
+            // other, 123.5 with selects in every batch; 20K 21.2 without, 21.5 with it).
             const auto blend = [&](int k, auto select) {
                 const float4 e0 = s0[k], e1 = s1[k];
                 const float2 e2 = s2[k];
@@ -839,16 +845,51 @@ __device__ __forceinline__ int term_of_lane(int l) {
     return (l & 2) ? 8 : ((l >> 4) & 1) * 4 + ((l >> 2) & 1) * 2 + ((l >> 3) & 1);
 }
 
+// Backward of one pixel by its lane, an atomic per term of each entry that it blends.
+__device__ __forceinline__ void backward_alone(const float4* __restrict__ trec,
+                                               const uint32_t* __restrict__ ids, uint32_t stop,
+                                               float pxc, float pyc, float T, float g0, float g1,
+                                               float g2, const TrainBwdParams& bp) {
+    float behind = bp.bg[0] * g0 + bp.bg[1] * g1 + bp.bg[2] * g2;
+#pragma unroll 1
+    for (uint32_t e = stop; e-- > 0;) {
+        const size_t gi = ids[e];
+        const float4 r0 = trec[3 * gi + 0], r1 = trec[3 * gi + 1], r2 = trec[3 * gi + 2];
+        const Splat s = splat_at(pxc, pyc, r0.x, r0.y, r1.x, r1.y, r1.z, r0.z);
+        const float alpha = fminf(s.raw, bp.alpha_max);
+        if (!(alpha >= bp.alpha_min)) continue;
+        T = T * __builtin_amdgcn_rcpf(1.0f - alpha);
+        const float d = __builtin_fmaf(r2.x, g0, __builtin_fmaf(r2.y, g1, r2.z * g2)) - behind;
+        behind = __builtin_fmaf(alpha, d, behind);
+        const float at = alpha * T;
+        const float dop = s.raw > bp.alpha_max ? 0.0f : T * d;
+        const float dp = s.power <= 0.0f ? dop * s.raw : 0.0f;
+        const float dpx = dp * s.dx, dpy = dp * s.dy;
+        float* const dst = bp.grad2d + 9 * gi;
+        atomicAdd(dst + 0, dp * __builtin_fmaf(r1.y, s.dy, s.adx));
+        atomicAdd(dst + 1, dp * __builtin_fmaf(r1.y, s.dx, s.cdy));
+        atomicAdd(dst + 2, -0.5f * dpx * s.dx);
+        atomicAdd(dst + 3, -dpx * s.dy);
+        atomicAdd(dst + 4, -0.5f * dpy * s.dy);
+        atomicAdd(dst + 5, dop * s.w);
+        atomicAdd(dst + 6, at * g0);
+        atomicAdd(dst + 7, at * g1);
+        atomicAdd(dst + 8, at * g2);
+    }
+}
+
 // Backward of one band: entries from the last one any of its pixels considered
 // down to the first; per pixel the reverse recursion T_i = T_{i+1}/(1 - alpha_i)
 // and, with s_i = c_i . g, behind_i = behind_{i+1} + alpha_{i+1} (s_{i+1} -
 // behind_{i+1}) starting from the background's bg . g (the colours behind an
 // entry are only ever needed through their product with the pixel's gradient),
 // dL/dalpha_i = T_i (s_i - behind_i). A lane that does not blend the entry has
-// alpha 0, which leaves T as it is, keeps its behind (by a select: the entry's colour
-// may not be finite) and contributes exact zeros: where a gradient of the band's pixels is
-// not finite, by a select too, as the other entry of the two, or the padding, is summed
-// beside it (v_mul_legacy_f32 in every pair instead: 289 -> 296 us at 1M Gaussians).
+// alpha 0, which leaves T and behind as they are and contributes exact zeros - of finite
+// values. A pixel whose gradient is not finite, or that blends a colour that is not (its
+// image is not either), takes no part but goes its entries alone (backward_alone), and
+// the others see such a colour as 0. (287 -> 289 us at 1M Gaussians, 33.9 at 20K; by
+// selects, of behind in every pair and of the colours' terms in the bands of such
+// gradients, 292 and 34.8.)
 // The nine per-pair terms (dmx dmy dA dB dC dop dr dg db) of two entries at a
 // time are summed over the wave (sum_terms) and 18 lanes add them to the
 // Gaussians' accumulators, one atomic each. 1/(1 - alpha) is one reciprocal
@@ -859,6 +900,7 @@ __global__ __launch_bounds__(GS_WAVE) void k_train_bwd(const float4* __restrict_
                                                        TrainBwdParams bp) {
     __shared__ float4 s0[GS_WAVE], s1[GS_WAVE], s2[GS_WAVE];
     if (upstream_failed(bp.ctl)) return;
+    const bool any_odd = __builtin_amdgcn_readfirstlane((int)*bp.odd) != 0;
     const int lane = threadIdx.x;
     const int tile = blockIdx.x / kBandsPerTile, band = blockIdx.x % kBandsPerTile;
     const int tx = tile % bp.tiles_x, ty = tile / bp.tiles_x;
@@ -877,8 +919,6 @@ __global__ __launch_bounds__(GS_WAVE) void k_train_bwd(const float4* __restrict_
         g1 = bp.dimage[3 * p + 1];
         g2 = bp.dimage[3 * p + 2];
     }
-    const bool odd = __ballot(!(fabsf(g0) + fabsf(g1) + fabsf(g2) < __builtin_inff())) != 0ull;
-    float behind = bp.bg[0] * g0 + bp.bg[1] * g1 + bp.bg[2] * g2;
     // the band's last considered entry: entries past it are skipped
     uint32_t nmax = stop;
 #pragma unroll
@@ -896,8 +936,20 @@ __global__ __launch_bounds__(GS_WAVE) void k_train_bwd(const float4* __restrict_
     float4 r0 = trec[3 * (size_t)gi + 0], r1 = trec[3 * (size_t)gi + 1],
            r2 = trec[3 * (size_t)gi + 2];
     uint32_t gn = sid[start + max(hi - 1 - GS_WAVE - lane, 0)];
+    bool alone = !finite3(g0, g1, g2);
+    if (any_odd && inside) {
+        const float* img = bp.image + 3 * ((size_t)py * bp.width + px);
+        alone = alone || !finite3(img[0], img[1], img[2]);
+    }
+    if (__builtin_expect(alone, 0)) {
+        backward_alone(trec, sid + start, min(stop, end - start), pxc, pyc, T, g0, g1, g2, bp);
+        stop = 0;
+        g0 = g1 = g2 = 0.0f;
+    }
+    float behind = bp.bg[0] * g0 + bp.bg[1] * g1 + bp.bg[2] * g2;
     for (; hi > 0; hi -= GS_WAVE) {
         const bool keep = hi - 1 - lane >= 0 && band_keeps(r0, r1, bx0, by0);
+        if (any_odd && !finite3(r2.x, r2.y, r2.z)) r2 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         const uint64_t mask = __ballot(keep);
         const int cnt = __popcll(mask);
         __syncthreads();  // one wave: orders the LDS reads of the batch before
@@ -921,19 +973,19 @@ __global__ __launch_bounds__(GS_WAVE) void k_train_bwd(const float4* __restrict_
         __syncthreads();
         for (int k = 0; k < cnt; k += 2) {
             float v[2][9];
-            bool blends[2];
+            bool any = false;
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
                 const float4 e0 = s0[k + j], e1 = s1[k + j], e2 = s2[k + j];
                 const Splat s = splat_at(pxc, pyc, e0.x, e0.y, e0.w, e1.x, e1.y, e0.z);
                 const float alpha = fminf(s.raw, bp.alpha_max);
                 const bool live = __float_as_uint(e2.y) < stop && alpha >= bp.alpha_min;
-                blends[j] = live;
+                any = any || live;
                 const float a = live ? alpha : 0.0f;
                 const float Tn = T * __builtin_amdgcn_rcpf(1.0f - a);
                 const float d = __builtin_fmaf(e1.z, g0, __builtin_fmaf(e1.w, g1, e2.x * g2)) -
                                 behind;
-                behind = live ? __builtin_fmaf(a, d, behind) : behind;
+                behind = __builtin_fmaf(a, d, behind);
                 T = Tn;
                 const float at = a * Tn;
                 // no gradient through the clamps
@@ -950,13 +1002,7 @@ __global__ __launch_bounds__(GS_WAVE) void k_train_bwd(const float4* __restrict_
                 v[j][7] = at * g1;
                 v[j][8] = at * g2;
             }
-            if (__ballot(blends[0] || blends[1]) == 0ull) continue;
-            if (odd) {
-#pragma unroll
-                for (int j = 0; j < 2; ++j)
-#pragma unroll
-                    for (int c = 6; c < 9; ++c) v[j][c] = blends[j] ? v[j][c] : 0.0f;
-            }
+            if (__ballot(any) == 0ull) continue;
             const float sum = sum_terms(v[0], v[1], bit3, bit2, bit1);
             const uint32_t g = __float_as_uint(s2[k + (lane >> 5)].z);
             if (writes && sum != 0.0f) atomicAdd(bp.grad2d + 9 * (size_t)g + term, sum * scale);
